@@ -22,6 +22,7 @@ struct Sweep {
 };
 
 constexpr int TIMING_PAIRS = 256;
+enum : unsigned { FILL_V = 1u, FILL_KA = 2u };   // what fill_fields writes
 
 // A captured block of `len` steps of one gstate (replayed from an even step).
 struct StepGraph {
@@ -77,11 +78,13 @@ struct gpue_ctx {
   double* Kt = nullptr;
   double* At[3] = {};
   bool az_zero = true;
-  // time-dependent equation fields (V, K, Ax, Ay, Az): device programs evaluated
-  // per point inside the sweeps; tables of the same fields are filled at time
-  // t_last only for the energy
+  // time-dependent equation fields (V, K, Ax, Ay, Az): device programs, run into
+  // the fields' tables before each step (fill_fields) and, at t_last, for the energy
   gpue::EqnProg* deq[5] = {};
-  bool t_dep = false;          // some field depends on time (steps run one by one)
+  int deq_depth[5] = {};
+  double* Vt2 = nullptr;       // second table of a time-dependent V (v_table)
+  double* tbase = nullptr;     // device: step index of the captured block being replayed
+  bool t_dep = false;          // some field depends on time
   double t_last = 0.0;         // time of the last step, Dt * i
   double* vst[3] = {};         // the harmonic trap's per-axis terms (V_TRAP_A)
   int ramp_type = 0;           // -R: gauge exponent scaled per step (0 off, 1, 2)
@@ -112,7 +115,8 @@ struct gpue_ctx {
 
 namespace gpue {
 gpue_status fail(gpue_ctx* c, gpue_status s, const std::string& msg);
-Phys make_phys(const gpue_ctx* c, int gstate, double time);
+Phys make_phys(const gpue_ctx* c, int gstate, int step);
+double* v_table(const gpue_ctx* c, int step);
 double ramp_scale(const gpue_ctx* c, int step);
 void schedule(const gpue_ctx* c, int gstate, int i, bool pending, std::vector<Sweep>& out);
 void schedule_block(const gpue_ctx* c, int gstate, int first, int n, std::vector<Sweep>& out,

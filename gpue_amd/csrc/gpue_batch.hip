@@ -123,7 +123,7 @@ static bool fill_args(gpue_batch* b) {
             const bool in = b->active[idx] && ((s.mask >> par) & 1);
             any = any || in;
             const std::vector<Sweep>& sc = g.sched[gs][par];
-            const Phys phys = make_phys(c, gs, 0.0);
+            const Phys phys = make_phys(c, gs, 0);
             for (size_t k = 0; k < s.keys.size(); ++k) {
               const bool on = in && k < sc.size();
               const Sweep& sw = on ? sc[k] : s.keys[k];

@@ -82,7 +82,7 @@ static double* dev_copy(const std::vector<double>& v, hipError_t* e) {
   return p;
 }
 
-Phys gpue::make_phys(const gpue_ctx* c, int gstate, double time) {
+Phys gpue::make_phys(const gpue_ctx* c, int gstate, int step) {
   const gpue_params& p = c->p;
   Phys f;
   std::memset(&f, 0, sizeof(f));
@@ -101,16 +101,9 @@ Phys gpue::make_phys(const gpue_ctx* c, int gstate, double time) {
   f.g = p.g;
   f.cK = Dt / p.hbar;
   f.Dt = Dt;
-  f.hb2m = p.hbar * p.hbar / (2 * p.mass);
-  f.mass = p.mass;
   f.omega = p.omega;
   f.omegaX = p.omegaX;
   f.omegaY = p.omegaY;
-  f.omegaZe = p.dimnum == 3 ? p.omegaZ : 0.0;   // items[5] (src/operators.cu:765-767)
-  f.gammaY = p.gammaY;
-  f.x0 = p.x0_shift;
-  f.y0 = p.y0_shift;
-  f.z0e = p.dimnum == 3 ? p.z0_shift : 0.0;     // items[8]
   for (int a = 0; a < 3; ++a) {
     (&f.xg)[a] = c->dgrid[a];
     (&f.pxg)[a] = c->dgrid[a + 3];
@@ -120,21 +113,89 @@ Phys gpue::make_phys(const gpue_ctx* c, int gstate, double time) {
     f.ks[a] = c->ks[a];
     f.kf[a] = c->kf[gstate][a];
   }
-  f.Vt = c->Vt;
   f.Kt = c->Kt;
   for (int a = 0; a < 3; ++a) f.At[a] = c->At[a];
-  for (int k = 0; k < 5; ++k) f.eq[k] = c->deq[k];
+  // time-dependent fields are read from the tables fill_fields writes for the step
+  f.Vt = v_table(c, step);
+  f.Vt_next = v_table(c, step + 1);
+  if (f.v_kind == V_EQN || f.v_kind == V_TRAP_A) f.v_kind = V_TABLE;
+  if (f.k_kind == K_EQN) f.k_kind = K_TABLE;
+  if (f.a_kind == A_EQN) f.a_kind = A_TABLE;
+  return f;
+}
+
+// The V table of a step: V(t) alternates between two, so that a sweep that ends one
+// step and opens the next (bridge modes) reads both times.
+double* gpue::v_table(const gpue_ctx* c, int step) { return c->Vt2 && (step & 1) ? c->Vt2 : c->Vt; }
+
+// Queue the kernel that writes the time-dependent fields into their tables at
+// t = Dt * tstep: V into Vt (which: FILL_V), K and A (FILL_KA); a harmonic V over a
+// time-dependent A is written with the A (FILL_KA).  In a captured block the step
+// is counted from the block's first, whose index the host leaves in tbase.
+static gpue_status fill_fields(gpue_ctx* c, unsigned which, double* Vt, double Dt, double tstep, const double* tbase) {
+  if (!c->t_dep) return GPUE_OK;
+  const gpue_params& p = c->p;
+  FieldArgs f;
+  std::memset(&f, 0, sizeof(f));
+  f.trap = c->v_kind == V_TRAP_A;
+  int depth = 1;
+  bool any = false;
+  for (int k = 0; k < 5; ++k) {
+    if (!c->deq[k] || !(which & (k == 0 ? FILL_V : FILL_KA))) continue;
+    f.eq[k] = c->deq[k];
+    f.out[k] = k == 0 ? Vt : k == 1 ? c->Kt : c->At[k - 2];
+    depth = std::max(depth, c->deq_depth[k]);
+    any = true;
+  }
+  if (f.trap && (which & FILL_KA)) {
+    f.out[0] = c->Vt;
+    any = true;
+  }
+  if (!any) return GPUE_OK;
   for (int a = 0; a < 3; ++a) {
+    f.At[a] = c->At[a];
     f.vst[a] = c->vst[a];
     f.dxyz[a] = c->d[a];
   }
+  f.mass = p.mass;
+  f.xDim = c->dims[0];
+  f.yDim = c->dims[1];
+  f.zDim = c->dims[2];
+  f.N = c->N;
   // find_field's coordinates dx*i - xMax (src/dynamic.cu:613-615)
   f.org[0] = -p.xMax;
   f.org[1] = p.dimnum > 1 ? -p.yMax : 0.0;
   f.org[2] = p.dimnum > 2 ? -p.zMax : 0.0;
-  f.t = time;
-  f.eqk = c->t_dep ? 1 : 0;
-  return f;
+  f.tbase = tbase;
+  f.Dt = Dt;
+  f.tstep = tstep;
+  const hipError_t e = launch_fields_at(f, depth, c->stream);
+  return e == hipSuccess ? GPUE_OK : fail(c, GPUE_EHIP, std::string("field tables: ") + hipGetErrorString(e));
+}
+
+// Sweeps that end one step and open the next (bridge modes).
+static bool bridges(const Sweep& s) {
+  return s.row ? s.mode == RM_INV_FWD || s.mode == RM_GAUGE_FWD : s.mode == CM_GAUGE_FWD;
+}
+
+// The field tables a sweep of `step` reads, written before it: the step's own ahead
+// of its first sweep, and the next step's V ahead of a bridge.  v_done, ka_done: the
+// last steps filled.
+static gpue_status fill_for(gpue_ctx* c, const Sweep& s, int gstate, int step, const double* tbase, int* v_done,
+                            int* ka_done) {
+  if (!c->t_dep) return GPUE_OK;
+  const double Dt = gstate == 0 ? c->p.gdt : c->p.dt;
+  unsigned which = 0u;
+  if (*v_done < step) which |= FILL_V;
+  if (*ka_done < step) which |= FILL_KA;
+  gpue_status st = which ? fill_fields(c, which, v_table(c, step), Dt, step, tbase) : GPUE_OK;
+  *v_done = std::max(*v_done, step);
+  *ka_done = std::max(*ka_done, step);
+  if (st == GPUE_OK && bridges(s) && *v_done < step + 1) {
+    st = fill_fields(c, FILL_V, v_table(c, step + 1), Dt, step + 1, tbase);
+    *v_done = step + 1;
+  }
+  return st;
 }
 
 // -R ramp (src/evolution.cu:409-428, 811-832): GPUE raises the gauge operators
@@ -215,12 +276,10 @@ static bool opens_step(const Sweep& s) {
   return s.row ? s.mode == RM_FWD : s.mode == CM_FWD_V;
 }
 
-static int default_variant(const gpue_ctx* c, int axis);
-
 // An opening sweep that can reduce the previous step's norm partials itself
 // (part_norm needs workgroups of whole waves).
 static bool takes_deferred_norm(const gpue_ctx* c, const Sweep& s) {
-  const int var = c->t_dep ? default_variant(c, s.axis) : s.var >= 0 ? s.var : c->var[s.axis];
+  const int var = s.var >= 0 ? s.var : c->var[s.axis];
   return opens_step(s) && sweep_full_waves(c->prec, s.row, c->dims[s.axis], var);
 }
 
@@ -261,7 +320,7 @@ static gpue_status timing_flush(gpue_ctx* c) {
 // Workgroups (= partials written) of a sweep.
 static int sweep_nb(const gpue_ctx* c, const Sweep& s) {
   const int n = c->dims[s.axis];
-  const int var = c->t_dep ? default_variant(c, s.axis) : s.var >= 0 ? s.var : c->var[s.axis];
+  const int var = s.var >= 0 ? s.var : c->var[s.axis];
   return s.row ? sweep_blocks(c->prec, true, n, var, c->dims[1] * c->dims[2], 1)
                : sweep_blocks(c->prec, false, n, var, c->dims[0], s.axis == 1 ? c->dims[2] : c->dims[1]);
 }
@@ -296,8 +355,7 @@ static gpue_status settle_deferred(gpue_ctx* c) {
 // The variants every context starts with (no timing, so results never depend on
 // it): for small, latency-bound grids narrow lines with up-front twiddle loads
 // and quarter strided tiles (the autotuner's choice for 2D grids of
-// 128^2-512^2), wide lines otherwise.  Contexts with time-dependent fields
-// always run these (their EQ kernels exist for these variants only).
+// 128^2-512^2), wide lines otherwise.
 static int default_variant(const gpue_ctx* c, int axis) {
   const bool small = c->N <= (1L << 20);
   return axis == 0 ? (small ? 3 : 0) : (small ? 5 : 0);
@@ -305,7 +363,7 @@ static int default_variant(const gpue_ctx* c, int axis) {
 
 gpue_status gpue::launch(gpue_ctx* c, const Sweep& s, const Phys& ph, const void* in, void* out) {
   const int n = c->dims[s.axis];
-  const int var = c->t_dep ? default_variant(c, s.axis) : s.var >= 0 ? s.var : c->var[s.axis];
+  const int var = s.var >= 0 ? s.var : c->var[s.axis];
   SweepArgs a;
   std::memset(&a, 0, sizeof(a));
   a.active = 1;
@@ -507,6 +565,8 @@ void gpue_destroy(gpue_ctx* c) {
     if (c->dgrid[a]) (void)hipFree(c->dgrid[a]);
   for (int k = 0; k < 5; ++k)
     if (c->deq[k]) (void)hipFree(c->deq[k]);
+  if (c->Vt2) (void)hipFree(c->Vt2);
+  if (c->tbase) (void)hipFree(c->tbase);
   for (int a = 0; a < 3; ++a)
     if (c->vst[a]) (void)hipFree(c->vst[a]);
   for (auto& kv : c->tw) (void)hipFree(kv.second);
@@ -764,6 +824,10 @@ static gpue_status materialise_A(gpue_ctx* c, int skip) {
 static void clear_program(gpue_ctx* c, int k) {
   if (c->deq[k]) (void)hipFree(c->deq[k]);
   c->deq[k] = nullptr;
+  if (k == GPUE_FIELD_V && c->Vt2) {
+    (void)hipFree(c->Vt2);
+    c->Vt2 = nullptr;
+  }
   c->t_dep = false;
   for (int j = 0; j < 5; ++j) c->t_dep = c->t_dep || c->deq[j] != nullptr;
   if (k >= 2 && !c->deq[2] && !c->deq[3] && !c->deq[4] && c->a_kind == A_EQN) c->a_kind = A_TABLE;
@@ -817,6 +881,21 @@ static std::map<std::string, double> name_map(const char* const* names, const do
   return m;
 }
 
+// Mark the ops whose operands hold no coordinate (EQ_UNI).
+static void mark_uniform(EqnProg& p) {
+  std::vector<bool> st;
+  for (int i = 0; i < p.n; ++i) {
+    if (p.op[i] < EQ_OP) {
+      st.push_back(p.op[i] == EQ_CONST || p.op[i] == EQ_T);
+    } else {
+      const bool u = st[st.size() - 1] && st[st.size() - 2];
+      st.pop_back();
+      st.back() = u;
+      if (u) p.op[i] |= EQ_UNI;
+    }
+  }
+}
+
 gpue_status gpue_set_field_eqn(gpue_ctx* c, int which, const char* expr, const char* const* names,
                                const double* values, int n_names) {
   if (!c || !expr || which < GPUE_FIELD_V || which > GPUE_FIELD_AZ) return GPUE_EINVAL;
@@ -833,8 +912,7 @@ gpue_status gpue_set_field_eqn(gpue_ctx* c, int which, const char* expr, const c
   const gpue_params& p = c->p;
   const double xM = p.xMax, yM = p.dimnum > 1 ? p.yMax : 0.0, zM = p.dimnum > 2 ? p.zMax : 0.0;
   if (td) {
-    // evaluated per point inside the step's sweeps at the step's time (the EQ
-    // kernels); the field's table is only filled for the energy
+    // run into the field's table before each step (fill_fields)
     if (c->prec != 64)
       return fail(c, GPUE_EUNSUPPORTED, "time-dependent equation fields need an FP64 context (GPUE's precision)");
     if (dp.depth > EQ_REG_DEPTH)
@@ -848,8 +926,13 @@ gpue_status gpue_set_field_eqn(gpue_ctx* c, int which, const char* expr, const c
       gpue_status st = materialise_A(c, which - GPUE_FIELD_AX);
       if (st != GPUE_OK) return st;
     }
+    if (!c->tbase && hipMalloc((void**)&c->tbase, sizeof(double)) != hipSuccess) return fail(c, GPUE_ENOMEM, "field");
+    if (which == GPUE_FIELD_V && !c->Vt2 && hipMalloc((void**)&c->Vt2, c->N * sizeof(double)) != hipSuccess)
+      return fail(c, GPUE_ENOMEM, "field");
     if (!c->deq[k] && hipMalloc((void**)&c->deq[k], sizeof(EqnProg)) != hipSuccess)
       return fail(c, GPUE_ENOMEM, "equation program");
+    mark_uniform(dp);
+    c->deq_depth[k] = dp.depth;
     HIPCHK(c, hipMemcpy(c->deq[k], &dp, sizeof(EqnProg), hipMemcpyHostToDevice));
     c->t_dep = true;
     if (which == GPUE_FIELD_V) {
@@ -970,21 +1053,8 @@ gpue_status gpue_parsum(gpue_ctx* c) {
 // The fields the energy kernels read: time-dependent ones are filled into their
 // tables at the time of the last step (one kernel per energy evaluation).
 static gpue_status energy_phys(gpue_ctx* c, Phys* out, bool fill) {
-  Phys ph = make_phys(c, 0, c->t_last);
-  if (c->t_dep) {
-    if (fill) {
-      hipError_t e = launch_fields_at(ph, (ph.v_kind == V_EQN || ph.v_kind == V_TRAP_A) ? c->Vt : nullptr,
-                                      c->deq[1] ? c->Kt : nullptr, c->deq[2] ? c->At[0] : nullptr,
-                                      c->deq[3] ? c->At[1] : nullptr, c->deq[4] ? c->At[2] : nullptr, c->N, c->stream);
-      if (e != hipSuccess) return fail(c, GPUE_EHIP, std::string("field tables: ") + hipGetErrorString(e));
-    }
-    if (ph.v_kind == V_EQN || ph.v_kind == V_TRAP_A) ph.v_kind = V_TABLE;
-    if (ph.k_kind == K_EQN) ph.k_kind = K_TABLE;
-    if (ph.a_kind == A_EQN) ph.a_kind = A_TABLE;
-    ph.eqk = 0;
-  }
-  *out = ph;
-  return GPUE_OK;
+  *out = make_phys(c, 0, 0);
+  return c->t_dep && fill ? fill_fields(c, FILL_V | FILL_KA, c->Vt, c->t_last, 1.0, nullptr) : GPUE_OK;
 }
 
 gpue_status gpue::energy_launch(gpue_ctx* c, double* host_dst) {
@@ -1305,7 +1375,8 @@ static gpue_status autotune(gpue_ctx* c, int reps) {
   for (int gstate = 0; gstate < 2 && st == GPUE_OK; ++gstate) {
     for (int parity = 0; parity < 2 && st == GPUE_OK; ++parity) {
       schedule(c, gstate, parity, true, sched);
-      Phys ph = make_phys(c, gstate, 0.0);
+      Phys ph = make_phys(c, gstate, 0);
+      if (c->t_dep) st = fill_fields(c, FILL_V | FILL_KA, c->Vt, 0.0, 0.0, nullptr);
       for (Sweep s : sched) {
         for (int v = 0; v < N_VARIANTS && st == GPUE_OK; ++v) {
           if (s.row && v > 3) break;   // row sweeps: plan and twiddle loading only
@@ -1362,7 +1433,7 @@ void gpue::schedule_block(const gpue_ctx* c, int gstate, int first, int n, std::
       step_of.push_back(first + s);
     }
   }
-  if (gstate != 1 || c->t_dep || c->ramp_type) return;
+  if (gstate != 1 || c->a_kind == A_EQN || c->ramp_type) return;
   std::vector<Sweep> fused;
   std::vector<int> fstep;
   for (size_t k = 0; k < out.size(); ++k) {
@@ -1397,16 +1468,16 @@ extern "C" {
 static gpue_status build_graph(gpue_ctx* c, int gstate, int len, StepGraph** out) {
   std::vector<Sweep> sched;
   std::vector<int> step_of;
-  const double Dt = gstate == 0 ? c->p.gdt : c->p.dt;
   schedule_block(c, gstate, 0, len, sched, step_of);
   if (gstate == 0)
     for (size_t k = 0; k + 1 < sched.size(); ++k)
       if (step_of[k + 1] == step_of[k] + 1) defer_norm(c, sched[k], sched[k + 1]);
   HIPCHK(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
   gpue_status st = GPUE_OK;
+  int v_done = -1, ka_done = -1;
   for (size_t k = 0; k < sched.size() && st == GPUE_OK; ++k) {
-    const Phys ph = make_phys(c, gstate, Dt * step_of[k]);
-    st = launch(c, sched[k], ph, c->psi, c->psi);
+    st = fill_for(c, sched[k], gstate, step_of[k], c->tbase, &v_done, &ka_done);
+    if (st == GPUE_OK) st = launch(c, sched[k], make_phys(c, gstate, step_of[k]), c->psi, c->psi);
   }
   hipGraph_t g = nullptr;
   hipError_t e = hipStreamEndCapture(c->stream, &g);
@@ -1451,13 +1522,12 @@ static gpue_status step_graph(gpue_ctx* c, int gstate, int len, StepGraph** out)
 }
 
 // Steps of a captured block starting at step s of an evolve call (0: the step
-// is launched on its own): up to G steps (an even count, from an even step) when
-// the fields do not depend on time, ending before the next energy evaluation and
-// at the end of the call.
+// is launched on its own): up to G steps (an even count, from an even step),
+// ending before the next energy evaluation and at the end of the call.
 static int block_len(const gpue_ctx* c, int first_step, int nsteps, int s, int energy_every) {
   const int G = c->graph_steps;
   const int i = first_step + s;
-  if (!(G > 0 && !c->timing && !c->t_dep && !c->ramp_type && (i % 2) == 0)) return 0;
+  if (!(G > 0 && !c->timing && !c->ramp_type && (i % 2) == 0)) return 0;
   int L = std::min(G, nsteps - s);
   if (energy_every > 0) {
     const int nxt = ((i + energy_every - 1) / energy_every) * energy_every;   // first cadence step >= i
@@ -1494,6 +1564,10 @@ static gpue_status evolve_impl(gpue_ctx* c, int first_step, int nsteps, int gsta
       gpue_status st = step_graph(c, gstate, L, &sg);
       if (st != GPUE_OK) return st;
       sg->last_use = ++c->graph_clock;
+      if (c->t_dep) {   // the block's fills count time from its first step
+        HIPCHK(c, launch_set_double(c->tbase, (double)i, c->stream));
+        c->t_last = Dt * (i + L - 1);
+      }
       HIPCHK(c, hipGraphLaunch(sg->exec, c->stream));
       if (!c->gev) HIPCHK(c, hipEventCreateWithFlags(&c->gev, hipEventDisableTiming));
       HIPCHK(c, hipEventRecord(c->gev, c->stream));
@@ -1501,7 +1575,7 @@ static gpue_status evolve_impl(gpue_ctx* c, int first_step, int nsteps, int gsta
       s += L - 1;
       continue;
     }
-    Phys ph = make_phys(c, gstate, Dt * i);   // time = Dt*i (src/evolution.cu:408)
+    Phys ph = make_phys(c, gstate, i);
     if (c->ramp_type) ph.Dt = Dt * ramp_scale(c, i);
     c->t_last = Dt * i;
     schedule(c, gstate, i, c->pending_norm, sched);
@@ -1524,8 +1598,10 @@ static gpue_status evolve_impl(gpue_ctx* c, int first_step, int nsteps, int gsta
         c->defer_nb = nb;
       }
     }
+    int v_done = -1, ka_done = -1;
     for (const Sweep& sw : sched) {
-      gpue_status st = launch(c, sw, ph, c->psi, c->psi);
+      gpue_status st = fill_for(c, sw, gstate, i, nullptr, &v_done, &ka_done);
+      if (st == GPUE_OK) st = launch(c, sw, ph, c->psi, c->psi);
       if (st != GPUE_OK) return st;
     }
     if (gstate == 0) c->pending_norm = true;
@@ -1729,7 +1805,11 @@ gpue_status gpue_sweep_profile(gpue_ctx* c, int gstate, int reps, int max_kinds,
   hipEvent_t e0, e1;
   HIPCHK(c, hipEventCreate(&e0));
   HIPCHK(c, hipEventCreate(&e1));
-  const Phys ph = make_phys(c, gstate, 0.0);
+  const Phys ph = make_phys(c, gstate, 0);
+  if (c->t_dep) {   // the tables at t = 0
+    st = fill_fields(c, FILL_V | FILL_KA, c->Vt, 0.0, 0.0, nullptr);
+    if (st == GPUE_OK && c->Vt2) st = fill_fields(c, FILL_V, c->Vt2, 0.0, 0.0, nullptr);
+  }
   *n_kinds = (int)kinds.size();
   for (size_t k = 0; k < kinds.size() && st == GPUE_OK; ++k) {
     double us = 0.0;
@@ -1763,7 +1843,7 @@ gpue_status gpue_step_bytes(gpue_ctx* c, int gstate, double* bytes, double* swee
   if (!c || (gstate != 0 && gstate != 1)) return GPUE_EINVAL;
   // the sweeps the steady state runs: a captured block when graphs are on (real
   // time fuses the sweeps at step boundaries), else a step of each parity
-  const int G = c->graph_steps > 0 && !c->t_dep && !c->ramp_type ? c->graph_steps : 2;
+  const int G = c->graph_steps > 0 && !c->ramp_type ? c->graph_steps : 2;
   std::vector<Sweep> blk;
   std::vector<int> step_of;
   if (G == c->graph_steps) {

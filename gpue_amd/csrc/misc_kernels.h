@@ -9,8 +9,21 @@ constexpr int REDUCE_BLOCKS = 1024;   // grid of the standalone reductions
 struct EqnProg;
 hipError_t launch_eqn_field(const EqnProg& prog, double* out, int xDim, int yDim, int zDim, double dx, double dy,
                             double dz, double xMax, double yMax, double zMax, double t, hipStream_t s);
-hipError_t launch_fields_at(const Phys& p, double* V, double* K, double* A0, double* A1, double* A2, long N,
-                            hipStream_t s);
+// Time-dependent fields into their tables (k_fields_at).
+struct FieldArgs {
+  const EqnProg* eq[5];    // programs of V, K, Ax, Ay, Az; null where the field is static
+  double* out[5];          // their tables; null: not written
+  const double* At[3];     // trap: the static components of A
+  const double* vst[3];    // trap: per-axis terms of the harmonic trap without 1/2 m |A|^2
+  double mass;
+  int trap;                // out[0] is the harmonic trap plus 1/2 m |A|^2 (V_TRAP_A)
+  int xDim, yDim, zDim;
+  long N;
+  double org[3], dxyz[3];  // coordinates x = dx * xi - xMax (src/dynamic.cu:613-615)
+  const double* tbase;     // device: step index of the captured block's first step (null: 0)
+  double Dt, tstep;        // t = Dt * (*tbase + tstep) (src/evolution.cu:408)
+};
+hipError_t launch_fields_at(const FieldArgs& f, int depth, hipStream_t s);
 template <typename T>
 hipError_t launch_apply_norm(void* psi, long N, const double* norm, hipStream_t s);
 template <typename T>

@@ -67,11 +67,9 @@ __device__ __forceinline__ double abs2d(cx<T> v) {
 // ---------------------------------------------------------------------------
 template <typename T, int N, int RV, int MODE_>
 __device__ __forceinline__ void row_body(const SweepArgs& a, int bid, int nblk) {
-  // bit 16 of the mode: FP32 real-time kernels forming phase factors in FP64;
-  // bit 32: time-dependent equation fields evaluated per point (EQ kernels)
+  // bit 16 of the mode: FP32 real-time kernels forming phase factors in FP64
   constexpr int MODE = MODE_ & 15;
   constexpr bool X = (MODE_ & 16) != 0;
-  constexpr bool EQ = (MODE_ & 32) != 0;
   // bit 64: RM_INV / RM_INV_FWD compiled without the gauge branch, for sweeps
   // whose flags carry no F_GAUGE_POST (its three-transform path sets the
   // register count of the whole kernel, and so the waves per SIMD)
@@ -108,10 +106,10 @@ __device__ __forceinline__ void row_body(const SweepArgs& a, int bid, int nblk) 
     }
     if constexpr (PRE) twr.load(tid, tw);
     fft_regs_tw<T, N, V, ORD_REV, +1, PRE>(v, tid, tw, twr, lds, la, active);
-    if (flags & F_HALFV_POST) halfV_all<T, E, X, EQ>(p, v, pos0);
+    if (flags & F_HALFV_POST) halfV_all<T, E, X>(p, p.Vt, v, pos0);
     if (!NG && (flags & F_GAUGE_POST)) {
       fft_regs_tw<T, N, V, ORD_FWD, -1, PRE>(v, tid, tw, twr, lds, la, active);
-      if (!gauge_rot_lin<T, N, TPL, RFL, E, 0, X, EQ>(p, v, tid, yi, a.invN)) gauge_all<T, E, 0, X, EQ>(p, v, posL, a.invN);
+      if (!gauge_rot_lin<T, N, TPL, RFL, E, 0, X>(p, v, tid, yi, a.invN)) gauge_all<T, E, 0, X>(p, v, posL, a.invN);
       fft_regs_tw<T, N, V, ORD_REV, +1, PRE>(v, tid, tw, twr, lds, la, active);
     }
   } else {
@@ -136,22 +134,22 @@ __device__ __forceinline__ void row_body(const SweepArgs& a, int bid, int nblk) 
 #pragma unroll
         for (int r = 0; r < E; ++r) v[r] = scale_norm(v[r], inv);
       }
-      if (flags & F_HALFV_PRE) halfV_all<T, E, X, EQ>(p, v, pos0);
+      if (flags & F_HALFV_PRE) halfV_all<T, E, X>(p, p.Vt, v, pos0);
     }
     fft_regs_tw<T, N, V, ORD_FWD, -1, PRE>(v, tid, tw, twr, lds, la, active);
     if constexpr (MODE == RM_GAUGE || MODE == RM_GAUGE_FWD) {
-      if (!gauge_rot_lin<T, N, TPL, RFL, E, 0, X, EQ>(p, v, tid, yi, a.invN)) gauge_all<T, E, 0, X, EQ>(p, v, posL, a.invN);
+      if (!gauge_rot_lin<T, N, TPL, RFL, E, 0, X>(p, v, tid, yi, a.invN)) gauge_all<T, E, 0, X>(p, v, posL, a.invN);
       fft_regs_tw<T, N, V, ORD_REV, +1, PRE>(v, tid, tw, twr, lds, la, active);
     } else if constexpr (MODE == RM_K) {
-      kstep_all<T, E, X, EQ>(p, v, posL, a.invN);
+      kstep_all<T, E, X>(p, v, posL, a.invN);
       fft_regs_tw<T, N, V, ORD_REV, +1, PRE>(v, tid, tw, twr, lds, la, active);
     } else if constexpr (MODE == RM_FULL) {
-      kstep_all<T, E, X, EQ>(p, v, posL, a.invN);
+      kstep_all<T, E, X>(p, v, posL, a.invN);
       fft_regs_tw<T, N, V, ORD_REV, +1, PRE>(v, tid, tw, twr, lds, la, active);
-      if (flags & F_HALFV_POST) halfV_all<T, E, X, EQ>(p, v, pos0);
+      if (flags & F_HALFV_POST) halfV_all<T, E, X>(p, p.Vt, v, pos0);
       if (flags & F_GAUGE_POST) {
         fft_regs_tw<T, N, V, ORD_FWD, -1, PRE>(v, tid, tw, twr, lds, la, active);
-        if (!gauge_rot_lin<T, N, TPL, RFL, E, 0, X, EQ>(p, v, tid, yi, a.invN)) gauge_all<T, E, 0, X, EQ>(p, v, posL, a.invN);
+        if (!gauge_rot_lin<T, N, TPL, RFL, E, 0, X>(p, v, tid, yi, a.invN)) gauge_all<T, E, 0, X>(p, v, posL, a.invN);
         fft_regs_tw<T, N, V, ORD_REV, +1, PRE>(v, tid, tw, twr, lds, la, active);
       }
     } else if constexpr (MODE == RM_KSUM) {
@@ -171,7 +169,7 @@ __device__ __forceinline__ void row_body(const SweepArgs& a, int bid, int nblk) 
 
   // bridge modes continue with the next step's first row sweep
   if constexpr (MODE == RM_INV_FWD || MODE == RM_GAUGE_FWD) {
-    if (flags & F_HALFV_PRE) halfV_all<T, E, X, EQ>(p, v, pos0);
+    if (flags & F_HALFV_PRE) halfV_all<T, E, X>(p, p.Vt_next, v, pos0);
     fft_regs_tw<T, N, V, ORD_FWD, -1, PRE>(v, tid, tw, twr, lds, la, active);
   }
 
@@ -202,11 +200,9 @@ __device__ __forceinline__ void row_body(const SweepArgs& a, int bid, int nblk) 
 // ---------------------------------------------------------------------------
 template <typename T, int N, int CV, int MODE_>
 __device__ __forceinline__ void col_body(const SweepArgs& a, int bid, int nblk) {
-  // bit 16 of the mode: FP32 real-time kernels forming phase factors in FP64;
-  // bit 32: time-dependent equation fields evaluated per point (EQ kernels)
+  // bit 16 of the mode: FP32 real-time kernels forming phase factors in FP64
   constexpr int MODE = MODE_ & 15;
   constexpr bool X = (MODE_ & 16) != 0;
-  constexpr bool EQ = (MODE_ & 32) != 0;
   constexpr int V = CV & 1;
   constexpr bool PRE = (CV >> 1) != 0 && sizeof(T) == 8;
   using P = Plan<N, V>;
@@ -250,9 +246,9 @@ __device__ __forceinline__ void col_body(const SweepArgs& a, int bid, int nblk) 
   };
   auto gauge_here = [&](cx<T>* w) {
     if (a.axis == 1) {
-      if (!gauge_rot_lin<T, N, TPL, RFL, E, 1, X, EQ>(p, w, tid, xq, a.invN)) gauge_all<T, E, 1, X, EQ>(p, w, posL, a.invN);
+      if (!gauge_rot_lin<T, N, TPL, RFL, E, 1, X>(p, w, tid, xq, a.invN)) gauge_all<T, E, 1, X>(p, w, posL, a.invN);
     } else {
-      gauge_all<T, E, 2, X, EQ>(p, w, posL, a.invN);
+      gauge_all<T, E, 2, X>(p, w, posL, a.invN);
     }
   };
 
@@ -266,7 +262,7 @@ __device__ __forceinline__ void col_body(const SweepArgs& a, int bid, int nblk) 
     if constexpr (MODE == CM_INV_VG) {
       // the closing sweep of a step that leads with this axis: V/2, then this
       // axis' gauge operator
-      if (flags & F_HALFV_POST) halfV_all<T, E, X, EQ>(p, v, pos0);
+      if (flags & F_HALFV_POST) halfV_all<T, E, X>(p, p.Vt, v, pos0);
       if (flags & F_GAUGE_POST) {
         fft_regs_tw<T, N, V, ORD_FWD, -1, PRE>(v, tid, tw, twr, lds, la, active);
         gauge_here(v);
@@ -302,7 +298,7 @@ __device__ __forceinline__ void col_body(const SweepArgs& a, int bid, int nblk) 
 #pragma unroll
         for (int r = 0; r < E; ++r) v[r] = scale_norm(v[r], inv);
       }
-      if (flags & F_HALFV_PRE) halfV_all<T, E, X, EQ>(p, v, pos0);
+      if (flags & F_HALFV_PRE) halfV_all<T, E, X>(p, p.Vt, v, pos0);
     }
     auto epos = [&](int r) { return bpos<N, TPL, RFL>(tid, r); };
     fft_regs_tw<T, N, V, ORD_FWD, -1, PRE>(v, tid, tw, twr, lds, la, active);
@@ -327,15 +323,15 @@ __device__ __forceinline__ void col_body(const SweepArgs& a, int bid, int nblk) 
       }
     } else {
       if constexpr (MODE == CM_K) {
-        if (a.axis == 1) kstep_col<T, E, 1, X, EQ>(p, v, xq, o, epos, a.invN);
-        else kstep_col<T, E, 2, X, EQ>(p, v, xq, o, epos, a.invN);
+        if (a.axis == 1) kstep_col<T, E, 1, X>(p, v, xq, o, epos, a.invN);
+        else kstep_col<T, E, 2, X>(p, v, xq, o, epos, a.invN);
       } else {
         gauge_here(v);
       }
       fft_regs_tw<T, N, V, ORD_REV, +1, PRE>(v, tid, tw, twr, lds, la, active);
       if constexpr (MODE == CM_GAUGE_FWD) {
         // bridge: the next step's V/2 and its first transform along this axis
-        if (flags & F_HALFV_PRE) halfV_all<T, E, X, EQ>(p, v, pos0);
+        if (flags & F_HALFV_PRE) halfV_all<T, E, X>(p, p.Vt_next, v, pos0);
         fft_regs_tw<T, N, V, ORD_FWD, -1, PRE>(v, tid, tw, twr, lds, la, active);
         if (active) {
 #pragma unroll

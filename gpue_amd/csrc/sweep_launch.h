@@ -13,65 +13,8 @@ inline int col_blocks(int xDim, int others) {
 
 // FP32 real-time steps run the kernels whose mode carries bit 16 (phase factors
 // and their products in FP64, sweep_kernels.h); every other launch the plain ones.
-// Kernels with time-dependent equation fields evaluated per point (bit 32 of
-// the mode): only for the default variants (wide lines, or narrow lines with
-// quarter strided tiles), which contexts with such fields always use; no
-// bridge modes (their steps run one by one).
-// FP64 only: GPUE's fields are FP64, and FP32 contexts reject time-dependent ones.
-template <typename T, int RV>
-constexpr bool row_eq_variant() { return sizeof(T) == 8 && (RV == 0 || RV == 3); }
-template <typename T, int CV>
-constexpr bool col_eq_variant() { return sizeof(T) == 8 && (CV == 0 || CV == 5); }
-
-template <typename T, int N, int V>
-hipError_t launch_row_eq(int mode, const SweepArgs& a, hipStream_t s) {
-  if constexpr (row_eq_variant<T, V>()) {
-    dim3 grid(row_blocks<N, V>(a.lines)), block(RowCfg<N, V>::WG);
-#define GPUE_ROW_EQ(M_)                                                                          \
-  hipLaunchKernelGGL((row_sweep<T, N, V, M_ | 32>), grid, block, 0, s, a);                       \
-  break;
-    switch (mode) {
-      case RM_FWD: GPUE_ROW_EQ(RM_FWD)
-      case RM_INV: GPUE_ROW_EQ(RM_INV)
-      case RM_GAUGE: GPUE_ROW_EQ(RM_GAUGE)
-      case RM_FULL: GPUE_ROW_EQ(RM_FULL)
-      case RM_K: GPUE_ROW_EQ(RM_K)
-      default: return hipErrorInvalidValue;
-    }
-#undef GPUE_ROW_EQ
-    return hipGetLastError();
-  } else {
-    (void)mode; (void)a; (void)s;
-    return hipErrorInvalidValue;
-  }
-}
-
-template <typename T, int N, int V>
-hipError_t launch_col_eq(int mode, const SweepArgs& a, hipStream_t s) {
-  if constexpr (col_eq_variant<T, V>()) {
-    const int others = a.axis == 1 ? a.ph.zDim : a.ph.yDim;
-    dim3 grid(col_blocks<T, N, V>(a.ph.xDim, others)), block(ColCfg<T, N, V>::WG);
-#define GPUE_COL_EQ(M_)                                                                          \
-  hipLaunchKernelGGL((col_sweep<T, N, V, M_ | 32>), grid, block, 0, s, a);                       \
-  break;
-    switch (mode) {
-      case CM_K: GPUE_COL_EQ(CM_K)
-      case CM_GAUGE: GPUE_COL_EQ(CM_GAUGE)
-      case CM_FWD_V: GPUE_COL_EQ(CM_FWD_V)
-      case CM_INV_VG: GPUE_COL_EQ(CM_INV_VG)
-      default: return hipErrorInvalidValue;
-    }
-#undef GPUE_COL_EQ
-    return hipGetLastError();
-  } else {
-    (void)mode; (void)a; (void)s;
-    return hipErrorInvalidValue;
-  }
-}
-
 template <typename T, int N, int V>
 hipError_t launch_row_t(int mode, const SweepArgs& a, hipStream_t s) {
-  if (a.ph.eqk && mode != RM_KSUM) return launch_row_eq<T, N, V>(mode, a, s);
   dim3 grid(row_blocks<N, V>(a.lines)), block(RowCfg<N, V>::WG);
   // closing sweeps with no gauge operator take the kernels compiled without it
   const bool ng = !(a.flags & F_GAUGE_POST);
@@ -118,8 +61,6 @@ hipError_t launch_row_t(int mode, const SweepArgs& a, hipStream_t s) {
 
 template <typename T, int N, int V>
 hipError_t launch_col_t(int mode, const SweepArgs& a, hipStream_t s) {
-  if (a.ph.eqk && (mode == CM_K || mode == CM_GAUGE || mode == CM_FWD_V || mode == CM_INV_VG))
-    return launch_col_eq<T, N, V>(mode, a, s);
   const int others = a.axis == 1 ? a.ph.zDim : a.ph.yDim;
   dim3 grid(col_blocks<T, N, V>(a.ph.xDim, others)), block(ColCfg<T, N, V>::WG);
   if constexpr (sizeof(T) == 4) {
