@@ -116,22 +116,25 @@ RM = {"row_fwd": 0, "row_inv": 1, "row_gauge": 2, "row_full": 3, "row_ksum": 4, 
 CM = {"fwd": 0, "inv": 1, "k": 2, "gauge": 3, "ksum": 4, "fwdv": 5, "invvg": 6, "gauge_fwd": 7}
 
 
-def kernel_symbol(name, prec, n_axis, variant):
+def kernel_symbol(name, prec, n_axis, variant, gstate=0):
     """The template instance rocprofv3 reports for a sweep name (row sweeps
     are instantiated per plan and twiddle loading, variants 0..3 with 4, 5
     acting as 2, 3; strided sweeps per full variant). Closing row sweeps
     without the gauge operator after them ("+gx") run the instance compiled
-    without it (mode bit 64)."""
+    without it (mode bit 64); sweeps with operators have real-time instances
+    (gstate 1, mode bit 16)."""
     t = "double" if prec == 64 else "float"
     parts = name.split("+")
     base = parts[0]
     if base.startswith("row"):
-        mode = RM[base]
+        mode = RM[base] | (16 if gstate and base != "row_ksum" else 0)
         if base in ("row_inv", "row_inv_fwd") and "gx" not in parts[1:]:
             mode |= 64
         return f"gpue::row_sweep<{t}, {n_axis[0]}, {(variant[0] & 1) + (2 if variant[0] > 1 else 0)}, {mode}>"
     axis = 1 if base.startswith("coly") else 2
-    return f"gpue::col_sweep<{t}, {n_axis[axis]}, {variant[axis]}, {CM[base.split('_', 1)[1]]}>"
+    kind = base.split("_", 1)[1]
+    mode = CM[kind] | (16 if gstate and kind not in ("fwd", "inv", "ksum") else 0)
+    return f"gpue::col_sweep<{t}, {n_axis[axis]}, {variant[axis]}, {mode}>"
 
 
 def kernel_table(ctx, prec, variants, steps_by_gstate, reps=50):
@@ -145,7 +148,7 @@ def kernel_table(ctx, prec, variants, steps_by_gstate, reps=50):
         if nsteps <= 0:
             continue
         for k in ctx.sweep_profile(gstate, reps):
-            rows.append(dict(kernel=k["name"], gstate=gstate, symbol=kernel_symbol(k["name"], prec, dims, variants),
+            rows.append(dict(kernel=k["name"], gstate=gstate, symbol=kernel_symbol(k["name"], prec, dims, variants, gstate),
                              us_per_launch=round(k["us"], 3), launches_per_step=k["per_step"],
                              job_ms=round(k["us"] * k["per_step"] * nsteps / 1e3, 3),
                              GBps=round(bytes_per_launch / (k["us"] * 1e-6) / 1e9, 1)))

@@ -375,42 +375,27 @@ struct LdsCol {
 
 // Full transform on registers: input in boundary layout of first radix,
 // output in boundary layout of last radix.  Inner passes exchange via LDS.
-// `active` predicates LDS traffic for padding threads (they still hit barriers).
+// Lanes past the last line take part (they have LDS of their own and load some valid
+// line): a branch around loads or LDS traffic would make every later wait conservative.
 template <typename T, int N, int V, int ORD, int SIGN, bool PRE, int P, typename LA>
 __device__ __forceinline__ void fft_from_pass(cx<T>* v, int tid, const typename TwE<T>::type* __restrict__ tw,
-                                              const typename TwE<T>::type* w, cx<T>* lds, const LA& la,
-                                              bool active) {
+                                              const typename TwE<T>::type* w, cx<T>* lds, const LA& la) {
   using S = Seq<N, V, ORD>;
   constexpr int NP = Plan<N, V>::NP, E = Plan<N, V>::E, TPL = Plan<N, V>::TPL;
   if constexpr (P < NP) {
     if constexpr (P > 0) {
       constexpr int RP = S::radix(P - 1), LP = S::Lbefore(P - 1);
       __syncthreads();  // previous users of LDS are done
-      if (active) {
 #pragma unroll
-        for (int r = 0; r < E; ++r) lds[la.at(pass_out<N, TPL, RP, LP>(tid, r / RP, r % RP))] = v[r];
-      }
+      for (int r = 0; r < E; ++r) lds[la.at(pass_out<N, TPL, RP, LP>(tid, r / RP, r % RP))] = v[r];
       __syncthreads();
-      if (active) {
 #pragma unroll
-        for (int r = 0; r < E; ++r) v[r] = lds[la.at(bpos<N, TPL, S::radix(P)>(tid, r))];
-      }
+      for (int r = 0; r < E; ++r) v[r] = lds[la.at(bpos<N, TPL, S::radix(P)>(tid, r))];
     }
     pass_compute<T, N, E, S::radix(P), S::Lbefore(P), SIGN, PRE>(v, tid, tw + TwTab<N, V>::template off<ORD>(P),
                                                                  w + TwPlan<N, V, ORD>::off(P));
-    fft_from_pass<T, N, V, ORD, SIGN, PRE, P + 1>(v, tid, tw, w, lds, la, active);
+    fft_from_pass<T, N, V, ORD, SIGN, PRE, P + 1>(v, tid, tw, w, lds, la);
   }
-}
-
-// PRE: load every twiddle of the transform before its first pass (for
-// latency-bound launches with registers to spare); otherwise per pass.
-template <typename T, int N, int V, int ORD, int SIGN, bool PRE, typename LA>
-__device__ __forceinline__ void fft_regs(cx<T>* v, int tid, const typename TwE<T>::type* __restrict__ tw, cx<T>* lds,
-                                         const LA& la,
-                                         bool active) {
-  typename TwE<T>::type w[PRE ? TwPlan<N, V, ORD>::total() : 1];
-  if constexpr (PRE) tw_load<T, N, V, ORD>(tid, tw, w);
-  fft_from_pass<T, N, V, ORD, SIGN, PRE, 0>(v, tid, tw, w, lds, la, active);
 }
 
 // The twiddles of both orders, loaded once at the start of a sweep (PRE
@@ -426,14 +411,15 @@ struct TwRegs {
   }
 };
 
-// fft_regs on preloaded twiddles (PRE) or from the table.
+// A transform on preloaded twiddles (PRE: for latency-bound launches with registers to
+// spare) or from the table, pass by pass.
 template <typename T, int N, int V, int ORD, int SIGN, bool PRE, typename LA>
 __device__ __forceinline__ void fft_regs_tw(cx<T>* v, int tid, const typename TwE<T>::type* __restrict__ tw,
-                                            const TwRegs<T, N, V>& wr, cx<T>* lds, const LA& la, bool active) {
+                                            const TwRegs<T, N, V>& wr, cx<T>* lds, const LA& la) {
   if constexpr (PRE)
-    fft_from_pass<T, N, V, ORD, SIGN, true, 0>(v, tid, tw, ORD == ORD_FWD ? wr.f : wr.r, lds, la, active);
+    fft_from_pass<T, N, V, ORD, SIGN, true, 0>(v, tid, tw, ORD == ORD_FWD ? wr.f : wr.r, lds, la);
   else
-    fft_from_pass<T, N, V, ORD, SIGN, false, 0>(v, tid, tw, wr.f, lds, la, active);
+    fft_from_pass<T, N, V, ORD, SIGN, false, 0>(v, tid, tw, wr.f, lds, la);
 }
 
 }  // namespace gpue

@@ -41,8 +41,8 @@ hipError_t launch_sweep(int prec, bool row, int N, int var, int mode, const Swee
                         bool* handled);
 int sweep_blocks(int prec, bool row, int N, int var, int lines_or_xdim, int others);
 bool sweep_full_waves(int prec, bool row, int N, int var);
-hipError_t launch_sweep_batched(int prec, bool row, int N, int var, int mode, const SweepArgs* d, int ninst, int lx,
-                                int others, hipStream_t s, bool* handled);
+hipError_t launch_sweep_batched(int prec, bool row, int N, int var, int mode, unsigned flags, int gstate,
+                                const SweepArgs* d, int ninst, int lx, int others, hipStream_t s, bool* handled);
 
 // Second stage of a batched reduction: one workgroup per instance.
 struct FinArgs {

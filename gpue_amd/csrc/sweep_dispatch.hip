@@ -32,6 +32,7 @@ hipError_t launch_sweep(int prec, bool row, int N, int var, int mode, const Swee
                         bool* handled) {
   *handled = true;
   const int pv = var & 1, nw = var >> 1;
+  mode = row ? row_kernel(mode, a.flags, a.ph.gstate) : col_kernel(mode, a.ph.gstate);
 #define GPUE_CASE(N_)                                                                         \
   case N_:                                                                                    \
     if (pv == 0)                                                                              \
@@ -46,10 +47,12 @@ hipError_t launch_sweep(int prec, bool row, int N, int var, int mode, const Swee
 #undef GPUE_CASE
 }
 
-hipError_t launch_sweep_batched(int prec, bool row, int N, int var, int mode, const SweepArgs* d, int ninst, int lx,
-                                int others, hipStream_t s, bool* handled) {
+// `flags`, `gstate`: those of every instance's sweep.
+hipError_t launch_sweep_batched(int prec, bool row, int N, int var, int mode, unsigned flags, int gstate,
+                                const SweepArgs* d, int ninst, int lx, int others, hipStream_t s, bool* handled) {
   *handled = true;
   const int pv = var & 1, nw = var >> 1;
+  mode = row ? row_kernel(mode, flags, gstate) : col_kernel(mode, gstate);
 #define GPUE_CASE(N_)                                                                                  \
   case N_:                                                                                             \
     if (pv == 0)                                                                                       \

@@ -54,7 +54,7 @@ struct ColCfg {
 // fused form multiplies by its reciprocal (within 1 ulp of the quotient).
 template <typename T>
 __device__ __forceinline__ cx<T> scale_norm(cx<T> v, T inv) {
-  return mk(v.x * inv, v.y * inv);
+  return scaled(v, inv);
 }
 
 template <typename T>
@@ -62,95 +62,208 @@ __device__ __forceinline__ double abs2d(cx<T> v) {
   return (double)v.x * (double)v.x + (double)v.y * (double)v.y;
 }
 
+// Mode bits above the sweep kind (RM_*, CM_*): 16, the real-time kernel (phases;
+// the plain one is imaginary time); 64, RM_INV compiled without the gauge operator
+// (its three-transform path sets the register count of the whole kernel, and so
+// the waves per SIMD), for sweeps whose flags carry no F_GAUGE_POST.
+
+// The pending norm's reciprocal for the sweep that opens an imaginary-time step.
+struct NormIn {
+  PartNorm part;
+  __device__ __forceinline__ void load(const SweepArgs& a) {
+    if (a.flags & F_SCALE_PART) part.load(a.partials, a.norm_nb);
+  }
+  // a deferred renormalisation: the norm reduced here from the previous sweep's
+  // partials by every wave (all lanes active), stored once by block 0
+  __device__ __forceinline__ double inverse(const SweepArgs& a, int bid) {
+    double nrm;
+    if (a.flags & F_SCALE_PART) {
+      nrm = part.norm(a.partials, a.norm_nb, a.norm_scale);
+      if (bid == 0 && threadIdx.x == 0) *a.norm_out = nrm;
+    } else {
+      nrm = *a.norm_in;
+    }
+    return 1.0 / nrm;
+  }
+};
+
+// Brings the scalar arguments of a sweep into registers in one go at its start: left
+// to their places of use they are separate scalar loads (selects between them become
+// loads through selected addresses), each with its own wait in the serial chain ahead
+// of psi's loads and of the operators.
+// (Pointers go through the asm as global ones, or their loads would become flat.)
+template <typename U>
+__device__ __forceinline__ void pin_ptr(U*& p) {
+  auto g = (__attribute__((address_space(1))) U*)p;
+  asm volatile("" : "+s"(g));
+  p = (U*)g;
+}
+template <typename... P>
+__device__ __forceinline__ void pin_ptrs(P&... p) { (pin_ptr(p), ...); }
+#define GPUE_PIN(...) asm volatile("" : __VA_ARGS__)
+template <bool VHALF, bool KSTEP, bool GAUGE, bool OPENS>
+__device__ __forceinline__ void pin_args(SweepArgs& a) {
+  Phys& p = a.ph;
+  pin_ptrs(a.in, a.out, a.tw);
+  GPUE_PIN("+s"(a.flags), "+s"(p.yDim), "+s"(p.zDim), "+s"(p.xDim));
+  if constexpr (VHALF) {
+    pin_ptrs(p.vs[0], p.vs[1], p.vs[2], p.vsf[0], p.vsf[1], p.vsf[2], p.Vt, p.Vt_next);
+    GPUE_PIN("+s"(p.v_kind), "+s"(p.cV), "+s"(p.g), "+s"(p.cH), "+s"(p.gpe));
+  }
+  if constexpr (KSTEP) {
+    pin_ptrs(p.kf[0], p.kf[1], p.kf[2], p.kff[0], p.kff[1], p.kff[2], p.Kt);
+    GPUE_PIN("+s"(p.k_kind), "+s"(a.invN));
+  }
+  if constexpr (GAUGE) {
+    pin_ptrs(p.xg, p.yg, p.pxg, p.pyg, p.pzg, p.At[0], p.At[1], p.At[2]);
+    GPUE_PIN("+s"(p.a_kind), "+s"(p.omega), "+s"(p.omegaX), "+s"(p.omegaY), "+s"(p.Dt), "+s"(a.invN));
+  }
+  if constexpr (OPENS) {
+    pin_ptrs(a.partials, a.norm_in, a.norm_out);
+    GPUE_PIN("+s"(a.norm_nb), "+s"(a.norm_scale));
+  }
+}
+#undef GPUE_PIN
+
 // ---------------------------------------------------------------------------
 // Row sweep: lines are contiguous x-rows, line = y + yDim*z.
 // ---------------------------------------------------------------------------
 template <typename T, int N, int RV, int MODE_>
-__device__ __forceinline__ void row_body(const SweepArgs& a, int bid, int nblk) {
-  // bit 16 of the mode: FP32 real-time kernels forming phase factors in FP64
+__device__ __forceinline__ void row_body(SweepArgs a, int bid, int nblk) {
   constexpr int MODE = MODE_ & 15;
-  constexpr bool X = (MODE_ & 16) != 0;
-  // bit 64: RM_INV / RM_INV_FWD compiled without the gauge branch, for sweeps
-  // whose flags carry no F_GAUGE_POST (its three-transform path sets the
-  // register count of the whole kernel, and so the waves per SIMD)
-  constexpr bool NG = (MODE_ & 64) != 0;
+  constexpr bool REAL = (MODE_ & 16) != 0, NG = (MODE_ & 64) != 0;
   constexpr int V = RV & 1;
-  constexpr bool PRE = (RV >> 1) != 0;
+  constexpr bool PRE = (RV >> 1) != 0;   // operands and twiddles loaded up front
+  constexpr bool GAUGE = (MODE == RM_INV && !NG) || MODE == RM_GAUGE || MODE == RM_GAUGE_FWD || MODE == RM_FULL;
+  constexpr bool KSTEP = MODE == RM_K || MODE == RM_FULL;
+  constexpr bool OPENS = !REAL && (MODE == RM_FWD || MODE == RM_FULL);
+  constexpr bool GEARLY = PRE && sizeof(T) == 8;
+  constexpr bool VHALF = MODE != RM_GAUGE && MODE != RM_K && MODE != RM_KSUM;
   using P = Plan<N, V>;
   constexpr int TPL = P::TPL, E = P::E, LPW = RowCfg<N, RV>::LPW;
   constexpr int FOOT = LdsRow::footprint(N);
   __shared__ cx<T> lds[P::NP > 1 ? LPW * FOOT : 1];
   __shared__ double sh[64];
+  if constexpr (PRE) pin_args<VHALF, KSTEP, GAUGE, OPENS>(a);
   const Phys& p = a.ph;
   const unsigned flags = a.flags;
   const int tid = threadIdx.x % TPL, lw = threadIdx.x / TPL;
   const int line = bid * LPW + lw;
   const bool active = line < a.lines;
-  const int yi = active ? line % p.yDim : 0, zi = active ? line / p.yDim : 0;
-  const cx<T>* __restrict__ in = (const cx<T>*)a.in + (long)(active ? line : 0) * N;
-  cx<T>* __restrict__ out = (cx<T>*)a.out + (long)(active ? line : 0) * N;
+  const int ln = active ? line : 0;
+  int yi = ln, zi = 0;
+  if (p.zDim > 1) {
+    zi = ln / p.yDim;
+    yi = ln - zi * p.yDim;
+  }
+  const LineAt l{0, tid, (long)ln * N, 1, yi, zi};
+  const cx<T>* __restrict__ in = (const cx<T>*)a.in + l.base;
+  cx<T>* __restrict__ out = (cx<T>*)a.out + l.base;
   const auto* __restrict__ tw = (const typename TwE<T>::type*)a.tw;
   const LdsRow la{lw * FOOT};
   constexpr int RF0 = Seq<N, V, ORD_FWD>::first(), RFL = Seq<N, V, ORD_FWD>::last();
+  constexpr int RIN = MODE == RM_INV || MODE == RM_INV_FWD ? RFL : RF0;
   cx<T> v[E];
   double acc = 0.0;
-  TwRegs<T, N, V> twr;   // PRE: every twiddle of the sweep, loaded after psi
-  // grid indices of register slot r in the boundary layouts of the first / last radix
-  auto pos0 = [&](int r) { return Pt{bpos<N, TPL, RF0>(tid, r), yi, zi}; };
-  auto posL = [&](int r) { return Pt{bpos<N, TPL, RFL>(tid, r), yi, zi}; };
+  TwRegs<T, N, V> twr;
+  NormIn nin;
+  VOp<T, N, TPL, RF0, E> vo;          // V/2 sits between transforms: first-radix layout
+  KOp<T, N, TPL, RFL, E, REAL> ko;    // K and A in the last radix's
+  GOp<T, N, TPL, RFL, E, REAL> go;
+  const double* __restrict__ Vt = MODE == RM_GAUGE_FWD ? p.Vt_next : p.Vt;
+  auto fwd = [&]() { fft_regs_tw<T, N, V, ORD_FWD, -1, PRE>(v, tid, tw, twr, lds, la); };
+  auto inv = [&]() { fft_regs_tw<T, N, V, ORD_REV, +1, PRE>(v, tid, tw, twr, lds, la); };
+  auto half = [&]() {
+    if constexpr (PRE) vo.ready();
+    else vo.load(p, Vt, l);
+    vo.template half<REAL>(p, l, v);
+  };
+  auto kstep = [&]() {
+    if constexpr (PRE) ko.ready();
+    else ko.load(p, l);
+    ko.apply(p, l, v, a.invN);
+  };
+  auto gauge = [&]() {
+    if constexpr (!PRE) {
+      go.load(p, l);
+      go.prep(p, l, a.invN);
+    }
+    go.apply(p, v, l, a.invN, GEARLY);
+  };
+
+  if constexpr (PRE && GAUGE) go.load(p, l);
+  if constexpr (OPENS) nin.load(a);
+#pragma unroll
+  for (int r = 0; r < E; ++r) v[r] = in[bpos<N, TPL, RIN>(tid, r)];
+  if constexpr (PRE) {
+    if constexpr (VHALF) vo.load(p, Vt, l);
+    if constexpr (KSTEP) ko.load(p, l);
+    if constexpr (GAUGE && GEARLY) {
+      if (p.a_kind == A_TABLE) go.load_points(p, l);
+    }
+    twr.load(tid, tw);
+    if constexpr (GAUGE) go.prep(p, l, a.invN);
+  }
 
   if constexpr (MODE == RM_INV || MODE == RM_INV_FWD) {
-    if (active) {
+    inv();
+    if constexpr (MODE == RM_INV_FWD && sizeof(T) == 8) {
+      // the closing V/2 of this step and the opening one of the next: phases, which
+      // leave |psi|^2, so one phase of the summed exponents
+      if constexpr (PRE) vo.ready();
+      else vo.load(p, Vt, l);
+      T arg[E];
+      vo.args(p, l, v, arg);
+      if (p.Vt_next != p.Vt) {   // V(t): the next step's table
+        VOp<T, N, TPL, RF0, E> vn;
+        vn.load(p, p.Vt_next, l);
+        T arg2[E];
+        vn.args(p, l, v, arg2);
 #pragma unroll
-      for (int r = 0; r < E; ++r) v[r] = in[bpos<N, TPL, RFL>(tid, r)];
-    }
-    if constexpr (PRE) twr.load(tid, tw);
-    fft_regs_tw<T, N, V, ORD_REV, +1, PRE>(v, tid, tw, twr, lds, la, active);
-    if (flags & F_HALFV_POST) halfV_all<T, E, X>(p, p.Vt, v, pos0);
-    if (!NG && (flags & F_GAUGE_POST)) {
-      fft_regs_tw<T, N, V, ORD_FWD, -1, PRE>(v, tid, tw, twr, lds, la, active);
-      if (!gauge_rot_lin<T, N, TPL, RFL, E, 0, X>(p, v, tid, yi, a.invN)) gauge_all<T, E, 0, X>(p, v, posL, a.invN);
-      fft_regs_tw<T, N, V, ORD_REV, +1, PRE>(v, tid, tw, twr, lds, la, active);
+        for (int r = 0; r < E; ++r) arg[r] += arg2[r];
+      } else {
+#pragma unroll
+        for (int r = 0; r < E; ++r) arg[r] += arg[r];
+      }
+      apply_phase_all<T, E, REAL>(v, arg, 1.0);
+      fwd();
+    } else if constexpr (MODE == RM_INV_FWD) {
+      half();   // FP32 (static V): each half's phase rounds psi, as in single steps
+      half();
+      fwd();
+    } else {
+      if (flags & F_HALFV_POST) half();
+      if constexpr (GAUGE) {
+        fwd();
+        gauge();
+        inv();
+      }
     }
   } else {
-    if (active) {
-#pragma unroll
-      for (int r = 0; r < E; ++r) v[r] = in[bpos<N, TPL, RF0>(tid, r)];
-    }
-    if constexpr (PRE) twr.load(tid, tw);
-    if constexpr (MODE == RM_FWD || MODE == RM_FULL) {
+    if constexpr (OPENS) {
       if (flags & F_SCALE_IN) {
-        // a deferred renormalisation: the norm reduced here from the previous
-        // sweep's partials by every wave (all lanes active; psi is already in
-        // flight), stored once by block 0
-        double nrm;
-        if (MODE == RM_FWD && (flags & F_SCALE_PART)) {
-          nrm = part_norm(a.partials, a.norm_nb, a.norm_scale);
-          if (bid == 0 && threadIdx.x == 0) *a.norm_out = nrm;
-        } else {
-          nrm = *a.norm_in;
-        }
-        const T inv = (T)(1.0 / nrm);
+        const T s = (T)nin.inverse(a, bid);
 #pragma unroll
-        for (int r = 0; r < E; ++r) v[r] = scale_norm(v[r], inv);
+        for (int r = 0; r < E; ++r) v[r] = scale_norm(v[r], s);
       }
-      if (flags & F_HALFV_PRE) halfV_all<T, E, X>(p, p.Vt, v, pos0);
     }
-    fft_regs_tw<T, N, V, ORD_FWD, -1, PRE>(v, tid, tw, twr, lds, la, active);
+    if constexpr (MODE == RM_FWD || MODE == RM_FULL) {
+      if (flags & F_HALFV_PRE) half();
+    }
+    fwd();
     if constexpr (MODE == RM_GAUGE || MODE == RM_GAUGE_FWD) {
-      if (!gauge_rot_lin<T, N, TPL, RFL, E, 0, X>(p, v, tid, yi, a.invN)) gauge_all<T, E, 0, X>(p, v, posL, a.invN);
-      fft_regs_tw<T, N, V, ORD_REV, +1, PRE>(v, tid, tw, twr, lds, la, active);
-    } else if constexpr (MODE == RM_K) {
-      kstep_all<T, E, X>(p, v, posL, a.invN);
-      fft_regs_tw<T, N, V, ORD_REV, +1, PRE>(v, tid, tw, twr, lds, la, active);
-    } else if constexpr (MODE == RM_FULL) {
-      kstep_all<T, E, X>(p, v, posL, a.invN);
-      fft_regs_tw<T, N, V, ORD_REV, +1, PRE>(v, tid, tw, twr, lds, la, active);
-      if (flags & F_HALFV_POST) halfV_all<T, E, X>(p, p.Vt, v, pos0);
-      if (flags & F_GAUGE_POST) {
-        fft_regs_tw<T, N, V, ORD_FWD, -1, PRE>(v, tid, tw, twr, lds, la, active);
-        if (!gauge_rot_lin<T, N, TPL, RFL, E, 0, X>(p, v, tid, yi, a.invN)) gauge_all<T, E, 0, X>(p, v, posL, a.invN);
-        fft_regs_tw<T, N, V, ORD_REV, +1, PRE>(v, tid, tw, twr, lds, la, active);
+      gauge();
+      inv();
+    } else if constexpr (KSTEP) {
+      kstep();
+      inv();
+      if constexpr (MODE == RM_FULL) {
+        if (flags & F_HALFV_POST) half();
+        if (flags & F_GAUGE_POST) {
+          fwd();
+          gauge();
+          inv();
+        }
       }
     } else if constexpr (MODE == RM_KSUM) {
       if (active) {
@@ -165,30 +278,26 @@ __device__ __forceinline__ void row_body(const SweepArgs& a, int bid, int nblk) 
         }
       }
     }
-  }
-
-  // bridge modes continue with the next step's first row sweep
-  if constexpr (MODE == RM_INV_FWD || MODE == RM_GAUGE_FWD) {
-    if (flags & F_HALFV_PRE) halfV_all<T, E, X>(p, p.Vt_next, v, pos0);
-    fft_regs_tw<T, N, V, ORD_FWD, -1, PRE>(v, tid, tw, twr, lds, la, active);
+    if constexpr (MODE == RM_GAUGE_FWD) {   // continue with the next step's first row sweep
+      half();
+      fwd();
+    }
   }
 
   // store: forward sweeps leave the forward layout (last radix), the others the first radix
-  if constexpr (MODE == RM_FWD || MODE == RM_INV_FWD || MODE == RM_GAUGE_FWD) {
-    if (active) {
-#pragma unroll
-      for (int r = 0; r < E; ++r) out[bpos<N, TPL, RFL>(tid, r)] = v[r];
-    }
-  } else if constexpr (MODE != RM_KSUM) {
+  constexpr bool FWD_OUT = MODE == RM_FWD || MODE == RM_INV_FWD || MODE == RM_GAUGE_FWD;
+  constexpr int ROUT = FWD_OUT ? RFL : RF0;
+  constexpr bool NORM = !REAL && !FWD_OUT && MODE != RM_KSUM;
+  if constexpr (MODE != RM_KSUM) {
     if (active) {
 #pragma unroll
       for (int r = 0; r < E; ++r) {
-        out[bpos<N, TPL, RF0>(tid, r)] = v[r];
-        if (flags & F_NORM) acc += abs2d(v[r]);
+        out[bpos<N, TPL, ROUT>(tid, r)] = v[r];
+        if (NORM && (flags & F_NORM)) acc += abs2d(v[r]);
       }
     }
   }
-  if (MODE == RM_KSUM || (flags & F_NORM)) {
+  if (MODE == RM_KSUM || (NORM && (flags & F_NORM))) {
     double pv[1] = {acc};
     block_partial<1>(pv, a.partials, sh, bid, nblk);
   }
@@ -199,156 +308,140 @@ __device__ __forceinline__ void row_body(const SweepArgs& a, int bid, int nblk) 
 // xDim*yDim); a workgroup owns TC adjacent x-lines, lanes vary fastest in x.
 // ---------------------------------------------------------------------------
 template <typename T, int N, int CV, int MODE_>
-__device__ __forceinline__ void col_body(const SweepArgs& a, int bid, int nblk) {
-  // bit 16 of the mode: FP32 real-time kernels forming phase factors in FP64
+__device__ __forceinline__ void col_body(SweepArgs a, int bid, int nblk) {
   constexpr int MODE = MODE_ & 15;
-  constexpr bool X = (MODE_ & 16) != 0;
+  constexpr bool REAL = (MODE_ & 16) != 0;
   constexpr int V = CV & 1;
-  constexpr bool PRE = (CV >> 1) != 0 && sizeof(T) == 8;
+  constexpr bool EARLY = (CV >> 1) != 0;               // operands loaded up front
+  constexpr bool PRE = EARLY && sizeof(T) == 8;        // and every twiddle
+  constexpr bool GAUGE = MODE == CM_INV_VG || MODE == CM_GAUGE || MODE == CM_GAUGE_FWD;
+  constexpr bool GEARLY = EARLY && sizeof(T) == 8;
+  constexpr bool VHALF = MODE == CM_FWD_V || MODE == CM_INV_VG || MODE == CM_GAUGE_FWD;
+  constexpr bool OPENS = !REAL && MODE == CM_FWD_V;
   using P = Plan<N, V>;
   constexpr int TC = ColCfg<T, N, CV>::TC, E = P::E, TPL = P::TPL;
   __shared__ cx<T> lds[P::NP > 1 ? TC * N : 1];
   __shared__ double sh[64];
+  if constexpr (EARLY) pin_args<VHALF, MODE == CM_K, GAUGE, OPENS>(a);
   const Phys& p = a.ph;
   const unsigned flags = a.flags;
   const int c = threadIdx.x % TC, tid = threadIdx.x / TC;
   const int tiles = (p.xDim + TC - 1) / TC;
-  const int xt = bid % tiles, o = bid / tiles;
+  const int o = bid / tiles, xt = bid - o * tiles;
   const int xi = xt * TC + c;
   const bool active = xi < p.xDim;
-  const int xq = active ? xi : 0;   // table index: lanes past xDim (a last partial tile) read column 0
-  const long es = (a.axis == 1) ? (long)p.xDim : (long)p.xDim * p.yDim;
-  const long base = (a.axis == 1) ? (long)(active ? xi : 0) + (long)o * p.xDim * p.yDim
-                                  : (long)(active ? xi : 0) + (long)o * p.xDim;
+  const int xq = active ? xi : 0;   // lanes past xDim (a last partial tile) read column 0
+  const bool ay = a.axis == 1;
+  const LineAt l{a.axis, tid, ay ? (long)xq + (long)o * p.xDim * p.yDim : (long)xq + (long)o * p.xDim,
+                 ay ? (long)p.xDim : (long)p.xDim * p.yDim, xq, o};
+  const long es = l.es;
   // a lane's points lie at (tid + bpos(0, r)) * es from the tile's base:
   // one per-lane pointer, then per register a uniform offset bpos(0, r) * es
   // (scalar arithmetic) instead of a 64-bit multiply per access
-  const cx<T>* __restrict__ in = (const cx<T>*)a.in + base + (long)tid * es;
-  cx<T>* __restrict__ out = (cx<T>*)a.out + base + (long)tid * es;
+  const cx<T>* __restrict__ in = (const cx<T>*)a.in + l.base + (long)tid * es;
+  cx<T>* __restrict__ out = (cx<T>*)a.out + l.base + (long)tid * es;
   const auto* __restrict__ tw = (const typename TwE<T>::type*)a.tw;
   const LdsCol la{c, TC};
   constexpr int RF0 = Seq<N, V, ORD_FWD>::first(), RFL = Seq<N, V, ORD_FWD>::last();
+  constexpr int RIN = MODE == CM_INV || MODE == CM_INV_VG ? RFL : RF0;
   cx<T> v[E];
   double acc = 0.0;
-  TwRegs<T, N, V> twr;   // PRE: every twiddle of the sweep, loaded after psi
-  // coordinates of element e along the axis
-  auto yz = [&](int e, int& yi, int& zi) {
-    if (a.axis == 1) { yi = e; zi = o; } else { yi = o; zi = e; }
+  TwRegs<T, N, V> twr;
+  NormIn nin;
+  VOp<T, N, TPL, RF0, E> vo;
+  KOp<T, N, TPL, RFL, E, REAL> ko;
+  GOp<T, N, TPL, RFL, E, REAL> go;
+  const double* __restrict__ Vt = MODE == CM_GAUGE_FWD ? p.Vt_next : p.Vt;
+  auto fwd = [&]() { fft_regs_tw<T, N, V, ORD_FWD, -1, PRE>(v, tid, tw, twr, lds, la); };
+  auto inv = [&]() { fft_regs_tw<T, N, V, ORD_REV, +1, PRE>(v, tid, tw, twr, lds, la); };
+  auto half = [&]() {
+    if constexpr (EARLY) vo.ready();
+    else vo.load(p, Vt, l);
+    vo.template half<REAL>(p, l, v);
   };
-  // grid indices of register slot r in the boundary layouts of the first / last radix
-  auto pos0 = [&](int r) {
-    const int e = bpos<N, TPL, RF0>(tid, r);
-    return a.axis == 1 ? Pt{xq, e, o} : Pt{xq, o, e};
-  };
-  auto posL = [&](int r) {
-    const int e = bpos<N, TPL, RFL>(tid, r);
-    return a.axis == 1 ? Pt{xq, e, o} : Pt{xq, o, e};
-  };
-  auto gauge_here = [&](cx<T>* w) {
-    if (a.axis == 1) {
-      if (!gauge_rot_lin<T, N, TPL, RFL, E, 1, X>(p, w, tid, xq, a.invN)) gauge_all<T, E, 1, X>(p, w, posL, a.invN);
-    } else {
-      gauge_all<T, E, 2, X>(p, w, posL, a.invN);
+  auto gauge = [&]() {
+    if constexpr (!EARLY) {
+      go.load(p, l);
+      go.prep(p, l, a.invN);
     }
+    go.apply(p, v, l, a.invN, GEARLY);
   };
 
-  if constexpr (MODE == CM_INV || MODE == CM_INV_VG) {
-    if (active) {
+  if constexpr (EARLY && GAUGE) go.load(p, l);
+  if constexpr (OPENS) nin.load(a);
 #pragma unroll
-      for (int r = 0; r < E; ++r) v[r] = in[bpos<N, TPL, RFL>(0, r) * es];
+  for (int r = 0; r < E; ++r) v[r] = in[bpos<N, TPL, RIN>(0, r) * es];
+  if constexpr (EARLY) {
+    if constexpr (VHALF) vo.load(p, Vt, l);
+    if constexpr (MODE == CM_K) ko.load(p, l);
+    if constexpr (GAUGE && GEARLY) {
+      if (p.a_kind == A_TABLE) go.load_points(p, l);
     }
-    if constexpr (PRE) twr.load(tid, tw);
-    fft_regs_tw<T, N, V, ORD_REV, +1, PRE>(v, tid, tw, twr, lds, la, active);
+  }
+  if constexpr (PRE) twr.load(tid, tw);
+  if constexpr (EARLY && GAUGE) go.prep(p, l, a.invN);
+
+  if constexpr (MODE == CM_INV || MODE == CM_INV_VG) {
+    inv();
     if constexpr (MODE == CM_INV_VG) {
       // the closing sweep of a step that leads with this axis: V/2, then this
       // axis' gauge operator
-      if (flags & F_HALFV_POST) halfV_all<T, E, X>(p, p.Vt, v, pos0);
-      if (flags & F_GAUGE_POST) {
-        fft_regs_tw<T, N, V, ORD_FWD, -1, PRE>(v, tid, tw, twr, lds, la, active);
-        gauge_here(v);
-        fft_regs_tw<T, N, V, ORD_REV, +1, PRE>(v, tid, tw, twr, lds, la, active);
-      }
-    }
-    if (active) {
-#pragma unroll
-      for (int r = 0; r < E; ++r) {
-        out[bpos<N, TPL, RF0>(0, r) * es] = v[r];
-        if (MODE == CM_INV_VG && (flags & F_NORM)) acc += abs2d(v[r]);
-      }
+      half();
+      fwd();
+      gauge();
+      inv();
     }
   } else {
-    if (active) {
-#pragma unroll
-      for (int r = 0; r < E; ++r) v[r] = in[bpos<N, TPL, RF0>(0, r) * es];
-    }
-    if constexpr (PRE) twr.load(tid, tw);
-    if constexpr (MODE == CM_FWD_V) {
-      // the opening sweep of a step that leads with this axis
+    if constexpr (OPENS) {   // the opening sweep of a step that leads with this axis
       if (flags & F_SCALE_IN) {
-        // a deferred renormalisation (as in the row sweep): the norm reduced
-        // here from the previous sweep's partials by every wave, stored once
-        double nrm;
-        if (flags & F_SCALE_PART) {
-          nrm = part_norm(a.partials, a.norm_nb, a.norm_scale);
-          if (bid == 0 && threadIdx.x == 0) *a.norm_out = nrm;
-        } else {
-          nrm = *a.norm_in;
-        }
-        const T inv = (T)(1.0 / nrm);
+        const T s = (T)nin.inverse(a, bid);
 #pragma unroll
-        for (int r = 0; r < E; ++r) v[r] = scale_norm(v[r], inv);
+        for (int r = 0; r < E; ++r) v[r] = scale_norm(v[r], s);
       }
-      if (flags & F_HALFV_PRE) halfV_all<T, E, X>(p, p.Vt, v, pos0);
     }
-    auto epos = [&](int r) { return bpos<N, TPL, RFL>(tid, r); };
-    fft_regs_tw<T, N, V, ORD_FWD, -1, PRE>(v, tid, tw, twr, lds, la, active);
-    if constexpr (MODE == CM_FWD || MODE == CM_FWD_V) {
-      if (active) {
-#pragma unroll
-        for (int r = 0; r < E; ++r) out[bpos<N, TPL, RFL>(0, r) * es] = v[r];
-      }
-    } else if constexpr (MODE == CM_KSUM) {
+    if constexpr (MODE == CM_FWD_V) half();
+    fwd();
+    if constexpr (MODE == CM_KSUM) {
       if (active) {
 #pragma unroll
         for (int r = 0; r < E; ++r) {
-          int yi, zi;
-          yz(bpos<N, TPL, RFL>(tid, r), yi, zi);
+          const int e = bpos<N, TPL, RFL>(tid, r);
+          const int yi = ay ? e : o, zi = ay ? o : e;
           const long gid = gid_of(p, xi, yi, zi);
-          const double w = (flags & F_ASUM)
-                               ? A_val(p, a.axis, xi, yi, zi, gid) * (a.axis == 1 ? p.pyg[yi] : p.pzg[zi])
-                           : (flags & F_KAX) ? (a.axis == 1 ? p.ks[1][yi] : p.ks[2][zi])
+          const double w = (flags & F_ASUM)  ? A_val(p, a.axis, xi, yi, zi, gid) * (ay ? p.pyg[yi] : p.pzg[zi])
+                           : (flags & F_KAX) ? (ay ? p.ks[1][yi] : p.ks[2][zi])
                                              : K_val(p, xi, yi, zi, gid);
           acc += w * abs2d(v[r]);
         }
       }
-    } else {
-      if constexpr (MODE == CM_K) {
-        if (a.axis == 1) kstep_col<T, E, 1, X>(p, v, xq, o, epos, a.invN);
-        else kstep_col<T, E, 2, X>(p, v, xq, o, epos, a.invN);
-      } else {
-        gauge_here(v);
-      }
-      fft_regs_tw<T, N, V, ORD_REV, +1, PRE>(v, tid, tw, twr, lds, la, active);
-      if constexpr (MODE == CM_GAUGE_FWD) {
-        // bridge: the next step's V/2 and its first transform along this axis
-        if (flags & F_HALFV_PRE) halfV_all<T, E, X>(p, p.Vt_next, v, pos0);
-        fft_regs_tw<T, N, V, ORD_FWD, -1, PRE>(v, tid, tw, twr, lds, la, active);
-        if (active) {
-#pragma unroll
-          for (int r = 0; r < E; ++r) out[bpos<N, TPL, RFL>(0, r) * es] = v[r];
-        }
-      } else {
-        if (active) {
-#pragma unroll
-          for (int r = 0; r < E; ++r) {
-            out[bpos<N, TPL, RF0>(0, r) * es] = v[r];
-            if (flags & F_NORM) acc += abs2d(v[r]);
-          }
-        }
+    } else if constexpr (MODE == CM_K) {
+      if constexpr (EARLY) ko.ready();
+      else ko.load(p, l);
+      ko.apply(p, l, v, a.invN);
+      inv();
+    } else if constexpr (GAUGE) {
+      gauge();
+      inv();
+      if constexpr (MODE == CM_GAUGE_FWD) {   // bridge: the next step's V/2 and its first transform along this axis
+        half();
+        fwd();
       }
     }
   }
-  if (MODE == CM_KSUM || (flags & F_NORM)) {
+
+  constexpr bool FWD_OUT = MODE == CM_FWD || MODE == CM_FWD_V || MODE == CM_GAUGE_FWD;
+  constexpr int ROUT = FWD_OUT ? RFL : RF0;
+  constexpr bool NORM = !REAL && (MODE == CM_INV_VG || MODE == CM_GAUGE);
+  if constexpr (MODE != CM_KSUM) {
+    if (active) {
+#pragma unroll
+      for (int r = 0; r < E; ++r) {
+        out[bpos<N, TPL, ROUT>(0, r) * es] = v[r];
+        if (NORM && (flags & F_NORM)) acc += abs2d(v[r]);
+      }
+    }
+  }
+  if (MODE == CM_KSUM || (NORM && (flags & F_NORM))) {
     double pv[1] = {acc};
     block_partial<1>(pv, a.partials, sh, bid, nblk);
   }

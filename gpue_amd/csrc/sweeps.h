@@ -14,6 +14,8 @@
 // (harmonic V, rotation A, standard K) or read from tables (equation-string
 // or file fields), so the only per-step HBM traffic is psi itself.
 #pragma once
+#include <type_traits>
+
 #include "fft_core.h"
 
 namespace gpue {
@@ -38,8 +40,7 @@ enum { K_SEP = 0, K_TABLE = 1, K_EQN = 2 };
 enum { RM_FWD = 0, RM_INV = 1, RM_GAUGE = 2, RM_FULL = 3, RM_KSUM = 4, RM_INV_FWD = 5, RM_GAUGE_FWD = 6, RM_K = 7 };
 enum { CM_FWD = 0, CM_INV = 1, CM_K = 2, CM_GAUGE = 3, CM_KSUM = 4, CM_FWD_V = 5, CM_INV_VG = 6, CM_GAUGE_FWD = 7 };
 
-// Strided-sweep modes that apply a phase operator (FP32 real time runs their
-// bit-16 kernels).
+// Strided-sweep modes that apply an operator (real time runs their bit-16 kernels).
 __host__ __device__ inline bool col_phase_mode(int mode) {
   return mode == CM_K || mode == CM_GAUGE || mode == CM_FWD_V || mode == CM_INV_VG || mode == CM_GAUGE_FWD;
 }
@@ -114,6 +115,11 @@ struct SweepArgs {
   double* norm_out;        // F_SCALE_PART: where block 0 stores the norm
 };
 
+// Of three scalar arguments the one of axis a, by value (an index or a select of
+// addresses would keep the arguments in memory).
+template <typename U>
+__device__ __forceinline__ U pick(int a, U x, U y, U z) { return a == 0 ? x : a == 1 ? y : z; }
+
 // ---------------------------------------------------------------------------
 // Field evaluation (GPUE operators.cu kernels restated per point)
 // ---------------------------------------------------------------------------
@@ -124,7 +130,7 @@ __device__ __forceinline__ double A_val(const Phys& p, int axis, int xi, int yi,
     return 0.0;
   }
   if (p.a_kind == A_ZERO) return 0.0;
-  return p.At[axis][gid];
+  return pick(axis, p.At[0], p.At[1], p.At[2])[gid];
 }
 
 // kharmonic_V (src/operators.cu:994-1008) is a sum of per-axis terms once the
@@ -298,18 +304,14 @@ __device__ __forceinline__ void sincos_cw(float x, float* s, float* c) {
   sincos_core(x, s, c);
 }
 
-// Transcendentals in the working precision: FP64 sweeps use the reduced forms
-// above; FP32 sweeps the FP32 library exp and the FP32 reduced sincos.
+// exp and sincos of the verification entry (gpue_math_eval) and of the library
+// fallback.
 template <typename T>
 struct WMath;
 template <>
 struct WMath<double> {
   static __device__ __forceinline__ double ex(double a) { return exp_cw(a); }
   static __device__ __forceinline__ void sc(double a, double* s, double* c) { sincos_cw(a, s, c); }
-  static __device__ __forceinline__ void sc_core(double a, double* s, double* c) { sincos_core(a, s, c); }
-  static __device__ __forceinline__ bool sc_ok(double a) { return sincos_fast_ok(a); }
-  static __device__ __forceinline__ bool sc_small_ok(double a) { return sincos_small_ok(a); }
-  static __device__ __forceinline__ void sc_small(double a, double* s, double* c) { sincos_poly(a, s, c); }
 };
 template <>
 struct WMath<float> {
@@ -318,48 +320,110 @@ struct WMath<float> {
   // adds |a|*2^-24 relative
   static __device__ __forceinline__ float ex(float a) { return __expf(a); }
   static __device__ __forceinline__ void sc(float a, float* s, float* c) { sincos_cw(a, s, c); }
-  static __device__ __forceinline__ void sc_core(float a, float* s, float* c) { sincos_core(a, s, c); }
-  static __device__ __forceinline__ bool sc_ok(float a) { return sincos_fast_ok(a); }
-  static __device__ __forceinline__ bool sc_small_ok(float a) { return sincos_small_ok(a); }
-  static __device__ __forceinline__ void sc_small(float a, float* s, float* c) { sincos_poly(a, s, c); }
-};
-
-struct Pt {
-  int x, y, z;
 };
 
 // ---------------------------------------------------------------------------
-// Batched forms of the pointwise operators for the E points a lane holds.  All
-// table loads of the E points are issued before any arithmetic and every
-// branch on a field kind or gstate is taken once, outside the point loop:
-// per-point branches around loads serialise one memory round trip per point.
-// pos(r) gives the (x, y, z) grid indices of register slot r.
+// Pointwise operators on the E points a lane holds of a line.
+//
+// Each operator comes in two parts: load() gathers what it needs from tables,
+// and the rest computes.  Sweeps of small grids are a serial chain (a 512^2 FP64
+// sweep is half a wave per SIMD; its waves waited 60 % of their life), so the
+// variants for them issue every load() of the sweep at its start, next to psi's
+// own, and derive factors that do not depend on psi while psi is on its way;
+// a load left to its place of use costs a further memory round trip of 0.5-1 us
+// in a sweep of 4-10 us.  At 512^2 FP64 with rotation (4 MiB psi, 32-step graphs)
+// loading up front took the step from 29.6 to 26.9 us in imaginary and from 26.2 to
+// 23.5 us in real time (sweeps 6.3-9.5 -> 6.1-8.9 and 6.4-10.9 -> 6.1-9.6 us), the
+// 256^2 step without rotation from 14.2 to 12.7 and from 9.8 to 8.8 us.  Sweeps of
+// large grids load at the place of use (other waves cover the wait, registers are
+// what they lack).
+//
+// The arithmetic runs in the working precision T: FP64 sweeps in double; FP32
+// sweeps in float, with table values held in double rounded once.  Reductions,
+// gauge factors and real-time phase factors stay in FP64 in the FP32 form.
 // ---------------------------------------------------------------------------
-// The operator arithmetic runs in the working precision T: FP64 sweeps in
-// double; FP32 sweeps in float, with the table values (held in double) rounded
-// once at load.  Only the reductions stay in FP64 in the FP32 form.
+// Marks loaded values as needed from here on.  Without it the compiler moves their
+// first arithmetic up to the loads (a sum of two table values next to them), and its
+// wait stands in front of every later load.
+template <typename U>
+__device__ __forceinline__ void arrive(U& x) { asm volatile("" : "+v"(x)); }
+template <typename U>
+__device__ __forceinline__ void arrive(cx<U>& x) {
+  arrive(x.x);
+  arrive(x.y);
+}
 
-// psi * exp(-arg) (imaginary time) or psi * exp(-i arg) (real time), times s
-// X (FP32 real-time kernels only): the phase factor is formed in FP32, then its
-// modulus is corrected in FP64 by one Newton step towards 1/sqrt(c^2 + s^2),
-// and the product is formed in FP64 and rounded to FP32 once.  A factor
-// rounded to FP32 carries a modulus error of ~1e-7 that is the same at every
-// step for static V, A and K, so the norm and energy would drift linearly with
-// the steps; after the Newton step the modulus is 1 within ~1e-14, and what is
-// left (the FP32 phase, ~1e-7 relative) acts like a rounded V and does not grow.
-// Separate kernels, so the imaginary-time ones keep their registers.
-template <typename T, int E, bool X = false>
-__device__ __forceinline__ void apply_phase_all(cx<T>* v, const T (&arg)[E], int gstate, double s_) {
-  const T s = (T)s_;
-  // FP64: a lane whose arguments are all small takes the short polynomials
-  bool tiny = false;
-  if constexpr (sizeof(T) == 8) {
-    tiny = true;
+// A scaled point.  FP32 rounds the product here: contracted into the butterfly that
+// follows it, results would depend on what the compiler sees next to each other.
+template <typename T>
+__device__ __forceinline__ cx<T> scaled(cx<T> v, T s) {
+  cx<T> r = cscale(v, s);
+  if constexpr (sizeof(T) == 4) arrive(r);
+  return r;
+}
+
+// A line of N points along axis ax: element e at flat index base + e*es; i0, i1:
+// the indices on the other two axes, in ascending order.  The lane holds points
+// tid + bpos(0, r).
+struct LineAt {
+  int ax, tid;
+  long base, es;
+  int i0, i1;
+  __device__ __forceinline__ int o0() const { return ax == 0 ? 1 : 0; }
+  __device__ __forceinline__ int o1() const { return ax == 2 ? 1 : 2; }
+};
+
+template <typename T>
+struct VTab;
+template <>
+struct VTab<double> {
+  static __device__ __forceinline__ const double* get(const Phys& p, int a) { return pick(a, p.vs[0], p.vs[1], p.vs[2]); }
+};
+template <>
+struct VTab<float> {
+  static __device__ __forceinline__ const float* get(const Phys& p, int a) { return pick(a, p.vsf[0], p.vsf[1], p.vsf[2]); }
+};
+
+// The sincos of E arguments that may need the library (huge, infinite, NaN): one
+// point at a time, the arrays rotating through their first slot, so that the kernel
+// holds one copy of the library code instead of E (they made up most of a sweep's
+// 36-107 KB) and no array is indexed by a variable.
+template <typename T, int E>
+__device__ __forceinline__ void sincos_any(T (&x)[E], T (&sn)[E], T (&cs)[E]) {
 #pragma unroll
-    for (int r = 0; r < E; ++r) tiny = tiny && fabs(arg[r]) <= SMALL_ARG;
+  for (int r = 0; r < E; ++r) sn[r] = cs[r] = (T)0;
+#pragma unroll 1
+  for (int k = 0; k < E; ++k) {
+    T s, c;
+    WMath<T>::sc(x[0], &s, &c);
+#pragma unroll
+    for (int r = 0; r + 1 < E; ++r) {
+      x[r] = x[r + 1];
+      sn[r] = sn[r + 1];
+      cs[r] = cs[r + 1];
+    }
+    sn[E - 1] = s;
+    cs[E - 1] = c;
   }
-  if (gstate == 0) {
+}
+
+// psi * exp(-arg) (imaginary time) or psi * exp(-i arg) (REAL), times s.
+// FP64: a lane whose arguments are all small takes the short polynomials.
+// FP32 real time: the phase factor is formed in FP32, then its modulus is
+// corrected in FP64 by one Newton step towards 1/sqrt(c^2 + s^2), and the
+// product is formed in FP64 and rounded to FP32 once.  A factor rounded to FP32
+// carries a modulus error of ~1e-7 that is the same at every step for static V,
+// A and K, so the norm and energy would drift linearly with the steps; after the
+// Newton step the modulus is 1 within ~1e-14, and what is left (the FP32 phase,
+// ~1e-7 relative) acts like a rounded V and does not grow.
+template <typename T, int E, bool REAL>
+__device__ __forceinline__ void apply_phase_all(cx<T>* v, const T (&arg)[E], double s_) {
+  const T s = (T)s_;
+  if constexpr (!REAL) {
     if constexpr (sizeof(T) == 8) {
+      bool tiny = true;
+#pragma unroll
+      for (int r = 0; r < E; ++r) tiny = tiny && fabs(arg[r]) <= SMALL_ARG;
       if (tiny) {
 #pragma unroll
         for (int r = 0; r < E; ++r) v[r] = cscale(v[r], exp_small(-arg[r]) * s);
@@ -367,351 +431,271 @@ __device__ __forceinline__ void apply_phase_all(cx<T>* v, const T (&arg)[E], int
       }
     }
 #pragma unroll
-    for (int r = 0; r < E; ++r) {
-      const T f = WMath<T>::ex(-arg[r]) * s;
-      v[r] = cscale(v[r], f);
-    }
-  } else if constexpr (X && sizeof(T) == 4) {
+    for (int r = 0; r < E; ++r) v[r] = scaled(v[r], WMath<T>::ex(-arg[r]) * s);
+  } else {
+    // one range check for the lane's E arguments, then branch-free forms
+    T x[E], sn[E], cs[E];
     bool small = true, fast = true;
 #pragma unroll
     for (int r = 0; r < E; ++r) {
-      small = small && sincos_small_ok(-arg[r]);
-      fast = fast && sincos_fast_ok(-arg[r]);
+      x[r] = -arg[r];
+      small = small && (sizeof(T) == 8 ? fabs((double)x[r]) <= SMALL_ARG : sincos_small_ok(x[r]));
+      fast = fast && sincos_fast_ok(x[r]);
     }
-    float sn[E], cs[E];
     if (small) {
 #pragma unroll
-      for (int r = 0; r < E; ++r) sincos_poly(-arg[r], &sn[r], &cs[r]);
+      for (int r = 0; r < E; ++r) {
+        if constexpr (sizeof(T) == 8) sincos_small(x[r], &sn[r], &cs[r]);
+        else sincos_poly(x[r], &sn[r], &cs[r]);
+      }
     } else if (fast) {
 #pragma unroll
-      for (int r = 0; r < E; ++r) sincos_core(-arg[r], &sn[r], &cs[r]);
+      for (int r = 0; r < E; ++r) sincos_core(x[r], &sn[r], &cs[r]);
     } else {
-#pragma unroll
-      for (int r = 0; r < E; ++r) sincos_cw(-arg[r], &sn[r], &cs[r]);
+      sincos_any<T, E>(x, sn, cs);
     }
 #pragma unroll
     for (int r = 0; r < E; ++r) {
-      const double c0 = cs[r], d0 = sn[r];
-      const double f = fma(-0.5, fma(c0, c0, d0 * d0), 1.5) * s_;
-      const double c = c0 * f, d = d0 * f, x = v[r].x, y = v[r].y;
-      v[r] = mk((float)(c * x - d * y), (float)(c * y + d * x));
-    }
-  } else {
-    // one range check for the lane's E arguments, then branch-free cores; a
-    // real-time phase is usually within pi/4 (no reduction needed)
-    bool small = true, fast = true;
-#pragma unroll
-    for (int r = 0; r < E; ++r) {
-      small = small && WMath<T>::sc_small_ok(-arg[r]);
-      fast = fast && WMath<T>::sc_ok(-arg[r]);
-    }
-    T sn[E], cs[E];
-    if constexpr (sizeof(T) == 8) {
-      if (tiny) {
-#pragma unroll
-        for (int r = 0; r < E; ++r) sincos_small(-arg[r], &sn[r], &cs[r]);
-#pragma unroll
-        for (int r = 0; r < E; ++r) v[r] = cmul(mk(cs[r] * s, sn[r] * s), v[r]);
-        return;
+      if constexpr (sizeof(T) == 8) {
+        v[r] = cmul(mk(cs[r] * s, sn[r] * s), v[r]);
+      } else {
+        const double c0 = cs[r], d0 = sn[r];
+        const double f = fma(-0.5, fma(c0, c0, d0 * d0), 1.5) * s_;
+        const double c = c0 * f, d = d0 * f, vx = v[r].x, vy = v[r].y;
+        v[r] = mk((float)(c * vx - d * vy), (float)(c * vy + d * vx));
       }
     }
-    if (small) {
-#pragma unroll
-      for (int r = 0; r < E; ++r) WMath<T>::sc_small(-arg[r], &sn[r], &cs[r]);
-    } else if (fast) {
-#pragma unroll
-      for (int r = 0; r < E; ++r) WMath<T>::sc_core(-arg[r], &sn[r], &cs[r]);
-    } else {
-#pragma unroll
-      for (int r = 0; r < E; ++r) WMath<T>::sc(-arg[r], &sn[r], &cs[r]);
-    }
-#pragma unroll
-    for (int r = 0; r < E; ++r) v[r] = cmul(mk(cs[r] * s, sn[r] * s), v[r]);
   }
 }
 
 // V/2 with the nonlinear density term: cMultDensity (src/kernels.cu:365-388)
 // with GV/EV (src/operators.cu:1081,1100) merged into one exponential.
-// In two parts: halfV_vargs gathers V*cV of the lane's points, halfV_apply
-// adds the density term and applies the phase (halfV_all does both in a row).
-template <typename T, int E, typename F>
-__device__ __forceinline__ void halfV_vargs(const Phys& p, const double* __restrict__ Vt, F pos, T (&arg)[E]) {
-  if (p.v_kind == V_SEP) {
+template <typename T, int N, int TPL, int R, int E>
+struct VOp {
+  T e[E], f0, f1;   // V = e + (f0 + f1): the line's own axis and the other two; a table: e
+  // no branch joins around the FP64 loads and f0, f1: a join copies registers, which
+  // waits for the values there
+  __device__ __forceinline__ void load(const Phys& p, const double* __restrict__ Vt, const LineAt& l) {
+    const bool sep = p.v_kind == V_SEP;
+    f0 = VTab<T>::get(p, l.o0())[l.i0];
+    f1 = VTab<T>::get(p, l.o1())[l.i1];
+    const double* vt = Vt + l.base + (long)l.tid * l.es;
+    if constexpr (sizeof(T) == 8) {
+      const double* ve = sep ? VTab<T>::get(p, l.ax) + l.tid : vt;
+      const long es = sep ? 1 : l.es;
 #pragma unroll
-    for (int r = 0; r < E; ++r) {
-      const Pt q = pos(r);
-      if constexpr (sizeof(T) == 4)
-        arg[r] = p.vsf[0][q.x] + p.vsf[1][q.y] + p.vsf[2][q.z];
-      else
-        arg[r] = p.vs[0][q.x] + p.vs[1][q.y] + p.vs[2][q.z];
-    }
-  } else {
+      for (int r = 0; r < E; ++r) e[r] = ve[bpos<N, TPL, R>(0, r) * es];
+    } else if (sep) {
+      const T* ve = VTab<T>::get(p, l.ax) + l.tid;
 #pragma unroll
-    for (int r = 0; r < E; ++r) {
-      const Pt q = pos(r);
-      arg[r] = (T)Vt[gid_of(p, q.x, q.y, q.z)];
-    }
-  }
-  const T cV = (T)p.cV;
-#pragma unroll
-  for (int r = 0; r < E; ++r) arg[r] = arg[r] * cV;
-}
-
-template <typename T, int E, bool X = false>
-__device__ __forceinline__ void halfV_apply(const Phys& p, cx<T>* v, T (&arg)[E]) {
-  if (p.gpe) {
-    const T g = (T)p.g, cH = (T)p.cH;
-#pragma unroll
-    for (int r = 0; r < E; ++r) {
-      const T d = v[r].x * v[r].x + v[r].y * v[r].y;
-      arg[r] += g * d * cH;
-    }
-  }
-  apply_phase_all<T, E, X>(v, arg, p.gstate, 1.0);
-}
-
-template <typename T, int E, bool X = false, typename F>
-__device__ __forceinline__ void halfV_all(const Phys& p, const double* __restrict__ Vt, cx<T>* v, F pos) {
-  T arg[E];
-  halfV_vargs<T, E>(p, Vt, pos, arg);
-  halfV_apply<T, E, X>(p, v, arg);
-}
-
-// gauge operator along AXIS: GpA*/EpA* (src/operators.cu:1089-1110) with both
-// 1/sqrt(n) of the axis transforms folded into invn.  gauge_args gathers the
-// exponents A*k*Dt of the lane's points; apply_phase_all applies the phase.
-template <typename T, int E, int AXIS, typename F>
-__device__ __forceinline__ void gauge_args(const Phys& p, F pos, T (&arg)[E]) {
-  if (p.a_kind == A_TABLE) {
-#pragma unroll
-    for (int r = 0; r < E; ++r) {
-      const Pt q = pos(r);
-      arg[r] = (T)p.At[AXIS][gid_of(p, q.x, q.y, q.z)];
-    }
-  } else {
-#pragma unroll
-    for (int r = 0; r < E; ++r) {
-      const Pt q = pos(r);
-      double A = 0.0;   // A_ZERO, and A_z of the rotation
-      if (p.a_kind == A_ROTATION) {
-        if constexpr (AXIS == 0) A = -p.yg[q.y] * p.omega * p.omegaX;
-        if constexpr (AXIS == 1) A = p.xg[q.x] * p.omega * p.omegaY;
-      }
-      arg[r] = (T)A;
-    }
-  }
-  const T Dt = (T)p.Dt;
-#pragma unroll
-  for (int r = 0; r < E; ++r) {
-    const Pt q = pos(r);
-    const T k = (T)(AXIS == 0 ? p.pxg[q.x] : AXIS == 1 ? p.pyg[q.y] : p.pzg[q.z]);
-    arg[r] = arg[r] * k * Dt;
-  }
-}
-
-template <typename T, int E, int AXIS, bool X = false, typename F>
-__device__ __forceinline__ void gauge_all(const Phys& p, cx<T>* v, F pos, double invn) {
-  T arg[E];
-  gauge_args<T, E, AXIS>(p, pos, arg);
-  apply_phase_all<T, E, X>(v, arg, p.gstate, invn);
-}
-
-// The rotation gauge on a line along AXIS (x: A_x = -y omega omegaX; y:
-// A_y = x omega omegaY; both constant along the line) multiplies the point of
-// signed wave-number index m by exp(-a m) (imaginary time) or exp(-i a m) (real
-// time), a = A dk Dt, dk = k[1].  In the boundary layout of radix R a lane holds
-// the points tid + TPL q + (N/R) s (r = q R + s), less N from the Nyquist index
-// on, so the E factors are products of four per-lane factors and their powers:
-// exp(-a tid), exp(-a N/R), exp(-a TPL) and exp(a N), i.e. three or four
-// exponentials per lane instead of E (each product adds a rounding: a few ulp).
-// FP64 kernels only; false (nothing applied) for other gauges, for FP32, or when
-// |a| N is large enough for exp(a N) to leave the double range.
-template <typename T, int N, int TPL, int R, int E, int AXIS, bool X>
-__device__ __forceinline__ bool gauge_rot_lin(const Phys& p, cx<T>* v, int tid, int other, double invn) {
-  if constexpr (sizeof(T) != 8 || X || AXIS == 2) {
-    return false;
-  } else {
-    if (p.a_kind != A_ROTATION) return false;
-    const double A = AXIS == 0 ? -p.yg[other] * p.omega * p.omegaX : p.xg[other] * p.omega * p.omegaY;
-    const double dk = AXIS == 0 ? p.pxg[1] : p.pyg[1];
-    const double a = A * dk * p.Dt;
-    if (!(fabs(a) * N <= 600.0)) return false;
-    constexpr int Q = E / R, NR = N / R;
-    if (p.gstate == 0) {
-      double w[R];
-      w[0] = WMath<double>::ex(-a * tid) * invn;
-      const double W = WMath<double>::ex(-a * NR), Z = WMath<double>::ex(a * N);
-      const double U = Q > 1 ? WMath<double>::ex(-a * TPL) : 1.0;
-#pragma unroll
-      for (int k = 1; k < R; ++k) w[k] = w[k - 1] * W;
-#pragma unroll
-      for (int q = 0; q < Q; ++q) {
-#pragma unroll
-        for (int k = 0; k < R; ++k) {
-          const int r = q * R + k;
-          const double f = (tid + TPL * q + NR * k >= N / 2) ? w[k] * Z : w[k];
-          v[r] = cscale(v[r], f);
-        }
-        if (q + 1 < Q) {
-#pragma unroll
-          for (int k = 0; k < R; ++k) w[k] *= U;
-        }
-      }
+      for (int r = 0; r < E; ++r) e[r] = ve[bpos<N, TPL, R>(0, r)];
     } else {
-      // exp(-i x) = (cos x, -sin x)
-      auto ph = [](double x) {
+#pragma unroll
+      for (int r = 0; r < E; ++r) e[r] = (T)vt[bpos<N, TPL, R>(0, r) * l.es];
+    }
+  }
+  __device__ __forceinline__ void ready() {
+    arrive(f0);
+    arrive(f1);
+#pragma unroll
+    for (int r = 0; r < E; ++r) arrive(e[r]);
+  }
+  // exponents of the half step on v.  FP32 adds the axes in the order x, y, z.
+  __device__ __forceinline__ void args(const Phys& p, const LineAt& l, const cx<T>* v, T (&arg)[E]) const {
+    const T cV = (T)p.cV;
+    if constexpr (sizeof(T) == 8) {
+      const T f = p.v_kind == V_SEP ? f0 + f1 : (T)0;
+#pragma unroll
+      for (int r = 0; r < E; ++r) arg[r] = (e[r] + f) * cV;
+    } else if (p.v_kind == V_SEP) {
+#pragma unroll
+      for (int r = 0; r < E; ++r) arg[r] = (l.ax == 2 ? (f0 + f1) + e[r] : (e[r] + f0) + f1) * cV;
+    } else {
+#pragma unroll
+      for (int r = 0; r < E; ++r) arg[r] = e[r] * cV;
+    }
+    if (p.gpe) {
+      const T g = (T)p.g, cH = (T)p.cH;
+#pragma unroll
+      for (int r = 0; r < E; ++r) {
+        if constexpr (sizeof(T) == 4) arrive(arg[r]);   // rounded before the sum
+        const T d = v[r].x * v[r].x + v[r].y * v[r].y;
+        arg[r] += g * d * cH;
+      }
+    }
+  }
+  template <bool REAL>
+  __device__ __forceinline__ void half(const Phys& p, const LineAt& l, cx<T>* v) const {
+    T arg[E];
+    args(p, l, v, arg);
+    apply_phase_all<T, E, REAL>(v, arg, 1.0);
+  }
+};
+
+// The gauge operator along the line's axis: GpA*/EpA* (src/operators.cu:1089-1110)
+// with both 1/sqrt(n) of the axis transforms folded into invn.
+//
+// The rotation gauge on a line along x (A_x = -y omega omegaX) or y (A_y = x omega
+// omegaY) is constant along the line, so the point of signed wave-number index m
+// is multiplied by exp(-a m) (imaginary time) or exp(-i a m) (real time), a = A dk
+// Dt, dk = k[1].  In the boundary layout of radix R a lane holds the points
+// tid + TPL q + (N/R) s (r = q R + s), less N from the Nyquist index on, so the E
+// factors are products of four per-lane factors and their powers: exp(-a tid),
+// exp(-a N/R), exp(-a TPL) and exp(a N), i.e. three or four exponentials per lane
+// instead of E (each product adds a rounding: a few ulp).  Other gauges, FP32, or an
+// |a| N large enough for exp(a N) to leave the double range take E exponentials.
+template <typename T, int N, int TPL, int R, int E, bool REAL>
+struct GOp {
+  static constexpr int Q = E / R, NR = N / R;
+  static constexpr bool LIN = sizeof(T) == 8;
+  double A, dk;
+  bool lin;
+  cx<double> b, W, U, Z;   // imaginary time: real factors, in .x
+  T at[E], kk[E];          // not lin: A and k of the points
+  __device__ __forceinline__ void load_points(const Phys& p, const LineAt& l) {
+    const double* kt = pick(l.ax, p.pxg, p.pyg, p.pzg) + l.tid;
+    const double* ap = pick(l.ax, p.At[0], p.At[1], p.At[2]) + l.base + (long)l.tid * l.es;
+#pragma unroll
+    for (int r = 0; r < E; ++r) kk[r] = (T)kt[bpos<N, TPL, R>(0, r)];
+    if (p.a_kind == A_TABLE) {
+#pragma unroll
+      for (int r = 0; r < E; ++r) at[r] = (T)ap[bpos<N, TPL, R>(0, r) * l.es];
+    }
+  }
+  __device__ __forceinline__ void load(const Phys& p, const LineAt& l) {
+    A = pick(l.ax, p.yg, p.xg, p.xg)[l.i0];   // the rotation's coordinate (A_z = 0)
+    dk = pick(l.ax, p.pxg, p.pyg, p.pzg)[1];
+  }
+  __device__ __forceinline__ void prep(const Phys& p, const LineAt& l, double invn) {
+    A = A * pick(l.ax, -p.omega, p.omega, p.omega) * pick(l.ax, p.omegaX, p.omegaY, p.omegaY);
+    A = p.a_kind == A_ROTATION && l.ax < 2 ? A : 0.0;
+    const double a = A * dk * p.Dt;
+    lin = LIN && p.a_kind != A_TABLE && fabs(a) * N <= 600.0;
+    if constexpr (!LIN) return;
+    if constexpr (!REAL) {
+      b.x = exp_cw(-a * l.tid) * invn;
+      W.x = exp_cw(-a * NR);
+      Z.x = exp_cw(a * N);
+      if constexpr (Q > 1) U.x = exp_cw(-a * TPL);
+    } else {
+      auto ph = [](double x) {   // exp(-i x)
         double sn, cs;
-        WMath<double>::sc(x, &sn, &cs);
+        sincos_core(x, &sn, &cs);
         return mk(cs, -sn);
       };
-      cx<double> w[R];
-      const cx<double> b = ph(a * tid);
-      w[0] = mk(b.x * invn, b.y * invn);
-      const cx<double> W = ph(a * NR), Zc = ph(a * N);
-      const cx<double> Z = mk(Zc.x, -Zc.y);   // exp(+i a N)
-      const cx<double> U = Q > 1 ? ph(a * TPL) : mk(1.0, 0.0);
+      const cx<double> b0 = ph(a * l.tid);
+      b = mk(b0.x * invn, b0.y * invn);
+      W = ph(a * NR);
+      Z = ph(-a * N);
+      if constexpr (Q > 1) U = ph(a * TPL);
+    }
+  }
+  __device__ __forceinline__ void apply_lin(cx<T>* v, const LineAt& l) const {
+    cx<double> w[R];
+    w[0] = b;
 #pragma unroll
-      for (int k = 1; k < R; ++k) w[k] = cmul(w[k - 1], W);
+    for (int k = 1; k < R; ++k) {
+      if constexpr (REAL) w[k] = cmul(w[k - 1], W);
+      else w[k].x = w[k - 1].x * W.x;
+    }
 #pragma unroll
-      for (int q = 0; q < Q; ++q) {
+    for (int q = 0; q < Q; ++q) {
+#pragma unroll
+      for (int k = 0; k < R; ++k) {
+        const int r = q * R + k;
+        const bool wrap = l.tid + TPL * q + NR * k >= N / 2;
+        if constexpr (REAL) v[r] = cmul(wrap ? cmul(w[k], Z) : w[k], v[r]);
+        else v[r] = cscale(v[r], wrap ? w[k].x * Z.x : w[k].x);
+      }
+      if (q + 1 < Q) {
 #pragma unroll
         for (int k = 0; k < R; ++k) {
-          const int r = q * R + k;
-          const cx<double> f = (tid + TPL * q + NR * k >= N / 2) ? cmul(w[k], Z) : w[k];
-          v[r] = cmul(f, v[r]);
-        }
-        if (q + 1 < Q) {
-#pragma unroll
-          for (int k = 0; k < R; ++k) w[k] = cmul(w[k], U);
+          if constexpr (REAL) w[k] = cmul(w[k], U);
+          else w[k].x *= U.x;
         }
       }
     }
-    return true;
   }
-}
-
-// Per-axis K factor table in the working precision.
-template <typename T>
-struct KTab {
-  static __device__ __forceinline__ const double* get(const Phys& p, int a) { return p.kf[a]; }
-};
-template <>
-struct KTab<float> {
-  static __device__ __forceinline__ const float* get(const Phys& p, int a) { return p.kff[a]; }
+  // `early`: load_points() was called up front where A is a table
+  __device__ __forceinline__ void apply(const Phys& p, cx<T>* v, const LineAt& l, double invn, bool early) {
+    if constexpr (LIN) {
+      if (lin) {
+        apply_lin(v, l);
+        return;
+      }
+    }
+    if (!(early && p.a_kind == A_TABLE)) load_points(p, l);
+    T arg[E];
+    const T Dt = (T)p.Dt;
+#pragma unroll
+    for (int r = 0; r < E; ++r) arg[r] = (p.a_kind == A_TABLE ? at[r] : (T)A) * kk[r] * Dt;
+    apply_phase_all<T, E, REAL>(v, arg, invn);
+  }
 };
 
 // K step: GK/EK (src/operators.cu:1082,1102) with both 1/sqrt(N) of
 // src/evolution.cu:761,777 folded into invN.  For the separable K the operator
-// is the product of per-axis factors (no transcendental per point).
-template <typename T, int E, bool X = false, typename F>
-__device__ __forceinline__ void kstep_all(const Phys& p, cx<T>* v, F pos, double invN_) {
-  const T invN = (T)invN_;
-  if constexpr (X && sizeof(T) == 4) {
-    if (p.k_kind == K_SEP && p.gstate != 0) {
-      // factor from the FP64 tables, product in FP64 (see apply_phase_all)
-#pragma unroll
-      for (int r = 0; r < E; ++r) {
-        const Pt q = pos(r);
-        const double* gx = p.kf[0] + 2 * q.x;
-        const double* gy = p.kf[1] + 2 * q.y;
-        const double* gz = p.kf[2] + 2 * q.z;
-        const double ar = gx[0] * gy[0] - gx[1] * gy[1], ai = gx[0] * gy[1] + gx[1] * gy[0];
-        const double br = (ar * gz[0] - ai * gz[1]) * invN_, bi = (ar * gz[1] + ai * gz[0]) * invN_;
-        const double x = v[r].x, y = v[r].y;
-        v[r] = mk((T)(br * x - bi * y), (T)(br * y + bi * x));
-      }
-      return;
-    }
+// is the product of per-axis factors (no transcendental per point): the other
+// two axes' product times the line's own.  FP32 real time reads the FP64 tables
+// and forms the product in FP64 (see apply_phase_all).
+template <typename T, int N, int TPL, int R, int E, bool REAL>
+struct KOp {
+  using F = typename std::conditional<REAL, double, T>::type;
+  cx<F> e[E], f0, f1;   // imaginary time: real factors, in .x; K tables: K itself in e.x
+  static __device__ __forceinline__ const F* tab(const Phys& p, int a) {
+    if constexpr (sizeof(F) == 4) return pick(a, p.kff[0], p.kff[1], p.kff[2]);
+    else return pick(a, p.kf[0], p.kf[1], p.kf[2]);
   }
-  if (p.k_kind == K_SEP) {
-    T f[E][6];
+  static __device__ __forceinline__ cx<F> one(const F* t, int i) {
+    return mk(t[2 * i], REAL ? t[2 * i + 1] : (F)0);
+  }
+  __device__ __forceinline__ void load(const Phys& p, const LineAt& l) {
+    f0 = one(tab(p, l.o0()), l.i0);
+    f1 = one(tab(p, l.o1()), l.i1);
+    if (p.k_kind == K_SEP) {
+      const F* t = tab(p, l.ax) + 2 * l.tid;
 #pragma unroll
-    for (int r = 0; r < E; ++r) {
-      const Pt q = pos(r);
-      const auto* fx = KTab<T>::get(p, 0) + 2 * q.x;
-      const auto* fy = KTab<T>::get(p, 1) + 2 * q.y;
-      const auto* fz = KTab<T>::get(p, 2) + 2 * q.z;
-      f[r][0] = (T)fx[0]; f[r][1] = (T)fx[1]; f[r][2] = (T)fy[0];
-      f[r][3] = (T)fy[1]; f[r][4] = (T)fz[0]; f[r][5] = (T)fz[1];
-    }
-    if (p.gstate == 0) {
-#pragma unroll
-      for (int r = 0; r < E; ++r) v[r] = cscale(v[r], f[r][0] * f[r][2] * f[r][4] * invN);
+      for (int r = 0; r < E; ++r) e[r] = one(t, bpos<N, TPL, R>(0, r));
     } else {
+      const double* kt = p.Kt + l.base + (long)l.tid * l.es;
 #pragma unroll
-      for (int r = 0; r < E; ++r) {
-        const T ar = f[r][0] * f[r][2] - f[r][1] * f[r][3], ai = f[r][0] * f[r][3] + f[r][1] * f[r][2];
-        const T br = (ar * f[r][4] - ai * f[r][5]) * invN, bi = (ar * f[r][5] + ai * f[r][4]) * invN;
-        v[r] = cmul(mk(br, bi), v[r]);
-      }
-    }
-    return;
-  }
-  T arg[E];
-  const T cK = (T)p.cK;
-#pragma unroll
-  for (int r = 0; r < E; ++r) {
-    const Pt q = pos(r);
-    arg[r] = (T)p.Kt[gid_of(p, q.x, q.y, q.z)] * cK;
-  }
-  apply_phase_all<T, E, X>(v, arg, p.gstate, invN_);
-}
-
-// K step on a strided line (axis AXIS = 1 or 2 varies along the line; x = xi
-// and the other coordinate o are fixed), separable K: the fixed axes' factors
-// are loaded once, only the varying axis' factor per point.  Same products as
-// kstep_all.
-template <typename T, int E, int AXIS>
-struct KCol {
-  T fx0, fx1, fo0, fo1, fe[E][2];
-  template <typename F>
-  __device__ __forceinline__ void load(const Phys& p, int xi, int o, F epos) {
-    const auto* fxp = KTab<T>::get(p, 0) + 2 * xi;
-    fx0 = (T)fxp[0];
-    fx1 = (T)fxp[1];
-    const auto* fop = KTab<T>::get(p, AXIS == 1 ? 2 : 1) + 2 * o;
-    fo0 = (T)fop[0];
-    fo1 = (T)fop[1];
-    const auto* fvp = KTab<T>::get(p, AXIS);
-#pragma unroll
-    for (int r = 0; r < E; ++r) {
-      const int e = epos(r);
-      fe[r][0] = (T)fvp[2 * e];
-      fe[r][1] = (T)fvp[2 * e + 1];
+      for (int r = 0; r < E; ++r) e[r] = mk((F)kt[bpos<N, TPL, R>(0, r) * l.es], (F)0);
     }
   }
-  __device__ __forceinline__ void apply(const Phys& p, cx<T>* v, double invN_) const {
-    const T invN = (T)invN_;
-    if (p.gstate == 0) {
+  __device__ __forceinline__ void ready() {
+    arrive(f0);
+    arrive(f1);
 #pragma unroll
-      for (int r = 0; r < E; ++r) {
-        const T fy0 = AXIS == 1 ? fe[r][0] : fo0, fz0 = AXIS == 1 ? fo0 : fe[r][0];
-        v[r] = cscale(v[r], fx0 * fy0 * fz0 * invN);
+    for (int r = 0; r < E; ++r) arrive(e[r]);
+  }
+  // FP32 imaginary time multiplies the axes' factors in the order x, y, z
+  __device__ __forceinline__ void apply(const Phys& p, const LineAt& l, cx<T>* v, double invN) const {
+    if (p.k_kind == K_SEP) {
+      if constexpr (REAL) {
+        const cx<double> f = cscale(cmul(f0, f1), invN);
+#pragma unroll
+        for (int r = 0; r < E; ++r) {
+          const cx<double> u = cmul(cmul(e[r], f), mk((double)v[r].x, (double)v[r].y));
+          v[r] = mk((T)u.x, (T)u.y);
+        }
+      } else if constexpr (sizeof(T) == 8) {
+        const T f = f0.x * f1.x * (T)invN;
+#pragma unroll
+        for (int r = 0; r < E; ++r) v[r] = cscale(v[r], e[r].x * f);
+      } else {
+#pragma unroll
+        for (int r = 0; r < E; ++r)
+          v[r] = scaled(v[r], (l.ax == 2 ? f0.x * f1.x * e[r].x : e[r].x * f0.x * f1.x) * (T)invN);
       }
     } else {
+      T arg[E];
+      const T cK = (T)p.cK;
 #pragma unroll
-      for (int r = 0; r < E; ++r) {
-        const T fy0 = AXIS == 1 ? fe[r][0] : fo0, fy1 = AXIS == 1 ? fe[r][1] : fo1;
-        const T fz0 = AXIS == 1 ? fo0 : fe[r][0], fz1 = AXIS == 1 ? fo1 : fe[r][1];
-        const T ar = fx0 * fy0 - fx1 * fy1, ai = fx0 * fy1 + fx1 * fy0;
-        const T br = (ar * fz0 - ai * fz1) * invN, bi = (ar * fz1 + ai * fz0) * invN;
-        v[r] = cmul(mk(br, bi), v[r]);
-      }
+      for (int r = 0; r < E; ++r) arg[r] = (T)e[r].x * cK;
+      apply_phase_all<T, E, REAL>(v, arg, invN);
     }
   }
 };
-
-template <typename T, int E, int AXIS, bool X = false, typename F>
-__device__ __forceinline__ void kstep_col(const Phys& p, cx<T>* v, int xi, int o, F epos, double invN_) {
-  if (p.k_kind != K_SEP || (X && sizeof(T) == 4 && p.gstate != 0)) {
-    kstep_all<T, E, X>(p, v, [&](int r) { const int e = epos(r); return AXIS == 1 ? Pt{xi, e, o} : Pt{xi, o, e}; },
-                           invN_);
-    return;
-  }
-  KCol<T, E, AXIS> kc;
-  kc.load(p, xi, o, epos);
-  kc.apply(p, v, invN_);
-}
 
 // ---------------------------------------------------------------------------
 // Deterministic two-stage reduction of NA doubles: every workgroup writes its
@@ -719,21 +703,49 @@ __device__ __forceinline__ void kstep_col(const Phys& p, cx<T>* v, int xi, int o
 // launched after it sums them in a fixed order.  The result is the same for
 // every run and independent of scheduling.
 // ---------------------------------------------------------------------------
+// Sum over the lanes of a wave (xor 1, 2, 4, 8 by DPP within rows of 16: once two
+// groups hold their own totals, mirroring pairs them as the xor would; 16 and 32 by
+// the row swaps), every lane gets it.  LDS-routed shuffles took ~130 cycles a level.
+template <int CTRL>
+__device__ __forceinline__ double dpp_move(double x) {
+  union { double d; int i[2]; } u, w;
+  u.d = x;
+  w.i[0] = __builtin_amdgcn_update_dpp(0, u.i[0], CTRL, 0xf, 0xf, false);
+  w.i[1] = __builtin_amdgcn_update_dpp(0, u.i[1], CTRL, 0xf, 0xf, false);
+  return w.d;
+}
+template <int ROW>
+__device__ __forceinline__ double row_swap_add(double x) {
+  union { double d; unsigned i[2]; } u, w0, w1;
+  u.d = x;
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    auto r = ROW == 16 ? __builtin_amdgcn_permlane16_swap(u.i[h], u.i[h], false, false)
+                       : __builtin_amdgcn_permlane32_swap(u.i[h], u.i[h], false, false);
+    w0.i[h] = r[0];
+    w1.i[h] = r[1];
+  }
+  return w0.d + w1.d;
+}
+__device__ __forceinline__ double wave_sum(double x, int width) {
+  x += dpp_move<0xB1>(x);    // quad_perm [1,0,3,2]
+  x += dpp_move<0x4E>(x);    // quad_perm [2,3,0,1]
+  x += dpp_move<0x141>(x);   // row_half_mirror
+  x += dpp_move<0x140>(x);   // row_mirror
+  if (width > 16) x = row_swap_add<16>(x);
+  if (width > 32) x = row_swap_add<32>(x);
+  return x;
+}
+
 template <int NA>
 __device__ __forceinline__ void block_sum(double (&v)[NA], double* sh /* >= NA * 16 */) {
   // a workgroup smaller than a wave (strided sweeps of 16- and 32-point lines
-  // with narrow tiles) has lanes past its end: the butterfly stays within the
-  // workgroup's lanes (the offsets not taken are >= blockDim.x)
-  const int wl = (int)blockDim.x;
+  // with narrow tiles) has lanes past its end: the sum stays within the
+  // workgroup's lanes
 #pragma unroll
-  for (int a = 0; a < NA; ++a) {
-    double x = v[a];
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1)
-      if (o < wl) x += __shfl_xor(x, o, 64);
-    v[a] = x;
-  }
+  for (int a = 0; a < NA; ++a) v[a] = wave_sum(v[a], (int)blockDim.x);
   const int w = threadIdx.x >> 6, nw = (blockDim.x + 63) >> 6;
+  if (nw == 1) return;   // every lane holds the total
   __syncthreads();
   if ((threadIdx.x & 63) == 0) {
 #pragma unroll
@@ -786,60 +798,60 @@ __device__ __forceinline__ double fin_sum8_at(const double* __restrict__ p, int 
 // The finalize block size for nb partials (launch_finalize).
 __host__ __device__ constexpr int fin_block(int nb) { return nb >= 4096 ? 1024 : 256; }
 
-// fin_sum_at(p, nb, t, 256) for the four lanes t = l + 64j (j < 4) of one
-// finalize block: in chunks of four consecutive elements per lane (k = 4c ..
-// 4c+3, element t + k*256; zero past nb), all sixteen loads of a chunk first,
-// then the same additions in the same order: a chunk is one iteration of the
-// first loop while t + (4c+3)*256 < nb (monotone in c), else its elements go
-// one by one into s0 as the second loop takes them (adding an exact zero
-// changes nothing).
-__device__ __forceinline__ void fin_sum4(const double* __restrict__ p, int nb, int l, double (&out)[4]) {
-  constexpr int B = 256;
-  double s[4][4] = {};
-  const int nch = (nb + 4 * B - 1) / (4 * B);
-  for (int c = 0; c < nch; ++c) {
-    double v[4][4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int i = l + 64 * j + (4 * c + q) * B;
-        v[j][q] = i < nb ? p[i] : 0.0;
-      }
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      if (l + 64 * j + (4 * c + 3) * B < nb) {
-#pragma unroll
-        for (int q = 0; q < 4; ++q) s[j][q] += v[j][q];
-      } else {
-#pragma unroll
-        for (int q = 0; q < 4; ++q) s[j][0] += v[j][q];
-      }
-    }
-  }
-#pragma unroll
-  for (int j = 0; j < 4; ++j) out[j] = (s[j][0] + s[j][1]) + (s[j][2] + s[j][3]);
-}
-
 // The parSum norm sqrt(sum * scale) of nb < 4096 partials, computed by one full
 // wave (every lane gets it; the host defers a norm only to sweeps whose
 // workgroups are whole waves) with the additions of k_finalize in its 256-lane
-// form, bit for bit: lane l stands for finalize lanes l + 64j (j < 4); each j
-// is one finalize wave, reduced by the same xor butterfly as block_sum (the
-// four run interleaved), and the four wave totals are added in order.
-__device__ __forceinline__ double part_norm(const double* __restrict__ p, int nb, double scale) {
-  const int l = threadIdx.x & 63;
-  double x[4];
-  fin_sum4(p, nb, l, x);
+// form, bit for bit.  Lane l stands for the finalize lanes t = l + 64j (j < 4): in
+// chunks of four consecutive elements per t (element t + (4c+q)*256, zero past
+// nb), a chunk is one iteration of fin_sum_at's first loop while t + (4c+3)*256 <
+// nb, else its elements go one by one into its s0, as the second loop takes them
+// (adding an exact zero changes nothing).  Each j is one finalize wave, reduced by
+// the same wave_sum, and the four wave totals are added in order.
+// load() issues the first chunk (1024 partials: all of them for most sweeps), so
+// that they are on their way before psi; indices are clamped, not branched on.
+struct PartNorm {
+  double v[4][4];
+  static __device__ __forceinline__ void chunk(const double* __restrict__ p, int nb, int c, double (&v)[4][4]) {
+    const int l = threadIdx.x & 63;
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1)
+    for (int q = 0; q < 4; ++q) {
+      const int e = (4 * c + q) * 256;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) x[j] += __shfl_xor(x[j], o, 64);
-  double tot = 0.0;
+      for (int j = 0; j < 4; ++j) {
+        const int i = e + l + 64 * j;
+        v[j][q] = p[i < nb ? i : nb - 1];
+      }
+    }
+  }
+  __device__ __forceinline__ void load(const double* __restrict__ p, int nb) { chunk(p, nb, 0, v); }
+  __device__ __forceinline__ double norm(const double* __restrict__ p, int nb, double scale) {
+    const int l = threadIdx.x & 63;
 #pragma unroll
-  for (int j = 0; j < 4; ++j) tot += x[j];
-  return sqrt(tot * scale);
-}
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) arrive(v[j][q]);
+    double s[4][4] = {};
+    const int nch = (nb + 1023) / 1024;
+    for (int c = 0; c < nch; ++c) {
+      if (c > 0) chunk(p, nb, c, v);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int i = 4 * c * 256 + l + 64 * j;
+        if (i + 3 * 256 < nb) {
+#pragma unroll
+          for (int q = 0; q < 4; ++q) s[j][q] += v[j][q];
+        } else {
+#pragma unroll
+          for (int q = 0; q < 4; ++q) s[j][0] += i + q * 256 < nb ? v[j][q] : 0.0;
+        }
+      }
+    }
+    double tot = 0.0;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) tot += wave_sum((s[j][0] + s[j][1]) + (s[j][2] + s[j][3]), 64);
+    return sqrt(tot * scale);
+  }
+};
 
 // Block b of nb (of one problem) stores its NA partial sums.
 template <int NA>
