@@ -361,10 +361,9 @@ static int default_variant(const gpue_ctx* c, int axis) {
   return axis == 0 ? (small ? 3 : 0) : (small ? 5 : 0);
 }
 
-gpue_status gpue::launch(gpue_ctx* c, const Sweep& s, const Phys& ph, const void* in, void* out) {
+static gpue_status sweep_args(gpue_ctx* c, const Sweep& s, const Phys& ph, const void* in, void* out, SweepArgs& a) {
   const int n = c->dims[s.axis];
   const int var = s.var >= 0 ? s.var : c->var[s.axis];
-  SweepArgs a;
   std::memset(&a, 0, sizeof(a));
   a.active = 1;
   a.in = in;
@@ -384,6 +383,17 @@ gpue_status gpue::launch(gpue_ctx* c, const Sweep& s, const Phys& ph, const void
     a.norm_nb = s.part_nb;
     a.norm_scale = c->d[0] * c->d[1] * c->d[2];
     a.norm_out = c->results + 0;
+  }
+  return GPUE_OK;
+}
+
+gpue_status gpue::launch(gpue_ctx* c, const Sweep& s, const Phys& ph, const void* in, void* out) {
+  const int n = c->dims[s.axis];
+  const int var = s.var >= 0 ? s.var : c->var[s.axis];
+  SweepArgs a;
+  {
+    const gpue_status st = sweep_args(c, s, ph, in, out, a);
+    if (st != GPUE_OK) return st;
   }
   int slot = -1;
   if (c->timing) {
@@ -1537,6 +1547,34 @@ static int block_len(const gpue_ctx* c, int first_step, int nsteps, int s, int e
   return L >= 2 ? L : 0;
 }
 
+// 1D: steps of an evolve call, from step s on, that run as one launch (line_steps);
+// 0: the step is launched on its own (fields that depend on time or ramp, kernel
+// timing).  A run ends with the next energy evaluation, the call, or 4096 steps (a
+// few milliseconds: no launch holds the device for long).
+static int line_len(const gpue_ctx* c, int first_step, int nsteps, int s, int energy_every) {
+  if (c->p.dimnum != 1 || c->graph_steps <= 0 || c->timing || c->t_dep || c->ramp_type) return 0;
+  const int i = first_step + s;
+  int L = std::min(nsteps - s, 4096);
+  if (energy_every > 0) L = std::min(L, ((i + energy_every - 1) / energy_every) * energy_every - i + 1);
+  return L;
+}
+
+// L steps of a 1D problem from the present psi (scaled by the norm slot, which holds
+// the pending norm or 1.0, in imaginary time).
+static gpue_status launch_steps_1d(gpue_ctx* c, int gstate, int L) {
+  std::vector<Sweep> sched;
+  schedule(c, gstate, 0, gstate == 0, sched);
+  SweepArgs a;
+  gpue_status st = sweep_args(c, sched[0], make_phys(c, gstate, 0), c->psi, c->psi, a);
+  if (st != GPUE_OK) return st;
+  a.norm_scale = c->d[0] * c->d[1] * c->d[2];
+  a.norm_out = c->results + 0;
+  bool handled = false;
+  const hipError_t e = launch_line(c->prec, c->dims[0], c->var[0] & 1, a, L, c->stream, &handled);
+  if (!handled) return fail(c, GPUE_EUNSUPPORTED, "no line kernel for n=" + std::to_string(c->dims[0]));
+  return e == hipSuccess ? GPUE_OK : fail(c, GPUE_EHIP, std::string("line launch: ") + hipGetErrorString(e));
+}
+
 static gpue_status evolve_impl(gpue_ctx* c, int first_step, int nsteps, int gstate, int energy_every,
                                double energy_thr, double* energies, int max_energies, gpue_evolve_result* res,
                                bool check_norm) {
@@ -1557,8 +1595,9 @@ static gpue_status evolve_impl(gpue_ctx* c, int first_step, int nsteps, int gsta
   // imaginary-time graph always rescales on entry (results[0] holds the
   // pending norm or 1.0, and x*1.0 is exact)
   for (s = 0; s < nsteps; ++s) {
-    const int i = first_step + s;
-    const int L = block_len(c, first_step, nsteps, s, energy_every);
+    int i = first_step + s;
+    const int L1 = line_len(c, first_step, nsteps, s, energy_every);
+    const int L = L1 > 0 ? 0 : block_len(c, first_step, nsteps, s, energy_every);
     if (L > 0) {
       StepGraph* sg = nullptr;
       gpue_status st = step_graph(c, gstate, L, &sg);
@@ -1575,36 +1614,45 @@ static gpue_status evolve_impl(gpue_ctx* c, int first_step, int nsteps, int gsta
       s += L - 1;
       continue;
     }
-    Phys ph = make_phys(c, gstate, i);
-    if (c->ramp_type) ph.Dt = Dt * ramp_scale(c, i);
-    c->t_last = Dt * i;
-    schedule(c, gstate, i, c->pending_norm, sched);
-    if (c->defer_nb > 0) {   // the previous step left its norm partials to this one
-      if (takes_deferred_norm(c, sched[0]) && (sched[0].flags & F_SCALE_IN)) {
-        sched[0].flags |= F_SCALE_PART;
-        sched[0].part_nb = c->defer_nb;
-        c->defer_nb = 0;
-      } else {
-        gpue_status st = settle_deferred(c);
+    if (L1 > 0) {
+      gpue_status st = launch_steps_1d(c, gstate, L1);
+      if (st != GPUE_OK) return st;
+      s += L1 - 1;
+      i += L1 - 1;
+      c->t_last = Dt * i;
+      if (gstate == 0) c->pending_norm = true;
+    } else {
+      Phys ph = make_phys(c, gstate, i);
+      if (c->ramp_type) ph.Dt = Dt * ramp_scale(c, i);
+      c->t_last = Dt * i;
+      schedule(c, gstate, i, c->pending_norm, sched);
+      if (c->defer_nb > 0) {   // the previous step left its norm partials to this one
+        if (takes_deferred_norm(c, sched[0]) && (sched[0].flags & F_SCALE_IN)) {
+          sched[0].flags |= F_SCALE_PART;
+          sched[0].part_nb = c->defer_nb;
+          c->defer_nb = 0;
+        } else {
+          gpue_status st = settle_deferred(c);
+          if (st != GPUE_OK) return st;
+        }
+      }
+      // leave this step's norm to the next one when that is an eager step too
+      if (gstate == 0 && c->p.dimnum >= 2 && s + 1 < nsteps && block_len(c, first_step, nsteps, s + 1, energy_every) == 0 &&
+          !(energy_every > 0 && i % energy_every == 0) && (sched.back().flags & F_NORM)) {
+        const int nb = sweep_nb(c, sched.back());
+        if (nb < 4096) {
+          sched.back().flags |= F_DEFER;
+          c->defer_nb = nb;
+        }
+      }
+      int v_done = -1, ka_done = -1;
+      for (const Sweep& sw : sched) {
+        gpue_status st = fill_for(c, sw, gstate, i, nullptr, &v_done, &ka_done);
+        if (st == GPUE_OK) st = launch(c, sw, ph, c->psi, c->psi);
         if (st != GPUE_OK) return st;
       }
+      if (gstate == 0) c->pending_norm = true;
     }
-    // leave this step's norm to the next one when that is an eager step too
-    if (gstate == 0 && c->p.dimnum >= 2 && s + 1 < nsteps && block_len(c, first_step, nsteps, s + 1, energy_every) == 0 &&
-        !(energy_every > 0 && i % energy_every == 0) && (sched.back().flags & F_NORM)) {
-      const int nb = sweep_nb(c, sched.back());
-      if (nb < 4096) {
-        sched.back().flags |= F_DEFER;
-        c->defer_nb = nb;
-      }
-    }
-    int v_done = -1, ka_done = -1;
-    for (const Sweep& sw : sched) {
-      gpue_status st = fill_for(c, sw, gstate, i, nullptr, &v_done, &ka_done);
-      if (st == GPUE_OK) st = launch(c, sw, ph, c->psi, c->psi);
-      if (st != GPUE_OK) return st;
-    }
-    if (gstate == 0) c->pending_norm = true;
     if (energy_every > 0 && i % energy_every == 0) {
       double E = 0, M = 0;
       gpue_status st = gpue_energy(c, &E, &M);
@@ -1654,7 +1702,7 @@ gpue_status gpue_evolve(gpue_ctx* c, int first_step, int nsteps, int gstate, int
 gpue_status gpue_prepare_evolve(gpue_ctx* c, int first_step, int nsteps, int gstate, int energy_every) {
   if (!c || nsteps < 0 || (gstate != 0 && gstate != 1) || first_step < 0) return GPUE_EINVAL;
   for (int s = 0; s < nsteps;) {
-    const int L = block_len(c, first_step, nsteps, s, energy_every);
+    const int L = c->p.dimnum == 1 && !c->t_dep ? 0 : block_len(c, first_step, nsteps, s, energy_every);
     if (L == 0) {
       ++s;
       continue;

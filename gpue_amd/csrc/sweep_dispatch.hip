@@ -6,6 +6,7 @@ namespace gpue {
 
 #define GPUE_DECL1(NAME_)                                                                         \
   hipError_t NAME_(bool row, int narrow, int mode, const SweepArgs& a, hipStream_t s);            \
+  hipError_t NAME_##_line(const SweepArgs& a, int nsteps, hipStream_t s);                          \
   hipError_t NAME_##_b(bool row, int narrow, int mode, const SweepArgs* d, int ninst, int lx, int others, \
                        hipStream_t s);
 #define GPUE_DECL(N_)                                                                     \
@@ -38,6 +39,22 @@ hipError_t launch_sweep(int prec, bool row, int N, int var, int mode, const Swee
     if (pv == 0)                                                                              \
       return prec == 64 ? sweep_f64_##N_##_v0(row, nw, mode, a, s) : sweep_f32_##N_##_v0(row, nw, mode, a, s); \
     return prec == 64 ? sweep_f64_##N_##_v1(row, nw, mode, a, s) : sweep_f32_##N_##_v1(row, nw, mode, a, s);
+  switch (N) {
+    GPUE_CASE(16) GPUE_CASE(32) GPUE_CASE(48) GPUE_CASE(64) GPUE_CASE(96) GPUE_CASE(128) GPUE_CASE(192) GPUE_CASE(256)
+    GPUE_CASE(384) GPUE_CASE(512) GPUE_CASE(1024) GPUE_CASE(2048)
+    GPUE_CASE(4096)
+    default: *handled = false; return hipErrorInvalidValue;
+  }
+#undef GPUE_CASE
+}
+
+// A run of whole steps of a 1D problem in one launch.
+hipError_t launch_line(int prec, int N, int plan, const SweepArgs& a, int nsteps, hipStream_t s, bool* handled) {
+  *handled = true;
+#define GPUE_CASE(N_)                                                                         \
+  case N_:                                                                                    \
+    if (plan == 0) return prec == 64 ? sweep_f64_##N_##_v0_line(a, nsteps, s) : sweep_f32_##N_##_v0_line(a, nsteps, s); \
+    return prec == 64 ? sweep_f64_##N_##_v1_line(a, nsteps, s) : sweep_f32_##N_##_v1_line(a, nsteps, s);
   switch (N) {
     GPUE_CASE(16) GPUE_CASE(32) GPUE_CASE(48) GPUE_CASE(64) GPUE_CASE(96) GPUE_CASE(128) GPUE_CASE(192) GPUE_CASE(256)
     GPUE_CASE(384) GPUE_CASE(512) GPUE_CASE(1024) GPUE_CASE(2048)

@@ -447,6 +447,98 @@ __device__ __forceinline__ void col_body(SweepArgs a, int bid, int nblk) {
   }
 }
 
+// ---------------------------------------------------------------------------
+// 1D problems: a run of whole steps in one launch.  The line fits one workgroup, so
+// psi stays in registers from step to step ([V/2, FFT, K, IFFT, V/2 (, gauge)], the
+// operators and their arithmetic as in RM_FULL) and the renormalisation is a block
+// sum, with the additions of a sweep's partial and its finalize: results are those
+// of steps launched one by one.  What bounds it is the dependent chain of a step
+// (N = 1024: eight passes and their exchanges, two V/2 and the block sum): about 4 us
+// at N = 1024 FP64, 1e2 steps in one launch, where a sweep and a finalize a step,
+// most of them launch and first loads, took 11.7 us.
+// The norm of the last step is left pending in *norm_out.
+// ---------------------------------------------------------------------------
+template <typename T, int N, int RV, bool REAL>
+__device__ __forceinline__ void line_body(const SweepArgs& a, int nsteps) {
+  constexpr int V = RV & 1;
+  constexpr bool PRE = (RV >> 1) != 0;   // twiddles in registers for the whole run
+  using P = Plan<N, V>;
+  constexpr int TPL = P::TPL, E = P::E, WG = RowCfg<N, RV>::WG, LPW = RowCfg<N, RV>::LPW, NW = (WG + 63) / 64;
+  constexpr int FOOT = LdsRow::footprint(N);
+  __shared__ cx<T> lds[P::NP > 1 ? LPW * FOOT : 1];
+  __shared__ double sh[16];
+  const Phys& p = a.ph;
+  const unsigned flags = a.flags;
+  const int tid = threadIdx.x % TPL, lw = threadIdx.x / TPL;
+  const bool active = lw == 0;   // further lines of the workgroup repeat line 0
+  const LineAt l{0, tid, 0, 1, 0, 0};
+  const auto* __restrict__ tw = (const typename TwE<T>::type*)a.tw;
+  const LdsRow la{lw * FOOT};
+  constexpr int RF0 = Seq<N, V, ORD_FWD>::first(), RFL = Seq<N, V, ORD_FWD>::last();
+  cx<T> v[E];
+  TwRegs<T, N, V> twr;
+  VOp<T, N, TPL, RF0, E> vo;
+  KOp<T, N, TPL, RFL, E, REAL> ko;
+  GOp<T, N, TPL, RFL, E, REAL> go;
+  const bool gauge = (flags & F_GAUGE_POST) != 0;
+#pragma unroll
+  for (int r = 0; r < E; ++r) v[r] = ((const cx<T>*)a.in)[bpos<N, TPL, RF0>(tid, r)];
+  vo.load(p, p.Vt, l);
+  ko.load(p, l);
+  if constexpr (PRE) twr.load(tid, tw);
+  if (gauge) {
+    go.load(p, l);
+    go.prep(p, l, a.invN);
+  }
+  double nrm = !REAL && (flags & F_SCALE_IN) ? *a.norm_in : 1.0;
+  auto fwd = [&]() { fft_regs_tw<T, N, V, ORD_FWD, -1, PRE>(v, tid, tw, twr, lds, la); };
+  auto inv = [&]() { fft_regs_tw<T, N, V, ORD_REV, +1, PRE>(v, tid, tw, twr, lds, la); };
+#pragma unroll 1
+  for (int s = 0; s < nsteps; ++s) {
+    if constexpr (!REAL) {
+      const T f = (T)(1.0 / nrm);
+#pragma unroll
+      for (int r = 0; r < E; ++r) v[r] = scale_norm(v[r], f);
+    }
+    vo.template half<REAL>(p, l, v);
+    fwd();
+    ko.apply(p, l, v, a.invN);
+    inv();
+    vo.template half<REAL>(p, l, v);
+    if (gauge) {
+      fwd();
+      go.apply(p, v, l, a.invN, false);
+      inv();
+    }
+    if constexpr (!REAL) {
+      double acc = 0.0;
+#pragma unroll
+      for (int r = 0; r < E; ++r)
+        if (active) acc += abs2d(v[r]);
+      double tot = wave_sum(acc, 64);
+      if constexpr (NW > 1) {
+        if constexpr (P::NP == 1) __syncthreads();   // else the exchanges' barriers follow the last read of sh
+        if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = tot;
+        __syncthreads();
+        tot = 0.0;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) tot += sh[w];
+      }
+      nrm = sqrt(tot * a.norm_scale);
+    }
+  }
+  if (active) {
+#pragma unroll
+    for (int r = 0; r < E; ++r) ((cx<T>*)a.out)[bpos<N, TPL, RF0>(tid, r)] = v[r];
+    if (!REAL && tid == 0) *a.norm_out = nrm;
+  }
+}
+
+template <typename T, int N, int V, bool REAL>
+__global__ void __launch_bounds__((RowCfg<N, V>::WG)) line_steps(SweepArgs a, int nsteps) {
+  line_body<T, N, V, REAL>(a, nsteps);
+}
+
 // One problem per launch (arguments by value) ...
 template <typename T, int N, int V, int MODE>
 __global__ void __launch_bounds__((RowCfg<N, V>::WG)) row_sweep(SweepArgs a) {

@@ -38,6 +38,17 @@ hipError_t launch_row_t(int m, const SweepArgs& a, hipStream_t s) {
   return hipGetLastError();
 }
 
+// 1D: nsteps whole steps of one line in one workgroup.  Twiddles in registers up to 256
+// lanes (one wave per SIMD); beyond, two waves share a SIMD's registers.
+template <typename T, int N, int V>
+hipError_t launch_line_t(const SweepArgs& a, int nsteps, hipStream_t s) {
+  constexpr int RV = V + (Plan<N, V>::TPL <= 256 ? 2 : 0);
+  dim3 grid(1), block(RowCfg<N, RV>::WG);
+  if (a.ph.gstate) hipLaunchKernelGGL((line_steps<T, N, RV, true>), grid, block, 0, s, a, nsteps);
+  else hipLaunchKernelGGL((line_steps<T, N, RV, false>), grid, block, 0, s, a, nsteps);
+  return hipGetLastError();
+}
+
 template <typename T, int N, int V>
 hipError_t launch_col_t(int m, const SweepArgs& a, hipStream_t s) {
   const int others = a.axis == 1 ? a.ph.zDim : a.ph.yDim;
@@ -98,6 +109,9 @@ hipError_t launch_col_b_t(int m, const SweepArgs* d, int ninst, int xDim, int ot
     if (narrow == 1) return launch_col_t<T_, N_, V_ + 2>(mode, a, s);                             \
     if (narrow == 2) return launch_col_t<T_, N_, V_ + 4>(mode, a, s);                             \
     return launch_col_t<T_, N_, V_>(mode, a, s);                                                  \
+  }                                                                                               \
+  hipError_t NAME_##_line(const SweepArgs& a, int nsteps, hipStream_t s) {                        \
+    return launch_line_t<T_, N_, V_>(a, nsteps, s);                                               \
   }                                                                                               \
   hipError_t NAME_##_b(bool row, int narrow, int mode, const SweepArgs* d, int ninst, int lx,     \
                        int others, hipStream_t s) {                                               \
