@@ -67,6 +67,7 @@ struct gpue_ctx {
   double* partials = nullptr;
   size_t partials_n = 0;
   double* results = nullptr;   // [0] norm  [1] kinetic  [2..5] position terms
+  double* hres = nullptr;      // pinned: scalars on their way to the host (16 doubles)
   int v_kind = gpue::V_SEP, a_kind = gpue::A_ROTATION, k_kind = gpue::K_SEP;
   bool v_user = false;         // V supplied by the caller (table or equation)
   double* vs[3] = {};          // separable V / K value tables
@@ -126,12 +127,16 @@ gpue_status apply_pending(gpue_ctx* c);
 gpue_status evolve_async(gpue_ctx* c, int first_step, int nsteps, int gstate);
 gpue_status energy_launch(gpue_ctx* c, double* host_dst);
 gpue_status energy_launch_graph(gpue_ctx* c, double* host_dst);
-// psi to the host, waiting on `ev` (recorded after the copy) rather than the stream.
-gpue_status download_wfc_ev(gpue_ctx* c, double* interleaved, hipEvent_t ev);
 // A context on a given stream (null: its own), and new parameters for one of the
 // same shape (no device allocation).
 gpue_status ctx_create(const gpue_params* p, hipStream_t ext_stream, gpue_ctx** out);
 gpue_status ctx_reset(gpue_ctx* c, const gpue_params* p);
 bool ctx_same_shape(const gpue_ctx* c, const gpue_params* p);
+// Pinned-chunk copies between the device and the caller's pageable memory (staging.hip);
+// the chunks are shared by all contexts, each of which holds an acquire.
+void staging_acquire();
+void staging_release();
+hipError_t copy_to_host(void* host, const void* dev, size_t n, size_t es, bool widen, int device, hipStream_t stream);
+hipError_t copy_to_device(void* dev, const void* host, size_t n, size_t es, bool narrow, int device, hipStream_t stream);
 void energy_combine(const gpue_ctx* c, const double* terms, double* energy, double* mu);
 }  // namespace gpue

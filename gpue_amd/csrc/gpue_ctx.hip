@@ -585,6 +585,8 @@ void gpue_destroy(gpue_ctx* c) {
   drop_graphs(c);
   if (c->gev) (void)hipEventDestroy(c->gev);
   if (c->stream && c->own_stream) (void)hipStreamDestroy(c->stream);
+  if (c->hres) (void)hipHostFree(c->hres);
+  staging_release();
   delete c;
 }
 
@@ -693,6 +695,7 @@ gpue_status gpue::ctx_create(const gpue_params* pin, hipStream_t ext_stream, gpu
   if (!pin || !out) return GPUE_EINVAL;
   *out = nullptr;
   gpue_ctx* c = new gpue_ctx();
+  staging_acquire();
   c->p = *pin;
   gpue_params& p = c->p;
   auto bail = [&](gpue_status s, const std::string& m) {
@@ -773,7 +776,8 @@ gpue_status gpue::ctx_create(const gpue_params* pin, hipStream_t ext_stream, gpu
   for (int a = 0; a < 3; ++a) c->var[a] = default_variant(c, a);
   c->partials_n = nb * 4;
   if (hipMalloc((void**)&c->partials, c->partials_n * sizeof(double)) != hipSuccess ||
-      hipMalloc((void**)&c->results, 16 * sizeof(double)) != hipSuccess)
+      hipMalloc((void**)&c->results, 16 * sizeof(double)) != hipSuccess ||
+      hipHostMalloc((void**)&c->hres, 16 * sizeof(double), hipHostMallocDefault) != hipSuccess)
     return bail(GPUE_ENOMEM, "reduction scratch");
   // on the context's own stream: other contexts' work on the device is not waited for
   if (hipMemsetAsync(c->results, 0, 16 * sizeof(double), c->stream) != hipSuccess ||
@@ -989,57 +993,24 @@ gpue_status gpue_set_field_eqn(gpue_ctx* c, int which, const char* expr, const c
   return st;
 }
 
+// psi as 2N numbers; FP32 contexts convert on the way.
 gpue_status gpue_upload_wfc(gpue_ctx* c, const double* il) {
   if (!c || !il) return GPUE_EINVAL;
-  if (c->prec == 64) {
-    HIPCHK(c, hipMemcpyAsync(c->psi, il, c->N * 16, hipMemcpyHostToDevice, c->stream));
-  } else {
-    std::vector<float> f(2 * c->N);
-    for (long i = 0; i < 2 * c->N; ++i) f[i] = (float)il[i];
-    HIPCHK(c, hipMemcpyAsync(c->psi, f.data(), c->N * 8, hipMemcpyHostToDevice, c->stream));
-  }
   HIPCHK(c, launch_set_double(c->results, 1.0, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
+  HIPCHK(c, copy_to_device(c->psi, il, 2 * c->N, c->esz / 2, c->prec == 32, c->p.device, c->stream));
   c->pending_norm = false;
   return GPUE_OK;
 }
 
+// Waits for the work queued before the copy, not for what another context queues on a
+// shared stream after it.
 gpue_status gpue_download_wfc(gpue_ctx* c, double* il) {
   if (!c || !il) return GPUE_EINVAL;
   gpue_status st = apply_pending(c);
   if (st != GPUE_OK) return st;
-  if (c->prec == 64) {
-    HIPCHK(c, hipMemcpyAsync(il, c->psi, c->N * 16, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-  } else {
-    std::vector<float> f(2 * c->N);
-    HIPCHK(c, hipMemcpyAsync(f.data(), c->psi, c->N * 8, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    for (long i = 0; i < 2 * c->N; ++i) il[i] = f[i];
-  }
+  HIPCHK(c, copy_to_host(il, c->psi, 2 * c->N, c->esz / 2, c->prec == 32, c->p.device, c->stream));
   return GPUE_OK;
 }
-
-}  // extern "C"
-
-gpue_status gpue::download_wfc_ev(gpue_ctx* c, double* il, hipEvent_t ev) {
-  gpue_status st = apply_pending(c);
-  if (st != GPUE_OK) return st;
-  if (c->prec == 64) {
-    HIPCHK(c, hipMemcpyAsync(il, c->psi, c->N * 16, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipEventRecord(ev, c->stream));
-    HIPCHK(c, hipEventSynchronize(ev));
-  } else {
-    std::vector<float> f(2 * c->N);
-    HIPCHK(c, hipMemcpyAsync(f.data(), c->psi, c->N * 8, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipEventRecord(ev, c->stream));
-    HIPCHK(c, hipEventSynchronize(ev));
-    for (long i = 0; i < 2 * c->N; ++i) il[i] = f[i];
-  }
-  return GPUE_OK;
-}
-
-extern "C" {
 
 gpue_status gpue_parsum(gpue_ctx* c) {
   if (!c) return GPUE_EINVAL;
@@ -1159,13 +1130,11 @@ extern "C" {
 
 gpue_status gpue_energy(gpue_ctx* c, double* energy, double* mu) {
   if (!c) return GPUE_EINVAL;
-  double r[6];
-  gpue_status st = energy_launch(c, nullptr);
+  gpue_status st = energy_launch(c, c->hres);
   if (st != GPUE_OK) return st;
-  HIPCHK(c, hipMemcpyAsync(r, c->results, sizeof(r), hipMemcpyDeviceToHost, c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
   double E = 0, M = 0;
-  energy_combine(c, r, &E, &M);
+  energy_combine(c, c->hres, &E, &M);
   if (energy) *energy = E;
   if (mu) *mu = M;
   if (!std::isfinite(E)) return fail(c, GPUE_ENONFINITE, "energy is not finite");
@@ -1193,8 +1162,8 @@ gpue_status gpue_energy_consistent(gpue_ctx* c, double* energy, double* mu) {
     st = launch(c, {a == 0, a, a == 0 ? (int)RM_KSUM : (int)CM_KSUM, F_ASUM, 1.0 / (double)c->dims[a]}, ph, c->psi,
                 c->psi);
   if (st != GPUE_OK) return st;
-  double r[9];
-  HIPCHK(c, hipMemcpyAsync(r, c->results, sizeof(r), hipMemcpyDeviceToHost, c->stream));
+  double* const r = c->hres;
+  HIPCHK(c, hipMemcpyAsync(r, c->results, 9 * sizeof(double), hipMemcpyDeviceToHost, c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
   if (p.corotating && p.dimnum > 1) {
     double s = 0.0;
@@ -1681,9 +1650,9 @@ static gpue_status evolve_impl(gpue_ctx* c, int first_step, int nsteps, int gsta
     if (st != GPUE_OK) return st;
   }
   if (check_norm && gstate == 0 && c->pending_norm) {
-    double nrm = 0;
-    HIPCHK(c, hipMemcpyAsync(&nrm, c->results, sizeof(double), hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(c, hipMemcpyAsync(c->hres, c->results, sizeof(double), hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
+    const double nrm = c->hres[0];
     if (!std::isfinite(nrm) || nrm == 0.0) return fail(c, GPUE_ENONFINITE, "norm is not finite");
   }
   if (res) *res = r;
@@ -1754,11 +1723,9 @@ gpue_status gpue_vortex_marker_2d(gpue_ctx* c, double radius, int* marker_out, i
   hipError_t e = c->prec == 64 ? launch_vortex<double>(c->psi, c->vmask, xDim, c->vcand, c->vmarker, c->vfound, c->stream)
                                : launch_vortex<float>(c->psi, c->vmask, xDim, c->vcand, c->vmarker, c->vfound, c->stream);
   if (e != hipSuccess) return fail(c, GPUE_EHIP, hipGetErrorString(e));
-  int f = 0;
-  HIPCHK(c, hipMemcpyAsync(marker_out, c->vmarker, (size_t)xDim * xDim * sizeof(int), hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipMemcpyAsync(&f, c->vfound, sizeof(int), hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
-  if (found) *found = f;
+  HIPCHK(c, hipMemcpyAsync(c->hres, c->vfound, sizeof(int), hipMemcpyDeviceToHost, c->stream));
+  HIPCHK(c, copy_to_host(marker_out, c->vmarker, (size_t)xDim * xDim, sizeof(int), false, c->p.device, c->stream));
+  if (found) std::memcpy(found, c->hres, sizeof(int));
   return GPUE_OK;
 }
 

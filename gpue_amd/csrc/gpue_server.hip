@@ -235,7 +235,7 @@ static void retire(gpue_server* sv, Slot* s) {
   r.t_start = s->t_start;
   if (s->ctx && s->req.r.psi_out && s->status == GPUE_OK) {
     // waits for this request's copy, not for the later work of the stream's other requests
-    const gpue_status st = download_wfc_ev(s->ctx, s->req.r.psi_out, s->ev);
+    const gpue_status st = gpue_download_wfc(s->ctx, s->req.r.psi_out);
     if (st != GPUE_OK) r.status = st;
   }
   r.t_done = sv->clock();
