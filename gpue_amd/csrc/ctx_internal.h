@@ -54,10 +54,13 @@ struct gpue_ctx {
   // steady-state step graphs: blocks of up to graph_steps consecutive steps (even
   // count, starting at an even step, norm pending) captured once per (gstate,
   // length) and replayed; shorter blocks cover the tail of an evolve call and the
-  // steps between energy evaluations
-  int graph_steps = 8;
+  // steps between energy evaluations.  A replay costs 15-25 us beside its steps (us a
+  // step in blocks of 2 / 8 / 32 / 96: 256^2 19.8 / 15.6 / 14.5 / 14.2, 512^2 with
+  // rotation 35.5 / 31.0 / 29.9 / 29.5, 128x128x96 88.9 / 82.6 / 81.0 / 80.6); a longer
+  // first capture is the price, and 32 leaves little to gain
+  int graph_steps = 32;
   std::vector<gpue::StepGraph> graphs;
-  hipEvent_t gev = nullptr;    // recorded after every graph replay (a shared stream is not waited for)
+  hipEvent_t gev = nullptr;    // recorded after the replays of an evolve call (a shared stream is not waited for)
   // the energy evaluation of gpue_batch_energy as one graph (energy_launch_graph),
   // with the host buffer its terms are copied to; dropped with the step graphs
   hipGraph_t egraph = nullptr;

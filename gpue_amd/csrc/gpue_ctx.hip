@@ -1491,13 +1491,10 @@ static gpue_status build_graph(gpue_ctx* c, int gstate, int len, StepGraph** out
   return GPUE_OK;
 }
 
-static gpue_status step_graph(gpue_ctx* c, int gstate, int len, StepGraph** out) {
+static StepGraph* find_graph(gpue_ctx* c, int gstate, int len) {
   for (StepGraph& g : c->graphs)
-    if (g.gstate == gstate && g.len == len) {
-      *out = &g;
-      return GPUE_OK;
-    }
-  return build_graph(c, gstate, len, out);
+    if (g.gstate == gstate && g.len == len) return &g;
+  return nullptr;
 }
 
 // Steps of a captured block starting at step s of an evolve call (0: the step
@@ -1544,6 +1541,22 @@ static gpue_status launch_steps_1d(gpue_ctx* c, int gstate, int L) {
   return e == hipSuccess ? GPUE_OK : fail(c, GPUE_EHIP, std::string("line launch: ") + hipGetErrorString(e));
 }
 
+// Leaves gev recorded after the replays an evolve call queued, once per call, on every
+// way out of it (an event between two replays is a packet of its own in the queue).
+struct ReplayMark {
+  gpue_ctx* c;
+  bool queued = false;
+  explicit ReplayMark(gpue_ctx* c_) : c(c_) {}
+  void mark() {
+    if (!queued) return;
+    queued = false;
+    if (!c->gev && hipEventCreateWithFlags(&c->gev, hipEventDisableTiming) != hipSuccess) c->gev = nullptr;
+    // without the event, drop_graphs and the eviction would have nothing to wait for
+    if (!c->gev || hipEventRecord(c->gev, c->stream) != hipSuccess) (void)hipStreamSynchronize(c->stream);
+  }
+  ~ReplayMark() { mark(); }
+};
+
 static gpue_status evolve_impl(gpue_ctx* c, int first_step, int nsteps, int gstate, int energy_every,
                                double energy_thr, double* energies, int max_energies, gpue_evolve_result* res,
                                bool check_norm) {
@@ -1563,13 +1576,18 @@ static gpue_status evolve_impl(gpue_ctx* c, int first_step, int nsteps, int gsta
   // steady state: captured blocks of steps (block_len) are replayed; the
   // imaginary-time graph always rescales on entry (results[0] holds the
   // pending norm or 1.0, and x*1.0 is exact)
+  ReplayMark replays(c);
   for (s = 0; s < nsteps; ++s) {
     int i = first_step + s;
     const int L1 = line_len(c, first_step, nsteps, s, energy_every);
     const int L = L1 > 0 ? 0 : block_len(c, first_step, nsteps, s, energy_every);
     if (L > 0) {
-      StepGraph* sg = nullptr;
-      gpue_status st = step_graph(c, gstate, L, &sg);
+      StepGraph* sg = find_graph(c, gstate, L);
+      gpue_status st = GPUE_OK;
+      if (!sg) {
+        replays.mark();   // a new block may evict one whose replay is queued
+        st = build_graph(c, gstate, L, &sg);
+      }
       if (st != GPUE_OK) return st;
       sg->last_use = ++c->graph_clock;
       if (c->t_dep) {   // the block's fills count time from its first step
@@ -1577,8 +1595,7 @@ static gpue_status evolve_impl(gpue_ctx* c, int first_step, int nsteps, int gsta
         c->t_last = Dt * (i + L - 1);
       }
       HIPCHK(c, hipGraphLaunch(sg->exec, c->stream));
-      if (!c->gev) HIPCHK(c, hipEventCreateWithFlags(&c->gev, hipEventDisableTiming));
-      HIPCHK(c, hipEventRecord(c->gev, c->stream));
+      replays.queued = true;
       if (gstate == 0) c->pending_norm = true;
       s += L - 1;
       continue;
@@ -1676,8 +1693,8 @@ gpue_status gpue_prepare_evolve(gpue_ctx* c, int first_step, int nsteps, int gst
       ++s;
       continue;
     }
-    StepGraph* sg = nullptr;
-    gpue_status st = step_graph(c, gstate, L, &sg);
+    StepGraph* sg = find_graph(c, gstate, L);
+    gpue_status st = sg ? GPUE_OK : build_graph(c, gstate, L, &sg);
     if (st != GPUE_OK) return st;
     sg->last_use = ++c->graph_clock;
     s += L;

@@ -163,7 +163,7 @@ gpue_status gpue_set_variants(gpue_ctx *c, const int *variants);
 /* The kernel variants in use per axis (what gpue_set_variants or an autotuner set). */
 gpue_status gpue_get_variants(const gpue_ctx *c, int *variants);
 /* Steady-state steps are captured as HIP graphs of up to `steps` consecutive
- * steps (even, default 8) and replayed; 0 launches every sweep individually.
+ * steps (even, default 32) and replayed; 0 launches every sweep individually.
  * No reference counterpart (GPUE launches each kernel from the host loop). */
 gpue_status gpue_set_graph_steps(gpue_ctx *c, int steps);
 /* Capture, without launching, the step blocks that gpue_evolve with the same
