@@ -390,8 +390,8 @@ class Context:
 
 class Batch:
     """Many independent contexts advanced together (gpue_batch): one launch per
-    sweep covers every instance of a shape; each shape group replays two steps
-    from a graph on its own stream."""
+    sweep covers every instance of a kind (small grids of any size) or of a shape;
+    each group replays blocks of steps from graphs on its own stream."""
 
     def __init__(self, contexts):
         self.contexts = list(contexts)
@@ -417,7 +417,7 @@ class Batch:
         return us.value, mode.value
 
     def set_graph_mode(self, mode):
-        """0: one graph per shape group (default); 1: one graph for the whole batch; 2: no graphs."""
+        """0: graphs per group (default); 1: one graph for the whole batch; 2: no graphs."""
         self._check(lib().gpue_batch_set_graph_mode(self._h, int(mode)), "set_graph_mode")
 
     def set_active(self, index, active):

@@ -32,9 +32,13 @@ template <typename T>
 __device__ __forceinline__ cx<T> operator+(cx<T> a, cx<T> b) { return mk(a.x + b.x, a.y + b.y); }
 template <typename T>
 __device__ __forceinline__ cx<T> operator-(cx<T> a, cx<T> b) { return mk(a.x - b.x, a.y - b.y); }
+// Products are fused by hand throughout (which of two products an add absorbs would be
+// the compiler's choice, different where the code around it is): a transform rounds the
+// same in every kernel that holds it, so a problem's results do not depend on whether
+// it runs alone, in a batch or with other operand loads.
 template <typename T>
 __device__ __forceinline__ cx<T> cmul(cx<T> a, cx<T> b) {
-  return mk(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
+  return mk(fma(-a.y, b.y, a.x * b.x), fma(a.y, b.x, a.x * b.y));
 }
 template <typename T>
 __device__ __forceinline__ cx<T> cscale(cx<T> a, T s) { return mk(a.x * s, a.y * s); }
@@ -101,7 +105,7 @@ __device__ __forceinline__ cx<T> twc(cx<T> a, int m) {
     return cmul_split(a, ch, sh, (float)(cd - (double)ch), (float)(sd - (double)sh));
   } else {
     const T c = (T)cd, s = (T)sd;
-    return mk(a.x * c - a.y * s, a.x * s + a.y * c);
+    return mk(fma(-a.y, s, a.x * c), fma(a.y, c, a.x * s));
   }
 }
 
@@ -363,13 +367,29 @@ __device__ __forceinline__ int pass_out(int tid, int q, int s) {
 
 // LDS addressing: element e of a line.  Row lines: base + pad(e); strided
 // lines: (e * LS + c) where LS = lines per tile (lanes vary in c fastest).
+// sync() orders the exchange: the workgroup's barrier, or, where the lines of one wave
+// have LDS of their own within a larger workgroup (ONEWAVE), program order, which the
+// LDS unit keeps for a wave.
+template <bool ONEWAVE>
+__device__ __forceinline__ void lds_sync() {
+  if constexpr (ONEWAVE) {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  } else {
+    __syncthreads();
+  }
+}
+template <bool ONEWAVE = false>
 struct LdsRow {
   int base;
+  static __device__ __forceinline__ void sync() { lds_sync<ONEWAVE>(); }
   __device__ __forceinline__ int at(int e) const { return base + e + (e >> 4); }
   static constexpr int footprint(int N) { return N + N / 16; }
 };
+template <bool ONEWAVE = false>
 struct LdsCol {
   int c, LS;
+  static __device__ __forceinline__ void sync() { lds_sync<ONEWAVE>(); }
   __device__ __forceinline__ int at(int e) const { return e * LS + c; }
 };
 
@@ -385,10 +405,10 @@ __device__ __forceinline__ void fft_from_pass(cx<T>* v, int tid, const typename 
   if constexpr (P < NP) {
     if constexpr (P > 0) {
       constexpr int RP = S::radix(P - 1), LP = S::Lbefore(P - 1);
-      __syncthreads();  // previous users of LDS are done
+      LA::sync();  // previous users of LDS are done
 #pragma unroll
       for (int r = 0; r < E; ++r) lds[la.at(pass_out<N, TPL, RP, LP>(tid, r / RP, r % RP))] = v[r];
-      __syncthreads();
+      LA::sync();
 #pragma unroll
       for (int r = 0; r < E; ++r) v[r] = lds[la.at(bpos<N, TPL, S::radix(P)>(tid, r))];
     }

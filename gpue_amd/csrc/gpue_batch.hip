@@ -1,19 +1,19 @@
 // gpue_batch.hip -- many independent problems advanced together.
 //
-// Instances with the same shape (precision, dimensions, grid sizes, kernel
-// variants, gauge/no gauge) form a group.  For every sweep of the step one
-// batched kernel covers every instance of the group: blocks [i*bpi, (i+1)*bpi)
-// work on instance i, whose SweepArgs live in a device array.  GPUE's gauge
+// Instances of one precision, dimension and gauge whose axes have merged kernels
+// (sweep_merged.h) form a merged group: every sweep of the step is one launch over all
+// of them, whatever their sizes.  Others group by shape (grid sizes and kernel variants
+// too): for every sweep one batched kernel covers the group, blocks [i*bpi, (i+1)*bpi)
+// working on instance i.  The instances' SweepArgs live in a device array.  GPUE's gauge
 // order alternates with the step parity (src/evolution.cu:837,842).  When the
-// odd-step sweep list is a prefix of the even-step one in kernel kind (the 2D
-// and rotation-about-z cases: [FWD][K][INV(+A_x)][A_y(+norm)] and
-// [FWD][K][INV][A_y][A_x+norm]) both parities share one launch per position,
-// with per-instance flags, and the extra position is inactive for odd
-// instances; otherwise each parity has its own sequence.  Every imaginary-time
-// sequence ends with one batched norm finalize.  The groups run on at most
+// odd-step sweep list is a prefix of the even-step one in kernel kind, both
+// parities share one launch per position, with per-instance flags; otherwise each parity
+// has its own sequence.  Imaginary-time norms are reduced in the next step's opening
+// sweep (groups whose partials allow it), with one batched finalize at the end of a
+// call, or else by a batched finalize after every step.  The groups run on at most
 // four streams (the process's hardware queues; the groups with the most work
-// get one each, the others share the last), with two consecutive steps of a
-// group captured once per gstate as a HIP graph and replayed, so the groups of
+// get one each, the others share the last), with blocks of 16 and 2 consecutive steps
+// of a group captured once per gstate as HIP graphs and replayed, so the groups of
 // different shapes (the small ones latency bound) overlap on the device.
 // Device memory is allocated only in gpue_batch_create.
 #include <hip/hip_runtime.h>
@@ -26,30 +26,88 @@
 #include <vector>
 
 #include "ctx_internal.h"
+#include "sweep_merged.h"
 
 using namespace gpue;
 
 namespace {
+
+struct Merged {                     // a merged launch (sweep_merged.h): which blocks a workgroup takes
+  MergeMap* map = nullptr;          // device array [grid]
+  int grid = 0, lds = 0;
+};
 
 struct BSeq {                       // one launch sequence of a group for (gstate, phase)
   std::vector<Sweep> keys;          // kernel kind per position (flags come per instance)
   int mask = 3;                     // step parities it serves (bit p: parity p)
   std::vector<SweepArgs*> dargs;    // per position: device array [members]
   std::vector<std::vector<SweepArgs>> hargs;
+  // imaginary time, groups that defer their norms: the opening sweep of a call's first
+  // step, which scales by the norm slot instead of the previous step's partials
+  SweepArgs* dopen = nullptr;
+  std::vector<SweepArgs> hopen;
+  std::vector<Merged> merged;       // per position, merged groups only
   FinArgs* dfin = nullptr;          // imaginary time: device array [members]
   std::vector<FinArgs> hfin;
   bool any = true;                  // some member takes this sequence (else it is not launched)
 };
 
+// Steps of a group's captured graphs: a replay costs some 10-20 us beside its steps,
+// the pair covers what is left.
+constexpr int kGraphLens[] = {16, 2};
+constexpr int kGraphKinds = 2;
+
 struct Group {
   std::vector<int> members;
   gpue_ctx* proto;                  // first member: shape and variants
+  bool merged = false;              // members of different shapes, launched together
+  bool defer = false;               // norms reduced in the next step's opening sweep
   std::vector<Sweep> sched[2][2];   // [gstate][parity]
   std::vector<BSeq> seqs[2][2];     // [gstate][phase]
   hipStream_t stream = nullptr;     // one of the batch's streams (not owned)
-  hipGraph_t graph[2] = {nullptr, nullptr};
-  hipGraphExec_t gexec[2] = {nullptr, nullptr};
+  hipGraph_t graph[2][kGraphKinds] = {};   // [gstate][kGraphLens]
+  hipGraphExec_t gexec[2][kGraphKinds] = {};
+  int var(const gpue_ctx* c, int axis) const { return !merged ? c->var[axis] : axis == 0 ? MERGE_ROW : MERGE_COL; }
 };
+
+// Problems that may share launches with others of their kind: every axis has a merged
+// kernel, and the variants are those it runs (the defaults of small grids).
+bool can_merge(const gpue_ctx* c) {
+  if (c->p.dimnum < 2) return false;
+  for (int a = 0; a < c->p.dimnum; ++a) {
+    int lds = 0;
+    if (!merged_shape(c->prec, a == 0, c->dims[a], &lds)) return false;
+    if (a == 0 ? c->var[a] != MERGE_ROW : c->var[a] != MERGE_COL) return false;
+  }
+  return true;
+}
+bool same_kind_of_problem(const gpue_ctx* a, const gpue_ctx* b) {
+  return a->prec == b->prec && a->p.dimnum == b->p.dimnum && a->p.corotating == b->p.corotating &&
+         a->az_zero == b->az_zero && a->p.device == b->p.device;
+}
+
+// Workgroups (= partials) of a member's sweep.
+int blocks_of(const Group& g, const gpue_ctx* c, const Sweep& s) {
+  const int n = c->dims[s.axis], var = g.var(c, s.axis);
+  return s.row ? sweep_blocks(c->prec, true, n, var, c->dims[1] * c->dims[2], 1)
+               : sweep_blocks(c->prec, false, n, var, c->dims[0], s.axis == 1 ? c->dims[2] : c->dims[1]);
+}
+
+// Whether every member's norm can be left to the next step's opening sweep (as
+// defer_norm decides for one context).
+bool can_defer(const Group& g, const std::vector<gpue_ctx*>& ctx) {
+  for (int idx : g.members) {
+    const gpue_ctx* c = ctx[idx];
+    if (c->p.dimnum < 2) return false;
+    for (int par = 0; par < 2; ++par) {
+      const Sweep& open = g.sched[0][par].front();
+      if (blocks_of(g, c, g.sched[0][par].back()) >= 4096 ||
+          !sweep_full_waves(c->prec, open.row, c->dims[open.axis], g.var(c, open.axis)))
+        return false;
+    }
+  }
+  return true;
+}
 
 bool same_shape(const gpue_ctx* a, const gpue_ctx* b) {
   return a->prec == b->prec && a->p.dimnum == b->p.dimnum && a->dims[0] == b->dims[0] && a->dims[1] == b->dims[1] &&
@@ -122,7 +180,9 @@ static bool fill_args(gpue_batch* b) {
             const int par = (b->cls[idx] + ph) % 2;   // the instance's step parity at this phase
             const bool in = b->active[idx] && ((s.mask >> par) & 1);
             any = any || in;
-            const std::vector<Sweep>& sc = g.sched[gs][par];
+            std::vector<Sweep> own;   // members of a merged group have their own normalisations
+            if (g.merged) schedule(c, gs, par, gs == 0, own);
+            const std::vector<Sweep>& sc = g.merged ? own : g.sched[gs][par];
             const Phys phys = make_phys(c, gs, 0);
             for (size_t k = 0; k < s.keys.size(); ++k) {
               const bool on = in && k < sc.size();
@@ -131,7 +191,7 @@ static bool fill_args(gpue_batch* b) {
               std::memset(&a, 0, sizeof(a));
               // every context holds the tables of both plans for each of its
               // axes; a missing one would leave the sweep off rather than fault
-              const auto twi = c->tw.find(2 * c->dims[sw.axis] + (c->var[sw.axis] & 1));
+              const auto twi = c->tw.find(2 * c->dims[sw.axis] + (g.var(c, sw.axis) & 1));
               a.active = on && twi != c->tw.end();
               a.in = c->psi;
               a.out = c->psi;
@@ -144,17 +204,21 @@ static bool fill_args(gpue_batch* b) {
               a.invN = sw.invN;
               a.norm_in = c->results;
               a.partials = c->partials;
+              if (k == 0 && s.dopen) {
+                s.hopen[m] = a;
+                // the previous step's norm from its partials (its last sweep's)
+                a.flags |= F_SCALE_PART;
+                a.norm_nb = blocks_of(g, c, g.sched[gs][1 - par].back());
+                a.norm_scale = c->d[0] * c->d[1] * c->d[2];
+                a.norm_out = c->results;
+              }
             }
             if (s.dfin) {
               // the partials come from the instance's F_NORM sweep (its last)
-              const Sweep& last = sc.back();
-              const int n = c->dims[last.axis];
-              const int var = c->var[last.axis];
               FinArgs& f = s.hfin[m];
               std::memset(&f, 0, sizeof(f));
               f.active = in;
-              f.nb = last.row ? sweep_blocks(c->prec, true, n, var, c->dims[1] * c->dims[2], 1)
-                              : sweep_blocks(c->prec, false, n, var, c->dims[0], last.axis == 1 ? c->dims[2] : c->dims[1]);
+              f.nb = blocks_of(g, c, sc.back());
               f.na = 1;
               f.mode = 1;
               f.scale = c->d[0] * c->d[1] * c->d[2];
@@ -176,53 +240,75 @@ static gpue_status upload_args(gpue_batch* b) {
           for (size_t k = 0; k < s.keys.size(); ++k)
             BHIP(b, hipMemcpy(s.dargs[k], s.hargs[k].data(), s.hargs[k].size() * sizeof(SweepArgs),
                               hipMemcpyHostToDevice));
+          if (s.dopen)
+            BHIP(b, hipMemcpy(s.dopen, s.hopen.data(), s.hopen.size() * sizeof(SweepArgs), hipMemcpyHostToDevice));
           if (s.dfin)
             BHIP(b, hipMemcpy(s.dfin, s.hfin.data(), s.hfin.size() * sizeof(FinArgs), hipMemcpyHostToDevice));
         }
   return GPUE_OK;
 }
 
-// One step (one phase) of group g for gstate, on the group's stream.
-static gpue_status launch_group_phase(gpue_batch* b, Group& g, int gs, int ph) {
-  {
-    gpue_ctx* c = g.proto;
-    for (BSeq& s : g.seqs[gs][ph]) {
-      if (!s.any) continue;   // the step parity no member has
-      for (size_t k = 0; k < s.keys.size(); ++k) {
-        const Sweep& sw = s.keys[k];
+// One step (one phase) of group g for gstate, on the group's stream.  `first`: the first
+// step of a call (deferring groups scale by the norm slot).  Groups that do not defer
+// close every imaginary-time step with their finalize.
+static gpue_status launch_group_phase(gpue_batch* b, Group& g, int gs, int ph, bool first) {
+  gpue_ctx* c = g.proto;
+  for (BSeq& s : g.seqs[gs][ph]) {
+    if (!s.any) continue;   // the step parity no member has
+    for (size_t k = 0; k < s.keys.size(); ++k) {
+      const Sweep& sw = s.keys[k];
+      const SweepArgs* args = k == 0 && first && s.dopen ? s.dopen : s.dargs[k];
+      bool handled = true;
+      hipError_t e;
+      if (g.merged) {
+        const Merged& m = s.merged[k];
+        e = launch_sweep_merged(c->prec, sw.row, sw.mode, sw.flags, gs, args, m.map, m.grid, m.lds, g.stream);
+      } else {
         const int n = c->dims[sw.axis];
         const int lx = sw.row ? c->dims[1] * c->dims[2] : c->dims[0];
         const int others = sw.row ? 1 : (sw.axis == 1 ? c->dims[2] : c->dims[1]);
-        bool handled = false;
-        hipError_t e = launch_sweep_batched(c->prec, sw.row, n, c->var[sw.axis], sw.mode, sw.flags, gs, s.dargs[k],
-                                            (int)g.members.size(), lx, others, g.stream, &handled);
-        if (!handled || e != hipSuccess) return bfail(b, GPUE_EHIP, "batched sweep launch");
+        e = launch_sweep_batched(c->prec, sw.row, n, c->var[sw.axis], sw.mode, sw.flags, gs, args,
+                                 (int)g.members.size(), lx, others, g.stream, &handled);
       }
-      if (s.dfin) {
-        hipError_t e = launch_finalize_batched(s.dfin, (int)g.members.size(), g.stream);
-        if (e != hipSuccess) return bfail(b, GPUE_EHIP, "batched finalize launch");
-      }
+      if (!handled || e != hipSuccess) return bfail(b, GPUE_EHIP, "batched sweep launch");
+    }
+    if (s.dfin && !g.defer) {
+      hipError_t e = launch_finalize_batched(s.dfin, (int)g.members.size(), g.stream);
+      if (e != hipSuccess) return bfail(b, GPUE_EHIP, "batched finalize launch");
     }
   }
   return GPUE_OK;
 }
 
-static gpue_status launch_phase(gpue_batch* b, int gs, int ph) {
-  for (Group& g : b->groups) {
-    gpue_status st = launch_group_phase(b, g, gs, ph);
+static gpue_status launch_phase(gpue_batch* b, int gs, int ph, bool first) {
+  for (size_t k : b->by_work) {
+    gpue_status st = launch_group_phase(b, b->groups[k], gs, ph, first);
     if (st != GPUE_OK) return st;
+  }
+  return GPUE_OK;
+}
+
+// The norms that deferring groups' last step (phase ph) left in its partials, into the
+// norm slots: every call ends with them there.
+static gpue_status settle_norms(gpue_batch* b, int ph) {
+  for (Group& g : b->groups) {
+    if (!g.defer) continue;
+    for (BSeq& s : g.seqs[0][ph])
+      if (s.any && launch_finalize_batched(s.dfin, (int)g.members.size(), g.stream) != hipSuccess)
+        return bfail(b, GPUE_EHIP, "batched finalize launch");
   }
   return GPUE_OK;
 }
 
 static void drop_batch_graphs(gpue_batch* b) {
   for (Group& grp : b->groups)
-    for (int g = 0; g < 2; ++g) {
-      if (grp.gexec[g]) (void)hipGraphExecDestroy(grp.gexec[g]);
-      if (grp.graph[g]) (void)hipGraphDestroy(grp.graph[g]);
-      grp.gexec[g] = nullptr;
-      grp.graph[g] = nullptr;
-    }
+    for (int g = 0; g < 2; ++g)
+      for (int j = 0; j < kGraphKinds; ++j) {
+        if (grp.gexec[g][j]) (void)hipGraphExecDestroy(grp.gexec[g][j]);
+        if (grp.graph[g][j]) (void)hipGraphDestroy(grp.graph[g][j]);
+        grp.gexec[g][j] = nullptr;
+        grp.graph[g][j] = nullptr;
+      }
   for (int g = 0; g < 2; ++g) {
     if (b->wexec[g]) (void)hipGraphExecDestroy(b->wexec[g]);
     if (b->wgraph[g]) (void)hipGraphDestroy(b->wgraph[g]);
@@ -247,8 +333,8 @@ static gpue_status build_whole_graph(gpue_batch* b, int gstate) {
   for (size_t k = 0; k < b->groups.size() && st == GPUE_OK && e == hipSuccess; ++k) {
     Group& grp = b->groups[k];
     e = hipStreamWaitEvent(grp.stream, b->fork_ev, 0);
-    if (e == hipSuccess) st = launch_group_phase(b, grp, gstate, 0);
-    if (st == GPUE_OK && e == hipSuccess) st = launch_group_phase(b, grp, gstate, 1);
+    if (e == hipSuccess) st = launch_group_phase(b, grp, gstate, 0, false);
+    if (st == GPUE_OK && e == hipSuccess) st = launch_group_phase(b, grp, gstate, 1, false);
     if (st == GPUE_OK && e == hipSuccess) e = hipEventRecord(b->join_ev[k], grp.stream);
     if (st == GPUE_OK && e == hipSuccess) e = hipStreamWaitEvent(b->origin, b->join_ev[k], 0);
   }
@@ -264,6 +350,66 @@ static gpue_status build_whole_graph(gpue_batch* b, int gstate) {
   }
   b->wgraph[gstate] = g;
   return GPUE_OK;
+}
+
+// Capture kGraphLens[j] steps (from phase 0, norms deferred where the group does) of a group.
+static gpue_status build_group_graph(gpue_batch* b, Group& grp, int gstate, int j) {
+  BHIP(b, hipStreamBeginCapture(grp.stream, hipStreamCaptureModeThreadLocal));
+  gpue_status st = GPUE_OK;
+  for (int s = 0; s < kGraphLens[j] && st == GPUE_OK; ++s) st = launch_group_phase(b, grp, gstate, s & 1, false);
+  hipGraph_t g = nullptr;
+  const hipError_t e = hipStreamEndCapture(grp.stream, &g);
+  if (st != GPUE_OK || e != hipSuccess) {
+    if (g) (void)hipGraphDestroy(g);
+    return st != GPUE_OK ? st : bfail(b, GPUE_EHIP, "batch graph capture");
+  }
+  if (hipGraphInstantiate(&grp.gexec[gstate][j], g, nullptr, nullptr, 0) != hipSuccess) {
+    (void)hipGraphDestroy(g);
+    grp.gexec[gstate][j] = nullptr;
+    return bfail(b, GPUE_EHIP, "batch graph instantiate");
+  }
+  grp.graph[gstate][j] = g;
+  return GPUE_OK;
+}
+
+// Lay out a merged launch: each member's blocks in runs of a workgroup's worth, the
+// members with the longest axes first (their blocks take longest).  Workgroups are dealt
+// to the 8 XCDs round robin; those whose tiles share 128-byte lines of psi (the quarter
+// tiles of one default tile) are given positions on one XCD, so that the lines are
+// fetched into one L2 (xcd_tile does this within a lone launch).
+static gpue_status build_map(gpue_batch* b, const Group& g, const Sweep& sw, Merged& out) {
+  constexpr int XCDS = 8;
+  std::vector<size_t> order(g.members.size());
+  std::iota(order.begin(), order.end(), size_t(0));
+  std::stable_sort(order.begin(), order.end(), [&](size_t x, size_t y) {
+    return b->ctx[g.members[x]]->dims[sw.axis] > b->ctx[g.members[y]]->dims[sw.axis];
+  });
+  std::vector<MergeMap> queue[XCDS];
+  for (size_t m : order) {
+    const gpue_ctx* c = b->ctx[g.members[m]];
+    const int n = c->dims[sw.axis], nblk = blocks_of(g, c, sw);
+    int lds = 0;
+    const int wg = merged_shape(c->prec, sw.row, n, &lds);
+    if (wg <= 0) return GPUE_EUNSUPPORTED;
+    out.lds = std::max(out.lds, lds);
+    const int per = MERGE_WG / wg;                              // blocks of a workgroup
+    const int share = sw.row ? per : std::max(per, MERGE_TILES);   // blocks that stay on one XCD
+    for (int k0 = 0; k0 < nblk; k0 += share) {
+      std::vector<MergeMap>* q = &queue[0];
+      for (int x = 1; x < XCDS; ++x)
+        if (queue[x].size() < q->size()) q = &queue[x];
+      for (int k = k0; k < std::min(k0 + share, nblk); k += per) q->push_back(MergeMap{(int)m, k, n, nblk});
+    }
+  }
+  size_t longest = 0;
+  for (const auto& q : queue) longest = std::max(longest, q.size());
+  std::vector<MergeMap> map(longest * XCDS, MergeMap{-1, 0, 0, 0});   // -1: nothing to do
+  for (int x = 0; x < XCDS; ++x)
+    for (size_t i = 0; i < queue[x].size(); ++i) map[i * XCDS + x] = queue[x][i];
+  out.grid = (int)map.size();
+  if (hipMalloc((void**)&out.map, map.size() * sizeof(MergeMap)) != hipSuccess) return GPUE_ENOMEM;
+  return hipMemcpy(out.map, map.data(), map.size() * sizeof(MergeMap), hipMemcpyHostToDevice) == hipSuccess ? GPUE_OK
+                                                                                                            : GPUE_EHIP;
 }
 
 extern "C" {
@@ -285,6 +431,9 @@ void gpue_batch_destroy(gpue_batch* b) {
           for (auto* p : s.dargs)
             if (p) (void)hipFree(p);
           if (s.dfin) (void)hipFree(s.dfin);
+          if (s.dopen) (void)hipFree(s.dopen);
+          for (Merged& m : s.merged)
+            if (m.map) (void)hipFree(m.map);
         }
   for (hipStream_t st : b->streams)
     if (st) (void)hipStreamDestroy(st);
@@ -327,8 +476,9 @@ gpue_status gpue_batch_create(gpue_ctx* const* ctxs, int n, gpue_batch** out) {
   }
   for (int i = 0; i < n; ++i) {
     bool placed = false;
+    const bool mg = can_merge(b->ctx[i]);
     for (Group& g : b->groups)
-      if (same_shape(g.proto, b->ctx[i])) {
+      if (mg ? g.merged && same_kind_of_problem(g.proto, b->ctx[i]) : !g.merged && same_shape(g.proto, b->ctx[i])) {
         g.members.push_back(i);
         placed = true;
         break;
@@ -336,6 +486,7 @@ gpue_status gpue_batch_create(gpue_ctx* const* ctxs, int n, gpue_batch** out) {
     if (!placed) {
       Group g;
       g.proto = b->ctx[i];
+      g.merged = mg;
       g.members.push_back(i);
       b->groups.push_back(g);
     }
@@ -348,7 +499,11 @@ gpue_status gpue_batch_create(gpue_ctx* const* ctxs, int n, gpue_batch** out) {
     // run one after another.
     std::vector<size_t> order(b->groups.size());
     std::iota(order.begin(), order.end(), size_t(0));
-    auto work = [&](size_t k) { return (double)b->groups[k].members.size() * (double)b->groups[k].proto->N; };
+    auto work = [&](size_t k) {
+      double n = 0.0;
+      for (int idx : b->groups[k].members) n += (double)b->ctx[idx]->N;
+      return n;
+    };
     std::stable_sort(order.begin(), order.end(), [&](size_t x, size_t y) { return work(x) > work(y); });
     const size_t ns = std::min<size_t>(b->groups.size(), kBatchStreams);
     for (size_t i = 0; i < ns; ++i) {
@@ -378,6 +533,7 @@ gpue_status gpue_batch_create(gpue_ctx* const* ctxs, int n, gpue_batch** out) {
       // imaginary time: the norm slot holds 1.0 whenever nothing is pending, so
       // the renormalising first sweep is always safe
       for (int par = 0; par < 2; ++par) schedule(g.proto, gs, par, gs == 0, g.sched[gs][par]);
+      if (gs == 0) g.defer = can_defer(g, b->ctx);
       const std::vector<Sweep>& s0 = g.sched[gs][0];
       const std::vector<Sweep>& s1 = g.sched[gs][1];
       for (int ph = 0; ph < 2; ++ph) {
@@ -402,6 +558,23 @@ gpue_status gpue_batch_create(gpue_ctx* const* ctxs, int n, gpue_batch** out) {
               gpue_batch_destroy(b);
               return GPUE_ENOMEM;
             }
+          if (g.merged) {
+            s.merged.resize(s.keys.size());
+            for (size_t k = 0; k < s.keys.size(); ++k) {
+              const gpue_status st = build_map(b, g, s.keys[k], s.merged[k]);
+              if (st != GPUE_OK) {
+                gpue_batch_destroy(b);
+                return st;
+              }
+            }
+          }
+          if (gs == 0 && g.defer) {
+            s.hopen.assign(M, SweepArgs{});
+            if (hipMalloc((void**)&s.dopen, M * sizeof(SweepArgs)) != hipSuccess) {
+              gpue_batch_destroy(b);
+              return GPUE_ENOMEM;
+            }
+          }
           if (gs == 0) {
             s.hfin.assign(M, FinArgs{});
             if (hipMalloc((void**)&s.dfin, M * sizeof(FinArgs)) != hipSuccess) {
@@ -454,12 +627,24 @@ gpue_status gpue_batch_evolve(gpue_batch* b, int nsteps, int gstate) {
     gpue_status st = upload_args(b);
     if (st != GPUE_OK) return st;
   }
-  int s = 0;
-  if (b->phase == 1 && s < nsteps) {   // finish a pair started by an odd call
-    gpue_status st = launch_phase(b, gstate, 1);
-    if (st != GPUE_OK) return st;
-    b->phase = 0;
+  int s = 0, last_phase = 0;
+  auto single = [&](bool first) {   // the next step, launched on its own
+    const gpue_status st = launch_phase(b, gstate, b->phase, first);
+    last_phase = b->phase;
+    b->phase ^= 1;
     ++s;
+    return st;
+  };
+  // imaginary time: the first step scales by the norm slots, not by partials of a call
+  // before (which other work may have replaced)
+  const bool slots = gstate == 0 && std::any_of(b->groups.begin(), b->groups.end(), [](const Group& g) { return g.defer; });
+  if (slots && s < nsteps) {
+    gpue_status st = single(true);
+    if (st != GPUE_OK) return st;
+  }
+  if (b->phase == 1 && s < nsteps) {   // up to the start of a pair
+    gpue_status st = single(false);
+    if (st != GPUE_OK) return st;
   }
   if (nsteps - s >= 2 && b->graph_mode == 1) {
     if (!b->wexec[gstate]) {
@@ -473,45 +658,38 @@ gpue_status gpue_batch_evolve(gpue_batch* b, int nsteps, int gstate) {
       BHIP(b, hipStreamWaitEvent(b->origin, b->join_ev[k], 0));
     }
     for (; nsteps - s >= 2; s += 2) BHIP(b, hipGraphLaunch(b->wexec[gstate], b->origin));
+    last_phase = 1;
     BHIP(b, hipEventRecord(b->fork_ev, b->origin));
     for (Group& grp : b->groups) BHIP(b, hipStreamWaitEvent(grp.stream, b->fork_ev, 0));
   }
   if (b->graph_mode == 2) {   // no graphs: every phase launched on its own (kernel traces)
-    for (; nsteps - s >= 2; s += 2) {
-      gpue_status st = launch_phase(b, gstate, 0);
-      if (st == GPUE_OK) st = launch_phase(b, gstate, 1);
+    while (nsteps - s >= 2) {
+      gpue_status st = single(false);
+      if (st == GPUE_OK) st = single(false);
       if (st != GPUE_OK) return st;
     }
   }
-  if (nsteps - s >= 2) {
-    for (Group& grp : b->groups) {
-      if (grp.gexec[gstate]) continue;
-      BHIP(b, hipStreamBeginCapture(grp.stream, hipStreamCaptureModeThreadLocal));
-      gpue_status st = launch_group_phase(b, grp, gstate, 0);
-      if (st == GPUE_OK) st = launch_group_phase(b, grp, gstate, 1);
-      hipGraph_t g = nullptr;
-      hipError_t e = hipStreamEndCapture(grp.stream, &g);
-      if (st != GPUE_OK) {
-        if (g) (void)hipGraphDestroy(g);
-        return st;
+  // blocks of steps, the groups' graphs interleaved across their streams, the group
+  // with the most work (the critical path) first
+  for (int j = 0; j < kGraphKinds; ++j) {
+    const int len = kGraphLens[j];
+    if (nsteps - s < len) continue;
+    for (Group& grp : b->groups)
+      if (!grp.gexec[gstate][j]) {
+        gpue_status st = build_group_graph(b, grp, gstate, j);
+        if (st != GPUE_OK) return st;
       }
-      if (e != hipSuccess) return bfail(b, GPUE_EHIP, "batch graph capture");
-      if (hipGraphInstantiate(&grp.gexec[gstate], g, nullptr, nullptr, 0) != hipSuccess) {
-        (void)hipGraphDestroy(g);
-        return bfail(b, GPUE_EHIP, "batch graph instantiate");
-      }
-      grp.graph[gstate] = g;
-    }
-    // pairs of steps, the groups' graphs interleaved across their streams, the
-    // group with the most work (the critical path) first
-    for (; nsteps - s >= 2; s += 2)
-      for (size_t k : b->by_work) BHIP(b, hipGraphLaunch(b->groups[k].gexec[gstate], b->groups[k].stream));
+    for (; nsteps - s >= len; s += len)
+      for (size_t k : b->by_work) BHIP(b, hipGraphLaunch(b->groups[k].gexec[gstate][j], b->groups[k].stream));
+    last_phase = 1;
   }
   if (s < nsteps) {
-    gpue_status st = launch_phase(b, gstate, 0);
+    gpue_status st = single(false);
     if (st != GPUE_OK) return st;
-    b->phase = 1;
-    ++s;
+  }
+  if (gstate == 0 && nsteps > 0) {
+    gpue_status st = settle_norms(b, last_phase);
+    if (st != GPUE_OK) return st;
   }
   {
     gpue_status st = sync_groups(b);
@@ -581,6 +759,7 @@ gpue_status gpue_batch_autotune(gpue_batch* b, int gstate, int steps, double* us
   });
   for (size_t k = 0; k < order.size() && st == GPUE_OK; ++k) {
     Group& g = b->groups[order[k]];
+    if (g.merged) continue;   // merged launches run one set of variants
     for (int a = 0; a < g.proto->p.dimnum && st == GPUE_OK; ++a) {
       const int keep = g.proto->var[a];
       int pick = keep;

@@ -45,6 +45,13 @@ bool sweep_full_waves(int prec, bool row, int N, int var);
 hipError_t launch_sweep_batched(int prec, bool row, int N, int var, int mode, unsigned flags, int gstate,
                                 const SweepArgs* d, int ninst, int lx, int others, hipStream_t s, bool* handled);
 
+// One launch over problems of different sizes (sweep_merged.h): lanes of a block and LDS
+// bytes of a workgroup for an axis length (0 lanes: no such kernel), and the launch.
+struct MergeMap;
+int merged_shape(int prec, bool row, int n, int* lds);
+hipError_t launch_sweep_merged(int prec, bool row, int mode, unsigned flags, int gstate, const SweepArgs* d,
+                               const MergeMap* map, int grid, int lds, hipStream_t s);
+
 // Second stage of a batched reduction: one workgroup per instance.
 struct FinArgs {
   int active;

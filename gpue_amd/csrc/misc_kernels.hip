@@ -219,7 +219,7 @@ __global__ void k_norm_sum(const cx<T>* psi, long N, double* partials) {
     acc += (double)v.x * (double)v.x + (double)v.y * (double)v.y;
   }
   double pv[1] = {acc};
-  block_partial<1>(pv, partials, sh, blockIdx.x, gridDim.x);
+  block_partial<1>(pv, partials, sh, blockIdx.x, gridDim.x, threadIdx.x, blockDim.x);
 }
 
 // Second stage of every reduction: one workgroup sums nb partials of each of
@@ -235,7 +235,7 @@ __global__ void __launch_bounds__(1024) k_finalize(const double* partials, int n
   __shared__ double sh[64];
   for (int a = 0; a < na; ++a) {
     double acc[1] = {fin_sum(partials + (size_t)a * nb, nb)};
-    block_sum<1>(acc, sh);
+    block_sum<1>(acc, sh, threadIdx.x, blockDim.x);
     if (threadIdx.x == 0) out[a] = mode == 1 ? sqrt(acc[0] * scale) : acc[0] * scale;
     __syncthreads();
   }
@@ -288,7 +288,7 @@ __global__ void k_energy_pos(const cx<T>* psi, Phys p, int gauge, double hbar, d
       acc[2] += wx * (-syy * hbar) - (-wy) * (sx * hbar);
     }
   }
-  block_partial<4>(acc, partials, sh, blockIdx.x, gridDim.x);
+  block_partial<4>(acc, partials, sh, blockIdx.x, gridDim.x, threadIdx.x, blockDim.x);
 }
 
 // ---------------------------------------------------------------------------
@@ -509,7 +509,7 @@ __global__ void __launch_bounds__(1024) k_finalize_b(const FinArgs* __restrict__
     const double* pa = f.partials + (size_t)a * f.nb;
     double acc[1] = {(int)threadIdx.x >= B ? 0.0
                      : B >= 1024 ? fin_sum8_at(pa, f.nb, threadIdx.x, B) : fin_sum_at(pa, f.nb, threadIdx.x, B)};
-    block_sum<1>(acc, sh);
+    block_sum<1>(acc, sh, threadIdx.x, blockDim.x);
     if (threadIdx.x == 0) f.out[a] = f.mode == 1 ? sqrt(acc[0] * f.scale) : acc[0] * f.scale;
     __syncthreads();
   }

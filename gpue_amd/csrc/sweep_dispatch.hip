@@ -86,6 +86,27 @@ hipError_t launch_sweep_batched(int prec, bool row, int N, int var, int mode, un
 #undef GPUE_CASE
 }
 
+#define GPUE_MERGED(P_, K_)                                                                                     \
+  hipError_t merged_##P_##_##K_(int m, const SweepArgs* d, const MergeMap* map, int grid, int lds, hipStream_t s); \
+  int merged_##P_##_##K_##_shape(int n, int* lds);
+GPUE_MERGED(f64, row) GPUE_MERGED(f64, col) GPUE_MERGED(f32, row) GPUE_MERGED(f32, col)
+#undef GPUE_MERGED
+
+int merged_shape(int prec, bool row, int n, int* lds) {
+  if (row) return prec == 64 ? merged_f64_row_shape(n, lds) : merged_f32_row_shape(n, lds);
+  return prec == 64 ? merged_f64_col_shape(n, lds) : merged_f32_col_shape(n, lds);
+}
+
+hipError_t launch_sweep_merged(int prec, bool row, int mode, unsigned flags, int gstate, const SweepArgs* d,
+                               const MergeMap* map, int grid, int lds, hipStream_t s) {
+  if (row) {
+    const int m = row_kernel(mode, flags, gstate);
+    return prec == 64 ? merged_f64_row(m, d, map, grid, lds, s) : merged_f32_row(m, d, map, grid, lds, s);
+  }
+  const int m = col_kernel(mode, gstate);
+  return prec == 64 ? merged_f64_col(m, d, map, grid, lds, s) : merged_f32_col(m, d, map, grid, lds, s);
+}
+
 // Whether the sweep's workgroups are whole waves (64 lanes or a multiple): the
 // deferred norm reduction inside a sweep needs full waves.
 bool sweep_full_waves(int prec, bool row, int N, int var) {

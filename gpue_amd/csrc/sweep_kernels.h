@@ -15,6 +15,7 @@ struct RowCfg {
   static constexpr int WGr = V == 0 ? 128 : 64;
   static constexpr int WG = TPL >= WGr ? TPL : WGr;
   static constexpr int LPW = WG / TPL;
+  static constexpr int LDS = Plan<N, V>::NP > 1 ? LPW * LdsRow<>::footprint(N) : 1;   // elements
 };
 
 // Strided sweeps read TC adjacent x-lines per row of the tile: at least one
@@ -47,6 +48,7 @@ struct ColCfg {
   static constexpr int TC = (TC0 >> NARROW) > 0 ? (TC0 >> NARROW) : 1;
   static constexpr int G = TC0 / TC;   // tiles per default-width tile
   static constexpr int WG = TPL * TC;
+  static constexpr int LDS = Plan<N, PV>::NP > 1 ? TC * N : 1;   // elements
   static_assert(TC0 >= 1 && G >= 1 && WG <= 1024, "strided tile does not fit a workgroup");
 };
 
@@ -59,13 +61,16 @@ __device__ __forceinline__ cx<T> scale_norm(cx<T> v, T inv) {
 
 template <typename T>
 __device__ __forceinline__ double abs2d(cx<T> v) {
-  return (double)v.x * (double)v.x + (double)v.y * (double)v.y;
+  return fma((double)v.x, (double)v.x, (double)v.y * (double)v.y);
 }
 
 // Mode bits above the sweep kind (RM_*, CM_*): 16, the real-time kernel (phases;
 // the plain one is imaginary time); 64, RM_INV compiled without the gauge operator
 // (its three-transform path sets the register count of the whole kernel, and so
 // the waves per SIMD), for sweeps whose flags carry no F_GAUGE_POST.
+
+using OpeningHalf = std::integral_constant<bool, false>;
+using ClosingHalf = std::integral_constant<bool, true>;
 
 // The pending norm's reciprocal for the sweep that opens an imaginary-time step.
 struct NormIn {
@@ -75,11 +80,11 @@ struct NormIn {
   }
   // a deferred renormalisation: the norm reduced here from the previous sweep's
   // partials by every wave (all lanes active), stored once by block 0
-  __device__ __forceinline__ double inverse(const SweepArgs& a, int bid) {
+  __device__ __forceinline__ double inverse(const SweepArgs& a, int bid, int tx) {
     double nrm;
     if (a.flags & F_SCALE_PART) {
       nrm = part.norm(a.partials, a.norm_nb, a.norm_scale);
-      if (bid == 0 && threadIdx.x == 0) *a.norm_out = nrm;
+      if (bid == 0 && tx == 0) *a.norm_out = nrm;
     } else {
       nrm = *a.norm_in;
     }
@@ -128,26 +133,27 @@ __device__ __forceinline__ void pin_args(SweepArgs& a) {
 // ---------------------------------------------------------------------------
 // Row sweep: lines are contiguous x-rows, line = y + yDim*z.
 // ---------------------------------------------------------------------------
-template <typename T, int N, int RV, int MODE_>
-__device__ __forceinline__ void row_body(SweepArgs a, int bid, int nblk) {
+// Block `bid` of nblk of a sweep, by the lanes tx = 0 .. RowCfg::WG - 1 on the LDS at
+// lds (RowCfg::LDS elements) and sh (16 doubles).  ONEWAVE: see lds_sync.
+template <typename T, int N, int RV, int MODE_, bool ONEWAVE = false, bool TWPRE = true>
+__device__ __forceinline__ void row_body(SweepArgs a, int bid, int nblk, int tx, cx<T>* lds, double* sh) {
   constexpr int MODE = MODE_ & 15;
   constexpr bool REAL = (MODE_ & 16) != 0, NG = (MODE_ & 64) != 0;
   constexpr int V = RV & 1;
-  constexpr bool PRE = (RV >> 1) != 0;   // operands and twiddles loaded up front
+  constexpr bool EARLY = (RV >> 1) != 0;     // operands loaded up front
+  constexpr bool PRE = EARLY && TWPRE;       // and every twiddle
   constexpr bool GAUGE = (MODE == RM_INV && !NG) || MODE == RM_GAUGE || MODE == RM_GAUGE_FWD || MODE == RM_FULL;
   constexpr bool KSTEP = MODE == RM_K || MODE == RM_FULL;
   constexpr bool OPENS = !REAL && (MODE == RM_FWD || MODE == RM_FULL);
-  constexpr bool GEARLY = PRE && sizeof(T) == 8;
+  constexpr bool GEARLY = EARLY && sizeof(T) == 8;
   constexpr bool VHALF = MODE != RM_GAUGE && MODE != RM_K && MODE != RM_KSUM;
   using P = Plan<N, V>;
   constexpr int TPL = P::TPL, E = P::E, LPW = RowCfg<N, RV>::LPW;
-  constexpr int FOOT = LdsRow::footprint(N);
-  __shared__ cx<T> lds[P::NP > 1 ? LPW * FOOT : 1];
-  __shared__ double sh[64];
-  if constexpr (PRE) pin_args<VHALF, KSTEP, GAUGE, OPENS>(a);
+  constexpr int FOOT = LdsRow<>::footprint(N);
+  if constexpr (EARLY) pin_args<VHALF, KSTEP, GAUGE, OPENS>(a);
   const Phys& p = a.ph;
   const unsigned flags = a.flags;
-  const int tid = threadIdx.x % TPL, lw = threadIdx.x / TPL;
+  const int tid = tx % TPL, lw = tx / TPL;
   const int line = bid * LPW + lw;
   const bool active = line < a.lines;
   const int ln = active ? line : 0;
@@ -160,7 +166,7 @@ __device__ __forceinline__ void row_body(SweepArgs a, int bid, int nblk) {
   const cx<T>* __restrict__ in = (const cx<T>*)a.in + l.base;
   cx<T>* __restrict__ out = (cx<T>*)a.out + l.base;
   const auto* __restrict__ tw = (const typename TwE<T>::type*)a.tw;
-  const LdsRow la{lw * FOOT};
+  const LdsRow<ONEWAVE> la{lw * FOOT};
   constexpr int RF0 = Seq<N, V, ORD_FWD>::first(), RFL = Seq<N, V, ORD_FWD>::last();
   constexpr int RIN = MODE == RM_INV || MODE == RM_INV_FWD ? RFL : RF0;
   cx<T> v[E];
@@ -173,35 +179,35 @@ __device__ __forceinline__ void row_body(SweepArgs a, int bid, int nblk) {
   const double* __restrict__ Vt = MODE == RM_GAUGE_FWD ? p.Vt_next : p.Vt;
   auto fwd = [&]() { fft_regs_tw<T, N, V, ORD_FWD, -1, PRE>(v, tid, tw, twr, lds, la); };
   auto inv = [&]() { fft_regs_tw<T, N, V, ORD_REV, +1, PRE>(v, tid, tw, twr, lds, la); };
-  auto half = [&]() {
-    if constexpr (PRE) vo.ready();
+  auto half = [&](auto closes) {
+    if constexpr (EARLY) vo.ready();
     else vo.load(p, Vt, l);
-    vo.template half<REAL>(p, l, v);
+    vo.template half<REAL, decltype(closes)::value>(p, l, v);
   };
   auto kstep = [&]() {
-    if constexpr (PRE) ko.ready();
+    if constexpr (EARLY) ko.ready();
     else ko.load(p, l);
     ko.apply(p, l, v, a.invN);
   };
   auto gauge = [&]() {
-    if constexpr (!PRE) {
+    if constexpr (!EARLY) {
       go.load(p, l);
       go.prep(p, l, a.invN);
     }
     go.apply(p, v, l, a.invN, GEARLY);
   };
 
-  if constexpr (PRE && GAUGE) go.load(p, l);
+  if constexpr (EARLY && GAUGE) go.load(p, l);
   if constexpr (OPENS) nin.load(a);
 #pragma unroll
   for (int r = 0; r < E; ++r) v[r] = in[bpos<N, TPL, RIN>(tid, r)];
-  if constexpr (PRE) {
+  if constexpr (EARLY) {
     if constexpr (VHALF) vo.load(p, Vt, l);
     if constexpr (KSTEP) ko.load(p, l);
     if constexpr (GAUGE && GEARLY) {
       if (p.a_kind == A_TABLE) go.load_points(p, l);
     }
-    twr.load(tid, tw);
+    if constexpr (PRE) twr.load(tid, tw);
     if constexpr (GAUGE) go.prep(p, l, a.invN);
   }
 
@@ -210,15 +216,15 @@ __device__ __forceinline__ void row_body(SweepArgs a, int bid, int nblk) {
     if constexpr (MODE == RM_INV_FWD && sizeof(T) == 8) {
       // the closing V/2 of this step and the opening one of the next: phases, which
       // leave |psi|^2, so one phase of the summed exponents
-      if constexpr (PRE) vo.ready();
+      if constexpr (EARLY) vo.ready();
       else vo.load(p, Vt, l);
       T arg[E];
-      vo.args(p, l, v, arg);
+      vo.template args<true>(p, l, v, arg);
       if (p.Vt_next != p.Vt) {   // V(t): the next step's table
         VOp<T, N, TPL, RF0, E> vn;
         vn.load(p, p.Vt_next, l);
         T arg2[E];
-        vn.args(p, l, v, arg2);
+        vn.template args<false>(p, l, v, arg2);
 #pragma unroll
         for (int r = 0; r < E; ++r) arg[r] += arg2[r];
       } else {
@@ -228,11 +234,11 @@ __device__ __forceinline__ void row_body(SweepArgs a, int bid, int nblk) {
       apply_phase_all<T, E, REAL>(v, arg, 1.0);
       fwd();
     } else if constexpr (MODE == RM_INV_FWD) {
-      half();   // FP32 (static V): each half's phase rounds psi, as in single steps
-      half();
+      half(ClosingHalf());   // FP32 (static V): each half's phase rounds psi, as in single steps
+      half(OpeningHalf());
       fwd();
     } else {
-      if (flags & F_HALFV_POST) half();
+      if (flags & F_HALFV_POST) half(ClosingHalf());
       if constexpr (GAUGE) {
         fwd();
         gauge();
@@ -242,13 +248,13 @@ __device__ __forceinline__ void row_body(SweepArgs a, int bid, int nblk) {
   } else {
     if constexpr (OPENS) {
       if (flags & F_SCALE_IN) {
-        const T s = (T)nin.inverse(a, bid);
+        const T s = (T)nin.inverse(a, bid, tx);
 #pragma unroll
         for (int r = 0; r < E; ++r) v[r] = scale_norm(v[r], s);
       }
     }
     if constexpr (MODE == RM_FWD || MODE == RM_FULL) {
-      if (flags & F_HALFV_PRE) half();
+      if (flags & F_HALFV_PRE) half(OpeningHalf());
     }
     fwd();
     if constexpr (MODE == RM_GAUGE || MODE == RM_GAUGE_FWD) {
@@ -258,7 +264,7 @@ __device__ __forceinline__ void row_body(SweepArgs a, int bid, int nblk) {
       kstep();
       inv();
       if constexpr (MODE == RM_FULL) {
-        if (flags & F_HALFV_POST) half();
+        if (flags & F_HALFV_POST) half(ClosingHalf());
         if (flags & F_GAUGE_POST) {
           fwd();
           gauge();
@@ -279,7 +285,7 @@ __device__ __forceinline__ void row_body(SweepArgs a, int bid, int nblk) {
       }
     }
     if constexpr (MODE == RM_GAUGE_FWD) {   // continue with the next step's first row sweep
-      half();
+      half(OpeningHalf());
       fwd();
     }
   }
@@ -299,7 +305,7 @@ __device__ __forceinline__ void row_body(SweepArgs a, int bid, int nblk) {
   }
   if (MODE == RM_KSUM || (NORM && (flags & F_NORM))) {
     double pv[1] = {acc};
-    block_partial<1>(pv, a.partials, sh, bid, nblk);
+    block_partial<1>(pv, a.partials, sh, bid, nblk, tx, RowCfg<N, RV>::WG);
   }
 }
 
@@ -307,30 +313,29 @@ __device__ __forceinline__ void row_body(SweepArgs a, int bid, int nblk) {
 // Strided sweep: lines along y (axis 1, stride xDim) or z (axis 2, stride
 // xDim*yDim); a workgroup owns TC adjacent x-lines, lanes vary fastest in x.
 // ---------------------------------------------------------------------------
-template <typename T, int N, int CV, int MODE_>
-__device__ __forceinline__ void col_body(SweepArgs a, int bid, int nblk) {
+template <typename T, int N, int CV, int MODE_, bool ONEWAVE = false, bool TWPRE = true>
+__device__ __forceinline__ void col_body(SweepArgs a, int bid, int nblk, int tx, cx<T>* lds, double* sh) {
   constexpr int MODE = MODE_ & 15;
   constexpr bool REAL = (MODE_ & 16) != 0;
   constexpr int V = CV & 1;
   constexpr bool EARLY = (CV >> 1) != 0;               // operands loaded up front
-  constexpr bool PRE = EARLY && sizeof(T) == 8;        // and every twiddle
+  constexpr bool PRE = EARLY && TWPRE && sizeof(T) == 8;   // and every twiddle
   constexpr bool GAUGE = MODE == CM_INV_VG || MODE == CM_GAUGE || MODE == CM_GAUGE_FWD;
   constexpr bool GEARLY = EARLY && sizeof(T) == 8;
   constexpr bool VHALF = MODE == CM_FWD_V || MODE == CM_INV_VG || MODE == CM_GAUGE_FWD;
   constexpr bool OPENS = !REAL && MODE == CM_FWD_V;
   using P = Plan<N, V>;
   constexpr int TC = ColCfg<T, N, CV>::TC, E = P::E, TPL = P::TPL;
-  __shared__ cx<T> lds[P::NP > 1 ? TC * N : 1];
-  __shared__ double sh[64];
   if constexpr (EARLY) pin_args<VHALF, MODE == CM_K, GAUGE, OPENS>(a);
   const Phys& p = a.ph;
   const unsigned flags = a.flags;
-  const int c = threadIdx.x % TC, tid = threadIdx.x / TC;
+  const int c = tx % TC, tid = tx / TC;
   const int tiles = (p.xDim + TC - 1) / TC;
-  const int o = bid / tiles, xt = bid - o * tiles;
+  const int bq = bid < nblk ? bid : 0;   // blocks past the last (parts of a merged workgroup) read block 0
+  const int o = bq / tiles, xt = bq - o * tiles;
   const int xi = xt * TC + c;
-  const bool active = xi < p.xDim;
-  const int xq = active ? xi : 0;   // lanes past xDim (a last partial tile) read column 0
+  const bool active = xi < p.xDim && bid < nblk;
+  const int xq = xi < p.xDim ? xi : 0;   // lanes past xDim (a last partial tile) read column 0
   const bool ay = a.axis == 1;
   const LineAt l{a.axis, tid, ay ? (long)xq + (long)o * p.xDim * p.yDim : (long)xq + (long)o * p.xDim,
                  ay ? (long)p.xDim : (long)p.xDim * p.yDim, xq, o};
@@ -341,7 +346,7 @@ __device__ __forceinline__ void col_body(SweepArgs a, int bid, int nblk) {
   const cx<T>* __restrict__ in = (const cx<T>*)a.in + l.base + (long)tid * es;
   cx<T>* __restrict__ out = (cx<T>*)a.out + l.base + (long)tid * es;
   const auto* __restrict__ tw = (const typename TwE<T>::type*)a.tw;
-  const LdsCol la{c, TC};
+  const LdsCol<ONEWAVE> la{c, TC};
   constexpr int RF0 = Seq<N, V, ORD_FWD>::first(), RFL = Seq<N, V, ORD_FWD>::last();
   constexpr int RIN = MODE == CM_INV || MODE == CM_INV_VG ? RFL : RF0;
   cx<T> v[E];
@@ -354,10 +359,10 @@ __device__ __forceinline__ void col_body(SweepArgs a, int bid, int nblk) {
   const double* __restrict__ Vt = MODE == CM_GAUGE_FWD ? p.Vt_next : p.Vt;
   auto fwd = [&]() { fft_regs_tw<T, N, V, ORD_FWD, -1, PRE>(v, tid, tw, twr, lds, la); };
   auto inv = [&]() { fft_regs_tw<T, N, V, ORD_REV, +1, PRE>(v, tid, tw, twr, lds, la); };
-  auto half = [&]() {
+  auto half = [&](auto closes) {
     if constexpr (EARLY) vo.ready();
     else vo.load(p, Vt, l);
-    vo.template half<REAL>(p, l, v);
+    vo.template half<REAL, decltype(closes)::value>(p, l, v);
   };
   auto gauge = [&]() {
     if constexpr (!EARLY) {
@@ -386,7 +391,7 @@ __device__ __forceinline__ void col_body(SweepArgs a, int bid, int nblk) {
     if constexpr (MODE == CM_INV_VG) {
       // the closing sweep of a step that leads with this axis: V/2, then this
       // axis' gauge operator
-      half();
+      half(ClosingHalf());
       fwd();
       gauge();
       inv();
@@ -394,12 +399,12 @@ __device__ __forceinline__ void col_body(SweepArgs a, int bid, int nblk) {
   } else {
     if constexpr (OPENS) {   // the opening sweep of a step that leads with this axis
       if (flags & F_SCALE_IN) {
-        const T s = (T)nin.inverse(a, bid);
+        const T s = (T)nin.inverse(a, bid, tx);
 #pragma unroll
         for (int r = 0; r < E; ++r) v[r] = scale_norm(v[r], s);
       }
     }
-    if constexpr (MODE == CM_FWD_V) half();
+    if constexpr (MODE == CM_FWD_V) half(OpeningHalf());
     fwd();
     if constexpr (MODE == CM_KSUM) {
       if (active) {
@@ -423,7 +428,7 @@ __device__ __forceinline__ void col_body(SweepArgs a, int bid, int nblk) {
       gauge();
       inv();
       if constexpr (MODE == CM_GAUGE_FWD) {   // bridge: the next step's V/2 and its first transform along this axis
-        half();
+        half(OpeningHalf());
         fwd();
       }
     }
@@ -443,7 +448,7 @@ __device__ __forceinline__ void col_body(SweepArgs a, int bid, int nblk) {
   }
   if (MODE == CM_KSUM || (NORM && (flags & F_NORM))) {
     double pv[1] = {acc};
-    block_partial<1>(pv, a.partials, sh, bid, nblk);
+    block_partial<1>(pv, a.partials, sh, bid, nblk, tx, ColCfg<T, N, CV>::WG);
   }
 }
 
@@ -463,9 +468,9 @@ __device__ __forceinline__ void line_body(const SweepArgs& a, int nsteps) {
   constexpr int V = RV & 1;
   constexpr bool PRE = (RV >> 1) != 0;   // twiddles in registers for the whole run
   using P = Plan<N, V>;
-  constexpr int TPL = P::TPL, E = P::E, WG = RowCfg<N, RV>::WG, LPW = RowCfg<N, RV>::LPW, NW = (WG + 63) / 64;
-  constexpr int FOOT = LdsRow::footprint(N);
-  __shared__ cx<T> lds[P::NP > 1 ? LPW * FOOT : 1];
+  constexpr int TPL = P::TPL, E = P::E, WG = RowCfg<N, RV>::WG, NW = (WG + 63) / 64;
+  constexpr int FOOT = LdsRow<>::footprint(N);
+  __shared__ cx<T> lds[RowCfg<N, RV>::LDS];
   __shared__ double sh[16];
   const Phys& p = a.ph;
   const unsigned flags = a.flags;
@@ -473,7 +478,7 @@ __device__ __forceinline__ void line_body(const SweepArgs& a, int nsteps) {
   const bool active = lw == 0;   // further lines of the workgroup repeat line 0
   const LineAt l{0, tid, 0, 1, 0, 0};
   const auto* __restrict__ tw = (const typename TwE<T>::type*)a.tw;
-  const LdsRow la{lw * FOOT};
+  const LdsRow<> la{lw * FOOT};
   constexpr int RF0 = Seq<N, V, ORD_FWD>::first(), RFL = Seq<N, V, ORD_FWD>::last();
   cx<T> v[E];
   TwRegs<T, N, V> twr;
@@ -500,11 +505,11 @@ __device__ __forceinline__ void line_body(const SweepArgs& a, int nsteps) {
 #pragma unroll
       for (int r = 0; r < E; ++r) v[r] = scale_norm(v[r], f);
     }
-    vo.template half<REAL>(p, l, v);
+    vo.template half<REAL, false>(p, l, v);
     fwd();
     ko.apply(p, l, v, a.invN);
     inv();
-    vo.template half<REAL>(p, l, v);
+    vo.template half<REAL, true>(p, l, v);
     if (gauge) {
       fwd();
       go.apply(p, v, l, a.invN, false);
@@ -542,7 +547,9 @@ __global__ void __launch_bounds__((RowCfg<N, V>::WG)) line_steps(SweepArgs a, in
 // One problem per launch (arguments by value) ...
 template <typename T, int N, int V, int MODE>
 __global__ void __launch_bounds__((RowCfg<N, V>::WG)) row_sweep(SweepArgs a) {
-  row_body<T, N, V, MODE>(a, blockIdx.x, gridDim.x);
+  __shared__ cx<T> lds[RowCfg<N, V>::LDS];
+  __shared__ double sh[16];
+  row_body<T, N, V, MODE>(a, blockIdx.x, gridDim.x, threadIdx.x, lds, sh);
 }
 // Workgroups are dealt to the 8 XCDs round robin (block b runs on XCD b % 8).
 // With narrowed tiles, the G tiles of one default-width tile (one 128-byte
@@ -563,7 +570,9 @@ __device__ __forceinline__ int xcd_tile(int b, int nblk) {
 
 template <typename T, int N, int CV, int MODE>
 __global__ void __launch_bounds__((ColCfg<T, N, CV>::WG)) col_sweep(SweepArgs a) {
-  col_body<T, N, CV, MODE>(a, xcd_tile<ColCfg<T, N, CV>::G>(blockIdx.x, gridDim.x), gridDim.x);
+  __shared__ cx<T> lds[ColCfg<T, N, CV>::LDS];
+  __shared__ double sh[16];
+  col_body<T, N, CV, MODE>(a, xcd_tile<ColCfg<T, N, CV>::G>(blockIdx.x, gridDim.x), gridDim.x, threadIdx.x, lds, sh);
 }
 
 // ... or many problems of one shape per launch: blocks [i*bpi, (i+1)*bpi) work
@@ -572,13 +581,17 @@ template <typename T, int N, int V, int MODE>
 __global__ void __launch_bounds__((RowCfg<N, V>::WG)) row_sweep_b(const SweepArgs* __restrict__ args, int bpi) {
   const SweepArgs& a = args[blockIdx.x / bpi];
   if (!a.active) return;
-  row_body<T, N, V, MODE>(a, blockIdx.x % bpi, bpi);
+  __shared__ cx<T> lds[RowCfg<N, V>::LDS];
+  __shared__ double sh[16];
+  row_body<T, N, V, MODE>(a, blockIdx.x % bpi, bpi, threadIdx.x, lds, sh);
 }
 template <typename T, int N, int CV, int MODE>
 __global__ void __launch_bounds__((ColCfg<T, N, CV>::WG)) col_sweep_b(const SweepArgs* __restrict__ args, int bpi) {
   const SweepArgs& a = args[blockIdx.x / bpi];
   if (!a.active) return;
-  col_body<T, N, CV, MODE>(a, blockIdx.x % bpi, bpi);
+  __shared__ cx<T> lds[ColCfg<T, N, CV>::LDS];
+  __shared__ double sh[16];
+  col_body<T, N, CV, MODE>(a, blockIdx.x % bpi, bpi, threadIdx.x, lds, sh);
 }
 
 }  // namespace gpue

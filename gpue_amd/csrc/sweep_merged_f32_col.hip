@@ -1,0 +1,8 @@
+// merged col sweeps, float
+#include "sweep_merged.h"
+namespace gpue {
+hipError_t merged_f32_col(int m, const SweepArgs* d, const MergeMap* map, int grid, int lds, hipStream_t s) {
+  return launch_col_merged<float>(m, d, map, grid, lds, s);
+}
+int merged_f32_col_shape(int n, int* lds) { return merged_col_shape<float>(n, lds); }
+}  // namespace gpue

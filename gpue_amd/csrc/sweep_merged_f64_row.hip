@@ -1,0 +1,8 @@
+// merged row sweeps, double
+#include "sweep_merged.h"
+namespace gpue {
+hipError_t merged_f64_row(int m, const SweepArgs* d, const MergeMap* map, int grid, int lds, hipStream_t s) {
+  return launch_row_merged<double>(m, d, map, grid, lds, s);
+}
+int merged_f64_row_shape(int n, int* lds) { return merged_row_shape<double>(n, lds); }
+}  // namespace gpue

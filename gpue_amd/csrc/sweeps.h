@@ -353,12 +353,12 @@ __device__ __forceinline__ void arrive(cx<U>& x) {
   arrive(x.y);
 }
 
-// A scaled point.  FP32 rounds the product here: contracted into the butterfly that
-// follows it, results would depend on what the compiler sees next to each other.
+// A scaled point, rounded here: contracted into the butterfly that follows it, results
+// would depend on what the compiler sees next to each other.
 template <typename T>
 __device__ __forceinline__ cx<T> scaled(cx<T> v, T s) {
   cx<T> r = cscale(v, s);
-  if constexpr (sizeof(T) == 4) arrive(r);
+  arrive(r);
   return r;
 }
 
@@ -426,7 +426,7 @@ __device__ __forceinline__ void apply_phase_all(cx<T>* v, const T (&arg)[E], dou
       for (int r = 0; r < E; ++r) tiny = tiny && fabs(arg[r]) <= SMALL_ARG;
       if (tiny) {
 #pragma unroll
-        for (int r = 0; r < E; ++r) v[r] = cscale(v[r], exp_small(-arg[r]) * s);
+        for (int r = 0; r < E; ++r) v[r] = scaled(v[r], exp_small(-arg[r]) * s);
         return;
       }
     }
@@ -500,7 +500,10 @@ struct VOp {
 #pragma unroll
     for (int r = 0; r < E; ++r) arrive(e[r]);
   }
-  // exponents of the half step on v.  FP32 adds the axes in the order x, y, z.
+  // exponents of the half step on v.  FP32 adds the axes in the order x, y, z, and the
+  // density takes the square of x after that of y in a step's first half, before it in
+  // its second (CLOSES): the roundings these steps have always had.
+  template <bool CLOSES>
   __device__ __forceinline__ void args(const Phys& p, const LineAt& l, const cx<T>* v, T (&arg)[E]) const {
     const T cV = (T)p.cV;
     if constexpr (sizeof(T) == 8) {
@@ -518,16 +521,16 @@ struct VOp {
       const T g = (T)p.g, cH = (T)p.cH;
 #pragma unroll
       for (int r = 0; r < E; ++r) {
-        if constexpr (sizeof(T) == 4) arrive(arg[r]);   // rounded before the sum
-        const T d = v[r].x * v[r].x + v[r].y * v[r].y;
-        arg[r] += g * d * cH;
+        arrive(arg[r]);   // rounded before the sum
+        const T d = CLOSES ? fma(v[r].x, v[r].x, v[r].y * v[r].y) : fma(v[r].y, v[r].y, v[r].x * v[r].x);
+        arg[r] = fma(g * d, cH, arg[r]);
       }
     }
   }
-  template <bool REAL>
+  template <bool REAL, bool CLOSES>
   __device__ __forceinline__ void half(const Phys& p, const LineAt& l, cx<T>* v) const {
     T arg[E];
-    args(p, l, v, arg);
+    args<CLOSES>(p, l, v, arg);
     apply_phase_all<T, E, REAL>(v, arg, 1.0);
   }
 };
@@ -605,7 +608,7 @@ struct GOp {
         const int r = q * R + k;
         const bool wrap = l.tid + TPL * q + NR * k >= N / 2;
         if constexpr (REAL) v[r] = cmul(wrap ? cmul(w[k], Z) : w[k], v[r]);
-        else v[r] = cscale(v[r], wrap ? w[k].x * Z.x : w[k].x);
+        else v[r] = scaled(v[r], wrap ? w[k].x * Z.x : w[k].x);
       }
       if (q + 1 < Q) {
 #pragma unroll
@@ -681,7 +684,7 @@ struct KOp {
       } else if constexpr (sizeof(T) == 8) {
         const T f = f0.x * f1.x * (T)invN;
 #pragma unroll
-        for (int r = 0; r < E; ++r) v[r] = cscale(v[r], e[r].x * f);
+        for (int r = 0; r < E; ++r) v[r] = scaled(v[r], e[r].x * f);
       } else {
 #pragma unroll
         for (int r = 0; r < E; ++r)
@@ -737,22 +740,24 @@ __device__ __forceinline__ double wave_sum(double x, int width) {
   return x;
 }
 
+// Lanes tx of a block of `width` (the workgroup, or a part of one whose other parts sum
+// in step); lane 0 gets the totals.
 template <int NA>
-__device__ __forceinline__ void block_sum(double (&v)[NA], double* sh /* >= NA * 16 */) {
+__device__ __forceinline__ void block_sum(double (&v)[NA], double* sh /* >= NA * 16 */, int tx, int width) {
   // a workgroup smaller than a wave (strided sweeps of 16- and 32-point lines
   // with narrow tiles) has lanes past its end: the sum stays within the
   // workgroup's lanes
 #pragma unroll
-  for (int a = 0; a < NA; ++a) v[a] = wave_sum(v[a], (int)blockDim.x);
-  const int w = threadIdx.x >> 6, nw = (blockDim.x + 63) >> 6;
+  for (int a = 0; a < NA; ++a) v[a] = wave_sum(v[a], width);
+  const int w = tx >> 6, nw = (width + 63) >> 6;
   if (nw == 1) return;   // every lane holds the total
   __syncthreads();
-  if ((threadIdx.x & 63) == 0) {
+  if ((tx & 63) == 0) {
 #pragma unroll
     for (int a = 0; a < NA; ++a) sh[a * 16 + w] = v[a];
   }
   __syncthreads();
-  if (threadIdx.x == 0) {
+  if (tx == 0) {
 #pragma unroll
     for (int a = 0; a < NA; ++a) {
       double s = 0.0;
@@ -856,9 +861,9 @@ struct PartNorm {
 // Block b of nb (of one problem) stores its NA partial sums.
 template <int NA>
 __device__ __forceinline__ void block_partial(double (&v)[NA], double* partials, double* sh, unsigned b,
-                                              unsigned nb) {
-  block_sum<NA>(v, sh);
-  if (threadIdx.x == 0) {
+                                              unsigned nb, int tx, int width) {
+  block_sum<NA>(v, sh, tx, width);
+  if (tx == 0 && b < nb) {
 #pragma unroll
     for (int a = 0; a < NA; ++a) partials[(size_t)a * nb + b] = v[a];
   }

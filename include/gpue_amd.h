@@ -215,16 +215,19 @@ gpue_status gpue_eqn_parse(const char *expr, const char *const *names, const dou
 double      gpue_eqn_eval(const gpue_eqn_node *nodes, int n_nodes, double x, double y, double z, double t);
 
 /* --- batched instances (no reference counterpart: GPUE solves one problem per
- * process; its bin/run.sh starts several processes).  Instances of one shape
- * share every sweep launch; the shape groups run on at most four streams (the
- * device's hardware queues per process: the three groups with the most work
- * get one each, the rest share the fourth), two steps of a group captured as
- * a HIP graph and replayed, so the groups overlap on the device.
- * The kernel variants are the contexts' own (equal within a group; a batch
- * may prefer other variants than a lone instance: the groups share the
- * device).  Contexts stay owned by the caller and must outlive the
- * batch; results are read through the contexts (gpue_energy, gpue_download_wfc).
- * Contexts with a time-dependent V or on different devices are rejected. --- */
+ * process; its bin/run.sh starts several processes).  2D and 3D instances of one
+ * precision, dimension and gauge whose axes are 64 to 512 points, with the
+ * variants small contexts start with, share every sweep launch, whatever their
+ * sizes.  Other instances form groups of one shape that share launches; groups
+ * run on at most four streams (the device's hardware queues per process: the
+ * three groups with the most work get one each, the rest share the fourth).
+ * Blocks of steps of a group are captured as HIP graphs and replayed.
+ * Outside merged launches the kernel variants are the contexts' own (equal
+ * within a group; a batch may prefer other variants than a lone instance: the
+ * groups share the device).  Contexts stay owned by the caller and must outlive
+ * the batch; results are read through the contexts (gpue_energy,
+ * gpue_download_wfc).  Contexts with a time-dependent V or on different devices
+ * are rejected. --- */
 typedef struct gpue_batch gpue_batch;
 gpue_status gpue_batch_create(gpue_ctx *const *ctxs, int n, gpue_batch **out);
 /* Exclude (0) or include (1) instance `index` from the following steps. */
@@ -239,8 +242,8 @@ gpue_status gpue_batch_evolve(gpue_batch *b, int nsteps, int gstate);
  * evaluation captured as one HIP graph at the first call and replayed after;
  * any change of its parameters, fields or variants drops the graph. */
 gpue_status gpue_batch_energy(gpue_batch *b, double *energy, double *mu);
-/* How pairs of steps are replayed: 0 (default) one graph per shape group on the
- * group's stream, launched group by group, most work first; 1 one graph for the whole batch, a
+/* How steps are replayed: 0 (default) graphs per group on the group's stream,
+ * launched group by group, most work first; 1 one graph for the whole batch, a
  * branch per group forked onto the group streams, so a pair of steps of every
  * instance is one launch; 2 no graphs (every sweep launched on its own, for
  * kernel tracers). */
@@ -248,7 +251,7 @@ gpue_status gpue_batch_set_graph_mode(gpue_batch *b, int mode);
 /* No counterpart in the reference (GPUE runs one problem per process): choose
  * the kernel variants of every shape group, and the graph mode, for the batch
  * as a whole (a lone instance's choice serves latency; in a batch the groups
- * share the device).  Coordinate descent over the groups, largest first, and
+ * share the device; merged launches have one set of variants).  Coordinate descent over the groups, largest first, and
  * their axes; each candidate is timed over `steps` steps of gstate of the whole
  * batch.  Every instance's psi, step counter and pending norm are restored
  * afterwards.  us_per_step, graph_mode (either may be NULL): the best time per
