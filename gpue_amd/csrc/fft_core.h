@@ -357,16 +357,44 @@ __device__ __forceinline__ void pass_compute(cx<T>* v, int tid, const typename T
   }
 }
 
-// Output position of register slot (q, s) after pass (R, L).
-template <int N, int TPL, int R, int L>
-__device__ __forceinline__ int pass_out(int tid, int q, int s) {
-  const int j = tid + TPL * q;
-  const int k = j % L;
-  return (j / L) * L * R + k + s * L;
+// The LDS layout of the exchange between pass (R, L) and the next one: element e of a
+// line lies at e + (e/B)*U.  C lanes with consecutive tid store 128 bytes, what the LDS
+// takes in a clock, if their places differ modulo C; pass (R, L) puts lane tid at
+// (tid/L)*L*R + tid%L, so unpadded blocks of L*R (even R) meet in the same banks.  A gap
+// of L after each block spreads them: (tid/L)*L*(R+1) for an even R.  Blocks shorter than
+// C take one gap per C elements; where L >= C lanes are contiguous already.  (R >= 8 for
+// L > 1, and for C = 2, keeps the gaps within 1/8 of the line.)  The reads that follow are
+// contiguous.
+// Rows have C = 8 (FP64) or 16, narrow strided tiles 2-4; tiles of whole 128-byte rows
+// C = 1, no gaps.  The former layouts (a gap per 16 elements in rows, none in strided
+// tiles) met 2-way conflicts in radix-8 and radix-4 rows, 4-way ones in quarter tiles.
+// 100 steps with energy and download (FP64): 384x192 field tables 2.59 -> 2.48 ms, 512^2
+// rotating 3.02 -> 2.96 (imaginary) and 2.77 -> 2.70 (real time), 256^2 1.45 -> 1.42;
+// 200 steps of sixteen FP32 problems 17.1 -> 16.2 ms.
+template <int R, int L, int C>
+struct LdsGap {
+  static constexpr bool POW2 = (L * R & (L * R - 1)) == 0;
+  static constexpr int B = POW2 && L * R < C ? C : L * R;
+  static constexpr int U = R % 2 == 0 && L < C && (R >= 8 || (L == 1 && C > 2)) && (L == 1 || L % 2 == 0) ? L : 0;
+  static constexpr int span(int N) { return N + (N - 1) / B * U; }
+};
+// Elements of LDS that a line needs over the exchanges of both orders of its plan.
+template <int N, int V, int C, int ORD, int P = 0>
+constexpr int lds_span_of() {
+  using S = Seq<N, V, ORD>;
+  if constexpr (P + 1 >= Plan<N, V>::NP) {
+    return N;
+  } else {
+    constexpr int a = LdsGap<S::radix(P), S::Lbefore(P), C>::span(N), b = lds_span_of<N, V, C, ORD, P + 1>();
+    return a > b ? a : b;
+  }
+}
+template <int N, int V, int C>
+constexpr int lds_span() {
+  constexpr int a = lds_span_of<N, V, C, ORD_FWD>(), b = lds_span_of<N, V, C, ORD_REV>();
+  return a > b ? a : b;
 }
 
-// LDS addressing: element e of a line.  Row lines: base + pad(e); strided
-// lines: (e * LS + c) where LS = lines per tile (lanes vary in c fastest).
 // sync() orders the exchange: the workgroup's barrier, or, where the lines of one wave
 // have LDS of their own within a larger workgroup (ONEWAVE), program order, which the
 // LDS unit keeps for a wave.
@@ -379,18 +407,44 @@ __device__ __forceinline__ void lds_sync() {
     __syncthreads();
   }
 }
-template <bool ONEWAVE = false>
-struct LdsRow {
+// A line's elements in LDS: LS apart (the lines of a strided tile lie side by side, and
+// its lanes vary in the line fastest; a row has LS = 1).
+template <typename T, int LS>
+constexpr int lds_lanes() {   // C of LdsGap
+  return 128 / (LS * 2 * (int)sizeof(T)) > 1 ? 128 / (LS * 2 * (int)sizeof(T)) : 1;
+}
+template <typename T, int LS, bool ONEWAVE = false>
+struct LdsLine {
+  static constexpr int C = lds_lanes<T, LS>();
   int base;
   static __device__ __forceinline__ void sync() { lds_sync<ONEWAVE>(); }
-  __device__ __forceinline__ int at(int e) const { return base + e + (e >> 4); }
-  static constexpr int footprint(int N) { return N + N / 16; }
-};
-template <bool ONEWAVE = false>
-struct LdsCol {
-  int c, LS;
-  static __device__ __forceinline__ void sync() { lds_sync<ONEWAVE>(); }
-  __device__ __forceinline__ int at(int e) const { return e * LS + c; }
+  // stores and loads of the exchange between pass (R, L) and the one of radix RN
+  template <int N, int TPL, int E, int R, int L>
+  __device__ __forceinline__ void put(cx<T>* lds, const cx<T>* v, int tid) const {
+    using G = LdsGap<R, L, C>;
+#pragma unroll
+    for (int q = 0; q < E / R; ++q) {
+      const int j = tid + TPL * q, e0 = j / L * (L * R), k = j % L;
+      cx<T>* p = lds + base + (e0 + k + e0 / G::B * G::U) * LS;   // no gap between the R of a lane
+#pragma unroll
+      for (int s = 0; s < R; ++s) p[s * L * LS] = v[q * R + s];
+    }
+  }
+  template <int N, int TPL, int E, int R, int L, int RN>
+  __device__ __forceinline__ void get(const cx<T>* lds, cx<T>* v, int tid) const {
+    using G = LdsGap<R, L, C>;
+    const cx<T>* p = lds + base + (tid + tid / G::B * G::U) * LS;
+#pragma unroll
+    for (int r = 0; r < E; ++r) {
+      const int off = bpos<N, TPL, RN>(0, r);
+      if (off % G::B == 0) {
+        v[r] = p[(off + off / G::B * G::U) * LS];
+      } else {
+        const int e = tid + off;
+        v[r] = lds[base + (e + e / G::B * G::U) * LS];
+      }
+    }
+  }
 };
 
 // Full transform on registers: input in boundary layout of first radix,
@@ -406,11 +460,9 @@ __device__ __forceinline__ void fft_from_pass(cx<T>* v, int tid, const typename 
     if constexpr (P > 0) {
       constexpr int RP = S::radix(P - 1), LP = S::Lbefore(P - 1);
       LA::sync();  // previous users of LDS are done
-#pragma unroll
-      for (int r = 0; r < E; ++r) lds[la.at(pass_out<N, TPL, RP, LP>(tid, r / RP, r % RP))] = v[r];
+      la.template put<N, TPL, E, RP, LP>(lds, v, tid);
       LA::sync();
-#pragma unroll
-      for (int r = 0; r < E; ++r) v[r] = lds[la.at(bpos<N, TPL, S::radix(P)>(tid, r))];
+      la.template get<N, TPL, E, RP, LP, S::radix(P)>(lds, v, tid);
     }
     pass_compute<T, N, E, S::radix(P), S::Lbefore(P), SIGN, PRE>(v, tid, tw + TwTab<N, V>::template off<ORD>(P),
                                                                  w + TwPlan<N, V, ORD>::off(P));

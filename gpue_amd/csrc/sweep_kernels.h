@@ -15,7 +15,10 @@ struct RowCfg {
   static constexpr int WGr = V == 0 ? 128 : 64;
   static constexpr int WG = TPL >= WGr ? TPL : WGr;
   static constexpr int LPW = WG / TPL;
-  static constexpr int LDS = Plan<N, V>::NP > 1 ? LPW * LdsRow<>::footprint(N) : 1;   // elements
+  // elements of a line (the larger of both precisions) and of the workgroup
+  static constexpr int FOOT64 = lds_span<N, V, lds_lanes<double, 1>()>(), FOOT32 = lds_span<N, V, lds_lanes<float, 1>()>();
+  static constexpr int FOOT = FOOT64 > FOOT32 ? FOOT64 : FOOT32;
+  static constexpr int LDS = Plan<N, V>::NP > 1 ? LPW * FOOT : 1;
 };
 
 // Strided sweeps read TC adjacent x-lines per row of the tile: at least one
@@ -48,7 +51,7 @@ struct ColCfg {
   static constexpr int TC = (TC0 >> NARROW) > 0 ? (TC0 >> NARROW) : 1;
   static constexpr int G = TC0 / TC;   // tiles per default-width tile
   static constexpr int WG = TPL * TC;
-  static constexpr int LDS = Plan<N, PV>::NP > 1 ? TC * N : 1;   // elements
+  static constexpr int LDS = Plan<N, PV>::NP > 1 ? TC * lds_span<N, PV, lds_lanes<T, TC>()>() : 1;   // elements
   static_assert(TC0 >= 1 && G >= 1 && WG <= 1024, "strided tile does not fit a workgroup");
 };
 
@@ -149,7 +152,6 @@ __device__ __forceinline__ void row_body(SweepArgs a, int bid, int nblk, int tx,
   constexpr bool VHALF = MODE != RM_GAUGE && MODE != RM_K && MODE != RM_KSUM;
   using P = Plan<N, V>;
   constexpr int TPL = P::TPL, E = P::E, LPW = RowCfg<N, RV>::LPW;
-  constexpr int FOOT = LdsRow<>::footprint(N);
   if constexpr (EARLY) pin_args<VHALF, KSTEP, GAUGE, OPENS>(a);
   const Phys& p = a.ph;
   const unsigned flags = a.flags;
@@ -166,7 +168,7 @@ __device__ __forceinline__ void row_body(SweepArgs a, int bid, int nblk, int tx,
   const cx<T>* __restrict__ in = (const cx<T>*)a.in + l.base;
   cx<T>* __restrict__ out = (cx<T>*)a.out + l.base;
   const auto* __restrict__ tw = (const typename TwE<T>::type*)a.tw;
-  const LdsRow<ONEWAVE> la{lw * FOOT};
+  const LdsLine<T, 1, ONEWAVE> la{lw * RowCfg<N, RV>::FOOT};
   constexpr int RF0 = Seq<N, V, ORD_FWD>::first(), RFL = Seq<N, V, ORD_FWD>::last();
   constexpr int RIN = MODE == RM_INV || MODE == RM_INV_FWD ? RFL : RF0;
   cx<T> v[E];
@@ -346,7 +348,7 @@ __device__ __forceinline__ void col_body(SweepArgs a, int bid, int nblk, int tx,
   const cx<T>* __restrict__ in = (const cx<T>*)a.in + l.base + (long)tid * es;
   cx<T>* __restrict__ out = (cx<T>*)a.out + l.base + (long)tid * es;
   const auto* __restrict__ tw = (const typename TwE<T>::type*)a.tw;
-  const LdsCol<ONEWAVE> la{c, TC};
+  const LdsLine<T, TC, ONEWAVE> la{c};
   constexpr int RF0 = Seq<N, V, ORD_FWD>::first(), RFL = Seq<N, V, ORD_FWD>::last();
   constexpr int RIN = MODE == CM_INV || MODE == CM_INV_VG ? RFL : RF0;
   cx<T> v[E];
@@ -469,7 +471,6 @@ __device__ __forceinline__ void line_body(const SweepArgs& a, int nsteps) {
   constexpr bool PRE = (RV >> 1) != 0;   // twiddles in registers for the whole run
   using P = Plan<N, V>;
   constexpr int TPL = P::TPL, E = P::E, WG = RowCfg<N, RV>::WG, NW = (WG + 63) / 64;
-  constexpr int FOOT = LdsRow<>::footprint(N);
   __shared__ cx<T> lds[RowCfg<N, RV>::LDS];
   __shared__ double sh[16];
   const Phys& p = a.ph;
@@ -478,7 +479,7 @@ __device__ __forceinline__ void line_body(const SweepArgs& a, int nsteps) {
   const bool active = lw == 0;   // further lines of the workgroup repeat line 0
   const LineAt l{0, tid, 0, 1, 0, 0};
   const auto* __restrict__ tw = (const typename TwE<T>::type*)a.tw;
-  const LdsRow<> la{lw * FOOT};
+  const LdsLine<T, 1> la{lw * RowCfg<N, RV>::FOOT};
   constexpr int RF0 = Seq<N, V, ORD_FWD>::first(), RFL = Seq<N, V, ORD_FWD>::last();
   cx<T> v[E];
   TwRegs<T, N, V> twr;
