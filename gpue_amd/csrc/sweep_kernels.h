@@ -49,7 +49,11 @@ struct ColCfg {
   static constexpr int TCm = 131072 / (N * 2 * (int)sizeof(T));
   static constexpr int TC0 = TCw < TCm ? TCw : TCm;
   static constexpr int TC = (TC0 >> NARROW) > 0 ? (TC0 >> NARROW) : 1;
-  static constexpr int G = TC0 / TC;   // tiles per default-width tile
+  // tiles that share 128-byte lines, or make up a default-width one: on one XCD (xcd_tile).
+  // (FP64 tiles of 2048 points are 4 columns, half lines; a line in two L2s made the K
+  // sweep of 2048^2 take 51 us next to 31 of a row sweep.  With it, and the exchange gaps
+  // of fft_core.h, an imaginary step there takes 101 instead of 112 us.)
+  static constexpr int G = TC0 < TCmin ? TCmin / TC : TC0 / TC;
   static constexpr int WG = TPL * TC;
   static constexpr int LDS = Plan<N, PV>::NP > 1 ? TC * lds_span<N, PV, lds_lanes<T, TC>()>() : 1;   // elements
   static_assert(TC0 >= 1 && G >= 1 && WG <= 1024, "strided tile does not fit a workgroup");
