@@ -211,6 +211,19 @@ double gpue::ramp_scale(const gpue_ctx* c, int step) {
   return w * (double)(step + 1) / (double)c->ramp_steps;
 }
 
+// Real-time strided sweeps on whole-width tiles hold complex factors of every point
+// beside psi: one or two waves per SIMD, or spills in 1024-lane workgroups.  Contexts that
+// run the default variants take narrower tiles, operands up front, for the K sweeps of
+// FP64 (quarter tiles in 3D, 192^3 186 -> 171 us a step, 256^3 377 -> 352; half tiles in 2D,
+// 2048 x 1024 53.8 -> 48.1; 384 and 4096 points would lose 1-5 %) and for all of FP32's in 2D
+// (2048^2 77.4 -> 65.8).  A tile's width changes no rounding in real time, which has no norm.
+static int realtime_variant(const gpue_ctx* c, int gstate, const Sweep& s) {
+  if (!c->var_default || !gstate || s.row || c->var[s.axis] != 0) return -1;
+  const int n = c->dims[s.axis];
+  if (c->p.dimnum == 3) return c->prec == 64 && s.mode == CM_K && (n == 192 || n == 256) ? 4 : -1;
+  return (n == 1024 || n == 2048) && (c->prec == 32 || s.mode == CM_K) ? 2 : -1;
+}
+
 // Sweeps of step i (src/evolution.cu:727-870): V/2, the forward transforms, K,
 // the inverse transforms, V/2, then the gauge operators in GPUE's order (x -> y
 // (-> z) on odd steps, (z ->) y -> x on even ones, src/evolution.cu:837,842).
@@ -268,6 +281,7 @@ void gpue::schedule(const gpue_ctx* c, int gstate, int i, bool pending, std::vec
   out.push_back(lead == 0 ? Sweep{true, 0, RM_INV, fc, invc} : Sweep{false, lead, CM_INV_VG, fc, invc});
   for (int k = 1; k < ng; ++k)
     out.push_back(G[k] == 0 ? Sweep{true, 0, RM_GAUGE, 0u, 1.0 / n[0]} : Sweep{false, G[k], CM_GAUGE, 0u, 1.0 / n[G[k]]});
+  for (Sweep& s : out) s.var = realtime_variant(c, gstate, s);
   if (gstate == 0) out.back().flags |= F_NORM;
 }
 
@@ -352,13 +366,38 @@ static gpue_status settle_deferred(gpue_ctx* c) {
   return GPUE_OK;
 }
 
-// The variants every context starts with (no timing, so results never depend on
-// it): for small, latency-bound grids narrow lines with up-front twiddle loads
-// and quarter strided tiles (the autotuner's choice for 2D grids of
-// 128^2-512^2), wide lines otherwise.
+// The variants every context starts with: a rule on sizes, no timing, so results never
+// depend on it.  (Figures: us a step, imaginary / real time, the former rule -> this one;
+// it had narrow lines and quarter tiles up to 2^20 points, wide ones beyond.)
+//  * Up to 2^18 points (2^20 in 3D) launches are latency bound: narrow lines, operands up
+//    front, quarter tiles (512^2 FP64 18.3 / 14.5, wide 25.3 / 20.5).
+//  * 2D to 2^20 points: waves enough that rows may load late, and past 2^19 long columns
+//    take half tiles, 64 bytes of a row (1024^2 rotating FP64 72.1 / 73.3 -> 67.3 / 61.5,
+//    FP32 48.6 / 44.5 -> 45.0 / 42.1; 512 x 1024 FP32 20.2 / 17.5 -> 19.5 / 17.0).
+//  * 2D beyond: whole-width tiles, and from 2^22 on FP64 rows of up to 2048 points spread
+//    over more lanes (2048^2 100.5 -> 95.7; 1024 x 2048 would lose 8 %).  FP32 columns of
+//    1024 and 2048 points are one 1024-lane workgroup of 128 KiB a CU: half tiles up to
+//    2^21 points (2048 x 1024 50.7 -> 44.3; 2048^2 would lose 2 %).
+//  * 3D beyond: wide tiles of lines up to 96 points are 64 columns in 64-96 KiB: quarter
+//    tiles, in FP64 of 8- or 12-point lanes (256 x 256 x 96 FP64 204 / 164 -> 188 / 152;
+//    192 x 192 x 64 rotating 105.8 / 108.0 -> 101.9 / 99.0); not 48, whose narrow plan has
+//    as many points a lane and a pass more.  FP64 lines of 128: 8 points a lane (128^3
+//    67.1 / 61.6 -> 61.3 / 53.2).  FP32 keeps its plans, so its rounding, and whole tiles
+//    below 64 points, where narrowed ones are less than a wave, and for 64 along y (64 x 64
+//    x 512 would lose 3 %).
 static int default_variant(const gpue_ctx* c, int axis) {
-  const bool small = c->N <= (1L << 20);
-  return axis == 0 ? (small ? 3 : 0) : (small ? 5 : 0);
+  const int n = c->dims[axis];
+  const bool f64 = c->prec == 64;
+  if (c->p.dimnum == 3) {
+    if (c->N <= (1L << 20)) return axis == 0 ? 3 : 5;
+    if (axis == 0) return 0;
+    if (!f64) return n == 96 || (n == 64 && axis == 2) ? 4 : 0;
+    return n <= 96 && n != 48 ? 5 : n == 128 ? 1 : 0;
+  }
+  if (c->N <= (1L << 18)) return axis == 0 ? 3 : 5;
+  if (c->N <= (1L << 20)) return axis == 0 ? 1 : c->N > (1L << 19) && n >= 512 ? 3 : 5;
+  if (axis == 0) return f64 && c->N >= (1L << 22) && n <= 2048 ? 1 : 0;
+  return !f64 && c->N <= (1L << 21) && (n == 1024 || n == 2048) ? 2 : 0;
 }
 
 static gpue_status sweep_args(gpue_ctx* c, const Sweep& s, const Phys& ph, const void* in, void* out, SweepArgs& a) {
@@ -774,6 +813,7 @@ gpue_status gpue::ctx_create(const gpue_params* pin, hipStream_t ext_stream, gpu
     if (p.dimnum > 2) nb = std::max<size_t>(nb, sweep_blocks(c->prec, false, p.zDim, v, p.xDim, p.yDim));
   }
   for (int a = 0; a < 3; ++a) c->var[a] = default_variant(c, a);
+  c->var_default = true;
   c->partials_n = nb * 4;
   if (hipMalloc((void**)&c->partials, c->partials_n * sizeof(double)) != hipSuccess ||
       hipMalloc((void**)&c->results, 16 * sizeof(double)) != hipSuccess ||
@@ -1347,6 +1387,7 @@ static gpue_status autotune(gpue_ctx* c, int reps) {
   HIPCHK(c, hipEventCreate(&e0));
   HIPCHK(c, hipEventCreate(&e1));
   double cost[3][N_VARIANTS] = {};
+  c->var_default = false;   // every sweep of an axis runs what is chosen for it
   std::vector<Sweep> sched;
   const bool timing = c->timing;
   c->timing = false;
@@ -1943,6 +1984,7 @@ gpue_status gpue_set_variants(gpue_ctx* c, const int* variants) {
     if (variants[a] < 0 || variants[a] >= N_VARIANTS) return fail(c, GPUE_EINVAL, "variant out of range");
   }
   for (int a = 0; a < 3; ++a) c->var[a] = variants[a];
+  c->var_default = false;
   drop_graphs(c);
   return GPUE_OK;
 }
