@@ -69,6 +69,12 @@ bool take(int device, Buffer& out) {
   return true;
 }
 
+// Whether the pool holds buffers for a transfer to overlap its halves.
+bool pooled(int device) {
+  std::lock_guard<std::mutex> lk(pool_mu);
+  return std::count_if(pool.begin(), pool.end(), [&](const Buffer& b) { return b.device == device; }) >= 2;
+}
+
 void give(Buffer& b) {
   {
     std::lock_guard<std::mutex> lk(pool_mu);
@@ -269,6 +275,9 @@ hipError_t copy_to_host(void* host, const void* dev, size_t n, size_t es, bool w
 
 // The other way (doubles rounded to floats with `narrow`); returns when the device
 // holds them.  64 MiB 2.3 -> 1.7 ms, 256 MiB 8.9 -> 5.9 ms, 256^3 FP32 38.1 -> 3.5 ms.
+// A program's first upload, without conversion, takes HIP's own path too: allocating the
+// ring (about 0.4 ms a buffer) would cost more than it saves (a new 128 x 128 x 96
+// context with its upload took 12.8 ms, with the ring 15.4).
 hipError_t copy_to_device(void* dev, const void* host, size_t n, size_t es, bool narrow, int device,
                           hipStream_t stream) {
   Job j;
@@ -279,7 +288,7 @@ hipError_t copy_to_device(void* dev, const void* host, size_t n, size_t es, bool
   j.conv = narrow;
   j.down = false;
   j.stream = stream;
-  if (!narrow && n * es < DIRECT_UP) {
+  if (!narrow && (n * es < DIRECT_UP || !pooled(device))) {
     hipError_t e = hipMemcpyAsync(dev, host, n * es, hipMemcpyHostToDevice, stream);
     if (e == hipSuccess) e = hipStreamSynchronize(stream);
     return e;
