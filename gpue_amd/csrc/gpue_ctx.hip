@@ -291,7 +291,7 @@ static bool opens_step(const Sweep& s) {
 }
 
 // An opening sweep that can reduce the previous step's norm partials itself
-// (part_norm needs workgroups of whole waves).
+// (PartNorm needs workgroups of whole waves).
 static bool takes_deferred_norm(const gpue_ctx* c, const Sweep& s) {
   const int var = s.var >= 0 ? s.var : c->var[s.axis];
   return opens_step(s) && sweep_full_waves(c->prec, s.row, c->dims[s.axis], var);
@@ -341,7 +341,7 @@ static int sweep_nb(const gpue_ctx* c, const Sweep& s) {
 
 // Deferred renormalisation: the norm sweep `last` of one imaginary step leaves
 // its partials to `next`, the first sweep of the following step, which reduces
-// them itself (part_norm, the same additions as the finalize) instead of a
+// them itself (PartNorm, the same additions as the finalize) instead of a
 // one-workgroup finalize kernel and its dispatch gap between the two.  Only
 // for fewer than 4096 partials (every workgroup of `next` sums all of them)
 // and when `next` is the row sweep that scales its input.
