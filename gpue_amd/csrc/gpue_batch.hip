@@ -42,8 +42,8 @@ struct BSeq {                       // one launch sequence of a group for (gstat
   int mask = 3;                     // step parities it serves (bit p: parity p)
   std::vector<SweepArgs*> dargs;    // per position: device array [members]
   std::vector<std::vector<SweepArgs>> hargs;
-  // imaginary time, groups that defer their norms: the opening sweep of a call's first
-  // step, which scales by the norm slot instead of the previous step's partials
+  // imaginary time: the opening sweep of a call's first step, which scales by the norm
+  // slot also where the group defers its norms to the next step's opening sweep
   SweepArgs* dopen = nullptr;
   std::vector<SweepArgs> hopen;
   std::vector<Merged> merged;       // per position, merged groups only
@@ -61,13 +61,15 @@ struct Group {
   std::vector<int> members;
   gpue_ctx* proto;                  // first member: shape and variants
   bool merged = false;              // members of different shapes, launched together
-  bool defer = false;               // norms reduced in the next step's opening sweep
+  int vars[3] = {};                 // kernel variants (unmerged): its contexts' when the batch
+                                    // was created, then what its tuner chose
+  bool defer = false;               // norms reduced in the next step's opening sweep (can_defer, of vars)
   std::vector<Sweep> sched[2][2];   // [gstate][parity]
   std::vector<BSeq> seqs[2][2];     // [gstate][phase]
   hipStream_t stream = nullptr;     // one of the batch's streams (not owned)
   hipGraph_t graph[2][kGraphKinds] = {};   // [gstate][kGraphLens]
   hipGraphExec_t gexec[2][kGraphKinds] = {};
-  int var(const gpue_ctx* c, int axis) const { return !merged ? c->var[axis] : axis == 0 ? MERGE_ROW : MERGE_COL; }
+  int var(int axis) const { return !merged ? vars[axis] : axis == 0 ? MERGE_ROW : MERGE_COL; }
 };
 
 // Problems that may share launches with others of their kind: every axis has a merged
@@ -88,13 +90,14 @@ bool same_kind_of_problem(const gpue_ctx* a, const gpue_ctx* b) {
 
 // Workgroups (= partials) of a member's sweep.
 int blocks_of(const Group& g, const gpue_ctx* c, const Sweep& s) {
-  const int n = c->dims[s.axis], var = g.var(c, s.axis);
+  const int n = c->dims[s.axis], var = g.var(s.axis);
   return s.row ? sweep_blocks(c->prec, true, n, var, c->dims[1] * c->dims[2], 1)
                : sweep_blocks(c->prec, false, n, var, c->dims[0], s.axis == 1 ? c->dims[2] : c->dims[1]);
 }
 
 // Whether every member's norm can be left to the next step's opening sweep (as
-// defer_norm decides for one context).
+// defer_norm decides for one context).  Asked again whenever the variants change: some
+// have tiles of less than a wave for axes of 16 and 32 points.
 bool can_defer(const Group& g, const std::vector<gpue_ctx*>& ctx) {
   for (int idx : g.members) {
     const gpue_ctx* c = ctx[idx];
@@ -102,7 +105,7 @@ bool can_defer(const Group& g, const std::vector<gpue_ctx*>& ctx) {
     for (int par = 0; par < 2; ++par) {
       const Sweep& open = g.sched[0][par].front();
       if (blocks_of(g, c, g.sched[0][par].back()) >= 4096 ||
-          !sweep_full_waves(c->prec, open.row, c->dims[open.axis], g.var(c, open.axis)))
+          !sweep_full_waves(c->prec, open.row, c->dims[open.axis], g.var(open.axis)))
         return false;
     }
   }
@@ -191,7 +194,7 @@ static bool fill_args(gpue_batch* b) {
               std::memset(&a, 0, sizeof(a));
               // every context holds the tables of both plans for each of its
               // axes; a missing one would leave the sweep off rather than fault
-              const auto twi = c->tw.find(2 * c->dims[sw.axis] + (g.var(c, sw.axis) & 1));
+              const auto twi = c->tw.find(2 * c->dims[sw.axis] + (g.var(sw.axis) & 1));
               a.active = on && twi != c->tw.end();
               a.in = c->psi;
               a.out = c->psi;
@@ -206,11 +209,12 @@ static bool fill_args(gpue_batch* b) {
               a.partials = c->partials;
               if (k == 0 && s.dopen) {
                 s.hopen[m] = a;
-                // the previous step's norm from its partials (its last sweep's)
-                a.flags |= F_SCALE_PART;
-                a.norm_nb = blocks_of(g, c, g.sched[gs][1 - par].back());
-                a.norm_scale = c->d[0] * c->d[1] * c->d[2];
-                a.norm_out = c->results;
+                if (g.defer) {   // the previous step's norm from its partials (its last sweep's)
+                  a.flags |= F_SCALE_PART;
+                  a.norm_nb = blocks_of(g, c, g.sched[gs][1 - par].back());
+                  a.norm_scale = c->d[0] * c->d[1] * c->d[2];
+                  a.norm_out = c->results;
+                }
               }
             }
             if (s.dfin) {
@@ -267,7 +271,7 @@ static gpue_status launch_group_phase(gpue_batch* b, Group& g, int gs, int ph, b
         const int n = c->dims[sw.axis];
         const int lx = sw.row ? c->dims[1] * c->dims[2] : c->dims[0];
         const int others = sw.row ? 1 : (sw.axis == 1 ? c->dims[2] : c->dims[1]);
-        e = launch_sweep_batched(c->prec, sw.row, n, c->var[sw.axis], sw.mode, sw.flags, gs, args,
+        e = launch_sweep_batched(c->prec, sw.row, n, g.var(sw.axis), sw.mode, sw.flags, gs, args,
                                  (int)g.members.size(), lx, others, g.stream, &handled);
       }
       if (!handled || e != hipSuccess) return bfail(b, GPUE_EHIP, "batched sweep launch");
@@ -487,6 +491,7 @@ gpue_status gpue_batch_create(gpue_ctx* const* ctxs, int n, gpue_batch** out) {
       Group g;
       g.proto = b->ctx[i];
       g.merged = mg;
+      std::copy(g.proto->var, g.proto->var + 3, g.vars);
       g.members.push_back(i);
       b->groups.push_back(g);
     }
@@ -568,7 +573,7 @@ gpue_status gpue_batch_create(gpue_ctx* const* ctxs, int n, gpue_batch** out) {
               }
             }
           }
-          if (gs == 0 && g.defer) {
+          if (gs == 0) {
             s.hopen.assign(M, SweepArgs{});
             if (hipMalloc((void**)&s.dopen, M * sizeof(SweepArgs)) != hipSuccess) {
               gpue_batch_destroy(b);
@@ -718,6 +723,8 @@ static gpue_status time_batch(gpue_batch* b, int gstate, int steps, double* us) 
 // Every member of group g takes variant v on axis a; the launch arguments and
 // graphs of the batch follow.
 static gpue_status set_group_variant(gpue_batch* b, Group& g, int a, int v) {
+  g.vars[a] = v;
+  g.defer = can_defer(g, b->ctx);
   for (int idx : g.members) {
     gpue_ctx* c = b->ctx[idx];
     int vars[3] = {c->var[0], c->var[1], c->var[2]};
@@ -761,7 +768,7 @@ gpue_status gpue_batch_autotune(gpue_batch* b, int gstate, int steps, double* us
     Group& g = b->groups[order[k]];
     if (g.merged) continue;   // merged launches run one set of variants
     for (int a = 0; a < g.proto->p.dimnum && st == GPUE_OK; ++a) {
-      const int keep = g.proto->var[a];
+      const int keep = g.vars[a];
       int pick = keep;
       // row sweeps: plan and twiddle loading (variants 0-3); strided: plan and tile width (0-5)
       const int nv = a == 0 ? 4 : N_VARIANTS;
@@ -775,7 +782,7 @@ gpue_status gpue_batch_autotune(gpue_batch* b, int gstate, int steps, double* us
           pick = v;
         }
       }
-      if (st == GPUE_OK && g.proto->var[a] != pick) st = set_group_variant(b, g, a, pick);
+      if (st == GPUE_OK && g.vars[a] != pick) st = set_group_variant(b, g, a, pick);
     }
   }
   // then the graph mode: per-group graphs or one graph for the whole batch

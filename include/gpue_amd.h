@@ -224,12 +224,13 @@ double      gpue_eqn_eval(const gpue_eqn_node *nodes, int n_nodes, double x, dou
  * run on at most four streams (the device's hardware queues per process: the
  * three groups with the most work get one each, the rest share the fourth).
  * Blocks of steps of a group are captured as HIP graphs and replayed.
- * Outside merged launches the kernel variants are the contexts' own (equal
- * within a group; a batch may prefer other variants than a lone instance: the
- * groups share the device).  Contexts stay owned by the caller and must outlive
- * the batch; results are read through the contexts (gpue_energy,
- * gpue_download_wfc).  Contexts with a time-dependent V or on different devices
- * are rejected. --- */
+ * Outside merged launches the kernel variants are those the contexts have when
+ * the batch is created (equal within a group; a batch may prefer other variants
+ * than a lone instance: the groups share the device), until gpue_batch_autotune
+ * chooses others; gpue_set_variants on a member changes what it runs alone.
+ * Contexts stay owned by the caller and must outlive the batch; results are read
+ * through the contexts (gpue_energy, gpue_download_wfc).  Contexts with a
+ * time-dependent V or on different devices are rejected. --- */
 typedef struct gpue_batch gpue_batch;
 gpue_status gpue_batch_create(gpue_ctx *const *ctxs, int n, gpue_batch **out);
 /* Exclude (0) or include (1) instance `index` from the following steps. */

@@ -1,0 +1,184 @@
+// The library's host code on the runtime of fake_hip.cpp: what it launches and with
+// which arguments, and what it leaves behind where memory runs out.  Built and run by
+// tests/test_host_logic.py, one argument: the check to run.
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <functional>
+#include <map>
+#include <string>
+#include <vector>
+
+#include "../../gpue_amd/csrc/ctx_internal.h"
+#include "../../gpue_amd/csrc/sweep_merged.h"
+#include "fake_hip.h"
+
+using namespace gpue;
+
+static int failures = 0;
+#define CHECK(cond, ...)                                          \
+  do {                                                            \
+    if (!(cond) && ++failures <= 20) {                            \
+      std::printf("%s:%d: %s: ", __FILE__, __LINE__, #cond);      \
+      std::printf(__VA_ARGS__);                                   \
+      std::printf("\n");                                          \
+    }                                                             \
+  } while (0)
+
+// Looks at every launch: a sweep's kernel is built for the length of the axis that its
+// arguments name, its psi is as large as its grid, and the norm an imaginary step divides
+// by is there: reduced by a finalize into the slot, or by the opening sweep itself from
+// all the partials of the sweep before, in workgroups of whole waves.
+struct Audit {
+  struct Norm {
+    int nb = 0;
+    bool settled = true;
+  };
+  std::map<const void*, Norm> norms;   // by partials
+  long sweeps = 0, from_partials = 0;
+  std::map<std::string, long> kernels;
+
+  void sweep(const fake::Launch& l, const SweepArgs& a, int n, int nblk, int wg, int mode, bool row) {
+    if (!a.active) return;
+    ++sweeps;
+    const int dims[3] = {a.ph.xDim, a.ph.yDim, a.ph.zDim};
+    CHECK(a.axis >= 0 && a.axis < 3 && (a.axis == 0) == row && dims[a.axis] == n, "%s on axis %d of %d x %d x %d",
+          l.kernel.c_str(), a.axis, dims[0], dims[1], dims[2]);
+    const size_t es = l.kernel.find("<double") != std::string::npos ? 16 : 8;
+    CHECK(fake::bytes_at(a.in) >= es * dims[0] * dims[1] * dims[2], "%s: psi", l.kernel.c_str());
+    CHECK(fake::bytes_at(a.tw) > 0, "%s: twiddles", l.kernel.c_str());
+    Norm& m = norms[a.partials];
+    const bool ksum = (mode & 15) == (row ? (int)RM_KSUM : (int)CM_KSUM);
+    if (a.flags & F_SCALE_IN) {
+      if (a.flags & F_SCALE_PART) {
+        ++from_partials;
+        CHECK(wg % 64 == 0, "%s: %d lanes reduce a norm", l.kernel.c_str(), wg);
+        CHECK(a.norm_nb < 4096 && a.norm_nb == m.nb, "%s: norm of %d partials, there are %d", l.kernel.c_str(), a.norm_nb,
+              m.nb);
+      } else {
+        CHECK(m.settled, "%s: the norm is still in its partials", l.kernel.c_str());
+      }
+      m.settled = true;
+    }
+    if (ksum) m.nb = -1;
+    if (a.flags & F_NORM) m = Norm{nblk, false};
+  }
+  void finalize(const void* partials, int nb, int mode) {
+    Norm& m = norms[partials];
+    if (mode != 1) return;
+    CHECK(m.nb == nb || m.settled, "finalize of %d partials, there are %d", nb, m.nb);
+    m.settled = true;
+  }
+  void operator()(const fake::Launch& l) {
+    const std::string& k = l.kernel;
+    ++kernels[k.substr(0, k.find('<'))];
+    if (k.rfind("gpue::k_finalize_b", 0) == 0) {
+      const FinArgs* f = *(const FinArgs**)l.args[0];
+      for (unsigned i = 0; i < l.grid; ++i)
+        if (f[i].active) finalize(f[i].partials, f[i].nb, f[i].mode);
+      return;
+    }
+    if (k.rfind("gpue::k_finalize", 0) == 0) {
+      finalize(*(const void**)l.args[0], *(int*)l.args[1], *(int*)l.args[3]);
+      return;
+    }
+    const bool row = k.rfind("gpue::row_", 0) == 0, col = k.rfind("gpue::col_", 0) == 0;
+    if (!row && !col) return;
+    const char* t = k.c_str() + k.find(", ") + 2;   // after the type
+    if (k.find("_merged<") != std::string::npos) {
+      const SweepArgs* d = *(const SweepArgs**)l.args[0];
+      const MergeMap* map = *(const MergeMap**)l.args[1];
+      std::map<int, bool> seen;
+      for (unsigned i = 0; i < l.grid; ++i)
+        if (map[i].inst >= 0 && !seen[map[i].inst]) {
+          seen[map[i].inst] = true;
+          sweep(l, d[map[i].inst], map[i].n, map[i].nblk, 64, std::atoi(t), row);
+        }
+      return;
+    }
+    int n = 0, var = 0, mode = 0;
+    std::sscanf(t, "%d, %d, %d", &n, &var, &mode);
+    if (k.find("_sweep_b<") != std::string::npos) {
+      const SweepArgs* d = *(const SweepArgs**)l.args[0];
+      const int bpi = *(int*)l.args[1];
+      for (unsigned i = 0; i < l.grid / bpi; ++i) sweep(l, d[i], n, bpi, l.block, mode, row);
+    } else {
+      sweep(l, *(const SweepArgs*)l.args[0], n, (int)l.grid, l.block, mode, row);
+    }
+  }
+};
+
+static gpue_ctx* make(std::vector<int> n, int prec, int gauge) {
+  gpue_params p;
+  gpue_params_default(&p);
+  p.dimnum = (int)n.size();
+  n.resize(3, 1);
+  p.xDim = n[0];
+  p.yDim = n[1];
+  p.zDim = n[2];
+  p.hbar = p.mass = p.omegaX = p.omegaY = p.omegaZ = 1.0;
+  p.xMax = p.yMax = p.zMax = 6.0;
+  p.g = 10.0;
+  p.gpe = 1;
+  p.omega = 0.3;
+  p.corotating = gauge;
+  p.precision = prec;
+  gpue_ctx* c = nullptr;
+  if (gpue_create(&p, &c) != GPUE_OK) {
+    std::printf("gpue_create failed\n");
+    std::exit(1);
+  }
+  return c;
+}
+
+// A batch whose instances (a shape without merged kernels) defer their norms runs the
+// variants its tuner tries, in both precisions and step parities: axes of 16 and 32
+// points have tiles of less than a wave in some variants.  A member whose variants are
+// set by hand stays in step with its group.
+static void batch_norms() {
+  const std::vector<std::vector<int>> shapes = {{64, 16}, {64, 32}, {48, 16}, {16, 48, 32}, {32, 16, 16}};
+  for (int prec : {64, 32})
+    for (const auto& shape : shapes)
+      for (int gauge : {0, 1}) {
+        Audit audit;
+        fake::on_launch = [&](const fake::Launch& l) { audit(l); };
+        gpue_ctx* c[2] = {make(shape, prec, gauge), make(shape, prec, gauge)};
+        gpue_batch* b = nullptr;
+        CHECK(gpue_batch_create(c, 2, &b) == GPUE_OK, "batch");
+        CHECK(gpue_batch_evolve(b, 5, 0) == GPUE_OK, "evolve");
+        CHECK(audit.from_partials > 0, "no norm was deferred");
+        CHECK(gpue_batch_autotune(b, 0, 4, nullptr, nullptr) == GPUE_OK, "autotune");
+        CHECK(gpue_batch_evolve(b, 37, 0) == GPUE_OK, "evolve");
+        CHECK(gpue_batch_set_graph_mode(b, 2) == GPUE_OK, "graph mode");
+        for (int v = 0; v < N_VARIANTS; ++v) {
+          const int vars[3] = {v, v, v};
+          gpue_set_variants(c[0], vars);
+          CHECK(gpue_batch_evolve(b, 3, 0) == GPUE_OK, "evolve");
+          gpue_set_variants(c[1], vars);
+          CHECK(gpue_batch_evolve(b, 2, 0) == GPUE_OK, "evolve");
+          gpue_batch_set_active(b, 0, v % 2);
+          CHECK(gpue_batch_evolve(b, 3, 0) == GPUE_OK, "evolve");
+        }
+        double e[2], m[2];
+        CHECK(gpue_batch_evolve(b, 2, 1) == GPUE_OK && gpue_batch_evolve(b, 2, 0) == GPUE_OK, "evolve");
+        (void)gpue_batch_energy(b, e, m);
+        CHECK(gpue_batch_evolve(b, 3, 0) == GPUE_OK, "evolve");
+        gpue_batch_destroy(b);
+        gpue_destroy(c[0]);
+        gpue_destroy(c[1]);
+      }
+}
+
+int main(int argc, char** argv) {
+  const std::map<std::string, std::function<void()>> checks = {
+      {"batch_norms", batch_norms},
+  };
+  const auto it = checks.find(argc > 1 ? argv[1] : "");
+  if (it == checks.end()) {
+    std::printf("no such check\n");
+    return 2;
+  }
+  it->second();
+  std::printf(failures ? "%d failures\n" : "ok\n", failures);
+  return failures != 0;
+}
