@@ -95,6 +95,14 @@ int blocks_of(const Group& g, const gpue_ctx* c, const Sweep& s) {
                : sweep_blocks(c->prec, false, n, var, c->dims[0], s.axis == 1 ? c->dims[2] : c->dims[1]);
 }
 
+// The normalisation of a member's sweep (schedule's, for its own sizes): of the whole
+// transform where K is applied, of the axis with a gauge operator.
+double inv_n(const gpue_ctx* c, const Sweep& s) {
+  if (s.invN == 0.0) return 0.0;
+  const bool k = s.row ? s.mode == RM_K || s.mode == RM_FULL : s.mode == CM_K;
+  return k ? 1.0 / (double)c->N : 1.0 / c->dims[s.axis];
+}
+
 // Whether every member's norm can be left to the next step's opening sweep (as
 // defer_norm decides for one context).  Asked again whenever the variants change: some
 // have tiles of less than a wave for axes of 16 and 32 points.
@@ -183,9 +191,9 @@ static bool fill_args(gpue_batch* b) {
             const int par = (b->cls[idx] + ph) % 2;   // the instance's step parity at this phase
             const bool in = b->active[idx] && ((s.mask >> par) & 1);
             any = any || in;
-            std::vector<Sweep> own;   // members of a merged group have their own normalisations
-            if (g.merged) schedule(c, gs, par, gs == 0, own);
-            const std::vector<Sweep>& sc = g.merged ? own : g.sched[gs][par];
+            // The group's schedule, which the launches and their maps were laid out for: a
+            // member's own may change after (A_z set to a field leads even steps along z).
+            const std::vector<Sweep>& sc = g.sched[gs][par];
             const Phys phys = make_phys(c, gs, 0);
             for (size_t k = 0; k < s.keys.size(); ++k) {
               const bool on = in && k < sc.size();
@@ -204,7 +212,7 @@ static bool fill_args(gpue_batch* b) {
               a.axis = sw.axis;
               a.gauge_axis = sw.axis;
               a.flags = sw.flags;
-              a.invN = sw.invN;
+              a.invN = inv_n(c, sw);
               a.norm_in = c->results;
               a.partials = c->partials;
               if (k == 0 && s.dopen) {

@@ -228,6 +228,8 @@ double      gpue_eqn_eval(const gpue_eqn_node *nodes, int n_nodes, double x, dou
  * the batch is created (equal within a group; a batch may prefer other variants
  * than a lone instance: the groups share the device), until gpue_batch_autotune
  * chooses others; gpue_set_variants on a member changes what it runs alone.
+ * The sweeps of a step are also those of that moment: an A_z field set on a member
+ * later is not applied by the batch.
  * Contexts stay owned by the caller and must outlive the batch; results are read
  * through the contexts (gpue_energy, gpue_download_wfc).  Contexts with a
  * time-dependent V or on different devices are rejected. --- */

@@ -47,6 +47,13 @@ struct Audit {
     const size_t es = l.kernel.find("<double") != std::string::npos ? 16 : 8;
     CHECK(fake::bytes_at(a.in) >= es * dims[0] * dims[1] * dims[2], "%s: psi", l.kernel.c_str());
     CHECK(fake::bytes_at(a.tw) > 0, "%s: twiddles", l.kernel.c_str());
+    const double all = 1.0 / ((double)dims[0] * dims[1] * dims[2]), one = 1.0 / dims[a.axis];
+    const int op = mode & 15;
+    const bool k_op = row ? op == RM_K || op == RM_FULL : op == CM_K;
+    const bool a_op = row ? op == RM_GAUGE || op == RM_GAUGE_FWD || (op == RM_INV && (a.flags & F_GAUGE_POST))
+                          : op == CM_GAUGE || op == CM_GAUGE_FWD || (op == CM_INV_VG && (a.flags & F_GAUGE_POST));
+    CHECK(!k_op || a.invN == all, "%s: K normalised by %g", l.kernel.c_str(), a.invN);
+    CHECK(!a_op || a.invN == one, "%s: A normalised by %g", l.kernel.c_str(), a.invN);
     Norm& m = norms[a.partials];
     const bool ksum = (mode & 15) == (row ? (int)RM_KSUM : (int)CM_KSUM);
     if (a.flags & F_SCALE_IN) {
@@ -169,9 +176,36 @@ static void batch_norms() {
       }
 }
 
+// A batch goes on with the schedule it was created for when a member's A_z becomes a
+// field, which would lead the member's own even steps along z: kernels, axes and
+// normalisations stay in step.  (Merged boxes of different sizes, and a group of one
+// shape without merged kernels.)
+static void batch_members_change() {
+  const std::vector<std::vector<int>> shapes = {{64, 128, 64}, {64, 64, 96}, {128, 64, 64}, {48, 64, 16}, {48, 64, 16}};
+  for (int prec : {64, 32}) {
+    Audit audit;
+    fake::on_launch = [&](const fake::Launch& l) { audit(l); };
+    std::vector<gpue_ctx*> c;
+    for (const auto& s : shapes) c.push_back(make(s, prec, 1));
+    gpue_batch* b = nullptr;
+    CHECK(gpue_batch_create(c.data(), (int)c.size(), &b) == GPUE_OK, "batch");
+    CHECK(gpue_batch_set_graph_mode(b, 2) == GPUE_OK, "graph mode");
+    for (size_t k = 0; k < c.size(); ++k) {
+      const std::vector<double> az(c[k]->N, 0.1 + (double)k);
+      CHECK(gpue_set_field(c[k], GPUE_FIELD_AZ, az.data()) == GPUE_OK, "A_z");
+      CHECK(gpue_batch_set_active(b, (int)k, 0) == GPUE_OK && gpue_batch_set_active(b, (int)k, 1) == GPUE_OK, "active");
+      for (int gstate : {0, 1}) CHECK(gpue_batch_evolve(b, 3, gstate) == GPUE_OK, "evolve");
+    }
+    CHECK(audit.kernels["gpue::col_merged"] > 0 && audit.kernels["gpue::col_sweep_b"] > 0, "kernels");
+    gpue_batch_destroy(b);
+    for (gpue_ctx* x : c) gpue_destroy(x);
+  }
+}
+
 int main(int argc, char** argv) {
   const std::map<std::string, std::function<void()>> checks = {
       {"batch_norms", batch_norms},
+      {"batch_members_change", batch_members_change},
   };
   const auto it = checks.find(argc > 1 ? argv[1] : "");
   if (it == checks.end()) {
