@@ -974,20 +974,49 @@ gpue_status gpue_set_field_eqn(gpue_ctx* c, int which, const char* expr, const c
                                             std::to_string(EQ_REG_DEPTH));
     drop_graphs(c);
     const int k = which;   // GPUE_FIELD_V, _K, _AX, _AY, _AZ = 0..4
+    const bool trap = which >= GPUE_FIELD_AX && !c->v_user;   // V = trap + 1/2 m |A(t)|^2, per point
+    // all that can fail comes first: the field stays as it is unless everything is there
+    // (a table that nothing refers to yet may stay for the next call)
     double** slot = which == GPUE_FIELD_V ? &c->Vt : which == GPUE_FIELD_K ? &c->Kt : &c->At[which - GPUE_FIELD_AX];
     if (!*slot && hipMalloc((void**)slot, c->N * sizeof(double)) != hipSuccess) return fail(c, GPUE_ENOMEM, "field");
-    if (which >= GPUE_FIELD_AX) {
-      gpue_status st = materialise_A(c, which - GPUE_FIELD_AX);
-      if (st != GPUE_OK) return st;
-    }
     if (!c->tbase && hipMalloc((void**)&c->tbase, sizeof(double)) != hipSuccess) return fail(c, GPUE_ENOMEM, "field");
-    if (which == GPUE_FIELD_V && !c->Vt2 && hipMalloc((void**)&c->Vt2, c->N * sizeof(double)) != hipSuccess)
-      return fail(c, GPUE_ENOMEM, "field");
-    if (!c->deq[k] && hipMalloc((void**)&c->deq[k], sizeof(EqnProg)) != hipSuccess)
-      return fail(c, GPUE_ENOMEM, "equation program");
+    if (trap) {
+      if (!c->Vt && hipMalloc((void**)&c->Vt, c->N * sizeof(double)) != hipSuccess) return fail(c, GPUE_ENOMEM, "V");
+      for (int a = 0; a < 3; ++a) {
+        if (c->vst[a]) continue;
+        std::vector<double> t(c->grid[a].size());
+        const double oZ = p.dimnum == 3 ? p.omegaZ : 0.0, z0 = p.dimnum == 3 ? p.z0_shift : 0.0;
+        for (size_t i = 0; i < t.size(); ++i) {
+          const double x = c->grid[a][i];
+          const double u = a == 0 ? p.omegaX * (x + p.x0_shift)
+                                  : a == 1 ? p.gammaY * p.omegaY * (x + p.y0_shift) : 1.0 * oZ * (x + z0);
+          t[i] = 0.5 * p.mass * (u * u);
+        }
+        hipError_t e = hipSuccess;
+        c->vst[a] = dev_copy(t, &e);
+        if (e != hipSuccess) return fail(c, GPUE_ENOMEM, "trap tables");
+      }
+    }
     mark_uniform(dp);
+    EqnProg* prog_d = nullptr;
+    double* vt2 = nullptr;
+    gpue_status st = GPUE_OK;
+    if (hipMalloc((void**)&prog_d, sizeof(EqnProg)) != hipSuccess)
+      st = fail(c, GPUE_ENOMEM, "equation program");
+    else if (hipMemcpy(prog_d, &dp, sizeof(EqnProg), hipMemcpyHostToDevice) != hipSuccess)
+      st = fail(c, GPUE_EHIP, "equation program");
+    else if (which == GPUE_FIELD_V && !c->Vt2 && hipMalloc((void**)&vt2, c->N * sizeof(double)) != hipSuccess)
+      st = fail(c, GPUE_ENOMEM, "field");
+    if (st == GPUE_OK && which >= GPUE_FIELD_AX) st = materialise_A(c, which - GPUE_FIELD_AX);
+    if (st != GPUE_OK) {
+      if (prog_d) (void)hipFree(prog_d);
+      if (vt2) (void)hipFree(vt2);
+      return st;
+    }
+    if (c->deq[k]) (void)hipFree(c->deq[k]);
+    c->deq[k] = prog_d;
     c->deq_depth[k] = dp.depth;
-    HIPCHK(c, hipMemcpy(c->deq[k], &dp, sizeof(EqnProg), hipMemcpyHostToDevice));
+    if (vt2) c->Vt2 = vt2;
     c->t_dep = true;
     if (which == GPUE_FIELD_V) {
       c->v_kind = V_EQN;
@@ -997,25 +1026,7 @@ gpue_status gpue_set_field_eqn(gpue_ctx* c, int which, const char* expr, const c
     } else {
       c->a_kind = A_EQN;
       if (which == GPUE_FIELD_AZ) c->az_zero = false;
-      if (!c->v_user) {   // V = trap + 1/2 m |A(t)|^2, per point
-        if (!c->Vt && hipMalloc((void**)&c->Vt, c->N * sizeof(double)) != hipSuccess)
-          return fail(c, GPUE_ENOMEM, "V");
-        for (int a = 0; a < 3 && !c->vst[a]; ++a) {
-          const gpue_params& q = c->p;
-          std::vector<double> t(c->grid[a].size());
-          const double oZ = q.dimnum == 3 ? q.omegaZ : 0.0, z0 = q.dimnum == 3 ? q.z0_shift : 0.0;
-          for (size_t i = 0; i < t.size(); ++i) {
-            const double x = c->grid[a][i];
-            const double u = a == 0 ? q.omegaX * (x + q.x0_shift)
-                                    : a == 1 ? q.gammaY * q.omegaY * (x + q.y0_shift) : 1.0 * oZ * (x + z0);
-            t[i] = 0.5 * q.mass * (u * u);
-          }
-          hipError_t e = hipSuccess;
-          c->vst[a] = dev_copy(t, &e);
-          if (e != hipSuccess) return fail(c, GPUE_ENOMEM, "trap tables");
-        }
-        c->v_kind = V_TRAP_A;
-      }
+      if (trap) c->v_kind = V_TRAP_A;
     }
     return GPUE_OK;
   }

@@ -42,6 +42,10 @@ static hipError_t release(void* p) {
   free(p);
   return hipSuccess;
 }
+size_t live() {
+  std::lock_guard<std::mutex> lk(mu);
+  return blocks().size();
+}
 size_t bytes_at(const void* p) {
   std::lock_guard<std::mutex> lk(mu);
   auto it = blocks().upper_bound((char*)p);

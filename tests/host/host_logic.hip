@@ -202,10 +202,61 @@ static void batch_members_change() {
   }
 }
 
+// What the steps read: the fields' kinds and, by step parity, the V table.
+struct Fields {
+  int v_kind, a_kind, k_kind;
+  bool az_zero, t_dep, two_v;
+  bool prog[5];
+  explicit Fields(const gpue_ctx* c)
+      : v_kind(c->v_kind), a_kind(c->a_kind), k_kind(c->k_kind), az_zero(c->az_zero), t_dep(c->t_dep),
+        two_v(v_table(c, 0) != v_table(c, 1)) {
+    for (int k = 0; k < 5; ++k) prog[k] = c->deq[k] != nullptr;
+  }
+  bool operator==(const Fields& o) const {
+    return v_kind == o.v_kind && a_kind == o.a_kind && k_kind == o.k_kind && az_zero == o.az_zero && t_dep == o.t_dep &&
+           two_v == o.two_v && std::memcmp(prog, o.prog, sizeof(prog)) == 0;
+  }
+};
+
+// Time-dependent fields where the n-th device allocation fails: the call reports it and
+// the fields stay as they were; with memory again it succeeds, and nothing leaks.
+static void field_out_of_memory() {
+  const char* td = "0.5*(x*x+y*y)*(1+0.1*sin(2*t))";
+  for (int before = 0; before < 4; ++before)   // trap; V(t); a table of V; a table of A_x
+    for (int which = GPUE_FIELD_V; which <= GPUE_FIELD_AZ; ++which) {
+      const size_t live = fake::live();
+      long fails = 0;
+      for (long n = 0;; ++n) {
+        gpue_ctx* c = make({32, 16, 16}, 64, 1);
+        const std::vector<double> table(c->N, 0.5);
+        if (before == 1) CHECK(gpue_set_field_eqn(c, GPUE_FIELD_V, td, nullptr, nullptr, 0) == GPUE_OK, "V(t)");
+        if (before == 2) CHECK(gpue_set_field(c, GPUE_FIELD_V, table.data()) == GPUE_OK, "V");
+        if (before == 3) CHECK(gpue_set_field(c, GPUE_FIELD_AX, table.data()) == GPUE_OK, "A_x");
+        const Fields was(c);
+        fake::mallocs_left = n;
+        const gpue_status st = gpue_set_field_eqn(c, which, td, nullptr, nullptr, 0);
+        fake::mallocs_left = -1;
+        if (st != GPUE_OK) {
+          ++fails;
+          CHECK(st == GPUE_ENOMEM && Fields(c) == was, "field %d, allocation %ld: half set", which, n);
+          CHECK(gpue_set_field_eqn(c, which, td, nullptr, nullptr, 0) == GPUE_OK, "with memory");
+        }
+        CHECK(c->t_dep && c->deq[which] && c->tbase && (which != GPUE_FIELD_V || c->Vt2), "field %d", which);
+        for (int a = 0; a < 3; ++a) CHECK(c->v_kind != V_TRAP_A || (c->Vt && c->vst[a]), "field %d: trap", which);
+        CHECK(gpue_evolve(c, 0, 4, 1, 0, -1.0, nullptr, 0, nullptr) == GPUE_OK, "evolve");
+        gpue_destroy(c);
+        CHECK(fake::live() == live, "%zu allocations left", fake::live() - live);
+        if (st == GPUE_OK) break;
+      }
+      CHECK(fails > 0, "no allocation failed");
+    }
+}
+
 int main(int argc, char** argv) {
   const std::map<std::string, std::function<void()>> checks = {
       {"batch_norms", batch_norms},
       {"batch_members_change", batch_members_change},
+      {"field_out_of_memory", field_out_of_memory},
   };
   const auto it = checks.find(argc > 1 ? argv[1] : "");
   if (it == checks.end()) {
