@@ -71,7 +71,8 @@ struct gpue_ctx {
   double* partials = nullptr;
   size_t partials_n = 0;
   double* results = nullptr;   // [0] norm  [1] kinetic  [2..5] position terms
-  double* hres = nullptr;      // pinned: scalars on their way to the host (16 doubles)
+  double* hres = nullptr;      // scalars on their way to the host (16 doubles), pinned where that can be had
+  bool hres_pinned = false;
   int v_kind = gpue::V_SEP, a_kind = gpue::A_ROTATION, k_kind = gpue::K_SEP;
   bool v_user = false;         // V supplied by the caller (table or equation)
   double* vs[3] = {};          // separable V / K value tables

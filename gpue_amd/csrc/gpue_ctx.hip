@@ -9,6 +9,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstdio>
+#include <cstdlib>
 #include <cstring>
 #include <map>
 #include <string>
@@ -63,6 +64,7 @@ static void pass_table(int n, const std::vector<int>& R, std::vector<int>& idx) 
   }
 }
 gpue_status gpue::fail(gpue_ctx* c, gpue_status s, const std::string& msg) {
+  (void)hipGetLastError();   // reported here, not by the next launch
   if (c) c->err = msg;
   return s;
 }
@@ -624,7 +626,8 @@ void gpue_destroy(gpue_ctx* c) {
   drop_graphs(c);
   if (c->gev) (void)hipEventDestroy(c->gev);
   if (c->stream && c->own_stream) (void)hipStreamDestroy(c->stream);
-  if (c->hres) (void)hipHostFree(c->hres);
+  if (c->hres_pinned) (void)hipHostFree(c->hres);
+  else std::free(c->hres);
   staging_release();
   delete c;
 }
@@ -741,6 +744,7 @@ gpue_status gpue::ctx_create(const gpue_params* pin, hipStream_t ext_stream, gpu
     c->err = m;
     std::fprintf(stderr, "gpue_create: %s\n", m.c_str());
     gpue_destroy(c);
+    (void)hipGetLastError();   // reported here, not by another context's next launch
     return s;
   };
   {
@@ -816,9 +820,14 @@ gpue_status gpue::ctx_create(const gpue_params* pin, hipStream_t ext_stream, gpu
   c->var_default = true;
   c->partials_n = nb * 4;
   if (hipMalloc((void**)&c->partials, c->partials_n * sizeof(double)) != hipSuccess ||
-      hipMalloc((void**)&c->results, 16 * sizeof(double)) != hipSuccess ||
-      hipHostMalloc((void**)&c->hres, 16 * sizeof(double), hipHostMallocDefault) != hipSuccess)
+      hipMalloc((void**)&c->results, 16 * sizeof(double)) != hipSuccess)
     return bail(GPUE_ENOMEM, "reduction scratch");
+  c->hres_pinned = hipHostMalloc((void**)&c->hres, 16 * sizeof(double), hipHostMallocDefault) == hipSuccess;
+  if (!c->hres_pinned) {   // copies of scalars then go through HIP's staging
+    (void)hipGetLastError();
+    c->hres = (double*)std::malloc(16 * sizeof(double));
+    if (!c->hres) return bail(GPUE_ENOMEM, "reduction scratch");
+  }
   // on the context's own stream: other contexts' work on the device is not waited for
   if (hipMemsetAsync(c->results, 0, 16 * sizeof(double), c->stream) != hipSuccess ||
       launch_set_double(c->results, 1.0, c->stream) != hipSuccess ||

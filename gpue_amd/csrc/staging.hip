@@ -12,7 +12,9 @@
 #include <algorithm>
 #include <atomic>
 #include <cstring>
+#include <memory>
 #include <mutex>
+#include <new>
 #include <system_error>
 #include <thread>
 #include <vector>
@@ -170,6 +172,31 @@ struct Job {
   }
 };
 
+// Without pinned memory to be had: HIP's own copies, conversions through a pageable chunk.
+hipError_t run_pageable(const Job& j) {
+  const size_t per = j.conv ? std::min(j.n, CHUNK / j.es) : j.n;
+  std::unique_ptr<float[]> f;
+  if (j.conv) {
+    f.reset(new (std::nothrow) float[per]);
+    if (!f) return hipErrorOutOfMemory;
+  }
+  for (size_t i = 0; i < j.n; i += per) {
+    const size_t c = std::min(per, j.n - i);
+    void* const dev = j.dev + i * j.es;
+    double* const d = (double*)j.host + i;   // conv
+    void* const host = j.conv ? (void*)f.get() : (void*)j.host;
+    if (j.conv && !j.down)
+      for (size_t k = 0; k < c; ++k) f[k] = (float)d[k];
+    hipError_t e = j.down ? hipMemcpyAsync(host, dev, c * j.es, hipMemcpyDeviceToHost, j.stream)
+                          : hipMemcpyAsync(dev, host, c * j.es, hipMemcpyHostToDevice, j.stream);
+    if (e == hipSuccess) e = hipStreamSynchronize(j.stream);
+    if (e != hipSuccess) return e;
+    if (j.conv && j.down)
+      for (size_t k = 0; k < c; ++k) d[k] = f[k];
+  }
+  return hipSuccess;
+}
+
 hipError_t run_on(Job& j, int device) {
   const size_t bytes = j.n * j.es;
   // one chunk up to 2 MiB, then chunks of 2 MiB up to 8 MiB: a chunk costs about 15 us
@@ -179,7 +206,7 @@ hipError_t run_on(Job& j, int device) {
   j.chunks = (int)((j.n + j.per - 1) / j.per);
   const int want = std::min(j.chunks, RING);
   for (j.nbuf = 0; j.nbuf < want && take(device, j.buf[j.nbuf]); ++j.nbuf) j.filled[j.nbuf] = 0;
-  if (j.nbuf == 0) return hipErrorOutOfMemory;
+  if (j.nbuf == 0) return run_pageable(j);
   std::vector<std::thread> th;
   if (bytes >= MT_BYTES) {
     const int hw = (int)std::thread::hardware_concurrency();

@@ -23,11 +23,12 @@ static std::map<const void*, std::string>& names() {   // registered before main
   return m;
 }
 static bool capturing = false;
+static hipError_t last_error = hipSuccess;
 static struct { dim3 grid, block; size_t shmem; hipStream_t stream; } pushed;
 
 static hipError_t alloc(void** p, size_t n, long* left, hipError_t none) {
   std::lock_guard<std::mutex> lk(mu);
-  if (*left == 0) return none;
+  if (*left == 0) return last_error = none;
   if (*left > 0) --*left;
   *p = calloc(1, n ? n : 1);
   blocks()[(char*)*p] = n;
@@ -119,7 +120,11 @@ hipError_t hipGetDevice(int* d) {
   return hipSuccess;
 }
 hipError_t hipSetDevice(int) { return hipSuccess; }
-hipError_t hipGetLastError() { return hipSuccess; }
+hipError_t hipGetLastError() {
+  const hipError_t e = last_error;
+  last_error = hipSuccess;
+  return e;
+}
 const char* hipGetErrorString(hipError_t e) { return e == hipErrorOutOfMemory ? "out of memory" : "error"; }
 
 hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) { return handle(s); }

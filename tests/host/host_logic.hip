@@ -239,6 +239,7 @@ static void field_out_of_memory() {
         if (st != GPUE_OK) {
           ++fails;
           CHECK(st == GPUE_ENOMEM && Fields(c) == was, "field %d, allocation %ld: half set", which, n);
+          CHECK(gpue_evolve(c, 0, 4, 1, 0, -1.0, nullptr, 0, nullptr) == GPUE_OK, "evolve after the failure");
           CHECK(gpue_set_field_eqn(c, which, td, nullptr, nullptr, 0) == GPUE_OK, "with memory");
         }
         CHECK(c->t_dep && c->deq[which] && c->tbase && (which != GPUE_FIELD_V || c->Vt2), "field %d", which);
@@ -252,11 +253,39 @@ static void field_out_of_memory() {
     }
 }
 
+// psi to the device and back where no pinned memory can be had, one or two buffers, or all:
+// parts of a chunk, several chunks, transfers that use threads.
+static void pinned_memory() {
+  const std::vector<std::vector<int>> shapes = {{16}, {512, 64}, {192, 192, 16}, {1024, 512}, {192, 96, 96}, {2048, 1024}};
+  for (long pinned : {0L, 1L, 2L, 3L, -1L})
+    for (int prec : {64, 32})
+      for (const auto& shape : shapes) {
+        const size_t live = fake::live();
+        fake::pinned_left = pinned;
+        gpue_ctx* c = make(shape, prec, 0);
+        std::vector<double> in(2 * c->N), out(2 * c->N, -1.0);
+        for (size_t k = 0; k < in.size(); ++k) in[k] = 0.1 * (double)(k % 9973) + (double)k;
+        for (int again = 0; again < 2; ++again) {
+          CHECK(gpue_upload_wfc(c, in.data()) == GPUE_OK, "upload: %s", gpue_last_error(c));
+          CHECK(gpue_download_wfc(c, out.data()) == GPUE_OK, "download: %s", gpue_last_error(c));
+          bool same = true;
+          for (size_t k = 0; k < in.size(); ++k) same = same && out[k] == (prec == 64 ? in[k] : (double)(float)in[k]);
+          CHECK(same, "%ld pinned allocations, %d bits, %ld points", pinned, prec, c->N);
+        }
+        double e = 0.0, m = 0.0;
+        CHECK(gpue_energy(c, &e, &m) == GPUE_OK, "energy: %s", gpue_last_error(c));
+        gpue_destroy(c);
+        fake::pinned_left = -1;
+        CHECK(fake::live() == live, "%zu allocations left", fake::live() - live);
+      }
+}
+
 int main(int argc, char** argv) {
   const std::map<std::string, std::function<void()>> checks = {
       {"batch_norms", batch_norms},
       {"batch_members_change", batch_members_change},
       {"field_out_of_memory", field_out_of_memory},
+      {"pinned_memory", pinned_memory},
   };
   const auto it = checks.find(argc > 1 ? argv[1] : "");
   if (it == checks.end()) {
