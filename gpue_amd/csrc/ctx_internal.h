@@ -31,8 +31,6 @@ struct StepGraph {
   hipGraphExec_t exec = nullptr;
   long last_use = 0;
 };
-constexpr int MAX_STEP_GRAPHS = 8;
-
 }  // namespace gpue
 
 struct gpue_ctx {
@@ -58,7 +56,7 @@ struct gpue_ctx {
   // steps between energy evaluations.  A replay costs 15-25 us beside its steps (us a
   // step in blocks of 2 / 8 / 32 / 96: 256^2 19.8 / 15.6 / 14.5 / 14.2, 512^2 with
   // rotation 35.5 / 31.0 / 29.9 / 29.5, 128x128x96 88.9 / 82.6 / 81.0 / 80.6); a longer
-  // first capture is the price, and 32 leaves little to gain
+  // first capture is the price (7-15 us a step, once per length), and 32 leaves little to gain
   int graph_steps = 32;
   std::vector<gpue::StepGraph> graphs;
   hipEvent_t gev = nullptr;    // recorded after the replays of an evolve call (a shared stream is not waited for)

@@ -280,12 +280,35 @@ static void pinned_memory() {
       }
 }
 
+// Step blocks of every length are captured once and kept, in both gstates.
+static void step_blocks() {
+  fake::on_launch = [&](const fake::Launch& l) {   // norms must be numbers
+    if (l.kernel.rfind("gpue::k_set_double", 0) == 0) **(double**)l.args[0] = *(double*)l.args[1];
+  };
+  gpue_ctx* c = make({64, 32}, 64, 1);
+  auto captures = [&](int n, int gstate) {
+    const long before = fake::captures;
+    CHECK(gpue_evolve(c, 0, n, gstate, 0, -1.0, nullptr, 0, nullptr) == GPUE_OK, "evolve: %s", gpue_last_error(c));
+    return fake::captures - before;
+  };
+  for (int round = 0; round < 3; ++round)
+    for (int gstate : {0, 1})
+      for (int n = 2; n <= 32; n += 2) {
+        const long got = captures(n, gstate);
+        CHECK(got == (round == 0), "%ld captures for %d steps in round %d", got, n, round);
+      }
+  CHECK(captures(100, 0) == 0 && captures(100, 1) == 0, "three blocks of 32 and a tail");
+  CHECK(gpue_set_g(c, 20.0) == GPUE_OK && captures(100, 0) == 2 && captures(100, 0) == 0, "dropped with the parameters");
+  gpue_destroy(c);
+}
+
 int main(int argc, char** argv) {
   const std::map<std::string, std::function<void()>> checks = {
       {"batch_norms", batch_norms},
       {"batch_members_change", batch_members_change},
       {"field_out_of_memory", field_out_of_memory},
       {"pinned_memory", pinned_memory},
+      {"step_blocks", step_blocks},
   };
   const auto it = checks.find(argc > 1 ? argv[1] : "");
   if (it == checks.end()) {
