@@ -1582,12 +1582,14 @@ static int block_len(const gpue_ctx* c, int first_step, int nsteps, int s, int e
 
 // 1D: steps of an evolve call, from step s on, that run as one launch (line_steps);
 // 0: the step is launched on its own (fields that depend on time or ramp, kernel
-// timing).  A run ends with the next energy evaluation, the call, or 4096 steps (a
-// few milliseconds: no launch holds the device for long).
+// timing).  A run ends with the next energy evaluation, the call, or 1024 steps (fewer
+// beyond 1024 points), so that no launch holds the device for longer than some 6 ms: a
+// step takes 1-2 us at 16 points, 3.2-6.1 at 1024, 6-17 at 4096 (both precisions, without
+// and with a gauge).  A launch more costs some 10 us.
 static int line_len(const gpue_ctx* c, int first_step, int nsteps, int s, int energy_every) {
   if (c->p.dimnum != 1 || c->graph_steps <= 0 || c->timing || c->t_dep || c->ramp_type) return 0;
   const int i = first_step + s;
-  int L = std::min(nsteps - s, 4096);
+  int L = std::min(nsteps - s, std::min(1024, (1 << 20) / c->dims[0]));
   if (energy_every > 0) L = std::min(L, ((i + energy_every - 1) / energy_every) * energy_every - i + 1);
   return L;
 }

@@ -302,6 +302,31 @@ static void step_blocks() {
   gpue_destroy(c);
 }
 
+// 1D runs: launches of at most 2^20 point steps and 1024 steps, up to each energy
+// evaluation, that make up the call.
+static void line_runs() {
+  for (int n : {16, 1024, 2048, 4096})
+    for (int every : {0, 700}) {
+      std::vector<int> runs;
+      fake::on_launch = [&](const fake::Launch& l) {
+        if (l.kernel.rfind("gpue::k_set_double", 0) == 0) **(double**)l.args[0] = *(double*)l.args[1];
+        if (l.kernel.rfind("gpue::line_steps", 0) == 0) runs.push_back(*(int*)l.args[1]);
+      };
+      gpue_ctx* c = make({n}, 64, 0);
+      double e[8];
+      CHECK(gpue_evolve(c, 0, 2500, 0, every, -1.0, e, 8, nullptr) == GPUE_OK, "evolve: %s", gpue_last_error(c));
+      int done = 0;
+      for (int r : runs) {
+        CHECK(r > 0 && r <= 1024 && (long)r * n <= 1 << 20, "%d steps of %d points in one launch", r, n);
+        if (every)
+          for (int i = done; i < done + r - 1; ++i) CHECK(i % every != 0, "energy step %d inside a launch", i);
+        done += r;
+      }
+      CHECK(done == 2500, "%d steps", done);
+      gpue_destroy(c);
+    }
+}
+
 int main(int argc, char** argv) {
   const std::map<std::string, std::function<void()>> checks = {
       {"batch_norms", batch_norms},
@@ -309,6 +334,7 @@ int main(int argc, char** argv) {
       {"field_out_of_memory", field_out_of_memory},
       {"pinned_memory", pinned_memory},
       {"step_blocks", step_blocks},
+      {"line_runs", line_runs},
   };
   const auto it = checks.find(argc > 1 ? argv[1] : "");
   if (it == checks.end()) {
