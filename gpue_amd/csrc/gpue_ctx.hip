@@ -1407,6 +1407,7 @@ static gpue_status autotune(gpue_ctx* c, int reps) {
   HIPCHK(c, hipEventCreate(&e0));
   HIPCHK(c, hipEventCreate(&e1));
   double cost[3][N_VARIANTS] = {};
+  const bool var_default = c->var_default;
   c->var_default = false;   // every sweep of an axis runs what is chosen for it
   std::vector<Sweep> sched;
   const bool timing = c->timing;
@@ -1431,7 +1432,10 @@ static gpue_status autotune(gpue_ctx* c, int reps) {
   c->timing = timing;
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
-  if (st != GPUE_OK) return st;
+  if (st != GPUE_OK) {   // nothing is chosen yet
+    c->var_default = var_default;
+    return st;
+  }
   for (int a = 0; a < 3; ++a) {
     int best = c->var[a];
     for (int v = 0; v < N_VARIANTS; ++v)

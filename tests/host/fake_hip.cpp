@@ -11,7 +11,7 @@
 
 namespace fake {
 std::function<void(const Launch&)> on_launch;
-long mallocs_left = -1, pinned_left = -1, mallocs = 0, captures = 0;
+long mallocs_left = -1, pinned_left = -1, instantiates_left = -1, mallocs = 0, captures = 0;
 
 static std::mutex mu;
 static std::map<char*, size_t>& blocks() {
@@ -151,7 +151,14 @@ hipError_t hipStreamEndCapture(hipStream_t, hipGraph_t* g) {
   capturing = false;
   return handle(g);
 }
-hipError_t hipGraphInstantiate(hipGraphExec_t* e, hipGraph_t, hipGraphNode_t*, char*, size_t) { return handle(e); }
+hipError_t hipGraphInstantiate(hipGraphExec_t* e, hipGraph_t, hipGraphNode_t*, char*, size_t) {
+  if (instantiates_left == 0) {
+    *e = nullptr;
+    return last_error = hipErrorOutOfMemory;
+  }
+  if (instantiates_left > 0) --instantiates_left;
+  return handle(e);
+}
 hipError_t hipGraphLaunch(hipGraphExec_t, hipStream_t) { return hipSuccess; }
 hipError_t hipGraphDestroy(hipGraph_t) { return hipSuccess; }
 hipError_t hipGraphExecDestroy(hipGraphExec_t) { return hipSuccess; }

@@ -327,6 +327,30 @@ static void line_runs() {
     }
 }
 
+// A tuner that fails before it has chosen anything leaves a context with its default
+// variants, the real-time choice (K sweeps of this box on quarter tiles) among them.
+static void tuner_fails() {
+  gpue_ctx* c = make({128, 64, 192}, 64, 0);
+  std::string kernels;
+  fake::on_launch = [&](const fake::Launch& l) { kernels += l.kernel + "\n"; };
+  auto step = [&]() {
+    kernels.clear();
+    CHECK(gpue_set_graph_steps(c, 0) == GPUE_OK && gpue_evolve(c, 0, 1, 1, 0, -1.0, nullptr, 0, nullptr) == GPUE_OK, "step");
+    return kernels;
+  };
+  const std::string before = step();
+  CHECK(before.find("col_sweep<double, 192, 4, 18>") != std::string::npos, "%s", before.c_str());
+  int was[3], now[3];
+  gpue_get_variants(c, was);
+  for (long n : {0L, 1L, 5L}) {
+    fake::instantiates_left = n;
+    CHECK(gpue_autotune(c, 2, now) != GPUE_OK, "the tuner");
+    fake::instantiates_left = -1;
+    CHECK(std::memcmp(was, now, sizeof(was)) == 0 && step() == before, "other kernels after a failed tuner");
+  }
+  gpue_destroy(c);
+}
+
 int main(int argc, char** argv) {
   const std::map<std::string, std::function<void()>> checks = {
       {"batch_norms", batch_norms},
@@ -335,6 +359,7 @@ int main(int argc, char** argv) {
       {"pinned_memory", pinned_memory},
       {"step_blocks", step_blocks},
       {"line_runs", line_runs},
+      {"tuner_fails", tuner_fails},
   };
   const auto it = checks.find(argc > 1 ? argv[1] : "");
   if (it == checks.end()) {
