@@ -1,5 +1,6 @@
 #include "fake_hip.h"
 
+#include <chrono>
 #include <cxxabi.h>
 #include <hip/hip_runtime_api.h>
 
@@ -8,10 +9,11 @@
 #include <cstring>
 #include <map>
 #include <mutex>
+#include <thread>
 
 namespace fake {
 std::function<void(const Launch&)> on_launch;
-long mallocs_left = -1, pinned_left = -1, instantiates_left = -1, mallocs = 0, captures = 0;
+long mallocs_left = -1, pinned_left = -1, instantiates_left = -1, capture_us = 0, replay_us = 0, mallocs = 0, captures = 0;
 
 static std::mutex mu;
 static std::map<char*, size_t>& blocks() {
@@ -145,6 +147,7 @@ hipError_t hipEventElapsedTime(float* ms, hipEvent_t, hipEvent_t) {
 hipError_t hipStreamBeginCapture(hipStream_t, hipStreamCaptureMode) {
   capturing = true;
   ++captures;
+  if (capture_us) std::this_thread::sleep_for(std::chrono::microseconds(capture_us));
   return hipSuccess;
 }
 hipError_t hipStreamEndCapture(hipStream_t, hipGraph_t* g) {
@@ -159,7 +162,10 @@ hipError_t hipGraphInstantiate(hipGraphExec_t* e, hipGraph_t, hipGraphNode_t*, c
   if (instantiates_left > 0) --instantiates_left;
   return handle(e);
 }
-hipError_t hipGraphLaunch(hipGraphExec_t, hipStream_t) { return hipSuccess; }
+hipError_t hipGraphLaunch(hipGraphExec_t, hipStream_t) {
+  if (replay_us) std::this_thread::sleep_for(std::chrono::microseconds(replay_us));
+  return hipSuccess;
+}
 hipError_t hipGraphDestroy(hipGraph_t) { return hipSuccess; }
 hipError_t hipGraphExecDestroy(hipGraphExec_t) { return hipSuccess; }
 }

@@ -17,6 +17,7 @@ extern std::function<void(const Launch&)> on_launch;
 extern long mallocs_left;        // device allocations that still succeed (negative: all)
 extern long pinned_left;         // pinned ones
 extern long instantiates_left;   // graph instantiations
+extern long capture_us, replay_us;   // what a capture, and a graph launch, takes
 extern long mallocs, captures;   // calls so far
 size_t live();                    // allocations not freed
 size_t bytes_at(const void* p);   // bytes from p to the end of its allocation (0: not in one)

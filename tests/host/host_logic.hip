@@ -351,6 +351,26 @@ static void tuner_fails() {
   gpue_destroy(c);
 }
 
+// The batch's tuner compares steps, not the captures before them: blocks of steps cost
+// less than pairs here, but their captures more.
+static void tuner_times_steps() {
+  for (int steps : {20, 19, 4, 3}) {
+    gpue_ctx* c[3] = {make({48, 64}, 64, 0), make({48, 64}, 64, 0), make({32, 64}, 64, 0)};
+    gpue_batch* b = nullptr;
+    CHECK(gpue_batch_create(c, 3, &b) == GPUE_OK, "batch");
+    fake::capture_us = 5000;
+    fake::replay_us = steps > 16 ? 200 : 0;
+    double us = 0.0;
+    int mode = -1;
+    CHECK(gpue_batch_autotune(b, 0, steps, &us, &mode) == GPUE_OK, "autotune");
+    fake::capture_us = fake::replay_us = 0;
+    CHECK(us < 1000.0, "%g us a step", us);
+    CHECK(steps < 16 || mode == 0, "mode %d", mode);
+    gpue_batch_destroy(b);
+    for (gpue_ctx* x : c) gpue_destroy(x);
+  }
+}
+
 int main(int argc, char** argv) {
   const std::map<std::string, std::function<void()>> checks = {
       {"batch_norms", batch_norms},
@@ -360,6 +380,7 @@ int main(int argc, char** argv) {
       {"step_blocks", step_blocks},
       {"line_runs", line_runs},
       {"tuner_fails", tuner_fails},
+      {"tuner_times_steps", tuner_times_steps},
   };
   const auto it = checks.find(argc > 1 ? argv[1] : "");
   if (it == checks.end()) {
