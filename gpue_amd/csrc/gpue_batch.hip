@@ -19,6 +19,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <array>
 #include <chrono>
 #include <cmath>
 #include <cstring>
@@ -138,18 +139,23 @@ bool mergeable(const std::vector<Sweep>& a, const std::vector<Sweep>& b) {
   return true;
 }
 
-}  // namespace
-
-struct gpue_batch {
-  int device = 0;
-  std::vector<gpue_ctx*> ctx;
-  std::vector<int> active;
-  std::vector<int> cls;            // parity class: the instance's step parity at phase 0
+// The instances as groups, and what belongs to them.
+struct Grouping {
   std::vector<Group> groups;
   // at most four streams (default priority), owned here: the groups with the
   // most work get one each, the others share the last
   std::vector<hipStream_t> streams;
   std::vector<size_t> by_work;     // group indices, most work first (launch order of the replays)
+  std::vector<hipEvent_t> join_ev;   // per group (graph mode 1)
+};
+
+}  // namespace
+
+struct gpue_batch : Grouping {
+  int device = 0;
+  std::vector<gpue_ctx*> ctx;
+  std::vector<int> active;
+  std::vector<int> cls;            // parity class: the instance's step parity at phase 0
   int phase = 0;
   // graph mode 1: one graph per pair of steps for the whole batch, captured on
   // `origin` with a branch per shape group (forked to the group streams and
@@ -157,7 +163,6 @@ struct gpue_batch {
   int graph_mode = 0;
   hipStream_t origin = nullptr;
   hipEvent_t fork_ev = nullptr;
-  std::vector<hipEvent_t> join_ev;   // per group
   hipGraph_t wgraph[2] = {nullptr, nullptr};
   hipGraphExec_t wexec[2] = {nullptr, nullptr};
   double* terms = nullptr;         // pinned: 6 energy terms per instance (gpue_batch_energy)
@@ -431,19 +436,13 @@ static gpue_status build_map(gpue_batch* b, const Group& g, const Sweep& sw, Mer
                                                                                                             : GPUE_EHIP;
 }
 
-extern "C" {
-
-void gpue_batch_destroy(gpue_batch* b) {
-  if (!b) return;
-  for (hipStream_t st : b->streams)
+static void free_grouping(Grouping& gr) {
+  for (hipStream_t st : gr.streams)
     if (st) (void)hipStreamSynchronize(st);
-  if (b->origin) (void)hipStreamSynchronize(b->origin);
-  drop_batch_graphs(b);
-  if (b->fork_ev) (void)hipEventDestroy(b->fork_ev);
-  for (hipEvent_t ev : b->join_ev)
+  for (Group& g : gr.groups) drop_group_graphs(g);
+  for (hipEvent_t ev : gr.join_ev)
     if (ev) (void)hipEventDestroy(ev);
-  if (b->origin) (void)hipStreamDestroy(b->origin);
-  for (Group& g : b->groups)
+  for (Group& g : gr.groups)
     for (int gs = 0; gs < 2; ++gs)
       for (int ph = 0; ph < 2; ++ph)
         for (BSeq& s : g.seqs[gs][ph]) {
@@ -454,8 +453,117 @@ void gpue_batch_destroy(gpue_batch* b) {
           for (Merged& m : s.merged)
             if (m.map) (void)hipFree(m.map);
         }
-  for (hipStream_t st : b->streams)
+  for (hipStream_t st : gr.streams)
     if (st) (void)hipStreamDestroy(st);
+  gr = Grouping();
+}
+
+// Group the instances (those with merged kernels together if `merge`) and lay out their
+// launches; a part of it may be there after a failure (free_grouping).
+static gpue_status make_grouping(gpue_batch* b, bool merge, Grouping& gr) {
+  for (int i = 0; i < (int)b->ctx.size(); ++i) {
+    bool placed = false;
+    const bool mg = merge && can_merge(b->ctx[i]);
+    for (Group& g : gr.groups)
+      if (mg ? g.merged && same_kind_of_problem(g.proto, b->ctx[i]) : !g.merged && same_shape(g.proto, b->ctx[i])) {
+        g.members.push_back(i);
+        placed = true;
+        break;
+      }
+    if (!placed) {
+      Group g;
+      g.proto = b->ctx[i];
+      g.merged = mg;
+      std::copy(g.proto->var, g.proto->var + 3, g.vars);
+      g.members.push_back(i);
+      gr.groups.push_back(g);
+    }
+  }
+  {
+    // A process gets four hardware queues (GPU_MAX_HW_QUEUES); more streams
+    // than that share queues in FIFO order wherever the runtime places them.
+    // So the groups are ranked by work (instances x points), the first three
+    // get a stream each and the rest share the last one, where their graphs
+    // run one after another.
+    std::vector<size_t> order(gr.groups.size());
+    std::iota(order.begin(), order.end(), size_t(0));
+    auto work = [&](size_t k) {
+      double n = 0.0;
+      for (int idx : gr.groups[k].members) n += (double)b->ctx[idx]->N;
+      return n;
+    };
+    std::stable_sort(order.begin(), order.end(), [&](size_t x, size_t y) { return work(x) > work(y); });
+    const size_t ns = std::min<size_t>(gr.groups.size(), kBatchStreams);
+    for (size_t i = 0; i < ns; ++i) {
+      hipStream_t st = nullptr;
+      if (hipStreamCreateWithFlags(&st, hipStreamNonBlocking) != hipSuccess) return GPUE_EHIP;
+      gr.streams.push_back(st);
+    }
+    for (size_t r = 0; r < order.size(); ++r) gr.groups[order[r]].stream = gr.streams[std::min(r, ns - 1)];
+    gr.by_work = order;
+  }
+  gr.join_ev.assign(gr.groups.size(), nullptr);
+  for (hipEvent_t& ev : gr.join_ev)
+    if (hipEventCreateWithFlags(&ev, hipEventDisableTiming) != hipSuccess) return GPUE_EHIP;
+  for (Group& g : gr.groups)
+    for (int gs = 0; gs < 2; ++gs) {
+      // imaginary time: the norm slot holds 1.0 whenever nothing is pending, so
+      // the renormalising first sweep is always safe
+      for (int par = 0; par < 2; ++par) schedule(g.proto, gs, par, gs == 0, g.sched[gs][par]);
+      if (gs == 0) g.defer = can_defer(g, b->ctx);
+      const std::vector<Sweep>& s0 = g.sched[gs][0];
+      const std::vector<Sweep>& s1 = g.sched[gs][1];
+      for (int ph = 0; ph < 2; ++ph) {
+        std::vector<BSeq>& seqs = g.seqs[gs][ph];
+        if (mergeable(s0, s1)) {
+          seqs.resize(1);
+          seqs[0].keys = s0.size() >= s1.size() ? s0 : s1;
+          seqs[0].mask = 3;
+        } else {
+          seqs.resize(2);
+          for (int par = 0; par < 2; ++par) {
+            seqs[par].keys = g.sched[gs][par];
+            seqs[par].mask = 1 << par;
+          }
+        }
+        const size_t M = g.members.size();
+        for (BSeq& s : seqs) {
+          s.hargs.assign(s.keys.size(), std::vector<SweepArgs>(M));
+          s.dargs.assign(s.keys.size(), nullptr);
+          for (size_t k = 0; k < s.keys.size(); ++k)
+            if (hipMalloc((void**)&s.dargs[k], M * sizeof(SweepArgs)) != hipSuccess) return GPUE_ENOMEM;
+          if (g.merged) {
+            s.merged.resize(s.keys.size());
+            for (size_t k = 0; k < s.keys.size(); ++k) {
+              const gpue_status st = build_map(b, g, s.keys[k], s.merged[k]);
+              if (st != GPUE_OK) return st;
+            }
+          }
+          if (gs == 0) {
+            s.hopen.assign(M, SweepArgs{});
+            if (hipMalloc((void**)&s.dopen, M * sizeof(SweepArgs)) != hipSuccess) return GPUE_ENOMEM;
+          }
+          if (gs == 0) {
+            s.hfin.assign(M, FinArgs{});
+            if (hipMalloc((void**)&s.dfin, M * sizeof(FinArgs)) != hipSuccess) return GPUE_ENOMEM;
+          }
+        }
+      }
+    }
+  return GPUE_OK;
+}
+
+extern "C" {
+
+void gpue_batch_destroy(gpue_batch* b) {
+  if (!b) return;
+  if (b->origin) (void)hipStreamSynchronize(b->origin);
+  for (hipStream_t st : b->streams)
+    if (st) (void)hipStreamSynchronize(st);
+  drop_batch_graphs(b);
+  free_grouping(*b);
+  if (b->fork_ev) (void)hipEventDestroy(b->fork_ev);
+  if (b->origin) (void)hipStreamDestroy(b->origin);
   if (b->terms) (void)hipHostFree(b->terms);
   delete b;
 }
@@ -493,118 +601,18 @@ gpue_status gpue_batch_create(gpue_ctx* const* ctxs, int n, gpue_batch** out) {
     gpue_batch_destroy(b);
     return GPUE_EHIP;
   }
-  for (int i = 0; i < n; ++i) {
-    bool placed = false;
-    const bool mg = can_merge(b->ctx[i]);
-    for (Group& g : b->groups)
-      if (mg ? g.merged && same_kind_of_problem(g.proto, b->ctx[i]) : !g.merged && same_shape(g.proto, b->ctx[i])) {
-        g.members.push_back(i);
-        placed = true;
-        break;
-      }
-    if (!placed) {
-      Group g;
-      g.proto = b->ctx[i];
-      g.merged = mg;
-      std::copy(g.proto->var, g.proto->var + 3, g.vars);
-      g.members.push_back(i);
-      b->groups.push_back(g);
-    }
-  }
-  {
-    // A process gets four hardware queues (GPU_MAX_HW_QUEUES); more streams
-    // than that share queues in FIFO order wherever the runtime places them.
-    // So the groups are ranked by work (instances x points), the first three
-    // get a stream each and the rest share the last one, where their graphs
-    // run one after another.
-    std::vector<size_t> order(b->groups.size());
-    std::iota(order.begin(), order.end(), size_t(0));
-    auto work = [&](size_t k) {
-      double n = 0.0;
-      for (int idx : b->groups[k].members) n += (double)b->ctx[idx]->N;
-      return n;
-    };
-    std::stable_sort(order.begin(), order.end(), [&](size_t x, size_t y) { return work(x) > work(y); });
-    const size_t ns = std::min<size_t>(b->groups.size(), kBatchStreams);
-    for (size_t i = 0; i < ns; ++i) {
-      hipStream_t st = nullptr;
-      if (hipStreamCreateWithFlags(&st, hipStreamNonBlocking) != hipSuccess) {
-        gpue_batch_destroy(b);
-        return GPUE_EHIP;
-      }
-      b->streams.push_back(st);
-    }
-    for (size_t r = 0; r < order.size(); ++r) b->groups[order[r]].stream = b->streams[std::min(r, ns - 1)];
-    b->by_work = order;
-  }
-  b->join_ev.assign(b->groups.size(), nullptr);
   if (hipStreamCreateWithFlags(&b->origin, hipStreamNonBlocking) != hipSuccess ||
       hipEventCreateWithFlags(&b->fork_ev, hipEventDisableTiming) != hipSuccess) {
     gpue_batch_destroy(b);
     return GPUE_EHIP;
   }
-  for (hipEvent_t& ev : b->join_ev)
-    if (hipEventCreateWithFlags(&ev, hipEventDisableTiming) != hipSuccess) {
+  {
+    const gpue_status st = make_grouping(b, true, *b);
+    if (st != GPUE_OK) {
       gpue_batch_destroy(b);
-      return GPUE_EHIP;
+      return st;
     }
-  for (Group& g : b->groups)
-    for (int gs = 0; gs < 2; ++gs) {
-      // imaginary time: the norm slot holds 1.0 whenever nothing is pending, so
-      // the renormalising first sweep is always safe
-      for (int par = 0; par < 2; ++par) schedule(g.proto, gs, par, gs == 0, g.sched[gs][par]);
-      if (gs == 0) g.defer = can_defer(g, b->ctx);
-      const std::vector<Sweep>& s0 = g.sched[gs][0];
-      const std::vector<Sweep>& s1 = g.sched[gs][1];
-      for (int ph = 0; ph < 2; ++ph) {
-        std::vector<BSeq>& seqs = g.seqs[gs][ph];
-        if (mergeable(s0, s1)) {
-          seqs.resize(1);
-          seqs[0].keys = s0.size() >= s1.size() ? s0 : s1;
-          seqs[0].mask = 3;
-        } else {
-          seqs.resize(2);
-          for (int par = 0; par < 2; ++par) {
-            seqs[par].keys = g.sched[gs][par];
-            seqs[par].mask = 1 << par;
-          }
-        }
-        const size_t M = g.members.size();
-        for (BSeq& s : seqs) {
-          s.hargs.assign(s.keys.size(), std::vector<SweepArgs>(M));
-          s.dargs.assign(s.keys.size(), nullptr);
-          for (size_t k = 0; k < s.keys.size(); ++k)
-            if (hipMalloc((void**)&s.dargs[k], M * sizeof(SweepArgs)) != hipSuccess) {
-              gpue_batch_destroy(b);
-              return GPUE_ENOMEM;
-            }
-          if (g.merged) {
-            s.merged.resize(s.keys.size());
-            for (size_t k = 0; k < s.keys.size(); ++k) {
-              const gpue_status st = build_map(b, g, s.keys[k], s.merged[k]);
-              if (st != GPUE_OK) {
-                gpue_batch_destroy(b);
-                return st;
-              }
-            }
-          }
-          if (gs == 0) {
-            s.hopen.assign(M, SweepArgs{});
-            if (hipMalloc((void**)&s.dopen, M * sizeof(SweepArgs)) != hipSuccess) {
-              gpue_batch_destroy(b);
-              return GPUE_ENOMEM;
-            }
-          }
-          if (gs == 0) {
-            s.hfin.assign(M, FinArgs{});
-            if (hipMalloc((void**)&s.dfin, M * sizeof(FinArgs)) != hipSuccess) {
-              gpue_batch_destroy(b);
-              return GPUE_ENOMEM;
-            }
-          }
-        }
-      }
-    }
+  }
   fill_args(b);
   if (upload_args(b) != GPUE_OK) {
     gpue_batch_destroy(b);
@@ -756,27 +764,16 @@ static gpue_status set_group_variant(gpue_batch* b, Group& g, int a, int v) {
   return upload_args(b);
 }
 
-gpue_status gpue_batch_autotune(gpue_batch* b, int gstate, int steps, double* us_per_step, int* graph_mode) {
-  if (!b || steps < 2 || (gstate != 0 && gstate != 1)) return GPUE_EINVAL;
-  gpue_status st = sync_groups(b);
-  if (st != GPUE_OK) return st;
-  // save every instance's state: psi into its scratch buffer, the step counter,
-  // the pending norm and its value
-  const size_t n = b->ctx.size();
-  std::vector<int> next(n), pend(n), cls = b->cls;
-  std::vector<double> nrm(n);
-  const int phase = b->phase;
-  for (size_t i = 0; i < n; ++i) {
-    gpue_ctx* c = b->ctx[i];
-    next[i] = c->next_step;
-    pend[i] = c->pending_norm;
-    BHIP(b, hipMemcpyAsync(c->tmp, c->psi, c->N * c->esz, hipMemcpyDeviceToDevice, c->stream));
-    BHIP(b, hipMemcpyAsync(&nrm[i], c->results, sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    BHIP(b, hipStreamSynchronize(c->stream));
-  }
-  double best = 0.0;
-  st = time_batch(b, gstate, steps, &best);
-  // coordinate descent: groups with the most points first, then each axis
+// The arguments of a grouping that has just come into use.
+static gpue_status load_grouping(gpue_batch* b) {
+  fill_args(b);
+  return upload_args(b);
+}
+
+// The time per step of the batch, and the variants of its unmerged groups that lower it:
+// coordinate descent over the groups, those with the most points first, then each axis.
+static gpue_status tune_groups(gpue_batch* b, int gstate, int steps, double* best) {
+  gpue_status st = time_batch(b, gstate, steps, best);
   std::vector<size_t> order(b->groups.size());
   for (size_t k = 0; k < order.size(); ++k) order[k] = k;
   std::sort(order.begin(), order.end(), [&](size_t x, size_t y) {
@@ -796,13 +793,74 @@ gpue_status gpue_batch_autotune(gpue_batch* b, int gstate, int steps, double* us
         st = set_group_variant(b, g, a, v);
         double us = 0.0;
         if (st == GPUE_OK) st = time_batch(b, gstate, steps, &us);
-        if (st == GPUE_OK && us < best) {
-          best = us;
+        if (st == GPUE_OK && us < *best) {
+          *best = us;
           pick = v;
         }
       }
       if (st == GPUE_OK && g.vars[a] != pick) st = set_group_variant(b, g, a, pick);
     }
+  }
+  return st;
+}
+
+gpue_status gpue_batch_autotune(gpue_batch* b, int gstate, int steps, double* us_per_step, int* graph_mode) {
+  if (!b || steps < 2 || (gstate != 0 && gstate != 1)) return GPUE_EINVAL;
+  gpue_status st = sync_groups(b);
+  if (st != GPUE_OK) return st;
+  // save every instance's state: psi into its scratch buffer, the step counter,
+  // the pending norm and its value
+  const size_t n = b->ctx.size();
+  std::vector<int> next(n), pend(n), cls = b->cls;
+  std::vector<double> nrm(n);
+  const int phase = b->phase;
+  for (size_t i = 0; i < n; ++i) {
+    gpue_ctx* c = b->ctx[i];
+    next[i] = c->next_step;
+    pend[i] = c->pending_norm;
+    BHIP(b, hipMemcpyAsync(c->tmp, c->psi, c->N * c->esz, hipMemcpyDeviceToDevice, c->stream));
+    BHIP(b, hipMemcpyAsync(&nrm[i], c->results, sizeof(double), hipMemcpyDeviceToHost, c->stream));
+    BHIP(b, hipStreamSynchronize(c->stream));
+  }
+  double best = 0.0;
+  st = tune_groups(b, gstate, steps, &best);
+  // Launches by shape, which have variants to choose, in place of merged ones: they win
+  // where a few groups fill the chip (us a step in imaginary time with rotation, merged /
+  // by shape and tuned: eight 512^2 FP64 84 / 73, sixty-four 256^2 FP64 138 / 120), and
+  // lose where there are more shapes than streams (fifteen 128^2-512^2 FP32 59 / 68).
+  // Merged launches stay unless more than the timings' noise is gained.
+  bool merged = false;
+  for (const Group& g : b->groups) merged = merged || g.merged;
+  if (st == GPUE_OK && merged) {
+    std::vector<std::array<int, 4>> vars(n);   // and whether they are the defaults
+    for (size_t i = 0; i < n; ++i) {
+      const gpue_ctx* c = b->ctx[i];
+      vars[i] = {c->var[0], c->var[1], c->var[2], c->var_default};
+    }
+    Grouping by_shape;
+    if (make_grouping(b, false, by_shape) != GPUE_OK) {
+      (void)hipGetLastError();   // no memory to try it: the batch stays merged
+    } else {
+      drop_batch_graphs(b);
+      std::swap((Grouping&)*b, by_shape);
+      double us = 0.0;
+      st = load_grouping(b);
+      if (st == GPUE_OK) st = tune_groups(b, gstate, steps, &us);
+      if (st == GPUE_OK && us < 0.99 * best) {
+        best = us;
+      } else {
+        (void)sync_groups(b);
+        drop_batch_graphs(b);
+        std::swap((Grouping&)*b, by_shape);
+        for (size_t i = 0; i < n; ++i) {
+          (void)gpue_set_variants(b->ctx[i], vars[i].data());
+          b->ctx[i]->var_default = vars[i][3] != 0;
+        }
+        const gpue_status back = load_grouping(b);
+        if (st == GPUE_OK) st = back;
+      }
+    }
+    free_grouping(by_shape);
   }
   // then the graph mode: per-group graphs or one graph for the whole batch
   if (st == GPUE_OK) {

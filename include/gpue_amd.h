@@ -256,9 +256,10 @@ gpue_status gpue_batch_set_graph_mode(gpue_batch *b, int mode);
 /* No counterpart in the reference (GPUE runs one problem per process): choose
  * the kernel variants of every shape group, and the graph mode, for the batch
  * as a whole (a lone instance's choice serves latency; in a batch the groups
- * share the device; merged launches have one set of variants).  Coordinate descent over the groups, largest first, and
- * their axes; each candidate is timed over `steps` steps of gstate of the whole
- * batch.  Every instance's psi, step counter and pending norm are restored
+ * share the device), and whether instances whose launches can be merged run merged
+ * or by shape (merged launches have one set of variants).  Coordinate descent over the
+ * groups, largest first, and their axes; each candidate is timed over `steps` steps of
+ * gstate of the whole batch.  Every instance's psi, step counter and pending norm are restored
  * afterwards.  us_per_step, graph_mode (either may be NULL): the best time per
  * batch step and the graph mode chosen. */
 gpue_status gpue_batch_autotune(gpue_batch *b, int gstate, int steps, double *us_per_step, int *graph_mode);

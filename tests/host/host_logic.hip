@@ -1,12 +1,14 @@
 // The library's host code on the runtime of fake_hip.cpp: what it launches and with
 // which arguments, and what it leaves behind where memory runs out.  Built and run by
 // tests/test_host_logic.py, one argument: the check to run.
+#include <chrono>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
 #include <functional>
 #include <map>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "../../gpue_amd/csrc/ctx_internal.h"
@@ -371,6 +373,40 @@ static void tuner_times_steps() {
   }
 }
 
+// The batch's tuner takes merged launches apart where launches by shape are faster, keeps
+// them (and the contexts' variants) where they are not or where there is no memory to try.
+static void tuner_regroups() {
+  for (int slow : {0, 1, 2}) {   // merged launches; launches by shape; those, and no memory
+    const size_t live = fake::live();
+    Audit audit;
+    std::vector<gpue_ctx*> c;
+    for (int n : {64, 128, 64, 96}) c.push_back(make({n, 64}, 64, 1));
+    c.push_back(make({48, 64}, 64, 1));   // has no merged kernels
+    gpue_batch* b = nullptr;
+    CHECK(gpue_batch_create(c.data(), (int)c.size(), &b) == GPUE_OK && gpue_batch_set_graph_mode(b, 2) == GPUE_OK, "batch");
+    fake::on_launch = [&](const fake::Launch& l) {
+      audit(l);
+      if ((l.kernel.find("_merged") != std::string::npos) == (slow == 0))
+        std::this_thread::sleep_for(std::chrono::microseconds(300));
+    };
+    fake::mallocs_left = slow == 2 ? 3 : -1;
+    CHECK(gpue_batch_autotune(b, 0, 4, nullptr, nullptr) == GPUE_OK, "%s", gpue_batch_last_error(b));
+    fake::mallocs_left = -1;
+    fake::on_launch = [&](const fake::Launch& l) { audit(l); };
+    audit.kernels.clear();
+    CHECK(gpue_batch_set_graph_mode(b, 2) == GPUE_OK && gpue_batch_set_active(b, 1, 0) == GPUE_OK, "active");
+    for (int gstate : {0, 1, 0}) CHECK(gpue_batch_evolve(b, 37, gstate) == GPUE_OK, "evolve");
+    CHECK((audit.kernels["gpue::row_merged"] == 0) == (slow == 0) && audit.kernels["gpue::row_sweep_b"] > 0,
+          "%ld merged row sweeps, slow %d", audit.kernels["gpue::row_merged"], slow);
+    if (slow)
+      for (int k = 0; k < 4; ++k)
+        CHECK(c[k]->var_default && c[k]->var[0] == MERGE_ROW && c[k]->var[1] == MERGE_COL, "variants of member %d", k);
+    gpue_batch_destroy(b);
+    for (gpue_ctx* x : c) gpue_destroy(x);
+    CHECK(fake::live() == live, "%zu allocations left", fake::live() - live);
+  }
+}
+
 int main(int argc, char** argv) {
   const std::map<std::string, std::function<void()>> checks = {
       {"batch_norms", batch_norms},
@@ -381,6 +417,7 @@ int main(int argc, char** argv) {
       {"line_runs", line_runs},
       {"tuner_fails", tuner_fails},
       {"tuner_times_steps", tuner_times_steps},
+      {"tuner_regroups", tuner_regroups},
   };
   const auto it = checks.find(argc > 1 ? argv[1] : "");
   if (it == checks.end()) {
