@@ -458,12 +458,29 @@ static void free_grouping(Grouping& gr) {
   gr = Grouping();
 }
 
+// Whether instances of c's kind run merged by default.  FP64 boxes do beyond four shapes
+// only: up to there each shape has a stream, and its own kernels, with twiddles up front
+// and the registers of one length, win (us a step, merged / by shape: eight 64^3 62.6 / 56.3
+// and rotating in real time 105.5 / 82.7, four 96^3 121 / 107, three shapes 52.4 / 39.0, four
+// rotating 201 / 170; six rotating 123 / 143, twelve 189 / 334).  FP32 boxes and planes gain
+// from merging with equal shapes too (sweep_merged.h).
+static bool merge_pays(const gpue_batch* b, const gpue_ctx* c) {
+  if (c->p.dimnum != 3 || c->prec != 64) return true;
+  std::vector<const gpue_ctx*> shapes;
+  for (const gpue_ctx* x : b->ctx) {
+    if (!can_merge(x) || !same_kind_of_problem(x, c)) continue;
+    if (std::none_of(shapes.begin(), shapes.end(), [&](const gpue_ctx* y) { return same_shape(x, y); })) shapes.push_back(x);
+    if (shapes.size() > kBatchStreams) return true;
+  }
+  return false;
+}
+
 // Group the instances (those with merged kernels together if `merge`) and lay out their
 // launches; a part of it may be there after a failure (free_grouping).
 static gpue_status make_grouping(gpue_batch* b, bool merge, Grouping& gr) {
   for (int i = 0; i < (int)b->ctx.size(); ++i) {
     bool placed = false;
-    const bool mg = merge && can_merge(b->ctx[i]);
+    const bool mg = merge && can_merge(b->ctx[i]) && merge_pays(b, b->ctx[i]);
     for (Group& g : gr.groups)
       if (mg ? g.merged && same_kind_of_problem(g.proto, b->ctx[i]) : !g.merged && same_shape(g.proto, b->ctx[i])) {
         g.members.push_back(i);

@@ -10,7 +10,9 @@
 // the whole batch is four launches.
 // Measured on those sixteen problems (imaginary time, us a step): launches per size on
 // four streams 110 in FP32 and 138 in FP64, merged 65 and 82; three of 512^2 alone 53
-// and 69, now 37 and 54.  A merged sweep takes 13-20 us, in which its waves wait half
+// and 69, now 37 and 54.  Equal shapes gain too, by shape / merged: sixteen 128^2 FP64 with
+// rotation 27.7 / 27.3, sixteen 256^2 FP32 57 / 38, thirty-two 512^2 FP64 372 / 260, thirty-two
+// 64^3 FP32 164 / 127; not FP64 boxes (merge_pays).  A merged sweep takes 13-20 us, in which its waves wait half
 // of their life for memory and exchanges.
 #pragma once
 #include "sweep_launch.h"

@@ -220,7 +220,7 @@ double      gpue_eqn_eval(const gpue_eqn_node *nodes, int n_nodes, double x, dou
  * process; its bin/run.sh starts several processes).  2D and 3D instances of one
  * precision, dimension and gauge whose axes are 64 to 512 points, with the
  * variants small contexts start with, share every sweep launch, whatever their
- * sizes.  Other instances form groups of one shape that share launches; groups
+ * sizes (3D FP64 ones where they have more than four shapes).  Other instances form groups of one shape that share launches; groups
  * run on at most four streams (the device's hardware queues per process: the
  * three groups with the most work get one each, the rest share the fourth).
  * Blocks of steps of a group are captured as HIP graphs and replayed.

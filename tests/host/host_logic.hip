@@ -183,7 +183,8 @@ static void batch_norms() {
 // normalisations stay in step.  (Merged boxes of different sizes, and a group of one
 // shape without merged kernels.)
 static void batch_members_change() {
-  const std::vector<std::vector<int>> shapes = {{64, 128, 64}, {64, 64, 96}, {128, 64, 64}, {48, 64, 16}, {48, 64, 16}};
+  const std::vector<std::vector<int>> shapes = {{64, 128, 64}, {64, 64, 96}, {128, 64, 64}, {64, 96, 64}, {64, 64, 64},
+                                                 {48, 64, 16},  {48, 64, 16}};
   for (int prec : {64, 32}) {
     Audit audit;
     fake::on_launch = [&](const fake::Launch& l) { audit(l); };
@@ -407,6 +408,27 @@ static void tuner_regroups() {
   }
 }
 
+// FP64 boxes share merged launches beyond four shapes, FP32 ones and planes always.
+static void batch_boxes() {
+  const std::vector<std::vector<int>> shapes = {{64, 64, 64}, {64, 64, 96}, {64, 96, 64}, {96, 64, 64}, {64, 64, 128}};
+  for (int prec : {64, 32})
+    for (int kinds = 1; kinds <= 5; ++kinds) {
+      Audit audit;
+      std::vector<gpue_ctx*> c;
+      for (int k = 0; k < kinds + 2; ++k) c.push_back(make(shapes[k % kinds], prec, 1));
+      c.push_back(make({64, 96}, prec, 1));
+      gpue_batch* b = nullptr;
+      CHECK(gpue_batch_create(c.data(), (int)c.size(), &b) == GPUE_OK, "batch");
+      fake::on_launch = [&](const fake::Launch& l) { audit(l); };
+      CHECK(gpue_batch_evolve(b, 3, 0) == GPUE_OK && gpue_batch_evolve(b, 3, 1) == GPUE_OK, "evolve");
+      const bool by_shape = audit.kernels["gpue::col_sweep_b"] > 0;
+      CHECK(audit.kernels["gpue::col_merged"] > 0, "the plane");
+      CHECK(by_shape == (prec == 64 && kinds <= 4), "%d kinds of boxes, %d bits", kinds, prec);
+      gpue_batch_destroy(b);
+      for (gpue_ctx* x : c) gpue_destroy(x);
+    }
+}
+
 int main(int argc, char** argv) {
   const std::map<std::string, std::function<void()>> checks = {
       {"batch_norms", batch_norms},
@@ -416,6 +438,7 @@ int main(int argc, char** argv) {
       {"step_blocks", step_blocks},
       {"line_runs", line_runs},
       {"tuner_fails", tuner_fails},
+      {"batch_boxes", batch_boxes},
       {"tuner_times_steps", tuner_times_steps},
       {"tuner_regroups", tuner_regroups},
   };
