@@ -156,6 +156,7 @@ __device__ __forceinline__ void row_body(SweepArgs a, int bid, int nblk, int tx,
   constexpr bool VHALF = MODE != RM_GAUGE && MODE != RM_K && MODE != RM_KSUM;
   using P = Plan<N, V>;
   constexpr int TPL = P::TPL, E = P::E, LPW = RowCfg<N, RV>::LPW;
+  constexpr bool AHEAD = EARLY && E <= 8;   // see apply_phase_all
   if constexpr (EARLY) pin_args<VHALF, KSTEP, GAUGE, OPENS>(a);
   const Phys& p = a.ph;
   const unsigned flags = a.flags;
@@ -188,19 +189,23 @@ __device__ __forceinline__ void row_body(SweepArgs a, int bid, int nblk, int tx,
   auto half = [&](auto closes) {
     if constexpr (EARLY) vo.ready();
     else vo.load(p, Vt, l);
-    vo.template half<REAL, decltype(closes)::value>(p, l, v);
+    vo.template half<REAL, decltype(closes)::value, AHEAD>(p, l, v);
   };
   auto kstep = [&]() {
-    if constexpr (EARLY) ko.ready();
-    else ko.load(p, l);
-    ko.apply(p, l, v, a.invN);
+    if constexpr (!EARLY && REAL) {
+      ko.load_apply(p, l, v, a.invN);
+    } else {
+      if constexpr (EARLY) ko.ready();
+      else ko.load(p, l);
+      ko.template apply<AHEAD>(p, l, v, a.invN);
+    }
   };
   auto gauge = [&]() {
     if constexpr (!EARLY) {
       go.load(p, l);
       go.prep(p, l, a.invN);
     }
-    go.apply(p, v, l, a.invN, GEARLY);
+    go.template apply<AHEAD>(p, v, l, a.invN, GEARLY);
   };
 
   if constexpr (EARLY && GAUGE) go.load(p, l);
@@ -237,7 +242,7 @@ __device__ __forceinline__ void row_body(SweepArgs a, int bid, int nblk, int tx,
 #pragma unroll
         for (int r = 0; r < E; ++r) arg[r] += arg[r];
       }
-      apply_phase_all<T, E, REAL>(v, arg, 1.0);
+      apply_phase_all<T, E, REAL, AHEAD>(v, arg, 1.0);
       fwd();
     } else if constexpr (MODE == RM_INV_FWD) {
       half(ClosingHalf());   // FP32 (static V): each half's phase rounds psi, as in single steps
@@ -332,6 +337,7 @@ __device__ __forceinline__ void col_body(SweepArgs a, int bid, int nblk, int tx,
   constexpr bool OPENS = !REAL && MODE == CM_FWD_V;
   using P = Plan<N, V>;
   constexpr int TC = ColCfg<T, N, CV>::TC, E = P::E, TPL = P::TPL;
+  constexpr bool AHEAD = EARLY && E <= 8;   // see apply_phase_all
   if constexpr (EARLY) pin_args<VHALF, MODE == CM_K, GAUGE, OPENS>(a);
   const Phys& p = a.ph;
   const unsigned flags = a.flags;
@@ -368,14 +374,14 @@ __device__ __forceinline__ void col_body(SweepArgs a, int bid, int nblk, int tx,
   auto half = [&](auto closes) {
     if constexpr (EARLY) vo.ready();
     else vo.load(p, Vt, l);
-    vo.template half<REAL, decltype(closes)::value>(p, l, v);
+    vo.template half<REAL, decltype(closes)::value, AHEAD>(p, l, v);
   };
   auto gauge = [&]() {
     if constexpr (!EARLY) {
       go.load(p, l);
       go.prep(p, l, a.invN);
     }
-    go.apply(p, v, l, a.invN, GEARLY);
+    go.template apply<AHEAD>(p, v, l, a.invN, GEARLY);
   };
 
   if constexpr (EARLY && GAUGE) go.load(p, l);
@@ -426,9 +432,13 @@ __device__ __forceinline__ void col_body(SweepArgs a, int bid, int nblk, int tx,
         }
       }
     } else if constexpr (MODE == CM_K) {
-      if constexpr (EARLY) ko.ready();
-      else ko.load(p, l);
-      ko.apply(p, l, v, a.invN);
+      if constexpr (!EARLY && REAL) {
+        ko.load_apply(p, l, v, a.invN);
+      } else {
+        if constexpr (EARLY) ko.ready();
+        else ko.load(p, l);
+        ko.template apply<AHEAD>(p, l, v, a.invN);
+      }
       inv();
     } else if constexpr (GAUGE) {
       gauge();
@@ -510,14 +520,14 @@ __device__ __forceinline__ void line_body(const SweepArgs& a, int nsteps) {
 #pragma unroll
       for (int r = 0; r < E; ++r) v[r] = scale_norm(v[r], f);
     }
-    vo.template half<REAL, false>(p, l, v);
+    vo.template half<REAL, false, true>(p, l, v);
     fwd();
-    ko.apply(p, l, v, a.invN);
+    ko.template apply<true>(p, l, v, a.invN);
     inv();
-    vo.template half<REAL, true>(p, l, v);
+    vo.template half<REAL, true, true>(p, l, v);
     if (gauge) {
       fwd();
-      go.apply(p, v, l, a.invN, false);
+      go.template apply<true>(p, v, l, a.invN, false);
       inv();
     }
     if constexpr (!REAL) {

@@ -384,10 +384,23 @@ struct VTab<float> {
   static __device__ __forceinline__ const float* get(const Phys& p, int a) { return pick(a, p.vsf[0], p.vsf[1], p.vsf[2]); }
 };
 
-// The sincos of E arguments that may need the library (huge, infinite, NaN): one
-// point at a time, the arrays rotating through their first slot, so that the kernel
-// holds one copy of the library code instead of E (they made up most of a sweep's
-// 36-107 KB) and no array is indexed by a variable.
+// v times the phase (cs, sn) and s: see apply_phase_all.
+template <typename T>
+__device__ __forceinline__ cx<T> times_phase(cx<T> v, T cs, T sn, double s_) {
+  if constexpr (sizeof(T) == 8) {
+    return cmul(mk(cs * s_, sn * s_), v);
+  } else {
+    const double c0 = cs, d0 = sn;
+    const double f = fma(-0.5, fma(c0, c0, d0 * d0), 1.5) * s_;
+    const cx<double> w = cmul(mk(c0 * f, d0 * f), mk((double)v.x, (double)v.y));
+    return mk((float)w.x, (float)w.y);
+  }
+}
+
+// E points whose arguments may need the library (huge, infinite, NaN): one at a time,
+// the arrays rotating through their first slot, so that the kernel holds one copy of the
+// library code instead of E (they made up most of a sweep's 36-107 KB) and no array is
+// indexed by a variable.  The factors ...
 template <typename T, int E>
 __device__ __forceinline__ void sincos_any(T (&x)[E], T (&sn)[E], T (&cs)[E]) {
 #pragma unroll
@@ -406,6 +419,22 @@ __device__ __forceinline__ void sincos_any(T (&x)[E], T (&sn)[E], T (&cs)[E]) {
     cs[E - 1] = c;
   }
 }
+// ... or the points times their phases.
+template <typename T, int E>
+__device__ __forceinline__ void phase_any(cx<T>* v, T (&x)[E], double s) {
+#pragma unroll 1
+  for (int k = 0; k < E; ++k) {
+    T sn, cs;
+    WMath<T>::sc(x[0], &sn, &cs);
+    const cx<T> u = times_phase(v[0], cs, sn, s);
+#pragma unroll
+    for (int r = 0; r + 1 < E; ++r) {
+      x[r] = x[r + 1];
+      v[r] = v[r + 1];
+    }
+    v[E - 1] = u;
+  }
+}
 
 // psi * exp(-arg) (imaginary time) or psi * exp(-i arg) (REAL), times s.
 // FP64: a lane whose arguments are all small takes the short polynomials.
@@ -416,7 +445,14 @@ __device__ __forceinline__ void sincos_any(T (&x)[E], T (&sn)[E], T (&cs)[E]) {
 // A and K, so the norm and energy would drift linearly with the steps; after the
 // Newton step the modulus is 1 within ~1e-14, and what is left (the FP32 phase,
 // ~1e-7 relative) acts like a rounded V and does not grow.
-template <typename T, int E, bool REAL>
+// AHEAD (real time): all factors before the first product, for serial chains with
+// registers to spare (line_body, and sweeps of small grids with up to 8 points a lane).
+// Elsewhere each branch finishes its points: factors kept across the join, and through the
+// loop of the library branch, are 4 registers a point, which left FP64 lanes of 16 points
+// one wave per SIMD and made 1024-lane workgroups spill (real time, us a step, with / without:
+// 384 x 4096 FP32 69 / 46, 1024 x 4096 FP64 107 / 81, 64 x 64 x 512 FP64 61.6 / 54.9; the other
+// way a line of 4096 points takes 8.4 / 10.1, one of 1024 3.19 / 3.27, 384^2 loses 1 %).
+template <typename T, int E, bool REAL, bool AHEAD>
 __device__ __forceinline__ void apply_phase_all(cx<T>* v, const T (&arg)[E], double s_) {
   const T s = (T)s_;
   if constexpr (!REAL) {
@@ -434,7 +470,7 @@ __device__ __forceinline__ void apply_phase_all(cx<T>* v, const T (&arg)[E], dou
     for (int r = 0; r < E; ++r) v[r] = scaled(v[r], WMath<T>::ex(-arg[r]) * s);
   } else {
     // one range check for the lane's E arguments, then branch-free forms
-    T x[E], sn[E], cs[E];
+    T x[E];
     bool small = true, fast = true;
 #pragma unroll
     for (int r = 0; r < E; ++r) {
@@ -442,28 +478,39 @@ __device__ __forceinline__ void apply_phase_all(cx<T>* v, const T (&arg)[E], dou
       small = small && (sizeof(T) == 8 ? fabs((double)x[r]) <= SMALL_ARG : sincos_small_ok(x[r]));
       fast = fast && sincos_fast_ok(x[r]);
     }
-    if (small) {
+    if constexpr (AHEAD) {
+      T sn[E], cs[E];
+      if (small) {
+#pragma unroll
+        for (int r = 0; r < E; ++r) {
+          if constexpr (sizeof(T) == 8) sincos_small(x[r], &sn[r], &cs[r]);
+          else sincos_poly(x[r], &sn[r], &cs[r]);
+        }
+      } else if (fast) {
+#pragma unroll
+        for (int r = 0; r < E; ++r) sincos_core(x[r], &sn[r], &cs[r]);
+      } else {
+        sincos_any<T, E>(x, sn, cs);
+      }
+#pragma unroll
+      for (int r = 0; r < E; ++r) v[r] = times_phase(v[r], cs[r], sn[r], s_);
+    } else if (small) {
 #pragma unroll
       for (int r = 0; r < E; ++r) {
-        if constexpr (sizeof(T) == 8) sincos_small(x[r], &sn[r], &cs[r]);
-        else sincos_poly(x[r], &sn[r], &cs[r]);
+        T sn, cs;
+        if constexpr (sizeof(T) == 8) sincos_small(x[r], &sn, &cs);
+        else sincos_poly(x[r], &sn, &cs);
+        v[r] = times_phase(v[r], cs, sn, s_);
       }
     } else if (fast) {
 #pragma unroll
-      for (int r = 0; r < E; ++r) sincos_core(x[r], &sn[r], &cs[r]);
-    } else {
-      sincos_any<T, E>(x, sn, cs);
-    }
-#pragma unroll
-    for (int r = 0; r < E; ++r) {
-      if constexpr (sizeof(T) == 8) {
-        v[r] = cmul(mk(cs[r] * s, sn[r] * s), v[r]);
-      } else {
-        const double c0 = cs[r], d0 = sn[r];
-        const double f = fma(-0.5, fma(c0, c0, d0 * d0), 1.5) * s_;
-        const double c = c0 * f, d = d0 * f, vx = v[r].x, vy = v[r].y;
-        v[r] = mk((float)(c * vx - d * vy), (float)(c * vy + d * vx));
+      for (int r = 0; r < E; ++r) {
+        T sn, cs;
+        sincos_core(x[r], &sn, &cs);
+        v[r] = times_phase(v[r], cs, sn, s_);
       }
+    } else {
+      phase_any<T, E>(v, x, s_);
     }
   }
 }
@@ -527,11 +574,11 @@ struct VOp {
       }
     }
   }
-  template <bool REAL, bool CLOSES>
+  template <bool REAL, bool CLOSES, bool AHEAD>
   __device__ __forceinline__ void half(const Phys& p, const LineAt& l, cx<T>* v) const {
     T arg[E];
     args<CLOSES>(p, l, v, arg);
-    apply_phase_all<T, E, REAL>(v, arg, 1.0);
+    apply_phase_all<T, E, REAL, AHEAD>(v, arg, 1.0);
   }
 };
 
@@ -620,6 +667,7 @@ struct GOp {
     }
   }
   // `early`: load_points() was called up front where A is a table
+  template <bool AHEAD>
   __device__ __forceinline__ void apply(const Phys& p, cx<T>* v, const LineAt& l, double invn, bool early) {
     if constexpr (LIN) {
       if (lin) {
@@ -632,7 +680,7 @@ struct GOp {
     const T Dt = (T)p.Dt;
 #pragma unroll
     for (int r = 0; r < E; ++r) arg[r] = (p.a_kind == A_TABLE ? at[r] : (T)A) * kk[r] * Dt;
-    apply_phase_all<T, E, REAL>(v, arg, invn);
+    apply_phase_all<T, E, REAL, AHEAD>(v, arg, invn);
   }
 };
 
@@ -671,31 +719,59 @@ struct KOp {
 #pragma unroll
     for (int r = 0; r < E; ++r) arrive(e[r]);
   }
-  // FP32 imaginary time multiplies the axes' factors in the order x, y, z
+  // A separable K: f0 f1 and 1/N once, then a factor a point.  FP32 imaginary time
+  // multiplies the axes' factors in the order x, y, z.
+  struct Sep {
+    cx<F> f0, f1, f;
+    double invN;
+    bool z;
+    __device__ __forceinline__ Sep(const LineAt& l, cx<F> f0_, cx<F> f1_, double invN_)
+        : f0(f0_), f1(f1_), invN(invN_), z(l.ax == 2) {
+      if constexpr (REAL) f = cscale(cmul(f0, f1), invN);
+      else f = mk(f0.x * f1.x * (F)invN, (F)0);
+    }
+    __device__ __forceinline__ cx<T> operator()(cx<F> e, cx<T> v) const {
+      if constexpr (REAL) {
+        const cx<double> u = cmul(cmul(e, f), mk((double)v.x, (double)v.y));
+        return mk((T)u.x, (T)u.y);
+      } else if constexpr (sizeof(T) == 8) {
+        return scaled(v, e.x * f.x);
+      } else {
+        return scaled(v, (z ? f0.x * f1.x * e.x : e.x * f0.x * f1.x) * (T)invN);
+      }
+    }
+  };
+  // on factors loaded up front
+  template <bool AHEAD>
   __device__ __forceinline__ void apply(const Phys& p, const LineAt& l, cx<T>* v, double invN) const {
     if (p.k_kind == K_SEP) {
-      if constexpr (REAL) {
-        const cx<double> f = cscale(cmul(f0, f1), invN);
+      const Sep k(l, f0, f1, invN);
 #pragma unroll
-        for (int r = 0; r < E; ++r) {
-          const cx<double> u = cmul(cmul(e[r], f), mk((double)v[r].x, (double)v[r].y));
-          v[r] = mk((T)u.x, (T)u.y);
-        }
-      } else if constexpr (sizeof(T) == 8) {
-        const T f = f0.x * f1.x * (T)invN;
-#pragma unroll
-        for (int r = 0; r < E; ++r) v[r] = scaled(v[r], e[r].x * f);
-      } else {
-#pragma unroll
-        for (int r = 0; r < E; ++r)
-          v[r] = scaled(v[r], (l.ax == 2 ? f0.x * f1.x * e[r].x : e[r].x * f0.x * f1.x) * (T)invN);
-      }
+      for (int r = 0; r < E; ++r) v[r] = k(e[r], v[r]);
     } else {
       T arg[E];
       const T cK = (T)p.cK;
 #pragma unroll
       for (int r = 0; r < E; ++r) arg[r] = (T)e[r].x * cK;
-      apply_phase_all<T, E, REAL>(v, arg, invN);
+      apply_phase_all<T, E, REAL, AHEAD>(v, arg, invN);
+    }
+  }
+  // Real time, loads included, each next to its use: held together, the factors take 4
+  // registers a point, and the widest workgroups spilled.  (Imaginary time has 2 a point,
+  // and gains 1-9 % from loading them together.)
+  static __device__ __forceinline__ void load_apply(const Phys& p, const LineAt& l, cx<T>* v, double invN) {
+    if (p.k_kind == K_SEP) {
+      const Sep k(l, one(tab(p, l.o0()), l.i0), one(tab(p, l.o1()), l.i1), invN);
+      const F* t = tab(p, l.ax) + 2 * l.tid;
+#pragma unroll
+      for (int r = 0; r < E; ++r) v[r] = k(one(t, bpos<N, TPL, R>(0, r)), v[r]);
+    } else {
+      const double* kt = p.Kt + l.base + (long)l.tid * l.es;
+      T arg[E];
+      const T cK = (T)p.cK;
+#pragma unroll
+      for (int r = 0; r < E; ++r) arg[r] = (T)kt[bpos<N, TPL, R>(0, r) * l.es] * cK;
+      apply_phase_all<T, E, REAL, false>(v, arg, invN);
     }
   }
 };
