@@ -48,7 +48,6 @@ struct gpue_ctx {
   double* dgrid[6] = {};
   std::map<int, void*> tw;   // 2*N + plan -> pass twiddle table (TwTab) in the working precision
   int var[3] = {0, 0, 0};      // kernel variant per axis (row sweeps: axis 0)
-  bool var_default = false;    // they are the defaults: neither set nor tuned
   bool tuned = false;
   // steady-state step graphs: blocks of up to graph_steps consecutive steps (even
   // count, starting at an even step, norm pending) captured once per (gstate,

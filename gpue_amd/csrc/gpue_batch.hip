@@ -849,11 +849,8 @@ gpue_status gpue_batch_autotune(gpue_batch* b, int gstate, int steps, double* us
   bool merged = false;
   for (const Group& g : b->groups) merged = merged || g.merged;
   if (st == GPUE_OK && merged) {
-    std::vector<std::array<int, 4>> vars(n);   // and whether they are the defaults
-    for (size_t i = 0; i < n; ++i) {
-      const gpue_ctx* c = b->ctx[i];
-      vars[i] = {c->var[0], c->var[1], c->var[2], c->var_default};
-    }
+    std::vector<std::array<int, 3>> vars(n);
+    for (size_t i = 0; i < n; ++i) std::copy(b->ctx[i]->var, b->ctx[i]->var + 3, vars[i].begin());
     Grouping by_shape;
     if (make_grouping(b, false, by_shape) != GPUE_OK) {
       (void)hipGetLastError();   // no memory to try it: the batch stays merged
@@ -869,10 +866,7 @@ gpue_status gpue_batch_autotune(gpue_batch* b, int gstate, int steps, double* us
         (void)sync_groups(b);
         drop_batch_graphs(b);
         std::swap((Grouping&)*b, by_shape);
-        for (size_t i = 0; i < n; ++i) {
-          (void)gpue_set_variants(b->ctx[i], vars[i].data());
-          b->ctx[i]->var_default = vars[i][3] != 0;
-        }
+        for (size_t i = 0; i < n; ++i) (void)gpue_set_variants(b->ctx[i], vars[i].data());
         const gpue_status back = load_grouping(b);
         if (st == GPUE_OK) st = back;
       }

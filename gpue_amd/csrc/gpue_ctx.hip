@@ -213,19 +213,6 @@ double gpue::ramp_scale(const gpue_ctx* c, int step) {
   return w * (double)(step + 1) / (double)c->ramp_steps;
 }
 
-// Real-time strided sweeps on whole-width tiles hold complex factors of every point
-// beside psi: one or two waves per SIMD, or spills in 1024-lane workgroups.  Contexts that
-// run the default variants take narrower tiles, operands up front, for the K sweeps of
-// FP64 (quarter tiles in 3D, 192^3 186 -> 171 us a step, 256^3 377 -> 352; half tiles in 2D,
-// 2048 x 1024 53.8 -> 48.1; 384 and 4096 points would lose 1-5 %) and for all of FP32's in 2D
-// (2048^2 77.4 -> 65.8).  A tile's width changes no rounding in real time, which has no norm.
-static int realtime_variant(const gpue_ctx* c, int gstate, const Sweep& s) {
-  if (!c->var_default || !gstate || s.row || c->var[s.axis] != 0) return -1;
-  const int n = c->dims[s.axis];
-  if (c->p.dimnum == 3) return c->prec == 64 && s.mode == CM_K && (n == 192 || n == 256) ? 4 : -1;
-  return (n == 1024 || n == 2048) && (c->prec == 32 || s.mode == CM_K) ? 2 : -1;
-}
-
 // Sweeps of step i (src/evolution.cu:727-870): V/2, the forward transforms, K,
 // the inverse transforms, V/2, then the gauge operators in GPUE's order (x -> y
 // (-> z) on odd steps, (z ->) y -> x on even ones, src/evolution.cu:837,842).
@@ -283,7 +270,6 @@ void gpue::schedule(const gpue_ctx* c, int gstate, int i, bool pending, std::vec
   out.push_back(lead == 0 ? Sweep{true, 0, RM_INV, fc, invc} : Sweep{false, lead, CM_INV_VG, fc, invc});
   for (int k = 1; k < ng; ++k)
     out.push_back(G[k] == 0 ? Sweep{true, 0, RM_GAUGE, 0u, 1.0 / n[0]} : Sweep{false, G[k], CM_GAUGE, 0u, 1.0 / n[G[k]]});
-  for (Sweep& s : out) s.var = realtime_variant(c, gstate, s);
   if (gstate == 0) out.back().flags |= F_NORM;
 }
 
@@ -817,7 +803,6 @@ gpue_status gpue::ctx_create(const gpue_params* pin, hipStream_t ext_stream, gpu
     if (p.dimnum > 2) nb = std::max<size_t>(nb, sweep_blocks(c->prec, false, p.zDim, v, p.xDim, p.yDim));
   }
   for (int a = 0; a < 3; ++a) c->var[a] = default_variant(c, a);
-  c->var_default = true;
   c->partials_n = nb * 4;
   if (hipMalloc((void**)&c->partials, c->partials_n * sizeof(double)) != hipSuccess ||
       hipMalloc((void**)&c->results, 16 * sizeof(double)) != hipSuccess)
@@ -1407,8 +1392,6 @@ static gpue_status autotune(gpue_ctx* c, int reps) {
   HIPCHK(c, hipEventCreate(&e0));
   HIPCHK(c, hipEventCreate(&e1));
   double cost[3][N_VARIANTS] = {};
-  const bool var_default = c->var_default;
-  c->var_default = false;   // every sweep of an axis runs what is chosen for it
   std::vector<Sweep> sched;
   const bool timing = c->timing;
   c->timing = false;
@@ -1432,10 +1415,7 @@ static gpue_status autotune(gpue_ctx* c, int reps) {
   c->timing = timing;
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
-  if (st != GPUE_OK) {   // nothing is chosen yet
-    c->var_default = var_default;
-    return st;
-  }
+  if (st != GPUE_OK) return st;
   for (int a = 0; a < 3; ++a) {
     int best = c->var[a];
     for (int v = 0; v < N_VARIANTS; ++v)
@@ -2016,7 +1996,6 @@ gpue_status gpue_set_variants(gpue_ctx* c, const int* variants) {
     if (variants[a] < 0 || variants[a] >= N_VARIANTS) return fail(c, GPUE_EINVAL, "variant out of range");
   }
   for (int a = 0; a < 3; ++a) c->var[a] = variants[a];
-  c->var_default = false;
   drop_graphs(c);
   return GPUE_OK;
 }

