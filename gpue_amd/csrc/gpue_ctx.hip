@@ -358,7 +358,9 @@ static gpue_status settle_deferred(gpue_ctx* c) {
 // depend on it.  (Figures: us a step, imaginary / real time, the former rule -> this one;
 // it had narrow lines and quarter tiles up to 2^20 points, wide ones beyond.)
 //  * Up to 2^18 points (2^20 in 3D) launches are latency bound: narrow lines, operands up
-//    front, quarter tiles (512^2 FP64 18.3 / 14.5, wide 25.3 / 20.5).
+//    front, quarter tiles (512^2 FP64 18.3 / 14.5, wide 25.3 / 20.5).  Not rows of 4096
+//    points in FP64, whose 16 points a lane leave no registers for operands (4096 x 64
+//    23.2 / 18.3 -> 22.1 / 17.2, rotating 35.5 / 43.1 -> 33.5 / 30.4).
 //  * 2D to 2^20 points: waves enough that rows may load late, and past 2^19 long columns
 //    take half tiles, 64 bytes of a row (1024^2 rotating FP64 72.1 / 73.3 -> 67.3 / 61.5,
 //    FP32 48.6 / 44.5 -> 45.0 / 42.1; 512 x 1024 FP32 20.2 / 17.5 -> 19.5 / 17.0).
@@ -376,13 +378,14 @@ static gpue_status settle_deferred(gpue_ctx* c) {
 static int default_variant(const gpue_ctx* c, int axis) {
   const int n = c->dims[axis];
   const bool f64 = c->prec == 64;
+  const int small_row = f64 && n == 4096 ? 1 : 3;
   if (c->p.dimnum == 3) {
-    if (c->N <= (1L << 20)) return axis == 0 ? 3 : 5;
+    if (c->N <= (1L << 20)) return axis == 0 ? small_row : 5;
     if (axis == 0) return 0;
     if (!f64) return n == 96 || (n == 64 && axis == 2) ? 4 : 0;
     return n <= 96 && n != 48 ? 5 : n == 128 ? 1 : 0;
   }
-  if (c->N <= (1L << 18)) return axis == 0 ? 3 : 5;
+  if (c->N <= (1L << 18)) return axis == 0 ? small_row : 5;
   if (c->N <= (1L << 20)) return axis == 0 ? 1 : c->N > (1L << 19) && n >= 512 ? 3 : 5;
   if (axis == 0) return f64 && c->N >= (1L << 22) && n <= 2048 ? 1 : 0;
   return !f64 && c->N <= (1L << 21) && (n == 1024 || n == 2048) ? 2 : 0;
