@@ -1044,8 +1044,8 @@ gpue_status gpue_set_field_eqn(gpue_ctx* c, int which, const char* expr, const c
 // psi as 2N numbers; FP32 contexts convert on the way.
 gpue_status gpue_upload_wfc(gpue_ctx* c, const double* il) {
   if (!c || !il) return GPUE_EINVAL;
-  HIPCHK(c, launch_set_double(c->results, 1.0, c->stream));
   HIPCHK(c, copy_to_device(c->psi, il, 2 * c->N, c->esz / 2, c->prec == 32, c->p.device, c->stream));
+  HIPCHK(c, launch_set_double(c->results, 1.0, c->stream));   // in stream order; the copy need not wait for it
   c->pending_norm = false;
   return GPUE_OK;
 }

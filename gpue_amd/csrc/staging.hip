@@ -31,6 +31,12 @@ constexpr int POOLED = 16;                  // free buffers kept (64 MiB pinned)
 constexpr int MAX_THREADS = 8;              // CPU threads of one large transfer
 constexpr size_t MT_BYTES = (size_t)16 << 20;   // from here on a transfer uses threads
 constexpr size_t DIRECT_UP = (size_t)8 << 20;   // smaller uploads: HIP's own path (66 us for 1 MiB, 148 for 4)
+// Downloads of more than 16 KiB up to DIRECT_DOWN, and conversions up to DIRECT_CONV (bytes
+// on the device), take HIP's own path too (us, HIP's / through a chunk: down 16 KiB 28 / 15,
+// 24 KiB 12 / 19, 256 KiB 22 / 30, 1 MiB 68 / 75, 1.5 MiB 97 / 98, 2.25 MiB 153 / 132; down and
+// up with conversion 16 KiB 23 / 15 and 17.6 / 17.7, 64 KiB 16 / 21 and 24 / 30, 192 KiB 25 / 27 and
+// 32 / 34, 512 KiB 48 / 45 and 50 / 49).
+constexpr size_t DIRECT_FROM = (size_t)16 << 10, DIRECT_DOWN = (size_t)3 << 19, DIRECT_CONV = (size_t)1 << 18;
 
 struct Buffer {
   void* p = nullptr;
@@ -172,7 +178,8 @@ struct Job {
   }
 };
 
-// Without pinned memory to be had: HIP's own copies, conversions through a pageable chunk.
+// HIP's own copies, conversions through a pageable chunk: small transfers, and where no
+// pinned memory is to be had.
 hipError_t run_pageable(const Job& j) {
   const size_t per = j.conv ? std::min(j.n, CHUNK / j.es) : j.n;
   std::unique_ptr<float[]> f;
@@ -258,6 +265,8 @@ hipError_t run_on(Job& j, int device) {
 // On the stream's device: the buffers' events belong to it.
 hipError_t run(Job& j, int device) {
   if (j.n == 0) return hipSuccess;
+  const size_t bytes = j.n * j.es;
+  if (bytes > DIRECT_FROM && (j.conv ? bytes < DIRECT_CONV : j.down && bytes < DIRECT_DOWN)) return run_pageable(j);
   int cur = device;
   hipError_t e = hipGetDevice(&cur);
   if (e == hipSuccess && cur != device) e = hipSetDevice(device);

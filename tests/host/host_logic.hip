@@ -259,7 +259,8 @@ static void field_out_of_memory() {
 // psi to the device and back where no pinned memory can be had, one or two buffers, or all:
 // parts of a chunk, several chunks, transfers that use threads.
 static void pinned_memory() {
-  const std::vector<std::vector<int>> shapes = {{16}, {512, 64}, {192, 192, 16}, {1024, 512}, {192, 96, 96}, {2048, 1024}};
+  const std::vector<std::vector<int>> shapes = {{16},          {32, 32},     {32, 48},   {128, 128},   {192, 192},    {384, 256},
+                                                 {192, 192, 16}, {1024, 512}, {512, 384}, {192, 96, 96}, {2048, 1024}};
   for (long pinned : {0L, 1L, 2L, 3L, -1L})
     for (int prec : {64, 32})
       for (const auto& shape : shapes) {
