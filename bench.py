@@ -126,6 +126,8 @@ def kernel_symbol(name, prec, n_axis, variant, gstate=0):
     t = "double" if prec == 64 else "float"
     parts = name.split("+")
     base = parts[0]
+    if base == "line_steps":
+        return base
     if base.startswith("row"):
         mode = RM[base] | (16 if gstate and base != "row_ksum" else 0)
         if base in ("row_inv", "row_inv_fwd") and "gx" not in parts[1:]:

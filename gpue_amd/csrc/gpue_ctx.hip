@@ -1573,21 +1573,25 @@ static int block_len(const gpue_ctx* c, int first_step, int nsteps, int s, int e
 // beyond 1024 points), so that no launch holds the device for longer than some 6 ms: a
 // step takes 1-2 us at 16 points, 3.2-6.1 at 1024, 6-17 at 4096 (both precisions, without
 // and with a gauge).  A launch more costs some 10 us.
+static bool runs_lines(const gpue_ctx* c) {
+  return c->p.dimnum == 1 && c->graph_steps > 0 && !c->t_dep && !c->ramp_type;
+}
+static int line_limit(const gpue_ctx* c) { return std::min(1024, (1 << 20) / c->dims[0]); }
 static int line_len(const gpue_ctx* c, int first_step, int nsteps, int s, int energy_every) {
-  if (c->p.dimnum != 1 || c->graph_steps <= 0 || c->timing || c->t_dep || c->ramp_type) return 0;
+  if (!runs_lines(c) || c->timing) return 0;
   const int i = first_step + s;
-  int L = std::min(nsteps - s, std::min(1024, (1 << 20) / c->dims[0]));
+  int L = std::min(nsteps - s, line_limit(c));
   if (energy_every > 0) L = std::min(L, ((i + energy_every - 1) / energy_every) * energy_every - i + 1);
   return L;
 }
 
-// L steps of a 1D problem from the present psi (scaled by the norm slot, which holds
+// L steps of a 1D problem from the state in psi (scaled by the norm slot, which holds
 // the pending norm or 1.0, in imaginary time).
-static gpue_status launch_steps_1d(gpue_ctx* c, int gstate, int L) {
+static gpue_status launch_steps_1d(gpue_ctx* c, int gstate, int L, void* psi) {
   std::vector<Sweep> sched;
   schedule(c, gstate, 0, gstate == 0, sched);
   SweepArgs a;
-  gpue_status st = sweep_args(c, sched[0], make_phys(c, gstate, 0), c->psi, c->psi, a);
+  gpue_status st = sweep_args(c, sched[0], make_phys(c, gstate, 0), psi, psi, a);
   if (st != GPUE_OK) return st;
   a.norm_scale = c->d[0] * c->d[1] * c->d[2];
   a.norm_out = c->results + 0;
@@ -1657,7 +1661,7 @@ static gpue_status evolve_impl(gpue_ctx* c, int first_step, int nsteps, int gsta
       continue;
     }
     if (L1 > 0) {
-      gpue_status st = launch_steps_1d(c, gstate, L1);
+      gpue_status st = launch_steps_1d(c, gstate, L1, c->psi);
       if (st != GPUE_OK) return st;
       s += L1 - 1;
       i += L1 - 1;
@@ -1851,6 +1855,22 @@ gpue_status gpue_timing_get(gpue_ctx* c, int kind, const char** name, long* laun
   return GPUE_OK;
 }
 
+// 1D: a run of steps as the step loop launches it, on a copy of psi in the scratch buffer;
+// the norm slot holds 1.0 before and after (nothing is pending).
+static gpue_status time_line(gpue_ctx* c, int gstate, int reps, hipEvent_t e0, hipEvent_t e1, double* us) {
+  HIPCHK(c, hipMemcpyAsync(c->tmp, c->psi, c->N * c->esz, hipMemcpyDeviceToDevice, c->stream));
+  gpue_status st = launch_steps_1d(c, gstate, line_limit(c), c->tmp);   // warm-up
+  HIPCHK(c, hipEventRecord(e0, c->stream));
+  for (int r = 0; r < reps && st == GPUE_OK; ++r) st = launch_steps_1d(c, gstate, line_limit(c), c->tmp);
+  HIPCHK(c, hipEventRecord(e1, c->stream));
+  HIPCHK(c, launch_set_double(c->results, 1.0, c->stream));
+  HIPCHK(c, hipEventSynchronize(e1));
+  float ms = 0.f;
+  HIPCHK(c, hipEventElapsedTime(&ms, e0, e1));
+  *us = ms * 1000.0 / reps;
+  return st;
+}
+
 // Per-kernel cost: every distinct sweep of the gstate schedules (both parities)
 // is timed by time_sweep (graph replays in place on copies of psi in the
 // scratch buffer; the state is untouched, the norm partials are not written).
@@ -1864,8 +1884,14 @@ gpue_status gpue_sweep_profile(gpue_ctx* c, int gstate, int reps, int max_kinds,
   std::vector<double> count;
   c->prof_names.clear();
   // the sweeps of an even/odd step pair as the step loop launches them (with
-  // the real-time step boundary fused when steps are replayed from graphs)
-  if (c->graph_steps > 0) {
+  // the real-time step boundary fused when steps are replayed from graphs); in 1D a
+  // run of steps
+  const bool lines = runs_lines(c);
+  if (lines) {
+    c->prof_names.push_back("line_steps");
+    kinds.push_back(Sweep{true, 0, RM_FULL, 0u, 0.0});
+    count.push_back(1.0 / line_limit(c));
+  } else if (c->graph_steps > 0) {
     schedule_block(c, gstate, 0, 2, sched, step_of);
   } else {
     std::vector<Sweep> one;
@@ -1901,7 +1927,7 @@ gpue_status gpue_sweep_profile(gpue_ctx* c, int gstate, int reps, int max_kinds,
   *n_kinds = (int)kinds.size();
   for (size_t k = 0; k < kinds.size() && st == GPUE_OK; ++k) {
     double us = 0.0;
-    st = time_sweep(c, kinds[k], ph, reps, e0, e1, &us);
+    st = lines ? time_line(c, gstate, reps, e0, e1, &us) : time_sweep(c, kinds[k], ph, reps, e0, e1, &us);
     if (st == GPUE_OK && (int)k < max_kinds) {
       if (names) names[k] = c->prof_names[k].c_str();
       if (us_per_launch) us_per_launch[k] = us;
@@ -1931,10 +1957,13 @@ gpue_status gpue_step_bytes(gpue_ctx* c, int gstate, double* bytes, double* swee
   if (!c || (gstate != 0 && gstate != 1)) return GPUE_EINVAL;
   // the sweeps the steady state runs: a captured block when graphs are on (real
   // time fuses the sweeps at step boundaries), else a step of each parity
-  const int G = c->graph_steps > 0 && !c->ramp_type ? c->graph_steps : 2;
+  // (1D: a run of steps reads and writes psi once)
+  const int G = runs_lines(c) ? line_limit(c) : c->graph_steps > 0 && !c->ramp_type ? c->graph_steps : 2;
   std::vector<Sweep> blk;
   std::vector<int> step_of;
-  if (G == c->graph_steps) {
+  if (runs_lines(c)) {
+    blk.resize(1);
+  } else if (G == c->graph_steps) {
     schedule_block(c, gstate, 0, G, blk, step_of);
   } else {
     std::vector<Sweep> a, b;

@@ -182,8 +182,9 @@ gpue_status gpue_set_timing(gpue_ctx *c, int on);
 gpue_status gpue_timing_get(gpue_ctx *c, int kind, const char **name, long *launches, double *ms);
 /* HBM bytes of psi one steady-state step moves in the current configuration:
  * 2 x (bytes of psi) per sweep, averaged over the step parities and, when graphs
- * are on, over a captured block (real time fuses the sweeps at step boundaries);
- * *sweeps_per_step receives the sweep count. */
+ * are on, over a captured block (real time fuses the sweeps at step boundaries) or,
+ * in 1D, over the longest run of steps of one launch; *sweeps_per_step receives the
+ * sweep count. */
 gpue_status gpue_step_bytes(gpue_ctx *c, int gstate, double *bytes_per_step, double *sweeps_per_step);
 /* Per-kernel cost of the step (no reference counterpart): each distinct sweep
  * of the gstate schedule is launched `reps` times back to back from a graph,
@@ -192,7 +193,7 @@ gpue_status gpue_step_bytes(gpue_ctx *c, int gstate, double *bytes_per_step, dou
  * 256 MiB and more in imaginary time, which run on one copy; HIP events on the context
  * stream.  Fills up to max_kinds entries: kernel name (owned by the
  * ctx, valid until the next call), microseconds per launch, launches per step
- * (averaged over the two gauge orders); *n_kinds = number of distinct sweeps. */
+ * (averaged over the two gauge orders; 1D: one entry "line_steps", a run of steps); *n_kinds = number of distinct sweeps. */
 gpue_status gpue_sweep_profile(gpue_ctx *c, int gstate, int reps, int max_kinds, int *n_kinds,
                                const char **names, double *us_per_launch, double *launches_per_step);
 /* The exp (fn 0), sin (1) and cos (2) the FP64 fused operators evaluate on the

@@ -331,6 +331,39 @@ static void line_runs() {
     }
 }
 
+// 1D: the profile and the traffic are those of the launches that the step loop makes.
+static void line_reports() {
+  for (int n : {64, 4096})
+    for (int gstate : {0, 1}) {
+      long lines = 0, sweeps = 0, steps = 0;
+      void *in = nullptr, *psi = nullptr;
+      fake::on_launch = [&](const fake::Launch& l) {
+        if (l.kernel.rfind("gpue::k_set_double", 0) == 0) **(double**)l.args[0] = *(double*)l.args[1];
+        if (l.kernel.rfind("gpue::line_steps", 0) == 0) {
+          ++lines;
+          steps = *(int*)l.args[1];
+          in = (void*)((const SweepArgs*)l.args[0])->in;
+        }
+        if (l.kernel.find("_sweep<") != std::string::npos) ++sweeps;
+      };
+      gpue_ctx* c = make({n}, 64, 1);
+      psi = c->psi;
+      int kinds = 0;
+      const char* names[4];
+      double us[4], per[4], bytes = 0.0, count = 0.0;
+      CHECK(gpue_sweep_profile(c, gstate, 5, 4, &kinds, names, us, per) == GPUE_OK, "profile: %s", gpue_last_error(c));
+      CHECK(kinds == 1 && std::string(names[0]) == "line_steps" && lines > 0 && sweeps == 0, "%d kinds, %s", kinds, names[0]);
+      CHECK(in != psi && c->psi == psi && c->results[0] == 1.0, "the state is untouched");
+      CHECK(per[0] == 1.0 / steps, "%g launches a step", per[0]);
+      CHECK(gpue_step_bytes(c, gstate, &bytes, &count) == GPUE_OK && count == 1.0 / steps && bytes == 32.0 * n / steps,
+            "%g bytes a step", bytes);
+      CHECK(gpue_set_graph_steps(c, 0) == GPUE_OK && gpue_step_bytes(c, gstate, &bytes, &count) == GPUE_OK && count == 1.0 &&
+                gpue_sweep_profile(c, gstate, 5, 4, &kinds, names, us, per) == GPUE_OK && kinds == 1 && per[0] == 1.0 && sweeps > 0,
+            "steps launched one by one");
+      gpue_destroy(c);
+    }
+}
+
 // A tuner that fails before it has chosen anything leaves a context with its default
 // variants: the kernels of a real-time step are those from before.
 static void tuner_fails() {
@@ -437,6 +470,7 @@ int main(int argc, char** argv) {
       {"pinned_memory", pinned_memory},
       {"step_blocks", step_blocks},
       {"line_runs", line_runs},
+      {"line_reports", line_reports},
       {"tuner_fails", tuner_fails},
       {"batch_boxes", batch_boxes},
       {"tuner_times_steps", tuner_times_steps},
