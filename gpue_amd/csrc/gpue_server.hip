@@ -139,6 +139,26 @@ static double footprint(const gpue_params& p) {
   return 2.0 * n * s + 4.0 * 1024 * 1024;   // psi, scratch psi, tables and partials
 }
 
+// Steps of the captured blocks of a phase whose chunks are `chunk` steps: the longest even
+// divisor, so that one block serves the phase.  Blocks live no longer than the phase (a
+// reset and a new interaction drop them), so a request pays for every capture, and a
+// second length costs most (ten requests of 128^2 FP64, ms, in blocks of 32 and the rest / of
+// one length: 40 steps 10.1 / 9.1, 60 steps 16.0 / 11.7, 100 steps 16.3 / 15.4; of 8 and the rest
+// 40 steps 9.0, 60 steps 11.2, 100 steps 15.7; quenches of 64^3, twice 20 steps 17 / 17, of 8 and
+// the rest 29, twice 40 steps 33 / 27).
+static int block_steps(int chunk) {
+  for (int g = 32; g >= 8; g -= 2)
+    if (chunk % g == 0) return g;
+  return 32;
+}
+
+// Start a phase of the request in s: `total` steps of gstate, looked at every `every` ones.
+static void start_phase(Slot* s, int gstate, int total, int every) {
+  s->gstate = gstate;
+  s->step = 0;
+  s->ctx->graph_steps = block_steps(std::min(every, total));   // no graphs are captured yet
+}
+
 // Queue a chunk: nsteps of the current phase, then the energy terms into pinned memory.
 static gpue_status issue_chunk(Slot* s, int nsteps) {
   gpue_ctx* c = s->ctx;
@@ -302,8 +322,7 @@ static void advance(gpue_server* sv, Slot* s) {
     if (conv || s->imag_done >= r.max_imag_steps) {
       if (r.real_steps > 0) {   // quench: new interaction, real time from the ground state
         gpue_set_g(c, c->p.g * r.quench_factor);
-        s->gstate = 1;
-        s->step = 0;
+        start_phase(s, 1, r.real_steps, every);
       } else {
         s->finished = true;
         return;
@@ -374,10 +393,11 @@ static void worker_main(gpue_server* sv) {
       const int every = r.check_every > 0 ? r.check_every : 100;
       if (s->status == GPUE_OK) {
         if (r.max_imag_steps > 0) {
+          start_phase(s, 0, r.max_imag_steps, every);
           s->status = issue_chunk(s, std::min(every, r.max_imag_steps));
         } else if (r.real_steps > 0) {   // straight to real time
           gpue_set_g(s->ctx, s->ctx->p.g * r.quench_factor);
-          s->gstate = 1;
+          start_phase(s, 1, r.real_steps, every);
           s->status = issue_chunk(s, std::min(every, r.real_steps));
         } else {
           s->finished = true;

@@ -364,6 +364,37 @@ static void line_reports() {
     }
 }
 
+// A request of the service captures one block a phase where its chunks allow it.
+static void service_captures() {
+  fake::on_launch = [&](const fake::Launch& l) {
+    if (l.kernel.rfind("gpue::k_set_double", 0) == 0) **(double**)l.args[0] = *(double*)l.args[1];
+  };
+  struct Case { int imag, real, every, captures; };
+  for (const Case& k : {Case{40, 0, 100, 1}, Case{60, 0, 100, 1}, Case{100, 0, 100, 1}, Case{200, 0, 100, 1}, Case{20, 40, 100, 2},
+                        Case{0, 90, 30, 1}, Case{41, 0, 100, 2}, Case{62, 0, 100, 2}, Case{4, 0, 100, 1}, Case{1, 0, 100, 0}}) {
+    gpue_server* sv = nullptr;
+    CHECK(gpue_server_create(0, 1e9, 2, &sv) == GPUE_OK, "server");
+    gpue_ctx* like = make({64, 64}, 64, 0);
+    for (int again = 0; again < 2; ++again) {   // a new context, then a reused one
+      gpue_request r;
+      std::memset(&r, 0, sizeof(r));
+      r.params = like->p;
+      r.max_imag_steps = k.imag;
+      r.real_steps = k.real;
+      r.check_every = k.every;
+      r.quench_factor = 1.1;
+      const long before = fake::captures;
+      CHECK(gpue_server_submit(sv, &r, 1) == GPUE_OK && gpue_server_drain(sv, 20.0) == GPUE_OK, "request");
+      gpue_result got;
+      CHECK(gpue_server_poll(sv, &got, 1) == 1 && got.status == GPUE_OK && got.imag_steps == k.imag && got.real_steps == k.real,
+            "status %d, %d + %d steps", got.status, (int)got.imag_steps, (int)got.real_steps);
+      CHECK(fake::captures - before == k.captures, "%d + %d steps: %ld captures", k.imag, k.real, fake::captures - before);
+    }
+    gpue_server_destroy(sv);
+    gpue_destroy(like);
+  }
+}
+
 // A tuner that fails before it has chosen anything leaves a context with its default
 // variants: the kernels of a real-time step are those from before.
 static void tuner_fails() {
@@ -470,6 +501,7 @@ int main(int argc, char** argv) {
       {"pinned_memory", pinned_memory},
       {"step_blocks", step_blocks},
       {"line_runs", line_runs},
+      {"service_captures", service_captures},
       {"line_reports", line_reports},
       {"tuner_fails", tuner_fails},
       {"batch_boxes", batch_boxes},

@@ -34,7 +34,7 @@ def exe(tmp_path_factory):
 
 
 @pytest.mark.parametrize("check", ["batch_norms", "batch_members_change", "field_out_of_memory", "pinned_memory",
-                                   "step_blocks", "line_runs", "line_reports", "tuner_fails", "tuner_times_steps",
+                                   "step_blocks", "line_runs", "line_reports", "service_captures", "tuner_fails", "tuner_times_steps",
                                    "tuner_regroups", "batch_boxes"])
 def test_host_logic(exe, check):
     r = subprocess.run([exe, check], capture_output=True, text=True, timeout=120)
