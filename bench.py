@@ -285,8 +285,8 @@ def config4_specs(n_inst=64, seed=4):
 
 def batched_sweep(G, n_inst=64, seed=4, max_steps=20000, tol=1e-8, force_mode=None, force_variants=None):
     """64 independent 2D imaginary-time solves on uneven grids, FP32 bulk with
-    FP64 norm/energy, advanced together through one batch (one launch per sweep
-    per shape, two steps per graph replay) until each instance's energy changes
+    FP64 norm/energy, advanced together through one batch (its tuner takes merged
+    launches or launches by shape; blocks of steps per graph replay) until each instance's energy changes
     by less than tol (relative) over 100 steps (at most max_steps).  psi0 is
     the noisy Gaussian exp(-r^2/2)(1 + 0.01 U[-1,1]), seeded per instance."""
     sizes, specs = config4_specs(n_inst, seed)
@@ -453,8 +453,8 @@ def main():
                     help="batched sweep: force the graph mode (2: no graphs, for kernel tracers)")
     ap.add_argument("--batch-variants", type=str, default=None, help="batched sweep: force the variants x,y,z")
     ap.add_argument("--graph-steps", type=int, default=32,
-                    help="steps per captured graph (library default 8; 32 saves ~1.5 %% of graph launch "
-                         "gaps here; 0: every sweep launched individually, e.g. under a tracer)")
+                    help="steps per captured graph (32 is the library's default; 0: every sweep launched "
+                         "individually, e.g. under a tracer)")
     ap.add_argument("--variants32", type=str, default=None,
                     help="kernel variants of the FP32 contexts (default: as --variants)")
     ap.add_argument("--variants", type=str, default=None,

@@ -1,8 +1,9 @@
 // gpue_batch.hip -- many independent problems advanced together.
 //
 // Instances of one precision, dimension and gauge whose axes have merged kernels
-// (sweep_merged.h) form a merged group: every sweep of the step is one launch over all
-// of them, whatever their sizes.  Others group by shape (grid sizes and kernel variants
+// (sweep_merged.h; FP64 boxes only where they have more shapes than there are streams) form
+// a merged group: every sweep of the step is one launch over all of them, whatever their
+// sizes.  Others group by shape (grid sizes and kernel variants
 // too): for every sweep one batched kernel covers the group, blocks [i*bpi, (i+1)*bpi)
 // working on instance i.  The instances' SweepArgs live in a device array.  GPUE's gauge
 // order alternates with the step parity (src/evolution.cu:837,842).  When the
@@ -15,7 +16,8 @@
 // get one each, the others share the last), with blocks of 16 and 2 consecutive steps
 // of a group captured once per gstate as HIP graphs and replayed, so the groups of
 // different shapes (the small ones latency bound) overlap on the device.
-// Device memory is allocated only in gpue_batch_create.
+// Device memory is allocated only in gpue_batch_create and by the tuner, which compares
+// merged launches with launches by shape.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

@@ -1443,9 +1443,10 @@ static gpue_status autotune(gpue_ctx* c, int reps) {
 
 // Sweeps of steps first..first+n-1 with, in real time, the sweep that ends a
 // step fused with the one that starts the next when both run along the same
-// axis (no norm stands between them, and the fields do not change): the pair's
-// arithmetic is unchanged, one read and one write of psi are saved.  With a
-// gauge this holds at every step boundary (GPUE's gauge order alternates, so
+// axis (no norm stands between them, and A does not change): one read and one write
+// of psi are saved.  FP64 takes the two V/2 that meet without a gauge operator as one
+// phase of the summed exponents, a rounding less than single steps; the arithmetic is
+// otherwise theirs.  With a gauge this holds at every step boundary (GPUE's gauge order alternates, so
 // a step ends on the axis the next one leads with): 2D real-time steps take 3
 // sweeps.
 void gpue::schedule_block(const gpue_ctx* c, int gstate, int first, int n, std::vector<Sweep>& out,

@@ -7,9 +7,9 @@
 //   3D: [V/2, FFTx] [FFTy] [FFTz, K, IFFTz] [IFFTy] [IFFTx, V/2 (,x-gauge)] (+gauge)
 //   1D: [V/2, FFT, K, IFFT, V/2 (,gauge)]
 // The imaginary-time renormalisation (parSum, src/split_op.cu:83-129) is
-// fused: the last sweep of a step leaves per-workgroup partial sums of |psi|^2,
-// the last workgroup to finish reduces them in a fixed order to
-// norm = sqrt(sum * dV), and the next step's first sweep divides by it.
+// fused: the last sweep of a step leaves per-workgroup partial sums of |psi|^2, a
+// finalize kernel or every wave of the next step's first sweep reduces them in one
+// fixed order to norm = sqrt(sum * dV), and that first sweep divides by it.
 // Operator fields are regenerated in-kernel from 1-D coordinate arrays
 // (harmonic V, rotation A, standard K) or read from tables (equation-string
 // or file fields), so the only per-step HBM traffic is psi itself.
@@ -549,7 +549,8 @@ struct VOp {
   }
   // exponents of the half step on v.  FP32 adds the axes in the order x, y, z, and the
   // density takes the square of x after that of y in a step's first half, before it in
-  // its second (CLOSES): the roundings these steps have always had.
+  // its second (CLOSES).  The order is fixed so that every kernel rounds alike; V cV is
+  // rounded before the density term for the same reason.
   template <bool CLOSES>
   __device__ __forceinline__ void args(const Phys& p, const LineAt& l, const cx<T>* v, T (&arg)[E]) const {
     const T cV = (T)p.cV;
