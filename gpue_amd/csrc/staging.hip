@@ -31,12 +31,6 @@ constexpr int POOLED = 16;                  // free buffers kept (64 MiB pinned)
 constexpr int MAX_THREADS = 8;              // CPU threads of one large transfer
 constexpr size_t MT_BYTES = (size_t)16 << 20;   // from here on a transfer uses threads
 constexpr size_t DIRECT_UP = (size_t)8 << 20;   // smaller uploads: HIP's own path (66 us for 1 MiB, 148 for 4)
-// Downloads of more than 16 KiB up to DIRECT_DOWN, and conversions up to DIRECT_CONV (bytes
-// on the device), take HIP's own path too (us, HIP's / through a chunk: down 16 KiB 28 / 15,
-// 24 KiB 12 / 19, 256 KiB 22 / 30, 1 MiB 68 / 75, 1.5 MiB 97 / 98, 2.25 MiB 153 / 132; down and
-// up with conversion 16 KiB 23 / 15 and 17.6 / 17.7, 64 KiB 16 / 21 and 24 / 30, 192 KiB 25 / 27 and
-// 32 / 34, 512 KiB 48 / 45 and 50 / 49).
-constexpr size_t DIRECT_FROM = (size_t)16 << 10, DIRECT_DOWN = (size_t)3 << 19, DIRECT_CONV = (size_t)1 << 18;
 
 struct Buffer {
   void* p = nullptr;
@@ -137,10 +131,16 @@ struct Job {
     char* d = dev + (size_t)k * per * es;
     hipError_t e = down ? hipMemcpyAsync(b.p, d, bytes, hipMemcpyDeviceToHost, stream)
                         : hipMemcpyAsync(d, b.p, bytes, hipMemcpyHostToDevice, stream);
-    if (e == hipSuccess) e = hipEventRecord(b.ev, stream);
+    if (e == hipSuccess && chunks > 1) e = hipEventRecord(b.ev, stream);
     if (e != hipSuccess) fail(e);
     issued.store(k + 1, std::memory_order_release);
   }
+  // Chunk k's DMA has ended.  A lone chunk is waited for with its stream: recording an
+  // event and waiting for that takes 6-15 us more (us, event / stream: down 64 KiB 19.9 / 13.1,
+  // 256 KiB 28.0 / 21.0, 1 MiB 69 / 62; 32 KiB FP32 down 19.6 / 12.4, up 30.2 / 14.4; HIP's own copies
+  // from and to pageable memory take 12-22 us up to 256 KiB where they find the memory pinned
+  // from the call before, and 50-190 where contexts of several sizes take turns).
+  hipError_t wait(int k) { return chunks > 1 ? hipEventSynchronize(buf[k % nbuf].ev) : hipStreamSynchronize(stream); }
   // The CPU's part of chunks, as they come; every wait ends with the DMA of an
   // earlier chunk, with another thread's chunk, or with the error flag.
   void consume() {
@@ -153,7 +153,7 @@ struct Job {
         std::this_thread::yield();
       }
       if (need > 0) {
-        const hipError_t e = hipEventSynchronize(buf[k % nbuf].ev);
+        const hipError_t e = wait(k);
         if (e != hipSuccess) {
           fail(e);
           return;
@@ -178,8 +178,7 @@ struct Job {
   }
 };
 
-// HIP's own copies, conversions through a pageable chunk: small transfers, and where no
-// pinned memory is to be had.
+// Without pinned memory to be had: HIP's own copies, conversions through a pageable chunk.
 hipError_t run_pageable(const Job& j) {
   const size_t per = j.conv ? std::min(j.n, CHUNK / j.es) : j.n;
   std::unique_ptr<float[]> f;
@@ -235,7 +234,7 @@ hipError_t run_on(Job& j, int device) {
       const int k = j.next.load();
       if (j.error.load()) break;
       if (j.down || k >= j.nbuf) {
-        const hipError_t e = hipEventSynchronize(j.buf[k % j.nbuf].ev);
+        const hipError_t e = j.wait(k);
         if (e != hipSuccess) {
           j.fail(e);
           break;
@@ -255,7 +254,7 @@ hipError_t run_on(Job& j, int device) {
   if (!j.down || j.error.load())
     for (int b = 0; b < j.nbuf; ++b)
       if (j.issued.load() > b) {
-        const hipError_t e = hipEventSynchronize(j.buf[b].ev);
+        const hipError_t e = j.wait(b);
         if (e != hipSuccess) j.fail(e);
       }
   for (int b = 0; b < j.nbuf; ++b) give(j.buf[b]);
@@ -265,8 +264,6 @@ hipError_t run_on(Job& j, int device) {
 // On the stream's device: the buffers' events belong to it.
 hipError_t run(Job& j, int device) {
   if (j.n == 0) return hipSuccess;
-  const size_t bytes = j.n * j.es;
-  if (bytes > DIRECT_FROM && (j.conv ? bytes < DIRECT_CONV : j.down && bytes < DIRECT_DOWN)) return run_pageable(j);
   int cur = device;
   hipError_t e = hipGetDevice(&cur);
   if (e == hipSuccess && cur != device) e = hipSetDevice(device);

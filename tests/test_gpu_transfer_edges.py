@@ -1,5 +1,5 @@
-"""psi transfers on either side of the sizes where the way they take changes: 16 KiB, 256
-KiB (conversions), 1.5 MiB (downloads) and 8 MiB (uploads) on the device."""
+"""psi transfers on either side of the sizes where the way they take changes: 2 MiB (one
+chunk), 8 MiB (chunk size, uploads) and 16 MiB (threads) on the device."""
 import numpy as np
 import pytest
 
@@ -9,8 +9,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("prec", [64, 32])
-@pytest.mark.parametrize("shape", [(32, 32), (32, 48), (32, 64), (48, 64), (128, 192), (128, 256), (256, 384), (384, 512),
-                                   (1024, 512), (1024, 1024)])
+@pytest.mark.parametrize("shape", [(32, 32), (32, 48), (32, 64), (48, 64), (128, 192), (128, 256), (256, 384), (256, 512),
+                                   (384, 512), (1024, 512), (1024, 1024)])
 def test_roundtrip(shape, prec):
     rng = np.random.default_rng(3)
     with G.Context(dimnum=2, xDim=shape[0], yDim=shape[1], xMax=5.0, yMax=5.0, precision=prec) as c:
