@@ -85,30 +85,48 @@ def run_schedule(ctx, imag, real):
 # (each scaled by its reading for a plain 256 MiB device copy: 2.0 and 1.0), per
 # kernel instance and workload; the passes and tables are in profiles/.
 MEASURED_TRAFFIC = {
-    "gpue::col_sweep<double, 512, 5, 2>@512sq": 8787797,
-    "gpue::col_sweep<double, 512, 5, 3>@512sq": 8784887,
-    "gpue::col_sweep<double, 512, 5, 5>@512sq": 8697118,
-    "gpue::col_sweep<double, 512, 5, 6>@512sq": 8936286,
-    "gpue::row_sweep<double, 512, 3, 0>@512sq": 8717749,
-    "gpue::row_sweep<double, 512, 3, 1>@512sq": 8972530,
-    "gpue::row_sweep<double, 512, 3, 2>@512sq": 8793964,
-    "gpue::row_sweep<double, 512, 3, 7>@512sq": 8841794,
-    "gpue::col_sweep<double, 256, 0, 0>@256cube": 536992027,
-    "gpue::col_sweep<double, 256, 0, 1>@256cube": 536993838,
-    "gpue::col_sweep<double, 256, 0, 2>@256cube": 537408139,
-    "gpue::col_sweep<double, 256, 0, 3>@256cube": 537402176,
-    "gpue::col_sweep<double, 256, 0, 5>@256cube": 537285972,
-    "gpue::col_sweep<double, 256, 0, 6>@256cube": 537569081,
-    "gpue::col_sweep<double, 256, 2, 2>@256cube": 537376379,
-    "gpue::col_sweep<float, 256, 0, 0>@256cube": 268548237,
-    "gpue::col_sweep<float, 256, 0, 1>@256cube": 268545933,
-    "gpue::col_sweep<float, 256, 0, 2>@256cube": 268798608,
-    "gpue::row_sweep<double, 256, 1, 0>@256cube": 537095067,
-    "gpue::row_sweep<double, 256, 1, 1>@256cube": 537334821,
-    "gpue::row_sweep<double, 256, 1, 2>@256cube": 538243034,
-    "gpue::row_sweep<double, 256, 1, 65>@256cube": 537835606,
-    "gpue::row_sweep<float, 256, 0, 0>@256cube": 268648607,
-    "gpue::row_sweep<float, 256, 0, 65>@256cube": 268896874,
+    "gpue::col_sweep<double, 512, 5, 2>@512sq": 8727099,
+    "gpue::col_sweep<double, 512, 5, 3>@512sq": 8684095,
+    "gpue::col_sweep<double, 512, 5, 5>@512sq": 8690393,
+    "gpue::col_sweep<double, 512, 5, 6>@512sq": 8810034,
+    "gpue::row_sweep<double, 512, 3, 0>@512sq": 8716892,
+    "gpue::row_sweep<double, 512, 3, 1>@512sq": 8839727,
+    "gpue::row_sweep<double, 512, 3, 2>@512sq": 8714814,
+    "gpue::row_sweep<double, 512, 3, 7>@512sq": 8774198,
+    "gpue::col_sweep<double, 512, 5, 18>@512sq": 8751672,
+    "gpue::col_sweep<double, 512, 5, 19>@512sq": 8687167,
+    "gpue::col_sweep<double, 512, 5, 21>@512sq": 8612422,
+    "gpue::col_sweep<double, 512, 5, 22>@512sq": 8798772,
+    "gpue::row_sweep<double, 512, 3, 16>@512sq": 8629828,
+    "gpue::row_sweep<double, 512, 3, 17>@512sq": 8856110,
+    "gpue::row_sweep<double, 512, 3, 18>@512sq": 8689214,
+    "gpue::row_sweep<double, 512, 3, 23>@512sq": 8803891,
+    "gpue::col_sweep<double, 256, 0, 0>@256cube": 536977111,
+    "gpue::col_sweep<double, 256, 0, 1>@256cube": 536962482,
+    "gpue::col_sweep<double, 256, 0, 2>@256cube": 537282287,
+    "gpue::col_sweep<double, 256, 0, 3>@256cube": 537329324,
+    "gpue::col_sweep<double, 256, 0, 5>@256cube": 537198124,
+    "gpue::col_sweep<double, 256, 0, 6>@256cube": 537400685,
+    "gpue::col_sweep<double, 256, 2, 0>@256cube": 536965816,
+    "gpue::col_sweep<double, 256, 2, 1>@256cube": 536965324,
+    "gpue::col_sweep<double, 256, 2, 2>@256cube": 537220267,
+    "gpue::col_sweep<double, 256, 2, 3>@256cube": 537249908,
+    "gpue::col_sweep<double, 256, 2, 5>@256cube": 537143985,
+    "gpue::col_sweep<double, 256, 2, 6>@256cube": 537302583,
+    "gpue::col_sweep<double, 256, 4, 2>@256cube": 537824655,
+    "gpue::col_sweep<float, 256, 0, 0>@256cube": 268532615,
+    "gpue::col_sweep<float, 256, 0, 1>@256cube": 268533639,
+    "gpue::col_sweep<float, 256, 0, 2>@256cube": 268689491,
+    "gpue::row_sweep<double, 256, 1, 0>@256cube": 537043172,
+    "gpue::row_sweep<double, 256, 1, 1>@256cube": 537208939,
+    "gpue::row_sweep<double, 256, 1, 2>@256cube": 538161396,
+    "gpue::row_sweep<double, 256, 1, 65>@256cube": 537806011,
+    "gpue::row_sweep<double, 256, 3, 0>@256cube": 537056380,
+    "gpue::row_sweep<double, 256, 3, 1>@256cube": 537201558,
+    "gpue::row_sweep<double, 256, 3, 2>@256cube": 538119443,
+    "gpue::row_sweep<double, 256, 3, 65>@256cube": 537818889,
+    "gpue::row_sweep<float, 256, 0, 0>@256cube": 268613997,
+    "gpue::row_sweep<float, 256, 0, 65>@256cube": 268859576,
 }
 
 RM = {"row_fwd": 0, "row_inv": 1, "row_gauge": 2, "row_full": 3, "row_ksum": 4, "row_inv_fwd": 5,
