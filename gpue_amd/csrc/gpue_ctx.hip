@@ -1050,8 +1050,8 @@ gpue_status gpue_upload_wfc(gpue_ctx* c, const double* il) {
   return GPUE_OK;
 }
 
-// Waits for the work queued before the copy, not for what another context queues on a
-// shared stream after it.
+// Waits for the work queued before the copy; up to 2 MiB for all of the stream, which is the
+// same where one thread queues on it (a context's own, or a service's worker).
 gpue_status gpue_download_wfc(gpue_ctx* c, double* il) {
   if (!c || !il) return GPUE_EINVAL;
   gpue_status st = apply_pending(c);
